@@ -26,6 +26,7 @@ struct seq_batch {
     uint64_t n_reads = 0, pres_total = 0;
     uint64_t n_items = 0;  // written on the device (k_seq_items) from the segments
     uint64_t n_items_sparse = 0;  // the first items: those of sparse jobs (layout)
+    uint64_t templates = 0, templates_sparse = 0;  // of all items, and of those
     uint32_t spi = 1;      // strata per item
     bool no_alloc = false;  // refuse jobs whose mutation table lacks an index for their genome
     scratch_builder sb;
@@ -271,7 +272,11 @@ void layout(seq_batch& P) {
         S.first_item = (uint32_t)P.n_items;
         if (S.T) P.n_items += (S.J + P.spi - 1) / P.spi;
         if (P.n_items >= (uint64_t(1) << 32)) psx_throw(PSX_EINVAL, "too many work items in one batch");
-        if (job_sparse(P, S.job)) P.n_items_sparse = P.n_items;
+        P.templates += S.T;
+        if (job_sparse(P, S.job)) {
+            P.n_items_sparse = P.n_items;
+            P.templates_sparse = P.templates;
+        }
     }
     for (uint32_t k = 0; k < (uint32_t)P.jobs.size(); ++k)
         if (P.cna_off[k] != SIZE_MAX) (job_sparse(P, k) ? P.cna_sparse : P.cna_dense) = true;
@@ -303,6 +308,13 @@ void launch_count(const seq_lane& lane, const psx_launch_config& c, const seq_la
     PSX_CASE(512, 512) PSX_CASE(512, 1024) PSX_CASE(512, 2048)
 #undef PSX_CASE
     psx_throw(PSX_EINVAL, "unsupported launch configuration");
+}
+
+// Items a block takes at a time: `work` templates' worth (run_of), but at
+// least `runs` runs per block, so that the last ones end together.
+uint32_t run_items(uint64_t items, uint64_t templates, uint64_t grid, uint64_t work, uint64_t runs) {
+    if (!items || !templates) return 1;
+    return (uint32_t)std::max<uint64_t>(1, std::min(work * items / templates, items / (runs * grid)));
 }
 
 seq_launch launch_desc(const seq_batch& P, uint8_t* base, unsigned long long* queue) {
@@ -384,15 +396,19 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
     const uint64_t ns = P->n_items_sparse, nd = P->n_items - ns;
     if (ns || !nd) {
         seq_launch Ls = L;
+        const uint64_t grid = std::max<uint64_t>(1, std::min(want, ns));
         Ls.n_items = ns;
-        launch_count(lane, cfg, Ls, (uint32_t)std::max<uint64_t>(1, std::min(want, ns)), P->cna_sparse, true);
+        Ls.chunk = run_items(ns, P->templates_sparse, grid, 8192, 4);
+        launch_count(lane, cfg, Ls, (uint32_t)grid, P->cna_sparse, true);
     }
     if (nd) {
         seq_launch Ld = L;
         Ld.items = L.items + ns;
         Ld.n_items = nd;
         Ld.queue = L.queue + 1;
-        launch_count(lane, cfg, Ld, (uint32_t)std::max<uint64_t>(1, std::min(want, nd)), P->cna_dense, false);
+        const uint64_t grid = std::max<uint64_t>(1, std::min(want, nd));
+        Ld.chunk = run_items(nd, P->templates - P->templates_sparse, grid, 8192, 4);
+        launch_count(lane, cfg, Ld, (uint32_t)grid, P->cna_dense, false);
     }
     PSX_HIP(hipGetLastError());
     if (timed) PSX_HIP(hipEventRecord(lane.ev1, lane.stream));
@@ -601,12 +617,13 @@ extern "C" psx_status psx_simulate_seq(psx_ctx* ctx, const psx_genome* g, const 
 // One persistent read-materialising launch: as many blocks as fit on every CU
 // at once (capped by the work items).
 template <int BLOCK, int CAP, bool STAGE, int NW, bool CNA = false>
-void launch_reads(psx_ctx* ctx, const seq_launch& L, size_t items, size_t stage) {
+void launch_reads(psx_ctx* ctx, seq_launch& L, size_t items, uint64_t templates, size_t stage) {
     int per_cu = 0;
     PSX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_seq_reads<BLOCK, CAP, STAGE, NW, CNA>, BLOCK,
                                                          stage));
     const uint64_t want = (uint64_t)ctx->n_cu * (uint64_t)std::max(per_cu, 1);
     const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, items));
+    L.chunk = run_items(items, templates, grid, 1024, 16);
     PSX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     hipLaunchKernelGGL((k_seq_reads<BLOCK, CAP, STAGE, NW, CNA>), dim3(grid), dim3(BLOCK), stage, ctx->stream, L);
 }
@@ -762,19 +779,19 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
         const size_t items = P.n_items;
         if (with_cn) {  // one instantiation with the copy-number path (any read size)
             if (8 * wave_stage <= STAGE_MAX)
-                launch_reads<512, CAP, true, 0, true>(ctx, L, items, 8 * wave_stage);
+                launch_reads<512, CAP, true, 0, true>(ctx, L, items, P.templates, 8 * wave_stage);
             else if (4 * wave_stage <= STAGE_MAX)
-                launch_reads<256, CAP, true, 0, true>(ctx, L, items, 4 * wave_stage);
+                launch_reads<256, CAP, true, 0, true>(ctx, L, items, P.templates, 4 * wave_stage);
             else
-                launch_reads<256, CAP, false, 0, true>(ctx, L, items, 0);
+                launch_reads<256, CAP, false, 0, true>(ctx, L, items, P.templates, 0);
         } else if (L.out_vec4 && L.read_words == 12) {  // 145-160 bp reads
-            launch_reads<512, CAP, true, 10>(ctx, L, items, 8 * wave_stage);
+            launch_reads<512, CAP, true, 10>(ctx, L, items, P.templates, 8 * wave_stage);
         } else if (8 * wave_stage <= STAGE_MAX) {
-            launch_reads<512, CAP, true, 0>(ctx, L, items, 8 * wave_stage);
+            launch_reads<512, CAP, true, 0>(ctx, L, items, P.templates, 8 * wave_stage);
         } else if (4 * wave_stage <= STAGE_MAX) {
-            launch_reads<256, CAP, true, 0>(ctx, L, items, 4 * wave_stage);
+            launch_reads<256, CAP, true, 0>(ctx, L, items, P.templates, 4 * wave_stage);
         } else {
-            launch_reads<256, CAP, false, 0>(ctx, L, items, 0);
+            launch_reads<256, CAP, false, 0>(ctx, L, items, P.templates, 0);
         }
     }
     PSX_HIP(hipGetLastError());

@@ -5,7 +5,7 @@
 // W = len - L + 1 template starts are cut into strata of PSX_STRATUM starts,
 // and stratum j owns a fixed number of templates (part of the sampling model,
 // so results do not depend on the launch). A work item is a run of strata of
-// one segment; persistent blocks pull items from a device counter.
+// one segment; persistent blocks pull runs of items from a device counter.
 //
 // Per stratum a block stages in LDS the mutation records the stratum's reads
 // can reach (pos, leaf range, packed info) with a 32-base bucket index, plus
@@ -117,10 +117,27 @@ struct seq_launch {
     const item_dev* items;
     uint64_t n_items;
     unsigned long long* queue;
+    uint32_t chunk;          // items taken at a time (run_of)
     uint32_t* reads_out;     // materialisation only
     uint32_t read_words;
     uint32_t out_vec4;       // read_words % 4 == 0 and reads_out 16-byte aligned
 };
+
+// The items of a persistent launch are handed out in runs of L.chunk: block b
+// takes run b without asking, later ones from the counter. Atomics on the one
+// counter serialise at about 12 ns each whatever the items hold, which set the
+// time of every launch of many small items (147,000 strata of a 10x run: 1.79
+// ms, of which the counter 1.76); in runs of about 8,192 templates the counter
+// costs 1.5 ps per template against the kernels' 5-11.
+struct item_run {
+    uint32_t first, end;
+};
+__device__ __forceinline__ item_run run_of(const seq_launch& L, uint32_t run) {
+    const uint64_t first = (uint64_t)run * L.chunk;
+    if (first >= L.n_items) return item_run{0u, 0u};
+    const uint64_t left = L.n_items - first;
+    return item_run{(uint32_t)first, (uint32_t)(first + (left < L.chunk ? left : L.chunk))};
+}
 
 // The job's inversion tables in LDS; the insert-size guide keeps 2^GB of the
 // host table's PSX_GUIDE entries (every 2^(PSX_GUIDE_BITS - GB)-th, the same
@@ -961,21 +978,19 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
     // the deferred form keeps a 256-entry guide (its LDS also holds the error-check rings),
     // the plain form a 1024-entry one
     __shared__ lds_tables_t<DEFER ? 8u : (CNA ? PSX_GUIDE_BITS : 10u)> s_tab;
-    __shared__ uint32_t s_item, s_acc;
+    __shared__ uint32_t s_run, s_acc;
     // per wave: the (lane, record) queue of a mate (also a slow template's errors on
     // the global path), and the deferred error checks
     __shared__ uint32_t s_wave[BLOCK / 64][ELIST];
     __shared__ uint32_t s_chk[BLOCK / 64][DEFER ? 3 * 128 : 1];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
-    for (;;) {
-        if (tid == 0) {
-            s_item = (uint32_t)atomicAdd(L.queue, 1ull);
-            s_acc = 0;
-        }
-        __syncthreads();
-        const uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
-        if (item >= L.n_items) break;
+    uint32_t in_tab = UNRESOLVED;  // the job whose tables s_tab holds
+    for (uint32_t run = blockIdx.x;;) {
+      const item_run R = run_of(L, run);
+      if (R.first == R.end) break;
+      if (tid == 0) s_run = gridDim.x + (uint32_t)atomicAdd(L.queue, 1ull);  // the block's next run
+      for (uint32_t item = R.first; item < R.end; ++item) {
         const item_dev it = uniform_at(L.items, item);
         // the segment's and the job's fields are read where they are used (scalar
         // loads from the constant address space) instead of being held in SGPRs
@@ -984,7 +999,11 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
         const job_dev& J = *(const job_dev*)((const __attribute__((address_space(4))) job_dev*)L.jobs + S.job);
         const uint32_t c2 = (S.chr << 16) | S.so;
         uint32_t acc = 0;  // accepted templates (copy-number events)
-        load_tables(J, s_tab, tid, BLOCK);
+        if (CNA && tid == 0) s_acc = 0;
+        if (in_tab != S.job) {
+            in_tab = S.job;
+            load_tables(J, s_tab, tid, BLOCK);
+        }
         __syncthreads();
         for (uint32_t j = it.j0; j < it.j1; ++j) {
             const stratum s = stratum_of(J, S, j);
@@ -1085,14 +1104,19 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
                 __syncthreads();
             } else {
                 count_stratum_global<BLOCK, CNA>(J, S, s_tab, s, j, c2, s_wave[wave], lane, wave, &acc);
+                __syncthreads();  // s_tab may be reloaded next
             }
         }
         if (CNA && S.n_cna) {
             if (acc) atomicAdd(&s_acc, acc);
             __syncthreads();
             if (tid == 0 && s_acc) atomicAdd(J.acc, (unsigned long long)s_acc * (J.pe + 1u));
+            __syncthreads();
         }
-        __syncthreads();
+      }
+      __syncthreads();
+      run = __builtin_amdgcn_readfirstlane(s_run);
+      __syncthreads();  // read by every wave before it is written again
     }
 }
 
@@ -1285,15 +1309,18 @@ __device__ __forceinline__ void apply_error(uint32_t* row, uint32_t o, uint32_t 
 // in the output. NW > 0: reads of NW base words (rows of whole 16-byte
 // vectors, built in registers); NW = 0: any read size. CNA: segments with
 // copy-number events keep only the templates whose copy slot is a copy of
-// their source (their reads from J.cn_row on); the others as without.
+// their source (their reads from J.cn_row on); the others as without. The
+// 512-thread forms are held to 80 VGPRs (the copy-number one spills two), so
+// that 3 blocks run per CU instead of 2: 5e7 single-end 100 bp reads 737 ->
+// 615 us, 2.7e7 reads with copy numbers 1290 -> 1100 us.
 template <int BLOCK, int CAP, bool STAGE, int NW, bool CNA = false>
-__global__ void __launch_bounds__(BLOCK) k_seq_reads(const seq_launch L) {
+__global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const seq_launch L) {
     constexpr uint32_t WAVES = BLOCK / 64;
     __shared__ uint32_t s_pos[CAP], s_lo[CAP], s_hi[CAP], s_info[CAP];
     __shared__ uint16_t s_bucket[NB_MAX];
     __shared__ uint32_t s_ref[REF_MAX];
     __shared__ lds_tables s_tab;
-    __shared__ uint32_t s_item;
+    __shared__ uint32_t s_run;
     __shared__ uint32_t s_cnt[WAVES];
     __shared__ uint32_t s_elist[WAVES][ELIST];  // per wave: errors of a slow template
     __shared__ uint32_t s_kept[WAVES];          // CNA: kept templates per wave in a round
@@ -1305,11 +1332,12 @@ __global__ void __launch_bounds__(BLOCK) k_seq_reads(const seq_launch L) {
     const bool vec4 = L.out_vec4 != 0;  // RW % 4 == 0 and a 16-byte aligned output
     uint32_t* stage = reinterpret_cast<uint32_t*>(s_stage4) + wave * 64u * RW;
     const uint4* stage4 = reinterpret_cast<const uint4*>(stage);
-    for (;;) {
-        if (tid == 0) s_item = (uint32_t)atomicAdd(L.queue, 1ull);
-        __syncthreads();
-        const uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
-        if (item >= L.n_items) break;
+    uint32_t in_tab = UNRESOLVED;  // the job whose tables s_tab holds
+    for (uint32_t run = blockIdx.x;;) {
+      const item_run R = run_of(L, run);
+      if (R.first == R.end) break;
+      if (tid == 0) s_run = gridDim.x + (uint32_t)atomicAdd(L.queue, 1ull);  // the block's next run
+      for (uint32_t item = R.first; item < R.end; ++item) {
         const item_dev it = uniform_at(L.items, item);
         const seg_dev S = uniform_at(L.segs, it.seg);
         const job_dev J = uniform_at(L.jobs, S.job);
@@ -1317,8 +1345,11 @@ __global__ void __launch_bounds__(BLOCK) k_seq_reads(const seq_launch L) {
         const uint32_t rpt = J.pe ? 2u : 1u;
         const uint32_t tpp = 64u / rpt;  // templates per pass
         const uint32_t chr_words = (S.len + 15u) >> 4;
-        load_tables(J, s_tab, tid, BLOCK);
-        __syncthreads();
+        if (in_tab != S.job) {
+            in_tab = S.job;
+            load_tables(J, s_tab, tid, BLOCK);
+            __syncthreads();
+        }
         for (uint32_t j = it.j0; j < it.j1; ++j) {
             const stratum s = stratum_of(J, S, j);
             const bool fits = s.n_win <= (uint32_t)CAP;
@@ -1474,7 +1505,10 @@ __global__ void __launch_bounds__(BLOCK) k_seq_reads(const seq_launch L) {
             }
             __syncthreads();
         }
-        __syncthreads();
+      }
+      __syncthreads();
+      run = __builtin_amdgcn_readfirstlane(s_run);
+      __syncthreads();  // read by every wave before it is written again
     }
 }
 

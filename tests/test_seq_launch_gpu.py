@@ -1,0 +1,56 @@
+"""Launch shapes of the sequencing kernels against the oracle, bit for bit, at
+the sizes where a launch rule changes."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import cases
+from oracle import oracle as O
+from process_amd import core
+
+pytestmark = pytest.mark.gpu
+
+
+class World:
+    """A two-species forest over a synthetic reference; the table is the GPU's own (its parity is tested elsewhere)."""
+
+    def __init__(self, ctx, lens, forest_kw, snv, seed=5, **eng):
+        self.lens = np.asarray(lens, np.uint32)
+        self.g = core.Genome(ctx, self.lens, seed=seed)
+        fd = cases.forest(**forest_kw)
+        self.of = O.Forest(fd["cell_id"], fd["parent"], fd["species"], fd["sample"], fd["birth"], fd["n_samples"])
+        self.pf = core.Forest(ctx, fd["cell_id"], fd["parent"], fd["species"], fd["sample"], fd["birth"],
+                              fd["n_samples"])
+        kw = dict(snv_rate=[snv, snv], indel_rate=[snv / 10, snv / 10], sbs=cases.signatures(1, 2), epoch_start=[0.0],
+                  exposure=[[1.0]], n_pre_snv=8, n_pre_indel=4)
+        kw.update(eng)
+        self.pm = core.Mutations.place(ctx, self.g, self.pf, seed + 1, **kw)
+        self.recs = self.pm.download()
+
+    def check(self, got, seed, kw):
+        oa, od, op, on = O.simulate_seq(self.lens, self.of, self.recs, seed, **kw)
+        a, d, p = got
+        assert np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op), kw
+        return on
+
+
+def test_runs_of_many_small_items(ctx):
+    """A launch of many strata with few templates each is handed out in runs of several strata, which cross segments
+    and jobs: 200 Mb over 22 chromosomes at 0.2-0.5x, three jobs of different read sizes, inserts and error rates."""
+    lens = np.full(22, 200_000_000 // 22) + np.arange(22) * 1000
+    w = World(ctx, lens, dict(n_cells=300, n_samples=2, sample_size=50, seed=3), 3e-9)
+    spec = [dict(coverage=0.3, read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=1e-2),
+            dict(coverage=0.5, read_size=100, error_rate=2e-2, purity=0.6),
+            dict(coverage=0.2, read_size=75, insert_size_mean=200, insert_size_stddev=5)]
+    jobs = [core.SeqJob(ctx, w.g, w.pf, w.pm, 40 + k, **kw) for k, kw in enumerate(spec)]
+    n = core.simulate_seq_batch(ctx, jobs)
+    assert n == sum(w.check(j.results(), 40 + k, kw) for k, (j, kw) in enumerate(zip(jobs, spec)))
+    # materialised reads: a chromosome's rows of the whole run are the oracle's reads of that chromosome alone
+    kw = dict(spec[0], with_normal_sample=False, samples=[1])
+    rows, n = core.simulate_seq_reads(ctx, w.g, w.pf, w.pm, 7, **kw)
+    per = [core.num_reads(w.g, w.pf, **dict(kw, chromosomes=[c])) for c in range(22)]
+    assert n == sum(per)
+    first = sum(per[:21])
+    alone = O.simulate_reads(w.lens, w.g.download(), w.of, w.recs, 7, per[21], **dict(kw, chromosomes=[21]))
+    assert len(alone) == per[21] and np.array_equal(rows.numpy()[first:first + per[21]], alone)
