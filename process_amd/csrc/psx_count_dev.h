@@ -1,0 +1,518 @@
+// The dense form of count-only sequencing on gfx950. Included once, by
+// psx_seq.hip, after psx_seq_dev.h.
+//
+// A block takes a window of one to eight strata of a segment, draws their
+// templates in rounds of about 5,600 reads and drops every read, one 32-bit
+// word, into the LDS bin of its start (start inside the bin | source copy);
+// then the window's records are dealt to the threads, several threads to a
+// record, and each scans the bins that can hold reads over its record's
+// position: two compares per read, the counts in registers. A read is
+// handled once when it is drawn and once per record near it, with no walk, no
+// queue and no LDS counters.
+//
+// Bound by vector instruction issue (4.4 cycles each; 6 waves per SIMD by
+// 80 VGPRs and 52 KB of LDS per block; 4 waves: 8.8 ms): on the plain-large
+// workload (200x, one record per 200 bases) 322 instructions per 64 templates
+// against 497 of a form that walked each read's records and queued (read,
+// record) pairs: 80 of them Philox, 80 the rest of the draw and the bins, 35
+// the window's set-up, 45 the scan, 80 the errors past their draw. 9.10 ->
+// 7.11 ms per 1.6e9 reads, 4.5 ms without errors; 10x single-end reads over
+// 300 Mb in windows of 8 strata 1.05 -> 0.57 ms.
+//
+// Sources are cells of the sample, not leaves: the cells that carry a record
+// are a range of the sample's cells (cells_below of its leaf range), so a
+// template needs no look-up of its leaf. Sequencing errors are drawn per
+// template, as in the model; an error matters only where a record lies, which
+// a bitmap of the window's record positions tells, and corrects the counts
+// there (error_fix).
+#pragma once
+#include "psx_seq_dev.h"
+
+namespace psxk {
+
+constexpr uint32_t DENSE_BLOCK = 512;
+constexpr uint32_t DENSE_WAVES = DENSE_BLOCK / 64;
+constexpr uint32_t BIN_SHIFT = 7;     // bins of 128 << lns starts (fewer where the chromosome has fewer than 8,192)
+constexpr uint32_t BIN_CAP = 120;     // reads a bin holds; the few beyond it are walked one by one
+constexpr uint32_t BIN_STRIDE = BIN_CAP + 4;  // words of a bin: those beyond it land in a slot nobody reads
+constexpr uint32_t BIN_READS = 88;    // expected reads of a bin in a round
+constexpr uint32_t MAX_BINS = (PSX_STRATUM + MAX_READ) >> BIN_SHIFT;
+
+// Dynamic LDS of a launch: the bitmap of record positions, the bins, their counts (two sets).
+__host__ __device__ __forceinline__ uint32_t dense_bit_words(uint32_t bits) { return (bits + 127u) / 128u * 4u; }
+__host__ __device__ __forceinline__ uint32_t dense_lds(uint32_t bins, uint32_t bits) {
+    return 4u * (dense_bit_words(bits) + bins * (BIN_STRIDE + 2u));
+}
+
+// A record as the scan sees it: position in the window, and the carrying
+// copies [low, low + len) of the word's copy field (allele above the cell).
+// Records alone at their position are counted by the scan alone; one that
+// shares its position is counted with it by the first of them (GROUP), as is
+// one whose carriers are no single range.
+struct scan_rec {
+    uint32_t p, low, len, kind;
+};
+enum : uint32_t { REC_NONE = 0, REC_SOLO = 1, REC_GROUP = 2 };
+
+__device__ __forceinline__ scan_rec load_rec(const job_dev& J, const seg_dev& S, uint32_t wb, uint32_t k0, uint32_t i,
+                                             uint32_t cb, uint32_t lw) {
+    const uint32_t q = k0 + i;
+    const uint32_t pos = J.pos[q], info = J.info[q];
+    const uint32_t nat = PSX_INFO_NATURE(info);
+    const bool normal_has = nat == PSX_GERMINAL || (nat == PSX_PRENEOPLASTIC && J.preneo);
+    uint32_t lo = 0, hi = normal_has ? 1u : 0u;  // the normal sample: one cell
+    bool one_range = true;
+    if (S.n_cells) {
+        lo = cells_below(J, S.sample, J.lo[q]);
+        hi = cells_below(J, S.sample, J.hi[q]);
+        if (normal_has && J.thr_normal) {  // reads of the normal genome carry it too (cell n_cells)
+            one_range = hi == S.n_cells || lo == hi;
+            lo = lo == hi ? S.n_cells : lo;
+            hi = S.n_cells + 1u;
+        }
+    }
+    scan_rec R;
+    R.p = pos - wb;
+    R.low = ((PSX_INFO_ALLELE(info) << cb) | lo) << lw;
+    R.len = (hi - lo) << lw;
+    const bool plain = one_range && PSX_INFO_HEAD(info) &&
+                       (PSX_INFO_KIND(info) != PSX_SNV || PSX_INFO_REF(info) != PSX_INFO_ALT(info));
+    if (PSX_INFO_SOLO(info)) R.kind = plain ? REC_SOLO : REC_GROUP;
+    else R.kind = i > 0 && J.pos[q - 1] == pos ? REC_NONE : REC_GROUP;
+    return R;
+}
+
+// The job's insert-size table in LDS: the thresholds and, per guide bucket,
+// the first and the last answer a draw of the bucket can have (one word).
+constexpr uint32_t DENSE_GUIDE_BITS = 10;
+struct dense_tables {
+    uint32_t ins[MAX_INS];
+    uint32_t guide[1u << DENSE_GUIDE_BITS];
+};
+
+__device__ __forceinline__ void load_dense_tables(const job_dev& J, dense_tables& t, uint32_t tid) {
+    constexpr uint32_t G = 1u << DENSE_GUIDE_BITS, STEP = 1u << (PSX_GUIDE_BITS - DENSE_GUIDE_BITS);
+    if (!J.pe) return;
+    for (uint32_t i = tid; i < J.ins_n; i += DENSE_BLOCK) t.ins[i] = J.ins_T[i];
+    for (uint32_t i = tid; i < G; i += DENSE_BLOCK)
+        t.guide[i] = (uint32_t)J.ins_guide[i * STEP] |
+                     (i + 1u < G ? (uint32_t)J.ins_guide[(i + 1u) * STEP] : J.ins_n - 1u) << 16;
+}
+
+// Insert-size pick (psx_guided_pick). Nearly every bucket holds at most one
+// threshold, so one compare settles it; where a lane's bucket holds more (the
+// tails: one wave in five), a binary search inside the buckets.
+__device__ __forceinline__ uint32_t pick_insert(const dense_tables& t, uint32_t u) {
+    const uint32_t g = t.guide[u >> (32u - DENSE_GUIDE_BITS)];
+    uint32_t lo = g & 0xFFFFu, hi = g >> 16;
+    const uint32_t first = t.ins[lo];  // lo < hi <= MAX_INS - 1, or the answer
+    const bool past = lo < hi && u >= first;
+    lo += past ? 1u : 0u;
+    if (__ballot(past && lo < hi)) {
+        hi = past ? hi : lo;
+        while (__ballot(lo < hi)) {
+            const uint32_t mid = (lo + hi) >> 1;
+            const bool below = u < t.ins[mid], on = lo < hi;
+            hi = on && below ? mid : hi;
+            lo = on && !below ? mid + 1u : lo;
+        }
+    }
+    return lo;
+}
+
+// A descriptor to be read again where it is used: the fields of the rare paths
+// are then loaded there instead of being held in scalar registers through the
+// hot loop, whose own values they would push into vector lanes.
+template <class T>
+__device__ __forceinline__ const T& reread(const T& x) {
+    uint64_t a = (uint64_t)(uintptr_t)&x;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(a));
+    return *(const T*)(const __attribute__((address_space(4))) T*)a;
+#else
+    return *(const T*)(uintptr_t)a;
+#endif
+}
+
+// The records of a window in global memory.
+__device__ __forceinline__ glb_view window_view(const job_dev& J, const seg_dev& S, uint32_t k0, uint32_t n) {
+    const uint64_t o = out_off(J, S) + k0;
+    return glb_view{J.pos + k0, J.lo + k0, J.hi + k0, J.info + k0, J.alt + o, J.depth + o, n};
+}
+
+__device__ __forceinline__ uint32_t leaf_of_cell(const job_dev& J, const seg_dev& S, uint32_t cell) {
+    return cell == S.n_cells || S.n_cells == 0 ? J.n_leaves : J.sample_leaves[S.leaf_off + cell];
+}
+
+// Rare work of a round, listed in LDS and done after its draws: an error of a
+// read at a position that holds a record, or a read whose bin is full.
+struct todo {
+    uint32_t at;    // position of the error or start of the read in the window | substitution << 18 | TODO_READ
+    uint32_t copy;  // the source copy
+};
+constexpr uint32_t TODO_READ = 1u << 20, TODO_POS = (1u << 18) - 1u;
+constexpr uint32_t TODO_CAP = 512;  // entries of a round; the ones beyond are done at once
+
+// The rare paths are functions of their own, called: inlined, their loops took
+// the scalar registers of the hot loop, which then read its own values back
+// from vector lanes (about 55 vector instructions per 64 templates).
+
+__device__ __attribute__((noinline)) void dense_todo(const job_dev* Jp, const seg_dev* Sp, todo T, uint32_t wb,
+                                                     uint32_t k0, uint32_t n_win, uint32_t cb) {
+    const job_dev& J = *Jp;
+    const seg_dev& S = *Sp;
+    const glb_view gv = window_view(J, S, k0, n_win);
+    const uint32_t P = wb + (T.at & TODO_POS);
+    const uint32_t al = T.copy >> cb, leaf = leaf_of_cell(J, S, T.copy & ((1u << cb) - 1u));
+    uint32_t i = gv.first(P);
+    if (!(T.at & TODO_READ)) {
+        error_fix(J, gv, i, al, leaf, (T.at >> 18) & 3u);
+    } else {
+        while (i < n_win && gv.pos[i] < P + J.L) i = count_group(J, gv, i, al, leaf, terr{0u, 0u}, 0u);
+    }
+}
+
+// Errors of a slow template into list; returns their number (all lanes of a wave call it).
+__device__ __attribute__((noinline)) uint32_t dense_slow(const job_dev* Jp, uint32_t r, uint32_t j, uint32_t c2,
+                                                         uint32_t* list) {
+    const job_dev& J = *Jp;
+    wave_sync();
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)J.seed);
+    const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(J.seed >> 32));
+    const uint32_t n =
+        wave_template_errors((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, r, j, c2, list, threadIdx.x & 63u);
+    wave_sync();
+    return n;
+}
+
+// The reads of one bin over a record that shares its position (or has no single range of carriers).
+__device__ __attribute__((noinline)) void dense_group(const job_dev* Jp, const seg_dev* Sp, const uint32_t* bin,
+                                                      uint32_t k, uint32_t n, uint32_t step, uint32_t elo, uint32_t elen,
+                                                      uint32_t lw, uint32_t cb, uint32_t k0, uint32_t n_win, uint32_t i) {
+    const job_dev& J = *Jp;
+    const seg_dev& S = *Sp;
+    const glb_view gv = window_view(J, S, k0, n_win);
+    for (; k < n; k += step) {
+        const uint32_t w = bin[k];
+        if (w - elo > elen) continue;
+        const uint32_t X = w & (0xFFFFFFFFu >> lw);
+        count_group(J, gv, i, X >> cb, leaf_of_cell(J, S, X & ((1u << cb) - 1u)), terr{0u, 0u}, 0u);
+    }
+}
+
+template <bool CNA>
+__global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch L) {
+    extern __shared__ uint4 s_dyn[];
+    __shared__ dense_tables s_tab;
+    __shared__ uint32_t s_run, s_acc, s_neff, s_todo_n[2];
+    __shared__ uint32_t s_list[DENSE_WAVES][ELIST];  // per wave: a slow template's errors
+    __shared__ todo s_todo[TODO_CAP];
+    uint32_t* const s_bits = (uint32_t*)s_dyn;
+    uint32_t* const s_bin = s_bits + L.bit_words;
+    uint32_t* const s_cnt = s_bin + L.bins * BIN_STRIDE;  // two sets: one fills while the other is cleared
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    uint32_t* const list = s_list[wave];
+    uint32_t in_tab = UNRESOLVED;
+    for (uint32_t run = blockIdx.x;;) {
+        const item_run R0 = run_of(L, run);
+        if (R0.first == R0.end) break;
+        if (tid == 0) s_run = gridDim.x + (uint32_t)atomicAdd(L.queue, 1ull);  // the block's next run
+        for (uint32_t item = R0.first; item < R0.end; ++item) {
+            const item_dev it = uniform_at(L.items, item);
+            const seg_dev& S = *(const seg_dev*)((const __attribute__((address_space(4))) seg_dev*)L.segs + it.seg);
+            const job_dev& J = *(const job_dev*)((const __attribute__((address_space(4))) job_dev*)L.jobs + S.job);
+            const uint32_t c2 = (S.chr << 16) | S.so;
+            const uint32_t lns = seg_lns(S), cb = seg_cb(S), lw = seg_lw(S), SH = 32u - lw;
+            const uint32_t nslot = DENSE_WAVES >> lns, slot = wave & (nslot - 1u);
+            const uint32_t RL = J.L, pe = J.pe, err_n = J.err_n, err_N = J.err_N, n_cells = S.n_cells;
+            const uint32_t starts_end = S.len - RL;  // the last start
+            const int ins_past = (int)J.ins_k0 - (int)RL;  // of the smallest insert size over the read size
+            // a diploid source without copy-number events is drawn here; normal_below: draws up to it take a copy of
+            // the normal genome (purity below 1)
+            const bool diploid = J.ploidy == 2u && !(CNA && S.n_cna != 0u);
+            const bool normal_some = n_cells != 0u && J.thr_normal != 0u;
+            const uint32_t normal_below = (uint32_t)(J.thr_normal - 1u), copies = n_cells ? 2u * n_cells : 2u;
+            uint32_t errT[4];  // thresholds of 1 to 4 errors past the table's first count (capped below)
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; ++q) errT[q] = q < err_n ? uniform_at(J.err_T, q) : 0xFFFFFFFFu;
+            if (CNA && tid == 0) s_acc = 0;
+            if (in_tab != S.job) {
+                in_tab = S.job;
+                load_dense_tables(J, s_tab, tid);
+            }
+            uint32_t acc = 0;  // accepted templates (copy-number events)
+            for (uint32_t jw = it.j0; jw < it.j1; jw += 1u << lns) {
+                const uint32_t wb = jw * PSX_STRATUM;
+                const uint32_t je = min(jw + (1u << lns), it.j1);
+                const uint32_t wend = min(S.len, min(je * PSX_STRATUM, S.W) - 1u + J.reach);
+                const uint32_t k0 = uniform_at(J.bucket, S.bucket_off + jw);
+                const uint32_t n_win = window_records(J, S, k0, wend);
+                // the window's record positions and how many of its records reads can reach
+                if (err_n)
+                    for (uint32_t i = tid; i < (wend - wb + 31u) >> 5; i += DENSE_BLOCK) s_bits[i] = 0;
+                for (uint32_t i = tid; i < L.bins; i += DENSE_BLOCK) s_cnt[i] = 0;
+                if (tid == 0) s_neff = s_todo_n[0] = 0;
+                __syncthreads();
+                for (uint32_t i0 = 0; i0 < n_win; i0 += DENSE_BLOCK) {
+                    const uint32_t i = i0 + tid;
+                    const uint32_t p = i < n_win ? J.pos[k0 + i] : wend;
+                    const bool in = p < wend;
+                    if (in && err_n) atomicOr(&s_bits[(p - wb) >> 5], 1u << ((p - wb) & 31u));
+                    const uint32_t n = (uint32_t)__popcll(__ballot(in));
+                    if (lane == 0 && n) atomicAdd(&s_neff, n);
+                }
+                __syncthreads();
+                const uint32_t n_rec = __builtin_amdgcn_readfirstlane(s_neff);
+                // threads per record: the most (up to 32) with all records at once
+                uint32_t lgt = 0;
+                while (lgt < 5u && (n_rec << (lgt + 1u)) <= DENSE_BLOCK) ++lgt;
+                const uint32_t sub = tid & ((1u << lgt) - 1u), step = 1u << lgt;
+                const uint32_t per_pass = DENSE_BLOCK >> lgt;
+                const bool one_pass = n_rec <= per_pass;
+                // the wave's stratum: its templates [t0, t1)
+                const uint32_t j = jw + wave / nslot;
+                const uint32_t b = j * PSX_STRATUM, e = min(b + PSX_STRATUM, S.W);
+                uint32_t t0 = 0, t1 = 0;
+                if (j < je) {
+                    const uint64_t below = templates_below(S, lane ? e : b);  // lane 0: its first template; lane 1: its end
+                    const uint32_t lo = (uint32_t)below, t_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
+                    const uint32_t nj = (uint32_t)__builtin_amdgcn_readlane((int)lo, 1) - t_b;
+                    if (seg_parts(S) == 1u) {
+                        t1 = nj;
+                    } else {
+                        const uint32_t share = (nj + seg_parts(S) - 1u) / seg_parts(S);
+                        t0 = min(nj, it.part * share);
+                        t1 = min(nj, t0 + share);
+                    }
+                }
+                // rounds: the same number for every wave, from a bound on any stratum's share
+                const uint32_t most = S.most, round_t = S.round_t;
+                scan_rec R{0, 0, 0, REC_NONE};
+                uint32_t dep = 0, alt = 0, set = 0;
+                for (uint32_t q0 = 0; q0 < most; q0 += round_t) {
+                    uint32_t* const cnt = s_cnt + set * L.bins;
+                    // ---- draw the round's templates, drop their reads into bins
+                    uint32_t pc = 0, px = 0, pd = 0, pX = 0, pr = 0;  // copy numbers: pending accepted templates
+                    const uint32_t end = min(t0 + q0 + round_t, t1);
+                    for (uint32_t g = t0 + q0 + slot * 64u;; g += nslot * 64u) {  // wave-uniform
+                        const bool more = g < end;
+                        bool have = more, on = false;
+                        uint32_t x = 0, d = 0, X = 0, r = g;  // start in the window, mate 2's offset, copy, index
+                        if (more) {
+                            on = g + lane < end;
+                            r = on ? g + lane : g;
+                            psx_u4 w;
+                            if (diploid) {
+                                w = psx_draw_u(J.seed, r, j, c2, PSX_P_TEMPLATE << 24);
+                                x = b - wb + psx_uniform32(w.x, e - b);
+                                uint32_t v = psx_uniform32(w.z, copies), cell = v >> 1;
+                                if (normal_some) {
+                                    const bool normal = w.y <= normal_below;
+                                    v = normal ? w.z >> 31 : v;
+                                    cell = normal ? n_cells : cell;
+                                }
+                                X = ((v & 1u) << cb) | cell;
+                            } else {
+                                const tmpl t = template_source<CNA, false>(J, S, r, j, b, e, w);
+                                x = t.x - wb;
+                                X = (t.allele << cb) | t.cell;
+                                if (CNA) on = on && t.ok;
+                            }
+                            if (pe) {
+                                const int I = (int)pick_insert(s_tab, w.w) + ins_past;
+                                d = min((uint32_t)max(I, 0), starts_end - wb - x);
+                            }
+                        }
+                        if (CNA) {
+                            // copy-number draws reject templates: the accepted ones are packed into the lanes of a
+                            // pending set, counted when the next group would overflow it (and at the end)
+                            acc += on ? 1u : 0u;
+                            const unsigned long long m = __ballot(on);
+                            const uint32_t n = (uint32_t)__popcll(m);
+                            const uint32_t cx = px, cd = pd, cX = pX, cr = pr, cn = pc;
+                            have = pc + n > 64u || (!more && pc);
+                            pc = have ? 0u : pc;
+                            const uint32_t below =
+                                __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                            const int a4 = (int)((on ? pc + below : (pc + n + (lane - below)) & 63u) * 4u);
+                            const uint32_t nx = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)x);
+                            const uint32_t nd = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)d);
+                            const uint32_t nX = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)X);
+                            const uint32_t nr = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)r);
+                            const bool recv = lane >= pc && lane < pc + n;
+                            px = recv ? nx : px;
+                            pd = recv ? nd : pd;
+                            pX = recv ? nX : pX;
+                            pr = recv ? nr : pr;
+                            pc += n;
+                            on = have && lane < cn;
+                            x = on ? cx : 0u;
+                            d = on ? cd : 0u;
+                            X = cX;
+                            r = on ? cr : (uint32_t)__builtin_amdgcn_readfirstlane((int)cr);
+                        }
+                        uint32_t ev = 0;  // the lane's rare events: full bins (bits 0, 1), errors at records (2, 3, 4)
+                        uint32_t P0 = 0, P1 = 0, P2 = 0, subs = 0;
+                        unsigned long long slow = 0;
+                        if (have) {
+                            auto put = [&](uint32_t xr) {  // whether the bin is full
+                                const uint32_t bin = xr >> lw;
+                                const uint32_t k = atomicAdd(&cnt[bin], 1u);
+                                s_bin[__umul24(bin, BIN_STRIDE) + min(k, BIN_CAP)] = (xr << SH) | X;
+                                return k >= BIN_CAP;
+                            };
+                            bool f0 = false, f1 = false;
+                            if (on) {
+                                f0 = put(x);
+                                if (pe) f1 = put(x + d);
+                            }
+                            if (__ballot(f0 || f1)) ev = (f0 ? 1u : 0u) | (f1 ? 2u : 0u);
+                            if (err_n) {
+                                // the template's errors (template_errors): all but the slow templates' are settled by
+                                // their first draw
+                                const psx_u4 w = psx_draw_u(J.seed, r, j, c2, PSX_P_ERROR << 24);
+                                uint32_t K = 0;
+#pragma unroll
+                                for (uint32_t q = 0; q < 4u; ++q) K += w.y >= errT[q] ? 1u : 0u;
+                                K = on ? J.err_k0 + min(K, err_n - 1u) : 0u;
+                                // position of base bi of the template; whether a record lies there
+                                const uint32_t x2 = x + d - RL;
+                                auto at = [&](uint32_t bi) { return bi + (bi >= RL ? x2 : x); };
+                                auto hit = [&](uint32_t p) { return (s_bits[p >> 5] >> (p & 31u)) & 1u; };
+                                const uint32_t b0 = psx_mulhi32(w.x, err_N);
+                                const unsigned long long m2 = __ballot(K >= 2u);
+                                if (m2) {  // a second and third error; slow templates (any repeated index among b0, b1, b2)
+                                    const uint32_t b1 = psx_mulhi32(w.z, err_N), b2 = psx_mulhi32(w.w, err_N);
+                                    slow = m2 & (__ballot(K > 3u) | __ballot(b1 == b0) | __ballot(b2 == b0) |
+                                                 __ballot(b2 == b1));
+                                    if (slow) K = (slow >> lane) & 1ull ? 0u : K;
+                                    if (K >= 2u) {
+                                        P1 = at(b1);
+                                        ev |= hit(P1) << 3;
+                                        if (K >= 3u) {
+                                            P2 = at(b2);
+                                            ev |= hit(P2) << 4;
+                                        }
+                                    }
+                                }
+                                if (K >= 1u) {
+                                    P0 = at(b0);
+                                    ev |= hit(P0) << 2;
+                                }
+                                if (__ballot(ev > 3u))
+                                    subs = (((w.x & 0xFFFFu) * 3u) >> 16) | ((((w.z & 0xFFFFu) * 3u) >> 16) << 2) |
+                                           ((((w.w & 0xFFFFu) * 3u) >> 16) << 4);
+                            }
+                        }
+                        // the group's rare events
+                        uint32_t sl_n = 0, sl_k = 0;  // the current slow template's errors and the next one
+                        uint32_t sx = 0, sd = 0, sX = 0;
+                        while (__ballot(ev != 0u) || slow || sl_k < sl_n) {
+                            bool add = false;
+                            todo q{0, 0};
+                            if (__ballot(ev != 0u)) {
+                                add = ev != 0u;
+                                const uint32_t f = add ? (uint32_t)__ffs((int)ev) - 1u : 0u;
+                                ev &= ev - 1u;
+                                q.at = f < 2u ? (x + (f ? d : 0u)) | TODO_READ
+                                              : (f == 2u ? P0 : (f == 3u ? P1 : P2)) | ((subs >> (2u * (f - 2u))) & 3u) << 18;
+                                q.copy = X;
+                            } else if (sl_k < sl_n) {
+                                const uint32_t k = sl_k + lane;
+                                const uint32_t w = k < sl_n ? list[k] : 0u, bi = w & 0xFFFFFu;
+                                const uint32_t p = bi + (bi >= RL ? sx + sd - RL : sx);
+                                add = k < sl_n && ((s_bits[p >> 5] >> (p & 31u)) & 1u);
+                                q.at = p | (w >> 20) << 18;
+                                q.copy = sX;
+                                sl_k += 64u;
+                            } else {  // wave-uniform
+                                const int ln = __ffsll((long long)slow) - 1;
+                                slow &= slow - 1ull;
+                                sx = (uint32_t)__builtin_amdgcn_readlane((int)x, ln);
+                                sd = (uint32_t)__builtin_amdgcn_readlane((int)d, ln);
+                                sX = (uint32_t)__builtin_amdgcn_readlane((int)X, ln);
+                                const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)r, ln);
+                                sl_n = (uint32_t)__builtin_amdgcn_readfirstlane((int)dense_slow(&J, rs, j, c2, list));
+                                sl_k = 0;
+                                continue;
+                            }
+                            if (add) {
+                                const uint32_t k = atomicAdd(&s_todo_n[set], 1u);
+                                if (k < TODO_CAP) s_todo[k] = q;
+                                else dense_todo(&J, &S, q, wb, k0, n_win, cb);
+                            }
+                        }
+                        if (!more) break;
+                    }
+                    __syncthreads();
+                    // ---- scan: each record's reads among the bins around it
+                    const uint32_t n_todo = min(s_todo_n[set], TODO_CAP);
+                    if (tid < n_todo) dense_todo(&J, &S, s_todo[tid], wb, k0, n_win, cb);
+                    set ^= 1u;
+                    for (uint32_t i = tid; i < L.bins; i += DENSE_BLOCK) s_cnt[set * L.bins + i] = 0;
+                    if (tid == 0) s_todo_n[set] = 0;
+                    const job_dev& Js = reread(J);
+                    const seg_dev& Ss = reread(S);
+                    for (uint32_t r0 = 0; r0 < n_rec; r0 += per_pass) {
+                        const uint32_t i = r0 + (tid >> lgt);
+                        if (!one_pass || q0 == 0u)
+                            R = i < n_rec ? load_rec(Js, Ss, wb, k0, i, cb, lw) : scan_rec{0, 0, 0, REC_NONE};
+                        const int lb = (int)(R.p - (RL - 1u));  // reads over it start at [lb, p]
+                        const uint32_t first = R.kind == REC_NONE ? 1u : (uint32_t)max(lb, 0) >> lw;
+                        const uint32_t last = R.kind == REC_NONE ? 0u : min(R.p >> lw, L.bins - 1u);
+                        for (uint32_t bn = first; bn <= last; ++bn) {
+                            const uint32_t n = min(cnt[bn], BIN_CAP);
+                            const int at = (int)(bn << lw);
+                            const uint32_t plo = (uint32_t)max(lb - at, 0), phi = min(R.p - (uint32_t)at, (1u << lw) - 1u);
+                            const uint32_t elo = plo << SH, elen = ((phi - plo + 1u) << SH) - 1u;
+                            const uint32_t* const bin = s_bin + bn * BIN_STRIDE;
+                            if (R.kind == REC_SOLO) {
+                                auto test = [&](uint32_t w) {
+                                    const bool over = w - elo <= elen;
+                                    dep += over ? 1u : 0u;
+                                    alt += over && (w << lw) - R.low < R.len ? 1u : 0u;
+                                };
+                                for (uint32_t k = sub; k < n >> 2; k += step) {
+                                    const uint4 w = ((const uint4*)bin)[k];
+                                    test(w.x);
+                                    test(w.y);
+                                    test(w.z);
+                                    test(w.w);
+                                }
+                                for (uint32_t k = (n & ~3u) + sub; k < n; k += step) test(bin[k]);
+                            } else {
+                                dense_group(&J, &S, bin, sub, n, step, elo, elen, lw, cb, k0, n_win, i);
+                            }
+                        }
+                        if (!one_pass || q0 + round_t >= most) {
+                            for (uint32_t m = 1; m < step; m <<= 1) {
+                                dep += (uint32_t)__shfl_xor((int)dep, (int)m);
+                                alt += (uint32_t)__shfl_xor((int)alt, (int)m);
+                            }
+                            if (sub == 0u && dep) {
+                                const uint64_t o = out_off(Js, Ss) + k0 + i;
+                                atomicAdd(Js.depth + o, (int32_t)dep);
+                                if (alt) atomicAdd(Js.alt + o, (int32_t)alt);
+                            }
+                            dep = alt = 0;
+                        }
+                    }
+                    __syncthreads();
+                }
+                __syncthreads();
+            }
+            if (CNA && S.n_cna) {
+                if (acc) atomicAdd(&s_acc, acc);
+                __syncthreads();
+                if (tid == 0 && s_acc) atomicAdd(J.acc, (unsigned long long)s_acc * (J.pe + 1u));
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+        run = __builtin_amdgcn_readfirstlane(s_run);
+        __syncthreads();  // read by every wave before it is written again
+    }
+}
+
+}  // namespace psxk

@@ -13,11 +13,18 @@
 #include <mutex>
 
 #include "psx_seq_dev.h"
+#include "psx_count_dev.h"
 #include "psx_seq_host.h"
 
 using namespace psxk;
 
 namespace psxh {
+
+// Covered positions per 64 templates from which a job counts by windows.
+constexpr double DENSE_COVER = 32.0, DENSE_COVER_NO_ERRORS = 4.0;
+// Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
+// templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves.
+constexpr uint64_t FEW_ITEMS = 2048, MANY_ITEMS = 4096;
 
 struct seq_batch {
     std::vector<job_dev> jobs;
@@ -28,12 +35,15 @@ struct seq_batch {
     uint64_t n_items_sparse = 0;  // the first items: those of sparse jobs (layout)
     uint64_t templates = 0, templates_sparse = 0;  // of all items, and of those
     uint32_t spi = 1;      // strata per item
+    bool count = true;      // descriptors of the count kernels (else of the read kernel: whole strata, no parts)
+    uint32_t dense_bins = 0, dense_bits = 0;  // of the largest window of the dense count kernel
     bool no_alloc = false;  // refuse jobs whose mutation table lacks an index for their genome
     scratch_builder sb;
     std::vector<size_t> tab_off;  // per job: insert thresholds, insert guide, error thresholds
     std::vector<size_t> cna_off;  // per job: copy-number events (SIZE_MAX: none)
     std::vector<uint64_t> job_reads;  // per job: reads of the sampling model without copy-number events
-    std::vector<double> job_cover;  // per job: expected covered positions per 64 templates (0: no errors)
+    std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
+    std::vector<uint8_t> job_fits;  // per job: its source copies fit the dense count kernel's words
     bool cna_sparse = false, cna_dense = false;  // copy-number events among the sparse / the other jobs
     size_t o_jobs = 0, o_segs = 0, o_items = 0, o_pres = 0, o_acc = 0;
     uint8_t* dev = nullptr;       // device base of the last upload
@@ -113,6 +123,12 @@ uint32_t out_samples(const psx_forest* f, const psx_seq_params* p) {
 }
 
 namespace {
+
+uint32_t bits_of(uint32_t x) {  // bits that represent x (at least 1)
+    uint32_t b = 1;
+    while (b < 32 && (x >> b) != 0) ++b;
+    return b;
+}
 
 // Validates one job and appends its descriptors; the ordering of output
 // samples and chromosomes follows the oracle. Nothing is appended when the
@@ -206,7 +222,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     P.cna_off.push_back(cdev.empty() ? SIZE_MAX : P.sb.put_vec(cdev));
     P.jobs.push_back(J);
     double cover = 0.0;
-    if (p->error_rate > 0.0) {
+    {
         // expected positions covered by 64 templates: records per base x bases read, times the share of
         // templates kept under copy numbers (ploidy / kmax, length-weighted)
         double recs = 0.0, bases = 0.0, kept = 0.0;
@@ -219,6 +235,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
         if (bases > 0.0) cover = 64.0 * (pe ? 2.0 : 1.0) * L * recs / bases * kept / bases;
     }
     P.job_cover.push_back(cover);
+    P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;
     for (uint32_t so = 0; so < n_out; ++so) {
         const bool normal = so == n_req;
@@ -239,7 +256,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
                                   ((double)S.kmax / (double)ploidy);
             if (!(t_real < 9.0e18)) psx_throw(PSX_EINVAL, "too many templates on chromosome %u", c);
             S.T = (uint64_t)std::llround(t_real);
-            S.out_off = (uint64_t)so * m->n;
+            S.sample = normal ? 0u : req[so];
             S.read_base = P.n_reads;
             S.chr_woff = g->woff[c];
             S.job = job; S.so = so; S.chr = c; S.len = g->len[c];
@@ -249,33 +266,86 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
                 psx_throw(PSX_EINVAL, "too many templates on chromosome %u (%llu over %u starts)", c,
                           (unsigned long long)S.T, S.W);
             S.bucket_off = (uint32_t)ix->bucket_off[c];
-            S.n_bucket = (uint32_t)(ix->bucket_off[c + 1] - ix->bucket_off[c]);
             S.leaf_off = leaf_off; S.n_cells = n_cells;
             P.n_reads += S.T * (pe ? 2u : 1u);  // template draws: an upper bound with copy-number events
+            // bits of a cell index (the sample's number of cells included) and of an allele in a 25-bit copy field
+            const uint32_t cb = bits_of(n_cells + 1u);
+            if (cb + bits_of(ploidy - 1u) > 32u - BIN_SHIFT) P.job_fits[job] = 0;
+            S.shape = cb;
             P.segs.push_back(S);  // its work items are numbered in layout()
         }
     }
     P.job_reads.push_back(P.n_reads - reads_before);
 }
 
-// A job whose reads cover fewer than 48 positions per 64 templates (or that
-// draws no errors) counts with errors checked per covered position.
-bool job_sparse(const seq_batch& P, uint32_t job) { return P.job_cover[job] < 48.0; }
+// A job whose reads cover few positions counts with errors checked per
+// covered position (k_seq_count), the others by windows (k_count_dense).
+bool job_sparse(const seq_batch& P, uint32_t job) {
+    return !P.job_fits[job] || P.job_cover[job] < (P.jobs[job].err_n ? DENSE_COVER : DENSE_COVER_NO_ERRORS);
+}
+
+// Strata, bins and items of a segment in the count kernels (parts: layout). A
+// dense window takes 2, 4 or 8 strata while their reads fit one round, in 64
+// bins of starts and as many more as mates reach past the window; on a
+// chromosome of less than a stratum the bins are narrower, at least 2 starts.
+void shape_segment(const seq_batch& P, seg_dev& S) {
+    const job_dev& J = P.jobs[S.job];
+    const uint32_t cb = seg_cb(S), copy_bits = cb + bits_of(J.ploidy - 1u), past = J.reach - J.L;
+    uint32_t lns = 0, lw = BIN_SHIFT;
+    S.spi = P.spi;
+    if (P.count && !job_sparse(P, S.job)) {
+        const double reads = (double)S.T * (J.pe + 1u) * PSX_STRATUM / (double)S.W;  // of a stratum
+        while (lns < (J.err_n ? 2u : 3u) && reads * (double)(2u << lns) <= 64.0 * BIN_READS * 0.9 &&
+               (1u << lns) < S.J && copy_bits + BIN_SHIFT + lns + 1u <= 32u)
+            ++lns;
+        lw += lns;
+        while (lw > 1 && (S.W >> lw) < 32u && ((S.W + past) >> (lw - 1u)) < MAX_BINS) --lw;
+        S.spi = std::max(P.spi, 1u << lns);
+    }
+    S.shape = cb | lns << 8 | lw << 12 | 1u << 16;
+}
 
 // Numbers the work items (the sparse jobs' segments first, so that each kind
 // of job is one range of items for its own kernel) and places the descriptors
 // of a prepared batch after the per-job tables.
 void layout(seq_batch& P) {
     std::stable_partition(P.segs.begin(), P.segs.end(), [&](const seg_dev& S) { return job_sparse(P, S.job); });
+    uint64_t items[2] = {0, 0};  // sparse, dense
+    for (seg_dev& S : P.segs) {
+        shape_segment(P, S);
+        if (S.T) items[job_sparse(P, S.job) ? 0 : 1] += (S.J + S.spi - 1) / S.spi;
+    }
     P.n_items = 0;
     for (seg_dev& S : P.segs) {
+        const bool sparse = job_sparse(P, S.job);
+        const uint64_t own = (S.J + S.spi - 1) / S.spi, all = items[sparse ? 0 : 1];
+        if (P.count && S.T && all < FEW_ITEMS) {
+            const uint64_t per_item = S.T / own, least = sparse ? 1024 : 32 * BIN_READS;
+            const uint64_t parts = std::min<uint64_t>((MANY_ITEMS + all - 1) / all, per_item / least);
+            S.shape = (S.shape & 0xFFFFu) | (uint32_t)std::max<uint64_t>(parts, 1) << 16;
+        }
         S.first_item = (uint32_t)P.n_items;
-        if (S.T) P.n_items += (S.J + P.spi - 1) / P.spi;
+        if (S.T) P.n_items += own * seg_parts(S);
         if (P.n_items >= (uint64_t(1) << 32)) psx_throw(PSX_EINVAL, "too many work items in one batch");
         P.templates += S.T;
-        if (job_sparse(P, S.job)) {
+        if (sparse) {
             P.n_items_sparse = P.n_items;
             P.templates_sparse = P.templates;
+        } else {
+            const job_dev& J = P.jobs[S.job];
+            const uint64_t starts = std::min<uint64_t>(S.W, (uint64_t)PSX_STRATUM << seg_lns(S));  // of a window
+            if (P.count) {
+                // a stratum's share, rounded up, in rounds of whole groups of 64 templates
+                const uint64_t stratum =
+                    (uint64_t)((double)S.T * std::min<double>(PSX_STRATUM, S.W) / (double)S.W) + 2;
+                const uint64_t most = stratum / seg_parts(S) + 1;
+                const uint64_t round_reads = BIN_READS * std::max<uint64_t>(1, starts >> seg_lw(S));
+                const uint64_t rounds = ((most * (J.pe + 1u) << seg_lns(S)) + round_reads - 1) / round_reads;
+                S.most = (uint32_t)std::min<uint64_t>(most, 0xFFFF0000u);
+                S.round_t = (uint32_t)(((most + rounds - 1) / rounds + 63) / 64 * 64);
+            }
+            P.dense_bins = std::max(P.dense_bins, (uint32_t)((starts - 1 + J.reach - J.L) >> seg_lw(S)) + 1u);
+            if (J.err_n) P.dense_bits = std::max(P.dense_bits, (PSX_STRATUM << seg_lns(S)) + J.reach);
         }
     }
     for (uint32_t k = 0; k < (uint32_t)P.jobs.size(); ++k)
@@ -289,21 +359,14 @@ void layout(seq_batch& P) {
 }
 
 template <int BLOCK, int CAP>
-void launch_count_t(const seq_lane& lane, const seq_launch& L, uint32_t grid, bool cna, bool defer) {
-    if (cna && defer)
-        hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, true, true>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
-    else if (cna)
-        hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, true, false>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
-    else if (defer)
-        hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, false, true>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
-    else
-        hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, false, false>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
+void launch_count_t(const seq_lane& lane, const seq_launch& L, uint32_t grid, bool cna) {
+    if (cna) hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, true>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
+    else hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, false>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
 }
 
-void launch_count(const seq_lane& lane, const psx_launch_config& c, const seq_launch& L, uint32_t grid, bool cna,
-                  bool defer) {
+void launch_count(const seq_lane& lane, const psx_launch_config& c, const seq_launch& L, uint32_t grid, bool cna) {
 #define PSX_CASE(B, C) \
-    if (c.block_threads == B && c.lds_records == C) return launch_count_t<B, C>(lane, L, grid, cna, defer);
+    if (c.block_threads == B && c.lds_records == C) return launch_count_t<B, C>(lane, L, grid, cna);
     PSX_CASE(256, 512) PSX_CASE(256, 1024) PSX_CASE(256, 2048)
     PSX_CASE(512, 512) PSX_CASE(512, 1024) PSX_CASE(512, 2048)
 #undef PSX_CASE
@@ -329,8 +392,9 @@ seq_launch launch_desc(const seq_batch& P, uint8_t* base, unsigned long long* qu
 
 }  // namespace
 
-seq_batch* batch_prepare(psx_ctx* ctx, const job_in* jobs, size_t n_jobs, uint32_t spi, bool no_alloc) {
+seq_batch* batch_prepare(psx_ctx* ctx, const job_in* jobs, size_t n_jobs, uint32_t spi, bool no_alloc, bool count) {
     auto P = std::make_unique<seq_batch>();
+    P->count = count;
     P->spi = spi;
     P->no_alloc = no_alloc;
     for (size_t k = 0; k < n_jobs; ++k) prepare_job(ctx, *P, jobs[k], spi);
@@ -376,7 +440,7 @@ void batch_upload(seq_batch* P, const seq_lane& lane) {
     if (P->n_items) {
         const uint32_t grid = (uint32_t)((P->n_items + 255) / 256);
         hipLaunchKernelGGL(k_seq_items, dim3(grid), dim3(256), 0, lane.stream, (const seg_dev*)(base + P->o_segs),
-                           (uint32_t)P->segs.size(), (item_dev*)(base + P->o_items), (uint32_t)P->n_items, P->spi);
+                           (uint32_t)P->segs.size(), (item_dev*)(base + P->o_items), (uint32_t)P->n_items);
         PSX_HIP(hipGetLastError());
     }
     P->dev = base;
@@ -399,7 +463,7 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
         const uint64_t grid = std::max<uint64_t>(1, std::min(want, ns));
         Ls.n_items = ns;
         Ls.chunk = run_items(ns, P->templates_sparse, grid, 8192, 4);
-        launch_count(lane, cfg, Ls, (uint32_t)grid, P->cna_sparse, true);
+        launch_count(lane, cfg, Ls, (uint32_t)grid, P->cna_sparse);
     }
     if (nd) {
         seq_launch Ld = L;
@@ -408,7 +472,13 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
         Ld.queue = L.queue + 1;
         const uint64_t grid = std::max<uint64_t>(1, std::min(want, nd));
         Ld.chunk = run_items(nd, P->templates - P->templates_sparse, grid, 8192, 4);
-        launch_count(lane, cfg, Ld, (uint32_t)grid, P->cna_dense, false);
+        Ld.bins = P->dense_bins;
+        Ld.bit_words = dense_bit_words(P->dense_bits);
+        const uint32_t lds = dense_lds(P->dense_bins, P->dense_bits);
+        if (P->cna_dense)
+            hipLaunchKernelGGL(k_count_dense<true>, dim3((uint32_t)grid), dim3(DENSE_BLOCK), lds, lane.stream, Ld);
+        else
+            hipLaunchKernelGGL(k_count_dense<false>, dim3((uint32_t)grid), dim3(DENSE_BLOCK), lds, lane.stream, Ld);
     }
     PSX_HIP(hipGetLastError());
     if (timed) PSX_HIP(hipEventRecord(lane.ev1, lane.stream));
@@ -733,7 +803,7 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
             psx_throw(PSX_EINVAL, "jobs of one read buffer need one read size (job %zu: %u words per read, job 0: %u)",
                       k, psx_read_words(in[k].p), rw);
     }
-    std::unique_ptr<seq_batch, void (*)(seq_batch*)> B(batch_prepare(ctx, in.data(), in.size(), 1), batch_free);
+    std::unique_ptr<seq_batch, void (*)(seq_batch*)> B(batch_prepare(ctx, in.data(), in.size(), 1, false, false), batch_free);
     seq_batch& P = *B;
     cn_rows cn;
     const bool with_cn = cn.prepare(P);
@@ -809,7 +879,7 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
 // (0 for chromosomes left out or shorter than a read): the closed form, or
 // with copy-number events the device count of kept templates.
 std::vector<uint64_t> psxh::segment_reads(psx_ctx* ctx, const job_in& in) {
-    std::unique_ptr<seq_batch, void (*)(seq_batch*)> B(batch_prepare(ctx, &in, 1, 1), batch_free);
+    std::unique_ptr<seq_batch, void (*)(seq_batch*)> B(batch_prepare(ctx, &in, 1, 1, false, false), batch_free);
     seq_batch& P = *B;
     cn_rows cn;
     if (cn.prepare(P)) {

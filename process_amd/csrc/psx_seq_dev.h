@@ -71,28 +71,43 @@ struct job_dev {
 
 struct seg_dev {
     uint64_t T;             // templates of the segment
-    uint64_t out_off;       // so * n_mut
-    uint64_t read_base;     // first read index of the segment (materialisation)
+    uint32_t sample;        // the forest sample (tumour samples)
+    uint32_t shape;         // count kernels: seg_cb | seg_lns << 8 | seg_lw << 12 | seg_parts << 16
+    union {
+        uint64_t read_base;  // materialisation: first read index of the segment
+        struct {             // dense count kernel: most templates of an item's part of a stratum, and of a round of it
+            uint32_t most, round_t;
+        };
+    };
     uint64_t chr_woff;      // first packed word of the chromosome
     uint32_t job, so, chr, len;
-    uint32_t W, J, bucket_off, n_bucket;
+    uint32_t W, J, bucket_off;
+    uint32_t spi;                // strata per work item
     uint32_t leaf_off, n_cells;  // n_cells == 0: normal sample
     uint32_t cna_off, n_cna;     // the chromosome's copy-number events (J.cna + cna_off)
     uint32_t kmax;               // copies drawn per template: the largest copy number, >= ploidy
-    uint32_t first_item;         // its work items: first_item .. first_item + ceil(J / strata per item) - 1
+    uint32_t first_item;         // its work items: first_item .. first_item + ceil(J / spi) seg_parts - 1
     uint32_t st_off;             // segments with copy-number events: index of its first stratum in J.cn_row
 };
 
+// Bits of a cell index of the segment's sample (its number of cells included); log2 of the strata of a window of the
+// dense count kernel and of the starts of its bins; the parts each item's templates are cut into (items of few strata
+// with many templates).
+__host__ __device__ __forceinline__ uint32_t seg_cb(const seg_dev& S) { return S.shape & 0xFFu; }
+__host__ __device__ __forceinline__ uint32_t seg_lns(const seg_dev& S) { return (S.shape >> 8) & 0xFu; }
+__host__ __device__ __forceinline__ uint32_t seg_lw(const seg_dev& S) { return (S.shape >> 12) & 0xFu; }
+__host__ __device__ __forceinline__ uint32_t seg_parts(const seg_dev& S) { return S.shape >> 16; }
+
 struct item_dev {
-    uint32_t seg, j0, j1, pad;
+    uint32_t seg, j0, j1, part;
 };
 
 // The work items of a batch, written on the device from the segments (the
 // host lists segments only): item q belongs to the last segment whose first
 // item is at or below q (a segment without templates has no items and shares
-// its successor's first item) and covers spi strata from its first.
+// its successor's first item) and covers its part of spi strata from its first.
 __global__ void __launch_bounds__(256) k_seq_items(const seg_dev* __restrict__ segs, uint32_t n_segs,
-                                                   item_dev* __restrict__ items, uint32_t n_items, uint32_t spi) {
+                                                   item_dev* __restrict__ items, uint32_t n_items) {
     const uint32_t q = blockIdx.x * 256u + threadIdx.x;
     if (q >= n_items) return;
     uint32_t a = 0, z = n_segs;
@@ -101,8 +116,9 @@ __global__ void __launch_bounds__(256) k_seq_items(const seg_dev* __restrict__ s
         if (segs[mid].first_item <= q) a = mid + 1; else z = mid;
     }
     const seg_dev& S = segs[a - 1];
-    const uint32_t j0 = (q - S.first_item) * spi;
-    items[q] = item_dev{a - 1, j0, min(S.J, j0 + spi), 0u};
+    const uint32_t run = (q - S.first_item) / seg_parts(S), part = (q - S.first_item) - run * seg_parts(S);
+    const uint32_t j0 = run * S.spi;
+    items[q] = item_dev{a - 1, j0, min(S.J, j0 + S.spi), part};
 }
 
 struct pres_dev {  // one per (job, output sample) for the init kernel
@@ -118,6 +134,8 @@ struct seq_launch {
     uint64_t n_items;
     unsigned long long* queue;
     uint32_t chunk;          // items taken at a time (run_of)
+    uint32_t bins;           // dense count kernel: bins of a window, words of its position bitmap
+    uint32_t bit_words;
     uint32_t* reads_out;     // materialisation only
     uint32_t read_words;
     uint32_t out_vec4;       // read_words % 4 == 0 and reads_out 16-byte aligned
@@ -279,6 +297,13 @@ __device__ __forceinline__ uint32_t leaf_of(const job_dev& J, const seg_dev& S, 
     return t.leaf;
 }
 
+// Cells of the sample with leaf ranks below x, from the sample's running counts.
+__device__ __forceinline__ uint32_t cells_below(const job_dev& J, uint32_t sample, uint32_t x) {
+    const uint4 e = J.leaf_count[(uint64_t)sample * J.leaf_blocks + (x >> 6)];
+    const uint64_t bits = (uint64_t)e.y | ((uint64_t)e.z << 32);
+    return e.x + (uint32_t)__popcll(bits & ((1ull << (x & 63u)) - 1ull));
+}
+
 __device__ __forceinline__ bool carried(const job_dev& J, uint32_t info, uint32_t lo, uint32_t hi, uint32_t leaf) {
     if (leaf == J.n_leaves) {
         const uint32_t nat = PSX_INFO_NATURE(info);
@@ -307,9 +332,10 @@ __device__ __forceinline__ uint32_t guided_pick_u(const uint32_t* T32, const uin
 }
 
 // Template r of stratum j without its mate (oracle: template_source): start,
-// source and, with copy-number events, whether the template is kept. w gets
-// the template draw (its word w is the insert size).
-template <bool CNA = false>
+// source and, with copy-number events, whether the template is kept; without
+// LEAF and events the source's leaf is left out. w gets the template draw
+// (its word w is the insert size).
+template <bool CNA = false, bool LEAF = true>
 __device__ __forceinline__ tmpl template_source(const job_dev& J, const seg_dev& S, uint32_t r, uint32_t j,
                                                 uint32_t b, uint32_t e, psx_u4& w) {
     const uint32_t c2 = (S.chr << 16) | S.so;
@@ -318,16 +344,16 @@ __device__ __forceinline__ tmpl template_source(const job_dev& J, const seg_dev&
     t.x = b + psx_uniform32(w.x, e - b);
     t.ok = 1u;
     if (!CNA || S.n_cna == 0) {
-        if (S.n_cells == 0 || (uint64_t)w.y < J.thr_normal) {
+        // a copy of a cell, or of the normal genome (cell n_cells)
+        const bool normal = S.n_cells == 0 || (uint64_t)w.y < J.thr_normal;
+        const uint32_t X = psx_uniform32(w.z, normal ? J.ploidy : S.n_cells * J.ploidy);
+        if (J.ploidy == 2) { t.cell = X >> 1; t.allele = X & 1u; }
+        else { t.cell = X / J.ploidy; t.allele = X - t.cell * J.ploidy; }
+        if (LEAF) {
             t.leaf = J.n_leaves;
-            t.cell = 0;
-            t.allele = psx_uniform32(w.z, J.ploidy);
-        } else {
-            const uint32_t X = psx_uniform32(w.z, S.n_cells * J.ploidy);
-            if (J.ploidy == 2) { t.cell = X >> 1; t.allele = X & 1u; }
-            else { t.cell = X / J.ploidy; t.allele = X - t.cell * J.ploidy; }
-            t.leaf = J.sample_leaves[S.leaf_off + t.cell];  // issued early: its latency overlaps the draws
+            if (!normal) t.leaf = J.sample_leaves[S.leaf_off + t.cell];  // issued early: its latency overlaps the draws
         }
+        t.cell = normal ? S.n_cells : t.cell;
     } else {
         // one of kmax copy slots per cell; the template is kept when the slot
         // is one of the source's copies at x, whose lineage it then reads
@@ -335,7 +361,7 @@ __device__ __forceinline__ tmpl template_source(const job_dev& J, const seg_dev&
         if (S.n_cells == 0 || (uint64_t)w.y < J.thr_normal) {
             const uint32_t k = psx_uniform32(w.z, K);
             t.leaf = J.n_leaves;
-            t.cell = 0;
+            t.cell = S.n_cells;
             t.allele = k;
             t.ok = k < J.ploidy;
         } else {
@@ -720,17 +746,14 @@ __device__ __forceinline__ void check_errors(const job_dev& J, const lds_view& v
 // (lane, mate, first record of the position) in the wave's LDS queue; the
 // queue is drained 64 entries at a time, one per lane, so the per-position
 // work runs on full waves instead of waiting for the lane whose reads cover
-// the most positions. Sequencing errors: with DEFER the reads are counted
-// with their true bases and each drained position whose observed base
-// matters goes to the deferred checks (with the lane's template index rr); otherwise the
-// template summaries e give the observed bases (slow templates are corrected
-// afterwards). Lanes with valid == false take no part (their starts must
-// still lie in the stratum).
-template <bool DEFER, class TAB>
+// the most positions. Sequencing errors: the reads are counted with their
+// true bases and each drained position whose observed base matters goes to
+// the deferred checks (with the lane's template index rr). Lanes with valid ==
+// false take no part (their starts must still lie in the stratum).
+template <class TAB>
 __device__ __forceinline__ void count_mates_wave(const job_dev& J, const seg_dev& S, const lds_view& v,
-                                                 const TAB& tab, tmpl& t, const terr& e, bool valid,
-                                                 uint32_t rr, uint32_t j, uint32_t c2, uint32_t* q, chk_ring& ck,
-                                                 uint32_t lane) {
+                                                 const TAB& tab, tmpl& t, bool valid, uint32_t rr, uint32_t j,
+                                                 uint32_t c2, uint32_t* q, chk_ring& ck, uint32_t lane) {
     uint32_t leaf = 0;  // the lane's source leaf, resolved once a read of it covers a record
     // allele | (x2 - x) << 8, for the drains (x2 - x < 2^13)
     const uint32_t ad = t.allele | ((t.x2 - t.x) << 8);
@@ -745,36 +768,31 @@ __device__ __forceinline__ void count_mates_wave(const job_dev& J, const seg_dev
         const uint32_t xo = (uint32_t)__shfl((int)t.x, (int)ol) + (mate ? ado >> 8 : 0u);  // the read's start
         const uint32_t in = v.info[ri], p = v.pos[ri];
         const bool grp = !PSX_INFO_SOLO(in);
-        terr eo{0u, 0u};
         const uint32_t boff = mate * J.L - xo;  // base index in the template of position p: p + boff
-        if (!DEFER) eo = shfl_terr(e, ol);
         if (__ballot(on && grp)) {
-            if (on && grp) count_group(J, v, ri, al, lo, eo, boff);
+            if (on && grp) count_group(J, v, ri, al, lo, terr{0u, 0u}, boff);
         }
         const bool one = on && !grp;
         const bool car = PSX_INFO_ALLELE(in) == al && carried(J, in, v.lo[ri], v.hi[ri], lo);
         const bool snv = PSX_INFO_KIND(in) == PSX_SNV;
         const uint32_t tb = snv && car ? PSX_INFO_ALT(in) : PSX_INFO_REF(in);
-        const uint32_t ob = DEFER ? tb : observe(eo, p + boff, tb);
         if (one) {
             v.add_dep(ri);
-            if (PSX_INFO_HEAD(in) && (snv ? ob == PSX_INFO_ALT(in) : car)) v.add_alt(ri);
+            if (PSX_INFO_HEAD(in) && (snv ? tb == PSX_INFO_ALT(in) : car)) v.add_alt(ri);
         }
-        if (DEFER) {
-            const bool chk = J.err_n && on && (grp || (snv && PSX_INFO_HEAD(in)));  // no errors: nothing to check
-            const unsigned long long m = __ballot(chk);
-            if (m) {
-                const uint32_t rank =
-                    __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                const uint32_t ro = (uint32_t)__shfl((int)rr, (int)ol);  // the entry's template
-                if (chk) {
-                    uint32_t* slot = ck.e + ((ck.head + ck.count + rank) & 127u) * 3u;
-                    slot[0] = ro;
-                    slot[1] = (p + boff) | (al << 13) | (ri << 21);
-                    slot[2] = lo;
-                }
-                ck.count += (uint32_t)__popcll(m);
+        const bool chk = J.err_n && on && (grp || (snv && PSX_INFO_HEAD(in)));  // no errors: nothing to check
+        const unsigned long long m = __ballot(chk);
+        if (m) {
+            const uint32_t rank =
+                __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            const uint32_t ro = (uint32_t)__shfl((int)rr, (int)ol);  // the entry's template
+            if (chk) {
+                uint32_t* slot = ck.e + ((ck.head + ck.count + rank) & 127u) * 3u;
+                slot[0] = ro;
+                slot[1] = (p + boff) | (al << 13) | (ri << 21);
+                slot[2] = lo;
             }
+            ck.count += (uint32_t)__popcll(m);
         }
     };
     uint32_t qn = 0;  // wave-uniform
@@ -822,14 +840,14 @@ __device__ __forceinline__ void count_mates_wave(const job_dev& J, const seg_dev
             drain(q + qn - 64u, 64u);
             qn -= 64u;
             wave_sync();
-            if (DEFER && ck.count >= 64u) check_errors(J, v, tab, j, c2, ck, 64u, lane);
+            if (ck.count >= 64u) check_errors(J, v, tab, j, c2, ck, 64u, lane);
         }
     }
     if (qn) {
         wave_sync();
         drain(q, qn);
         wave_sync();
-        if (DEFER && ck.count >= 64u) check_errors(J, v, tab, j, c2, ck, 64u, lane);
+        if (ck.count >= 64u) check_errors(J, v, tab, j, c2, ck, 64u, lane);
     }
 }
 
@@ -839,18 +857,45 @@ struct stratum {
     uint64_t nj, before;
 };
 
+// Templates that start below x: floor(T x / W) (T W < 2^64, x <= W) by a
+// double quotient and its exact remainder; a 64-bit integer division is over
+// a hundred instructions.
+__device__ __forceinline__ uint64_t templates_below(const seg_dev& S, uint32_t x) {
+    const uint64_t n = S.T * x, W = S.W;
+    uint64_t q = (uint64_t)((double)n / (double)W);
+    int64_t r = (int64_t)(n - q * W);
+    while (r < 0) {
+        --q;
+        r += (int64_t)W;
+    }
+    while (r >= (int64_t)W) {
+        ++q;
+        r -= (int64_t)W;
+    }
+    return q;
+}
+
+// Records of the stratum index from stratum j's first to the last that a read
+// below wend can reach (up to the end of wend's stratum).
+__device__ __forceinline__ uint32_t window_records(const job_dev& J, const seg_dev& S, uint32_t k0, uint32_t wend) {
+    const uint32_t last = (S.len + PSX_STRATUM - 1) / PSX_STRATUM;
+    return uniform_at(J.bucket, S.bucket_off + min((wend + PSX_STRATUM - 1) / PSX_STRATUM, last)) - k0;
+}
+
 __device__ __forceinline__ stratum stratum_of(const job_dev& J, const seg_dev& S, uint32_t j) {
     stratum s;
     s.b = j * PSX_STRATUM;
     s.e = min(s.b + PSX_STRATUM, S.W);
-    s.before = S.T * s.b / S.W;
-    s.nj = S.T * s.e / S.W - s.before;
+    s.before = templates_below(S, s.b);
+    s.nj = templates_below(S, s.e) - s.before;
     s.wend = min(S.len, s.e - 1 + J.reach);
     s.k0 = uniform_at(J.bucket, S.bucket_off + j);
-    const uint32_t kb = min((s.wend + PSX_STRATUM - 1) / PSX_STRATUM, S.n_bucket - 1);
-    s.n_win = uniform_at(J.bucket, S.bucket_off + kb) - s.k0;
+    s.n_win = window_records(J, S, s.k0, s.wend);
     return s;
 }
+
+// The segment's first entry of the count arrays.
+__device__ __forceinline__ uint64_t out_off(const job_dev& J, const seg_dev& S) { return (uint64_t)S.so * J.n_mut; }
 
 template <int BLOCK, int CAP>
 __device__ __forceinline__ void stage_window(const job_dev& J, const stratum& s, uint32_t* s_pos, uint32_t* s_lo,
@@ -942,12 +987,11 @@ __device__ __forceinline__ uint32_t stage_snvs(const job_dev& J, const seg_dev& 
 // code is shared by both mates).
 template <int BLOCK, bool CNA, class TAB>
 __device__ __forceinline__ void count_stratum_global(const job_dev& J, const seg_dev& S, const TAB& tab,
-                                                  const stratum& s, uint32_t j, uint32_t c2, uint32_t* list,
-                                                  uint32_t lane, uint32_t wave, uint32_t* acc) {
-    const glb_view v{J.pos + s.k0, J.lo + s.k0, J.hi + s.k0, J.info + s.k0, J.alt + S.out_off + s.k0,
-                     J.depth + S.out_off + s.k0, s.n_win};
-    const uint32_t nj = (uint32_t)s.nj;
-    for (uint32_t base = wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
+                                                  const stratum& s, uint32_t t0, uint32_t nj, uint32_t j, uint32_t c2,
+                                                  uint32_t* list, uint32_t lane, uint32_t wave, uint32_t* acc) {
+    const glb_view v{J.pos + s.k0, J.lo + s.k0, J.hi + s.k0, J.info + s.k0, J.alt + out_off(J, S) + s.k0,
+                     J.depth + out_off(J, S) + s.k0, s.n_win};
+    for (uint32_t base = t0 + wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
         const uint32_t r = base + lane;
         bool valid = r < nj;
         tmpl t = make_template<CNA>(J, S, tab, valid ? r : base, j, s.b, s.e);
@@ -963,26 +1007,23 @@ __device__ __forceinline__ void count_stratum_global(const job_dev& J, const seg
     }
 }
 
-// CNA: some job has copy-number events (templates may be rejected and are
-// counted); the plain instantiation carries none of that code. DEFER: the
-// jobs' reads cover few positions per wave (sparse tables, rejected
-// templates), so errors are drawn per covered position (deferred checks, one
-// draw per 64 positions) instead of per template; both give the same counts.
-// The deferred form is held to 6 waves per SIMD (80 VGPRs; a few spill), the
-// plain form to 7 (72 VGPRs, with a 1024-entry guide so that 7 blocks of 256
-// threads fit in LDS).
-template <int BLOCK, int CAP, bool CNA, bool DEFER>
-__global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(const seq_launch L) {
+// Jobs whose reads cover few positions: errors are checked per covered
+// position (deferred checks, one draw per 64 positions). The others' reads are
+// counted by windows (k_count_dense); both give the same counts. On a 1.6e9-read
+// run the two take the same time where 64 templates cover about 30 positions
+// (19: 5.9 against 6.2 ms; 48: 6.8 by windows). CNA: some job has copy-number
+// events (templates may be rejected and are counted); the plain instantiation
+// carries none of that code. Held to 6 waves per SIMD (80 VGPRs; a few spill).
+template <int BLOCK, int CAP, bool CNA>
+__global__ void __launch_bounds__(BLOCK, 6) k_seq_count(const seq_launch L) {
     __shared__ uint32_t s_pos[CAP], s_lo[CAP], s_hi[CAP], s_info[CAP], s_alt[CAP], s_dep[CAP];
     __shared__ uint16_t s_bucket[NB_MAX];
-    // the deferred form keeps a 256-entry guide (its LDS also holds the error-check rings),
-    // the plain form a 1024-entry one
-    __shared__ lds_tables_t<DEFER ? 8u : (CNA ? PSX_GUIDE_BITS : 10u)> s_tab;
+    __shared__ lds_tables_t<8u> s_tab;  // a 256-entry guide: the LDS also holds the error-check rings
     __shared__ uint32_t s_run, s_acc;
     // per wave: the (lane, record) queue of a mate (also a slow template's errors on
     // the global path), and the deferred error checks
     __shared__ uint32_t s_wave[BLOCK / 64][ELIST];
-    __shared__ uint32_t s_chk[BLOCK / 64][DEFER ? 3 * 128 : 1];
+    __shared__ uint32_t s_chk[BLOCK / 64][3 * 128];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     uint32_t in_tab = UNRESOLVED;  // the job whose tables s_tab holds
@@ -1007,39 +1048,19 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
         __syncthreads();
         for (uint32_t j = it.j0; j < it.j1; ++j) {
             const stratum s = stratum_of(J, S, j);
+            // the item's part of the stratum's templates
+            const uint32_t share = ((uint32_t)s.nj + seg_parts(S) - 1u) / seg_parts(S);
+            const uint32_t t0 = min((uint32_t)s.nj, it.part * share), nj = min((uint32_t)s.nj, t0 + share);
             if (s.n_win <= (uint32_t)CAP) {
                 stage_window<BLOCK, CAP>(J, s, s_pos, s_lo, s_hi, s_info, s_alt, s_dep, s_bucket, tid);
                 const lds_view v{s_pos, s_lo, s_hi, s_info, s_alt, s_dep, s_bucket, s.n_win, s.b};
-                const uint32_t nj = (uint32_t)s.nj;
                 chk_ring ck{s_chk[wave], 0u, 0u};
-                // the counting of a wave's templates t (lanes with valid; template indices rr)
-                auto count_wave = [&](tmpl& t, uint32_t rr, bool valid) {
-                    if (DEFER) {
-                        count_mates_wave<true>(J, S, v, s_tab, t, terr{0u, 0u}, valid, rr, j, c2, s_wave[wave], ck,
-                                               lane);
-                    } else {
-                        const terr e = J.err_n ? template_errors(J, s_tab, rr, j, c2, valid) : terr{0u, 0u};
-                        count_mates_wave<false>(J, S, v, s_tab, t, e, valid, rr, j, c2, s_wave[wave], ck, lane);
-                        if (J.err_n) count_slow_errors(J, v, s_tab, t, e, valid, rr, j, c2, s_wave[wave], lane);
-                    }
-                };
-                if (!CNA && DEFER) {
-                    for (uint32_t base = wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
+                if (!CNA) {
+                    for (uint32_t base = t0 + wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
                         const uint32_t r = base + lane;
                         const bool valid = r < nj;
                         tmpl t = make_template<CNA>(J, S, s_tab, valid ? r : base, j, s.b, s.e);
-                        count_mates_wave<true>(J, S, v, s_tab, t, terr{0u, 0u}, valid, valid ? r : base, j, c2,
-                                               s_wave[wave], ck, lane);
-                    }
-                } else if (!CNA) {
-                    for (uint32_t base = wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
-                        const uint32_t r = base + lane;
-                        const bool valid = r < nj;
-                        const uint32_t rv = valid ? r : base;
-                        tmpl t = make_template<CNA>(J, S, s_tab, rv, j, s.b, s.e);
-                        const terr e = J.err_n ? template_errors(J, s_tab, rv, j, c2, valid) : terr{0u, 0u};
-                        count_mates_wave<false>(J, S, v, s_tab, t, e, valid, rv, j, c2, s_wave[wave], ck, lane);
-                        if (J.err_n) count_slow_errors(J, v, s_tab, t, e, valid, rv, j, c2, s_wave[wave], lane);
+                        count_mates_wave(J, S, v, s_tab, t, valid, valid ? r : base, j, c2, s_wave[wave], ck, lane);
                     }
                 } else {
                     // copy-number draws reject templates: the accepted ones are packed
@@ -1056,10 +1077,10 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
                         t.leaf = pleaf;
                         t.cell = 0;
                         t.ok = 1;
-                        count_wave(t, pr, on);
+                        count_mates_wave(J, S, v, s_tab, t, on, pr, j, c2, s_wave[wave], ck, lane);
                         pc = 0;
                     };
-                    for (uint32_t base = wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
+                    for (uint32_t base = t0 + wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
                         const uint32_t r = base + lane;
                         bool valid = r < nj;
                         tmpl t = make_template<CNA>(J, S, s_tab, valid ? r : base, j, s.b, s.e);
@@ -1089,10 +1110,10 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
                     }
                     if (pc) flush();
                 }
-                if (DEFER && J.err_n && ck.count) check_errors(J, v, s_tab, j, c2, ck, ck.count, lane);
+                if (J.err_n && ck.count) check_errors(J, v, s_tab, j, c2, ck, ck.count, lane);
                 __syncthreads();
-                int32_t* ga = J.alt + S.out_off + s.k0;
-                int32_t* gd = J.depth + S.out_off + s.k0;
+                int32_t* ga = J.alt + out_off(J, S) + s.k0;
+                int32_t* gd = J.depth + out_off(J, S) + s.k0;
                 for (uint32_t i = tid; i < s.n_win; i += BLOCK) {
                     const uint32_t d = s_dep[i];
                     if (d) {
@@ -1103,7 +1124,7 @@ __global__ void __launch_bounds__(BLOCK, DEFER ? 6 : (CNA ? 1 : 7)) k_seq_count(
                 }
                 __syncthreads();
             } else {
-                count_stratum_global<BLOCK, CNA>(J, S, s_tab, s, j, c2, s_wave[wave], lane, wave, &acc);
+                count_stratum_global<BLOCK, CNA>(J, S, s_tab, s, t0, nj, j, c2, s_wave[wave], lane, wave, &acc);
                 __syncthreads();  // s_tab may be reloaded next
             }
         }
@@ -1136,14 +1157,7 @@ __device__ __forceinline__ bool record_present(const job_dev& J, const pres_dev&
     } else {
         pres = J.purity_lt1 && normal_has;
         if (!pres) {
-            // sample leaves of rank below x, from the sample's running counts
-            const uint4* lc = J.leaf_count + (uint64_t)P.sample * J.leaf_blocks;
-            auto below = [&](uint32_t x) {
-                const uint4 e = lc[x >> 6];
-                const uint64_t bits = (uint64_t)e.y | ((uint64_t)e.z << 32);
-                return e.x + (uint32_t)__popcll(bits & ((1ull << (x & 63u)) - 1ull));
-            };
-            pres = below(J.hi[m]) > below(J.lo[m]);
+            pres = cells_below(J, P.sample, J.hi[m]) > cells_below(J, P.sample, J.lo[m]);
         }
     }
     return pres;
@@ -1537,7 +1551,7 @@ __global__ void __launch_bounds__(256) k_cn_accept(const accept_args a) {
     const job_dev J = uniform_at(a.jobs, S.job);
     const uint32_t j = g - uniform_at(a.cn_first, lo);
     const uint32_t b = j * PSX_STRATUM, e = min(b + PSX_STRATUM, S.W);
-    const uint64_t nj = S.T * e / S.W - S.T * b / S.W;
+    const uint64_t nj = templates_below(S, e) - templates_below(S, b);
     uint64_t cnt = 0;
     for (uint64_t r0 = 0; r0 < nj; r0 += 64u) {
         const uint64_t r = r0 + lane;

@@ -37,9 +37,10 @@ struct seq_batch;  // descriptors of one launch over one or more jobs
 // Validates the jobs (psx_error on the first invalid one) and builds their
 // descriptors on the host. Builds a mutation table's stratum index for a
 // genome it was not indexed for yet (allocates and synchronises ctx's stream)
-// unless no_alloc, which refuses such a job instead.
+// unless no_alloc, which refuses such a job instead. count: descriptors for
+// the count kernels (else for the read kernel).
 seq_batch* batch_prepare(psx_ctx* ctx, const job_in* jobs, size_t n_jobs, uint32_t strata_per_item,
-                         bool no_alloc = false);
+                         bool no_alloc = false, bool count = true);
 void batch_free(seq_batch* b);
 size_t batch_desc_bytes(const seq_batch* b);
 uint64_t batch_reads(const seq_batch* b);

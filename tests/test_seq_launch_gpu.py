@@ -54,3 +54,53 @@ def test_runs_of_many_small_items(ctx):
     first = sum(per[:21])
     alone = O.simulate_reads(w.lens, w.g.download(), w.of, w.recs, 7, per[21], **dict(kw, chromosomes=[21]))
     assert len(alone) == per[21] and np.array_equal(rows.numpy()[first:first + per[21]], alone)
+
+
+@pytest.mark.parametrize("cov,kw", [
+    # windows of one stratum in several rounds, of 2 and 4 strata, of 8 (no errors), single- and paired-end
+    (900.0, dict(read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=1e-3)),
+    (45.0, dict(read_size=100, insert_size_mean=250, insert_size_stddev=15, error_rate=4e-3, purity=0.6)),
+    (20.0, dict(read_size=151, error_rate=1e-3, purity=0.8, preneoplastic_in_normal=True)),
+    (4.0, dict(read_size=75)),
+    # nearly every template with repeated or more than three errors, more of them at records than a round lists
+    (300.0, dict(read_size=120, insert_size_mean=300, insert_size_stddev=12, error_rate=0.05)),
+    # mates far from their reads
+    (60.0, dict(read_size=60, insert_size_mean=2500, insert_size_stddev=40, error_rate=1e-3, purity=0.0))])
+def test_windows_of_dense_tables(ctx, dense, cov, kw):
+    """Tables whose reads cover many positions are counted by windows (k_count_dense): strata per window, rounds, parts
+    of an item, chromosomes of a few starts, records that share positions, the normal genome."""
+    for w in dense:
+        a, d, p, n = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 17, coverage=cov, **kw)
+        assert n == w.check((a, d, p), 17, dict(kw, coverage=cov)) and d.sum() > 0
+
+
+@pytest.fixture(scope="module")
+def dense(ctx):
+    forest = dict(n_cells=600, n_samples=2, sample_size=70, seed=6)
+    lens = [70_001, 33_000, 8_192 + 149, 400, 153]
+    return [World(ctx, lens, forest, 3e-5, n_pre_snv=60),
+            World(ctx, [50_000, 2_600], forest, 4e-5, seed=8, infinite_sites=False, n_pre_snv=60)]
+
+
+def test_windows_with_copy_numbers(ctx):
+    """Copy-number events on a dense table: rejected draws, packed templates, accepted reads counted."""
+    from process_amd import _abi as A
+    lens = [60_000, 20_000]
+    cna = [(0, 0, 5_000, 30_000, 0, A.PSX_CNA_AMP, 2), (0, 1, 1_000, 9_000, 1, A.PSX_CNA_DEL, 0),
+           (1, 0, 0, 0, 0, A.PSX_CNA_WGD, 0)]
+    w = World(ctx, lens, dict(n_cells=500, n_samples=1, sample_size=90, seed=2), 6e-5, cna=cna)
+    for kw in (dict(coverage=400, read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=2e-3, purity=0.7),
+               dict(coverage=8, read_size=100)):
+        a, d, p, n = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)
+        oa, od, op, on = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), **kw)
+        assert n == on and np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op)
+
+
+def test_parts_of_few_strata(ctx):
+    """Few strata with many templates: items are cut into parts, in both count kernels."""
+    forest = dict(n_cells=300, n_samples=1, sample_size=60, seed=4)
+    for snv in (2e-7, 1e-4):
+        w = World(ctx, [20_000, 5_000], forest, snv)
+        for kw in (dict(coverage=6000, read_size=101, error_rate=5e-3, purity=0.7),
+                   dict(coverage=4000, read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=1e-3)):
+            w.check(core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 5, **kw)[:3], 5, kw)
