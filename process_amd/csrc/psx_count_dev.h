@@ -1,7 +1,10 @@
-// The dense form of count-only sequencing on gfx950. Included once, by
-// psx_seq.hip, after psx_seq_dev.h.
+// Count-only sequencing on gfx950. Included once, by psx_seq.hip, after
+// psx_seq_dev.h.
 //
-// A block takes a window of one to eight strata of a segment, draws their
+// Two forms with the same counts: k_count_sparse for tables whose records
+// reads rarely cover, k_count_dense for the others.
+//
+// Dense. A block takes a window of one to eight strata of a segment, draws their
 // templates in rounds of about 5,600 reads and drops every read, one 32-bit
 // word, into the LDS bin of its start (start inside the bin | source copy);
 // then the window's records are dealt to the threads, several threads to a
@@ -44,57 +47,20 @@ __host__ __device__ __forceinline__ uint32_t dense_lds(uint32_t bins, uint32_t b
     return 4u * (dense_bit_words(bits) + bins * (BIN_STRIDE + 2u));
 }
 
-// A record as the scan sees it: position in the window, and the carrying
-// copies [low, low + len) of the word's copy field (allele above the cell).
-// Records alone at their position are counted by the scan alone; one that
-// shares its position is counted with it by the first of them (GROUP), as is
-// one whose carriers are no single range.
-struct scan_rec {
-    uint32_t p, low, len, kind;
-};
-enum : uint32_t { REC_NONE = 0, REC_SOLO = 1, REC_GROUP = 2 };
-
-__device__ __forceinline__ scan_rec load_rec(const job_dev& J, const seg_dev& S, uint32_t wb, uint32_t k0, uint32_t i,
-                                             uint32_t cb, uint32_t lw) {
-    const uint32_t q = k0 + i;
-    const uint32_t pos = J.pos[q], info = J.info[q];
-    const uint32_t nat = PSX_INFO_NATURE(info);
-    const bool normal_has = nat == PSX_GERMINAL || (nat == PSX_PRENEOPLASTIC && J.preneo);
-    uint32_t lo = 0, hi = normal_has ? 1u : 0u;  // the normal sample: one cell
-    bool one_range = true;
-    if (S.n_cells) {
-        lo = cells_below(J, S.sample, J.lo[q]);
-        hi = cells_below(J, S.sample, J.hi[q]);
-        if (normal_has && J.thr_normal) {  // reads of the normal genome carry it too (cell n_cells)
-            one_range = hi == S.n_cells || lo == hi;
-            lo = lo == hi ? S.n_cells : lo;
-            hi = S.n_cells + 1u;
-        }
-    }
-    scan_rec R;
-    R.p = pos - wb;
-    R.low = ((PSX_INFO_ALLELE(info) << cb) | lo) << lw;
-    R.len = (hi - lo) << lw;
-    const bool plain = one_range && PSX_INFO_HEAD(info) &&
-                       (PSX_INFO_KIND(info) != PSX_SNV || PSX_INFO_REF(info) != PSX_INFO_ALT(info));
-    if (PSX_INFO_SOLO(info)) R.kind = plain ? REC_SOLO : REC_GROUP;
-    else R.kind = i > 0 && J.pos[q - 1] == pos ? REC_NONE : REC_GROUP;
-    return R;
-}
-
 // The job's insert-size table in LDS: the thresholds and, per guide bucket,
 // the first and the last answer a draw of the bucket can have (one word).
-constexpr uint32_t DENSE_GUIDE_BITS = 10;
-struct dense_tables {
+constexpr uint32_t COUNT_GUIDE_BITS = 10;
+struct count_tables {
     uint32_t ins[MAX_INS];
-    uint32_t guide[1u << DENSE_GUIDE_BITS];
+    uint32_t guide[1u << COUNT_GUIDE_BITS];
 };
 
-__device__ __forceinline__ void load_dense_tables(const job_dev& J, dense_tables& t, uint32_t tid) {
-    constexpr uint32_t G = 1u << DENSE_GUIDE_BITS, STEP = 1u << (PSX_GUIDE_BITS - DENSE_GUIDE_BITS);
+template <uint32_t BLOCK>
+__device__ __forceinline__ void load_count_tables(const job_dev& J, count_tables& t, uint32_t tid) {
+    constexpr uint32_t G = 1u << COUNT_GUIDE_BITS, STEP = 1u << (PSX_GUIDE_BITS - COUNT_GUIDE_BITS);
     if (!J.pe) return;
-    for (uint32_t i = tid; i < J.ins_n; i += DENSE_BLOCK) t.ins[i] = J.ins_T[i];
-    for (uint32_t i = tid; i < G; i += DENSE_BLOCK)
+    for (uint32_t i = tid; i < J.ins_n; i += BLOCK) t.ins[i] = J.ins_T[i];
+    for (uint32_t i = tid; i < G; i += BLOCK)
         t.guide[i] = (uint32_t)J.ins_guide[i * STEP] |
                      (i + 1u < G ? (uint32_t)J.ins_guide[(i + 1u) * STEP] : J.ins_n - 1u) << 16;
 }
@@ -102,8 +68,8 @@ __device__ __forceinline__ void load_dense_tables(const job_dev& J, dense_tables
 // Insert-size pick (psx_guided_pick). Nearly every bucket holds at most one
 // threshold, so one compare settles it; where a lane's bucket holds more (the
 // tails: one wave in five), a binary search inside the buckets.
-__device__ __forceinline__ uint32_t pick_insert(const dense_tables& t, uint32_t u) {
-    const uint32_t g = t.guide[u >> (32u - DENSE_GUIDE_BITS)];
+__device__ __forceinline__ uint32_t pick_insert(const count_tables& t, uint32_t u) {
+    const uint32_t g = t.guide[u >> (32u - COUNT_GUIDE_BITS)];
     uint32_t lo = g & 0xFFFFu, hi = g >> 16;
     const uint32_t first = t.ins[lo];  // lo < hi <= MAX_INS - 1, or the answer
     const bool past = lo < hi && u >= first;
@@ -200,10 +166,358 @@ __device__ __attribute__((noinline)) void dense_group(const job_dev* Jp, const s
     }
 }
 
+// The templates [t0, t1) of the item's part of stratum [b, e) (wave-uniform; all lanes of the wave call it).
+__device__ __forceinline__ void wave_share(const seg_dev& S, uint32_t part, uint32_t b, uint32_t e, uint32_t lane,
+                                           uint32_t& t0, uint32_t& t1) {
+    const uint32_t below = (uint32_t)templates_below(S, lane ? e : b);  // lane 0: its first template; lane 1: its end
+    const uint32_t nj = (uint32_t)__builtin_amdgcn_readlane((int)below, 1) -
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)below);
+    t0 = 0;
+    t1 = nj;
+    if (seg_parts(S) != 1u) {
+        const uint32_t share = (nj + seg_parts(S) - 1u) / seg_parts(S);
+        t0 = min(nj, part * share);
+        t1 = min(nj, t0 + share);
+    }
+}
+
+// What a segment's template draws use, read once per item. A diploid source
+// without copy-number events is drawn here, any other by template_source.
+struct source_draw {
+    uint32_t n_cells, copies, normal_below, starts_end, RL;
+    int ins_past;  // the smallest insert size over the read size
+    bool diploid, normal_some;
+    __device__ __forceinline__ source_draw(const job_dev& J, const seg_dev& S, bool cna)
+        : n_cells(S.n_cells), copies(S.n_cells ? 2u * S.n_cells : 2u), normal_below((uint32_t)(J.thr_normal - 1u)),
+          starts_end(S.len - J.L), RL(J.L), ins_past((int)J.ins_k0 - (int)J.L),
+          diploid(J.ploidy == 2u && !(cna && S.n_cna != 0u)), normal_some(S.n_cells != 0u && J.thr_normal != 0u) {}
+    // Template r of stratum j = [b, e): start in the window that begins at wb, mate 2's offset, source cell (n_cells: the
+    // normal genome) and allele; false when a copy-number draw rejects it.
+    template <bool CNA>
+    __device__ __forceinline__ bool draw(const job_dev& J, const seg_dev& S, const count_tables& tab, uint32_t r, uint32_t j,
+                                         uint32_t c2, uint32_t b, uint32_t e, uint32_t wb, uint32_t& x, uint32_t& d,
+                                         uint32_t& cell, uint32_t& al) const {
+        psx_u4 w;
+        bool ok = true;
+        if (diploid) {
+            w = psx_draw_u(J.seed, r, j, c2, PSX_P_TEMPLATE << 24);
+            x = b - wb + psx_uniform32(w.x, e - b);
+            uint32_t v = psx_uniform32(w.z, copies);
+            cell = v >> 1;
+            if (normal_some) {
+                const bool normal = w.y <= normal_below;
+                v = normal ? w.z >> 31 : v;
+                cell = normal ? n_cells : cell;
+            }
+            al = v & 1u;
+        } else {
+            const tmpl t = template_source<CNA, false>(J, S, r, j, b, e, w);
+            x = t.x - wb;
+            cell = t.cell;
+            al = t.allele;
+            if (CNA) ok = t.ok != 0u;
+        }
+        d = 0;
+        if (J.pe) {
+            const int I = (int)pick_insert(tab, w.w) + ins_past;
+            d = min((uint32_t)max(I, 0), starts_end - wb - x);
+        }
+        return ok;
+    }
+};
+
+// The carriers of record q among the reads of the segment's sample: cells [lo, lo + len) (the normal genome is cell
+// n_cells); false when they are no single range.
+__device__ __forceinline__ bool carrier_cells(const job_dev& J, const seg_dev& S, uint64_t q, uint32_t info, uint32_t& lo,
+                                              uint32_t& len) {
+    const uint32_t nat = PSX_INFO_NATURE(info);
+    const bool normal_has = nat == PSX_GERMINAL || (nat == PSX_PRENEOPLASTIC && J.preneo);
+    lo = 0;
+    uint32_t hi = normal_has ? 1u : 0u;  // the normal sample: one cell
+    bool one_range = true;
+    if (S.n_cells) {
+        lo = cells_below(J, S.sample, J.lo[q]);
+        hi = cells_below(J, S.sample, J.hi[q]);
+        if (normal_has && J.thr_normal) {  // reads of the normal genome carry it too
+            one_range = hi == S.n_cells || lo == hi;
+            lo = lo == hi ? S.n_cells : lo;
+            hi = S.n_cells + 1u;
+        }
+    }
+    len = hi - lo;
+    return one_range;
+}
+
+// Whether the carrier range decides an alternative read of a record alone at its position.
+__device__ __forceinline__ bool plain_record(uint32_t info) {
+    return PSX_INFO_HEAD(info) && (PSX_INFO_KIND(info) != PSX_SNV || PSX_INFO_REF(info) != PSX_INFO_ALT(info));
+}
+
+// ------------------------------------------------- tables with few mutations
+//
+// Where reads rarely cover a record, a template ends with one test per read:
+// a bit per 8 starts of the window says whether a read that starts there can
+// reach a record. The reads that can are queued by the wave and counted 64 at
+// a time, one per lane: the records each covers, found in LDS, the carriers as
+// ranges of the sample's cells, and the errors of its template, drawn only
+// then. Bound by vector instruction issue: 132 instructions per 64 templates
+// where nothing is covered (43 Philox, 20 the source, 20 the insert size, 20
+// the tests; 4.4-4.7 cycles each), and about 390 per 64 queued reads. The form
+// before walked every read's records and queued positions: 200 Mb at 30x with
+// one record per 13,000 bases 559 -> 357 us, 1.5 Mb at 2000x 500 -> 447 us.
+// With a bit per 32 starts instead of 8 (more reads queued in vain) 362 and
+// 486 us.
+
+// An entry of a wave's queue: a read.
+struct sparse_read {
+    uint32_t at;    // start in the window | mate << 18 | allele << 19
+    uint32_t cell;  // its source cell (the normal genome: n_cells)
+    uint32_t r;     // template index
+};
+
+constexpr uint32_t START_SHIFT = 3;  // starts per bit of the reach bitmap
+
+template <int BLOCK, int CAP>
+struct sparse_lds {
+    static constexpr uint32_t WAVES = BLOCK / 64;
+    static constexpr uint32_t START_BITS = ((PSX_STRATUM * WAVES + MAX_READ) >> START_SHIFT) + 1u;
+    count_tables tab;
+    uint32_t err[4];                         // thresholds of 1 to 4 errors, padded
+    uint32_t p[CAP], low[CAP], len[CAP], info[CAP];  // records: position in the window, cells [low, low + len)
+    uint32_t dep[CAP], alt[CAP];
+    uint32_t bits[(START_BITS + 31u) / 32u];
+    sparse_read queue[WAVES][128];
+    uint32_t run, acc;
+};
+static_assert(64 * sizeof(sparse_read) >= 4 * ELIST, "a slow template's errors take the place of the entries counted");
+
+// info word of a staged record: the table's, with bits 30 (counted with the first record of its position) and 31 (that
+// first record, or one whose carriers are no single range) set where the record is not counted alone
+constexpr uint32_t REC_SKIP = 1u << 30, REC_SHARED = 1u << 31;
+
+// The queued reads q[0, n) of a wave, one per lane; n_lds: records staged (0: the window has more, all in global memory).
+template <class LDS>
+__device__ __forceinline__ void stage_record(const job_dev& J, const seg_dev& S, LDS& lds, uint32_t k0, uint32_t i,
+                                             uint32_t p) {
+    const uint32_t q = k0 + i;
+    const uint32_t info = J.info[q];
+    uint32_t lo, len;
+    const bool one_range = carrier_cells(J, S, q, info, lo, len);
+    uint32_t flag = 0;
+    if (!PSX_INFO_SOLO(info)) flag = i > 0 && J.pos[q - 1] == J.pos[q] ? REC_SKIP : REC_SHARED;
+    else if (!one_range || !plain_record(info)) flag = REC_SHARED;
+    lds.p[i] = p;
+    lds.low[i] = lo;
+    lds.len[i] = len;
+    lds.info[i] = (info & ~(REC_SKIP | REC_SHARED)) | flag;
+}
+
+template <class LDS>
+__device__ __attribute__((noinline)) void count_queued(const job_dev* Jp, const seg_dev* Sp, LDS* lds,
+                                                       sparse_read* q, uint32_t n, uint32_t wb, uint32_t k0,
+                                                       uint32_t n_win, uint32_t n_lds, uint32_t j, uint32_t c2) {
+    const job_dev& J = *Jp;
+    const seg_dev& S = *Sp;
+    const uint32_t lane = threadIdx.x & 63u;
+    const bool on = lane < n;
+    const sparse_read R = on ? q[lane] : sparse_read{0u, 0u, 0u};
+    const uint32_t xr = R.at & 0x3FFFFu, mate = (R.at >> 18) & 1u, al = R.at >> 19;
+    const uint32_t leaf = on ? leaf_of_cell(J, S, R.cell) : 0u;
+    const uint32_t end = xr + J.L, boff = mate * J.L - xr;  // base index of position p in the template: p + boff
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)J.seed);
+    const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(J.seed >> 32));
+    const glb_view gv = window_view(J, S, k0, n_win);
+    terr e{0u, 0u};
+    if (J.err_n) e = template_errors(J, (uint64_t)s1 << 32 | s0, lds->err, R.r, j, c2, on);
+    if (n_lds) {
+        uint32_t a = 0, z = on ? n_lds : 0u;
+        while (a < z) {
+            const uint32_t mid = (a + z) >> 1;
+            if (lds->p[mid] < xr) a = mid + 1; else z = mid;
+        }
+        for (; on && a < n_lds; ++a) {
+            const uint32_t p = lds->p[a];
+            if (p >= end) break;
+            const uint32_t in = lds->info[a];
+            if (in & (REC_SKIP | REC_SHARED)) {
+                if (in & REC_SHARED) count_group(J, gv, a, al, leaf, e, boff - wb);
+                continue;
+            }
+            atomicAdd(&lds->dep[a], 1u);
+            const bool car = PSX_INFO_ALLELE(in) == al && R.cell - lds->low[a] < lds->len[a];
+            bool hit = car;
+            if (PSX_INFO_KIND(in) == PSX_SNV) {
+                const uint32_t tb = car ? PSX_INFO_ALT(in) : PSX_INFO_REF(in);
+                hit = observe(e, p + boff, tb) == PSX_INFO_ALT(in);
+            }
+            if (hit) atomicAdd(&lds->alt[a], 1u);
+        }
+    } else if (on) {
+        uint32_t i = gv.first(wb + xr);
+        while (i < n_win && gv.pos[i] < wb + end) i = count_group(J, gv, i, al, leaf, e, boff - wb);
+    }
+    // slow templates counted without errors: the wave generates each one's and corrects the counts at those of this mate
+    uint32_t* list = (uint32_t*)q;  // every lane has read its entry
+    unsigned long long sm = __ballot(on && e.slow());
+    while (sm) {
+        const int ln = __ffsll((long long)sm) - 1;
+        sm &= sm - 1ull;
+        const uint32_t xs = (uint32_t)__builtin_amdgcn_readlane((int)xr, ln), ms = (uint32_t)__builtin_amdgcn_readlane((int)mate, ln);
+        const uint32_t as = (uint32_t)__builtin_amdgcn_readlane((int)al, ln), ls = (uint32_t)__builtin_amdgcn_readlane((int)leaf, ln);
+        const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)R.r, ln);
+        wave_sync();
+        const uint32_t ne = wave_template_errors((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane);
+        wave_sync();
+        for (uint32_t k = lane; k < ne; k += 64u) {
+            const uint32_t w = list[k], bi = w & 0xFFFFFu;
+            if ((bi >= J.L ? 1u : 0u) != ms) continue;
+            const uint32_t P = wb + xs + bi - ms * J.L;
+            const uint32_t i = gv.first(P);
+            if (i < n_win && gv.pos[i] == P) error_fix(J, gv, i, as, ls, w >> 20);
+        }
+    }
+    wave_sync();
+}
+
+template <int BLOCK, int CAP, bool CNA>
+__global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
+    using LDS = sparse_lds<BLOCK, CAP>;
+    __shared__ LDS lds;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    sparse_read* const queue = lds.queue[wave];
+    uint32_t in_tab = UNRESOLVED;
+    for (uint32_t i = tid; i < (uint32_t)CAP; i += BLOCK) lds.dep[i] = lds.alt[i] = 0;
+    for (uint32_t i = tid; i < (LDS::START_BITS + 31u) / 32u; i += BLOCK) lds.bits[i] = 0;
+    __syncthreads();
+    for (uint32_t run = blockIdx.x;;) {
+        const item_run R0 = run_of(L, run);
+        if (R0.first == R0.end) break;
+        if (tid == 0) lds.run = gridDim.x + (uint32_t)atomicAdd(L.queue, 1ull);  // the block's next run
+        for (uint32_t item = R0.first; item < R0.end; ++item) {
+            const item_dev it = uniform_at(L.items, item);
+            const seg_dev& S = *(const seg_dev*)((const __attribute__((address_space(4))) seg_dev*)L.segs + it.seg);
+            const job_dev& J = *(const job_dev*)((const __attribute__((address_space(4))) job_dev*)L.jobs + S.job);
+            const uint32_t c2 = (S.chr << 16) | S.so;
+            const uint32_t lns = seg_lns(S), nslot = LDS::WAVES >> lns, slot = wave & (nslot - 1u);
+            const uint32_t RL = J.L, pe = J.pe;
+            const source_draw D(J, S, CNA);
+            if (CNA && tid == 0) lds.acc = 0;
+            if (in_tab != S.job) {
+                in_tab = S.job;
+                load_count_tables<BLOCK>(J, lds.tab, tid);
+                if (tid < 4u) lds.err[tid] = tid < J.err_n ? J.err_T[tid] : 0xFFFFFFFFu;
+            }
+            uint32_t acc = 0;  // accepted templates (wave-uniform)
+            for (uint32_t jw = it.j0; jw < it.j1; jw += 1u << lns) {
+                const uint32_t wb = jw * PSX_STRATUM, je = min(jw + (1u << lns), it.j1);
+                const uint32_t starts = min(je * PSX_STRATUM, S.W);
+                const uint32_t wend = min(S.len, starts - 1u + J.reach);
+                const uint32_t k0 = uniform_at(J.bucket, S.bucket_off + jw);
+                const uint32_t n_win = window_records(J, S, k0, wend);
+                const uint32_t n_lds = n_win <= (uint32_t)CAP ? n_win : 0u;
+                // the records, and the starts from which a read reaches one
+                for (uint32_t i = tid; i < n_win; i += BLOCK) {
+                    const uint32_t p = J.pos[k0 + i] - wb;
+                    if (n_lds) stage_record(J, S, lds, k0, i, p);
+                    if (p >= wend - wb) continue;
+                    const uint32_t f = (p + 1u > RL ? p + 1u - RL : 0u) >> START_SHIFT, l = p >> START_SHIFT;
+                    for (uint32_t w = f >> 5; w <= l >> 5; ++w) {
+                        const uint32_t from = w == f >> 5 ? f & 31u : 0u, to = w == l >> 5 ? l & 31u : 31u;
+                        atomicOr(&lds.bits[w], (0xFFFFFFFFu << from) & (0xFFFFFFFFu >> (31u - to)));
+                    }
+                }
+                __syncthreads();
+                const uint32_t j = jw + wave / nslot;
+                const uint32_t b = j * PSX_STRATUM, e = min(b + PSX_STRATUM, S.W);
+                uint32_t t0 = 0, t1 = 0;
+                if (j < je) wave_share(S, it.part, b, e, lane, t0, t1);
+                uint32_t qn = 0;
+                for (uint32_t g = t0 + slot * 64u; g < t1; g += nslot * 64u) {  // wave-uniform
+                    bool on = g + lane < t1;
+                    const uint32_t r = on ? g + lane : g;
+                    uint32_t x, d, cell, al;
+                    on = D.draw<CNA>(J, S, lds.tab, r, j, c2, b, e, wb, x, d, cell, al) && on;
+                    if (CNA) acc += (uint32_t)__popcll(__ballot(on));
+                    for (uint32_t m = 0; m <= pe; ++m) {
+                        const uint32_t xm = m ? x + d : x;
+                        const uint32_t bit = xm >> START_SHIFT;
+                        const bool add = on && ((lds.bits[bit >> 5] >> (bit & 31u)) & 1u);
+                        const unsigned long long mask = __ballot(add);
+                        if (!mask) continue;
+                        if (add)
+                            queue[qn + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u))] =
+                                sparse_read{xm | m << 18 | al << 19, cell, r};
+                        qn += (uint32_t)__popcll(mask);
+                        if (qn >= 64u) {
+                            qn -= 64u;
+                            wave_sync();
+                            count_queued(&J, &S, &lds, queue + qn, 64u, wb, k0, n_win, n_lds, j, c2);
+                        }
+                    }
+                }
+                if (qn) {
+                    wave_sync();
+                    count_queued(&J, &S, &lds, queue, qn, wb, k0, n_win, n_lds, j, c2);
+                }
+                __syncthreads();
+                for (uint32_t i = tid; i < n_lds; i += BLOCK) {
+                    const uint32_t dep = lds.dep[i], alt = lds.alt[i];
+                    if (dep) {
+                        const uint64_t o = out_off(J, S) + k0 + i;
+                        atomicAdd(J.depth + o, (int32_t)dep);
+                        if (alt) atomicAdd(J.alt + o, (int32_t)alt);
+                        lds.dep[i] = lds.alt[i] = 0;
+                    }
+                }
+                for (uint32_t i = tid; i < (((wend - wb) >> START_SHIFT) + 32u) >> 5; i += BLOCK) lds.bits[i] = 0;
+                __syncthreads();
+            }
+            if (CNA && S.n_cna) {
+                if (acc && lane == 0) atomicAdd(&lds.acc, acc);
+                __syncthreads();
+                if (tid == 0 && lds.acc) atomicAdd(J.acc, (unsigned long long)lds.acc * (J.pe + 1u));
+            }
+        }
+        __syncthreads();
+        run = __builtin_amdgcn_readfirstlane(lds.run);
+        __syncthreads();  // read by every wave before it is written again
+    }
+}
+
+// ---------------------------------------------- tables with many mutations
+
+// A record as the scan sees it: position in the window, and the carrying
+// copies [low, low + len) of the word's copy field (allele above the cell).
+// Records alone at their position are counted by the scan alone; one that
+// shares its position is counted with it by the first of them (GROUP), as is
+// one whose carriers are no single range.
+struct scan_rec {
+    uint32_t p, low, len, kind;
+};
+enum : uint32_t { REC_NONE = 0, REC_SOLO = 1, REC_GROUP = 2 };
+
+__device__ __forceinline__ scan_rec load_rec(const job_dev& J, const seg_dev& S, uint32_t wb, uint32_t k0, uint32_t i,
+                                             uint32_t cb, uint32_t lw) {
+    const uint32_t q = k0 + i;
+    const uint32_t pos = J.pos[q], info = J.info[q];
+    uint32_t lo, len;
+    const bool one_range = carrier_cells(J, S, q, info, lo, len);
+    scan_rec R;
+    R.p = pos - wb;
+    R.low = ((PSX_INFO_ALLELE(info) << cb) | lo) << lw;
+    R.len = len << lw;
+    if (PSX_INFO_SOLO(info)) R.kind = one_range && plain_record(info) ? REC_SOLO : REC_GROUP;
+    else R.kind = i > 0 && J.pos[q - 1] == pos ? REC_NONE : REC_GROUP;
+    return R;
+}
+
+
 template <bool CNA>
 __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch L) {
     extern __shared__ uint4 s_dyn[];
-    __shared__ dense_tables s_tab;
+    __shared__ count_tables s_tab;
     __shared__ uint32_t s_run, s_acc, s_neff, s_todo_n[2];
     __shared__ uint32_t s_list[DENSE_WAVES][ELIST];  // per wave: a slow template's errors
     __shared__ todo s_todo[TODO_CAP];
@@ -225,21 +539,15 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
             const uint32_t c2 = (S.chr << 16) | S.so;
             const uint32_t lns = seg_lns(S), cb = seg_cb(S), lw = seg_lw(S), SH = 32u - lw;
             const uint32_t nslot = DENSE_WAVES >> lns, slot = wave & (nslot - 1u);
-            const uint32_t RL = J.L, pe = J.pe, err_n = J.err_n, err_N = J.err_N, n_cells = S.n_cells;
-            const uint32_t starts_end = S.len - RL;  // the last start
-            const int ins_past = (int)J.ins_k0 - (int)RL;  // of the smallest insert size over the read size
-            // a diploid source without copy-number events is drawn here; normal_below: draws up to it take a copy of
-            // the normal genome (purity below 1)
-            const bool diploid = J.ploidy == 2u && !(CNA && S.n_cna != 0u);
-            const bool normal_some = n_cells != 0u && J.thr_normal != 0u;
-            const uint32_t normal_below = (uint32_t)(J.thr_normal - 1u), copies = n_cells ? 2u * n_cells : 2u;
+            const uint32_t RL = J.L, pe = J.pe, err_n = J.err_n, err_N = J.err_N;
+            const source_draw D(J, S, CNA);
             uint32_t errT[4];  // thresholds of 1 to 4 errors past the table's first count (capped below)
 #pragma unroll
             for (uint32_t q = 0; q < 4u; ++q) errT[q] = q < err_n ? uniform_at(J.err_T, q) : 0xFFFFFFFFu;
             if (CNA && tid == 0) s_acc = 0;
             if (in_tab != S.job) {
                 in_tab = S.job;
-                load_dense_tables(J, s_tab, tid);
+                load_count_tables<DENSE_BLOCK>(J, s_tab, tid);
             }
             uint32_t acc = 0;  // accepted templates (copy-number events)
             for (uint32_t jw = it.j0; jw < it.j1; jw += 1u << lns) {
@@ -274,18 +582,7 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                 const uint32_t j = jw + wave / nslot;
                 const uint32_t b = j * PSX_STRATUM, e = min(b + PSX_STRATUM, S.W);
                 uint32_t t0 = 0, t1 = 0;
-                if (j < je) {
-                    const uint64_t below = templates_below(S, lane ? e : b);  // lane 0: its first template; lane 1: its end
-                    const uint32_t lo = (uint32_t)below, t_b = (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
-                    const uint32_t nj = (uint32_t)__builtin_amdgcn_readlane((int)lo, 1) - t_b;
-                    if (seg_parts(S) == 1u) {
-                        t1 = nj;
-                    } else {
-                        const uint32_t share = (nj + seg_parts(S) - 1u) / seg_parts(S);
-                        t0 = min(nj, it.part * share);
-                        t1 = min(nj, t0 + share);
-                    }
-                }
+                if (j < je) wave_share(S, it.part, b, e, lane, t0, t1);
                 // rounds: the same number for every wave, from a bound on any stratum's share
                 const uint32_t most = S.most, round_t = S.round_t;
                 scan_rec R{0, 0, 0, REC_NONE};
@@ -302,27 +599,10 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                         if (more) {
                             on = g + lane < end;
                             r = on ? g + lane : g;
-                            psx_u4 w;
-                            if (diploid) {
-                                w = psx_draw_u(J.seed, r, j, c2, PSX_P_TEMPLATE << 24);
-                                x = b - wb + psx_uniform32(w.x, e - b);
-                                uint32_t v = psx_uniform32(w.z, copies), cell = v >> 1;
-                                if (normal_some) {
-                                    const bool normal = w.y <= normal_below;
-                                    v = normal ? w.z >> 31 : v;
-                                    cell = normal ? n_cells : cell;
-                                }
-                                X = ((v & 1u) << cb) | cell;
-                            } else {
-                                const tmpl t = template_source<CNA, false>(J, S, r, j, b, e, w);
-                                x = t.x - wb;
-                                X = (t.allele << cb) | t.cell;
-                                if (CNA) on = on && t.ok;
-                            }
-                            if (pe) {
-                                const int I = (int)pick_insert(s_tab, w.w) + ins_past;
-                                d = min((uint32_t)max(I, 0), starts_end - wb - x);
-                            }
+                            uint32_t cell, al;
+                            const bool ok = D.draw<CNA>(J, S, s_tab, r, j, c2, b, e, wb, x, d, cell, al);
+                            X = (al << cb) | cell;
+                            if (CNA) on = on && ok;
                         }
                         if (CNA) {
                             // copy-number draws reject templates: the accepted ones are packed into the lanes of a

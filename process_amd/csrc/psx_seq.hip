@@ -20,8 +20,9 @@ using namespace psxk;
 
 namespace psxh {
 
-// Covered positions per 64 templates from which a job counts by windows.
-constexpr double DENSE_COVER = 32.0, DENSE_COVER_NO_ERRORS = 4.0;
+// Covered positions per 64 templates from which a job counts by windows: on 1.6e9 reads with errors k_count_sparse takes
+// 3.8 ms at 10 and 5.2 at 19, k_count_dense 6.0 and 6.2; without errors 3.5 (10) and 4.7 (19) against 3.7 and 3.8.
+constexpr double DENSE_COVER = 28.0, DENSE_COVER_NO_ERRORS = 8.0;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
 // templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves.
 constexpr uint64_t FEW_ITEMS = 2048, MANY_ITEMS = 4096;
@@ -278,8 +279,8 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     P.job_reads.push_back(P.n_reads - reads_before);
 }
 
-// A job whose reads cover few positions counts with errors checked per
-// covered position (k_seq_count), the others by windows (k_count_dense).
+// A job whose reads cover few positions queues the reads that cover any
+// (k_count_sparse), the others count by windows (k_count_dense).
 bool job_sparse(const seq_batch& P, uint32_t job) {
     return !P.job_fits[job] || P.job_cover[job] < (P.jobs[job].err_n ? DENSE_COVER : DENSE_COVER_NO_ERRORS);
 }
@@ -288,11 +289,12 @@ bool job_sparse(const seq_batch& P, uint32_t job) {
 // dense window takes 2, 4 or 8 strata while their reads fit one round, in 64
 // bins of starts and as many more as mates reach past the window; on a
 // chromosome of less than a stratum the bins are narrower, at least 2 starts.
-void shape_segment(const seq_batch& P, seg_dev& S) {
+// Sparse windows take 2 or 4 strata where a wave would have fewer than 16
+// groups of 64 templates of one, as long as the launch keeps MANY_ITEMS.
+void shape_segment(const seq_batch& P, seg_dev& S, uint64_t strata) {
     const job_dev& J = P.jobs[S.job];
     const uint32_t cb = seg_cb(S), copy_bits = cb + bits_of(J.ploidy - 1u), past = J.reach - J.L;
     uint32_t lns = 0, lw = BIN_SHIFT;
-    S.spi = P.spi;
     if (P.count && !job_sparse(P, S.job)) {
         const double reads = (double)S.T * (J.pe + 1u) * PSX_STRATUM / (double)S.W;  // of a stratum
         while (lns < (J.err_n ? 2u : 3u) && reads * (double)(2u << lns) <= 64.0 * BIN_READS * 0.9 &&
@@ -300,8 +302,12 @@ void shape_segment(const seq_batch& P, seg_dev& S) {
             ++lns;
         lw += lns;
         while (lw > 1 && (S.W >> lw) < 32u && ((S.W + past) >> (lw - 1u)) < MAX_BINS) --lw;
-        S.spi = std::max(P.spi, 1u << lns);
+    } else if (P.count) {
+        const double templates = (double)S.T * PSX_STRATUM / (double)S.W;  // of a stratum
+        while (lns < 2u && templates * (double)(1u << lns) < 4096.0 && (1u << lns) < S.J && strata >> (lns + 1u) >= MANY_ITEMS)
+            ++lns;
     }
+    S.spi = std::max(P.spi, 1u << lns);
     S.shape = cb | lns << 8 | lw << 12 | 1u << 16;
 }
 
@@ -310,9 +316,11 @@ void shape_segment(const seq_batch& P, seg_dev& S) {
 // of a prepared batch after the per-job tables.
 void layout(seq_batch& P) {
     std::stable_partition(P.segs.begin(), P.segs.end(), [&](const seg_dev& S) { return job_sparse(P, S.job); });
-    uint64_t items[2] = {0, 0};  // sparse, dense
+    uint64_t items[2] = {0, 0}, strata[2] = {0, 0};  // sparse, dense
+    for (const seg_dev& S : P.segs)
+        if (S.T) strata[job_sparse(P, S.job) ? 0 : 1] += S.J;
     for (seg_dev& S : P.segs) {
-        shape_segment(P, S);
+        shape_segment(P, S, strata[job_sparse(P, S.job) ? 0 : 1]);
         if (S.T) items[job_sparse(P, S.job) ? 0 : 1] += (S.J + S.spi - 1) / S.spi;
     }
     P.n_items = 0;
@@ -360,8 +368,8 @@ void layout(seq_batch& P) {
 
 template <int BLOCK, int CAP>
 void launch_count_t(const seq_lane& lane, const seq_launch& L, uint32_t grid, bool cna) {
-    if (cna) hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, true>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
-    else hipLaunchKernelGGL((k_seq_count<BLOCK, CAP, false>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
+    if (cna) hipLaunchKernelGGL((k_count_sparse<BLOCK, CAP, true>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
+    else hipLaunchKernelGGL((k_count_sparse<BLOCK, CAP, false>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
 }
 
 void launch_count(const seq_lane& lane, const psx_launch_config& c, const seq_launch& L, uint32_t grid, bool cna) {

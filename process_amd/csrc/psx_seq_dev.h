@@ -424,10 +424,10 @@ struct terr {
 
 // The summary of template r of stratum j; lanes with want == false get none.
 // Every lane steps through the same count loop.
-template <class TAB>
-__device__ __forceinline__ terr template_errors(const job_dev& J, const TAB& tab, uint32_t r, uint32_t j,
-                                                uint32_t c2, bool want) {
-    const psx_u4 w = psx_draw_u(J.seed, r, j, c2, PSX_P_ERROR << 24);
+// err: the error table's first four thresholds (padded).
+__device__ __forceinline__ terr template_errors(const job_dev& J, uint64_t seed, const uint32_t* err, uint32_t r,
+                                                uint32_t j, uint32_t c2, bool want) {
+    const psx_u4 w = psx_draw_u(seed, r, j, c2, PSX_P_ERROR << 24);
     // K = err_k0 + the number of thresholds k < err_n - 1 with u >= T[k] (T is
     // non-decreasing, every kept threshold but the last below 2^32, the last and
     // the padding 2^32 - 1); only K <= 3 matters here, so four compares against
@@ -436,7 +436,7 @@ __device__ __forceinline__ terr template_errors(const job_dev& J, const TAB& tab
     // which only u = 2^32 - 1 reaches
     uint32_t k = 0;
 #pragma unroll
-    for (uint32_t q = 0; q < 4u; ++q) k += w.y >= tab.err[q] ? 1u : 0u;
+    for (uint32_t q = 0; q < 4u; ++q) k += w.y >= err[q] ? 1u : 0u;
     k = min(k, J.err_n ? J.err_n - 1u : 0u);
     const uint32_t K = want ? J.err_k0 + k : 0u;
     const uint32_t b0 = psx_mulhi32(w.x, J.err_N), b1 = psx_mulhi32(w.z, J.err_N), b2 = psx_mulhi32(w.w, J.err_N);
@@ -613,244 +613,6 @@ __device__ __forceinline__ void error_fix(const job_dev& J, const V& v, uint32_t
     }
 }
 
-// The slow templates among a wave's 64 (one per lane: t, e, template index
-// rr, counted when valid) were counted without errors: for each, the wave
-// generates its errors and each lane takes one, correcting the counts where
-// the error's base holds records. A read covering that position resolved its
-// template's leaf while it was counted.
-template <class V, class TAB>
-__device__ __forceinline__ void count_slow_errors(const job_dev& J, const V& v, const TAB& tab, const tmpl& t,
-                                                  const terr& e, bool valid, uint32_t rr, uint32_t j, uint32_t c2,
-                                                  uint32_t* list, uint32_t lane) {
-    unsigned long long sm = __ballot(valid && e.slow());
-    while (sm) {  // wave-uniform
-        const uint32_t sl = (uint32_t)__ffsll((long long)sm) - 1u;
-        sm &= sm - 1ull;
-        const uint32_t xs = (uint32_t)__builtin_amdgcn_readlane((int)t.x, (int)sl);
-        const uint32_t x2s = (uint32_t)__builtin_amdgcn_readlane((int)t.x2, (int)sl);
-        const uint32_t ls = (uint32_t)__builtin_amdgcn_readlane((int)t.leaf, (int)sl);
-        const uint32_t as = (uint32_t)__builtin_amdgcn_readlane((int)t.allele, (int)sl);
-        const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)rr, (int)sl);
-        wave_sync();
-        const uint32_t n = wave_template_errors(J.seed, J.err_n, J.err_k0, J.err_N, tab.err, rs, j, c2, list, lane);
-        wave_sync();
-        for (uint32_t k0 = 0; k0 < n; k0 += 64u) {
-            const uint32_t k = k0 + lane;
-            if (k < n) {
-                const uint32_t w = list[k];
-                const uint32_t b = w & 0xFFFFFu, sub = w >> 20;
-                const uint32_t m = b >= J.L ? 1u : 0u;
-                const uint32_t P = (m ? x2s : xs) + b - m * J.L;
-                const uint32_t i = v.first(P);
-                if (i < v.n && v.pos[i] == P) error_fix(J, v, i, as, ls, sub);
-            }
-        }
-    }
-}
-
-// One read [x, x + L) (mate `mate` of the lane's template; summary e): depth
-// for every record at a covered position, an alternative read for each SID
-// head whose alternative is observed (SNV) or carried (indel). Oracle:
-// seq_read. A record alone at its position (every record under the
-// infinite-sites model) takes one branch-free step of a wave-uniform loop; a
-// position shared by several records goes through count_group. Lanes with
-// valid == false take no part. Returns whether any lane's read covers a
-// record (wave-uniform).
-template <class V>
-__device__ __forceinline__ bool count_read(const job_dev& J, const seg_dev& S, const V& v, tmpl& t, const terr& e,
-                                           bool valid, uint32_t x, uint32_t mate) {
-    const uint32_t end = x + J.L;
-    uint32_t i = v.first_u(x);
-    bool go = valid && i < v.n && v.pos[v.at(i)] < end;
-    if (!__ballot(go)) return false;
-    uint32_t leaf = 0;
-    if (go) leaf = leaf_of(J, S, t);
-    const uint32_t boff = mate * J.L - x;  // base index of position p: p + boff
-    while (__ballot(go)) {
-        const uint32_t ic = go ? i : 0u;
-        const uint32_t p = v.pos[ic], in = v.info[ic];
-        if (__ballot(go && !PSX_INFO_SOLO(in))) {
-            if (go && !PSX_INFO_SOLO(in)) i = count_group(J, v, ic, t.allele, leaf, e, boff);
-        }
-        const bool one = go && PSX_INFO_SOLO(in);
-        const bool car = PSX_INFO_ALLELE(in) == t.allele && carried(J, in, v.lo[ic], v.hi[ic], leaf);
-        const bool snv = PSX_INFO_KIND(in) == PSX_SNV;
-        const uint32_t tb = snv && car ? PSX_INFO_ALT(in) : PSX_INFO_REF(in);
-        const uint32_t ob = observe(e, p + boff, tb);
-        if (one) {
-            v.add_dep(ic);
-            if (PSX_INFO_HEAD(in) && (snv ? ob == PSX_INFO_ALT(in) : car)) v.add_alt(ic);
-        }
-        i += one ? 1u : 0u;
-        go = go && i < v.n && v.pos[v.at(i)] < end;
-    }
-    return true;
-}
-
-// Deferred error checks of a wave (count kernel, LDS windows): a ring of
-// 128 entries of three words (template r; read base index b | allele << 13 |
-// record << 21; leaf), filled by the queue drains with every covered position
-// whose observed base matters (an SNV head, or several records) and checked
-// 64 at a time, so one draw per lane serves 64 covered positions instead of
-// one per template. head is 0 or 64 and count < 64 between drains.
-struct chk_ring {
-    uint32_t* e;  // 3 * 128 words, entry-major
-    uint32_t head, count;  // wave-uniform
-};
-
-// Checks the n <= 64 entries at the ring's head, one per lane: the entry's
-// template draws its error summary, and an error at the entry's base index
-// corrects the counts there (error_fix). The entries are read first, so a
-// slow template's error list can use their half of the ring. Oracle:
-// seq_read with the read's errors.
-template <class TAB>
-__device__ __forceinline__ void check_errors(const job_dev& J, const lds_view& v, const TAB& tab, uint32_t j,
-                                             uint32_t c2, chk_ring& q, uint32_t n, uint32_t lane) {
-    const bool on = lane < n;
-    uint32_t* half = q.e + q.head * 3u;
-    const uint32_t r = on ? half[lane * 3u] : 0u;
-    const uint32_t w = on ? half[lane * 3u + 1u] : 0u;
-    const uint32_t leaf = on ? half[lane * 3u + 2u] : 0u;
-    q.head = (q.head + 64u) & 127u;
-    q.count -= n;
-    const uint32_t b = w & 0x1FFFu, al = (w >> 13) & 0xFFu, ri = w >> 21;
-    const terr e = template_errors(J, tab, r, j, c2, on);
-    const uint32_t sub = error_sub(e, b);
-    if (on && sub < 4u) error_fix(J, v, ri, al, leaf, sub);
-    unsigned long long sm = __ballot(on && e.slow());
-    while (sm) {  // wave-uniform, rare
-        const uint32_t sl = (uint32_t)__ffsll((long long)sm) - 1u;
-        sm &= sm - 1ull;
-        const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)r, (int)sl);
-        const uint32_t bs = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)sl);
-        wave_sync();
-        const uint32_t ne = wave_template_errors(J.seed, J.err_n, J.err_k0, J.err_N, tab.err, rs, j, c2, half, lane);
-        wave_sync();
-        uint32_t found = 4u;  // at most one of the template's errors is at bs
-        for (uint32_t k0 = 0; k0 < ne; k0 += 64u) {
-            const uint32_t k = k0 + lane;
-            const uint32_t le = k < ne ? half[k] : 0u;
-            found = k < ne && (le & 0xFFFFFu) == bs ? le >> 20 : found;
-        }
-        const unsigned long long fm = __ballot(found < 4u);
-        if (fm) {
-            const uint32_t fs = (uint32_t)__builtin_amdgcn_readlane((int)found, (int)((uint32_t)__ffsll((long long)fm) - 1u));
-            if (lane == sl) error_fix(J, v, ri, al, leaf, fs);
-        }
-    }
-    wave_sync();  // the half is free again
-}
-
-// Both mates of 64 templates of a wave (one per lane): every lane walks the
-// positions its reads cover (mate 0's, then mate 1's, in one loop) and queues
-// (lane, mate, first record of the position) in the wave's LDS queue; the
-// queue is drained 64 entries at a time, one per lane, so the per-position
-// work runs on full waves instead of waiting for the lane whose reads cover
-// the most positions. Sequencing errors: the reads are counted with their
-// true bases and each drained position whose observed base matters goes to
-// the deferred checks (with the lane's template index rr). Lanes with valid ==
-// false take no part (their starts must still lie in the stratum).
-template <class TAB>
-__device__ __forceinline__ void count_mates_wave(const job_dev& J, const seg_dev& S, const lds_view& v,
-                                                 const TAB& tab, tmpl& t, bool valid, uint32_t rr, uint32_t j,
-                                                 uint32_t c2, uint32_t* q, chk_ring& ck, uint32_t lane) {
-    uint32_t leaf = 0;  // the lane's source leaf, resolved once a read of it covers a record
-    // allele | (x2 - x) << 8, for the drains (x2 - x < 2^13)
-    const uint32_t ad = t.allele | ((t.x2 - t.x) << 8);
-    // one drain: entries qb[0 .. count), one per lane
-    auto drain = [&](const uint32_t* qb, uint32_t count) {
-        const bool on = lane < count;
-        const uint32_t qe = on ? qb[lane] : 0u;
-        const uint32_t ol = qe >> 26, mate = (qe >> 25) & 1u, ri = qe & 0x1FFFFFFu;
-        const uint32_t lo = (uint32_t)__shfl((int)leaf, (int)ol);
-        const uint32_t ado = (uint32_t)__shfl((int)ad, (int)ol);
-        const uint32_t al = ado & 0xFFu;
-        const uint32_t xo = (uint32_t)__shfl((int)t.x, (int)ol) + (mate ? ado >> 8 : 0u);  // the read's start
-        const uint32_t in = v.info[ri], p = v.pos[ri];
-        const bool grp = !PSX_INFO_SOLO(in);
-        const uint32_t boff = mate * J.L - xo;  // base index in the template of position p: p + boff
-        if (__ballot(on && grp)) {
-            if (on && grp) count_group(J, v, ri, al, lo, terr{0u, 0u}, boff);
-        }
-        const bool one = on && !grp;
-        const bool car = PSX_INFO_ALLELE(in) == al && carried(J, in, v.lo[ri], v.hi[ri], lo);
-        const bool snv = PSX_INFO_KIND(in) == PSX_SNV;
-        const uint32_t tb = snv && car ? PSX_INFO_ALT(in) : PSX_INFO_REF(in);
-        if (one) {
-            v.add_dep(ri);
-            if (PSX_INFO_HEAD(in) && (snv ? tb == PSX_INFO_ALT(in) : car)) v.add_alt(ri);
-        }
-        const bool chk = J.err_n && on && (grp || (snv && PSX_INFO_HEAD(in)));  // no errors: nothing to check
-        const unsigned long long m = __ballot(chk);
-        if (m) {
-            const uint32_t rank =
-                __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            const uint32_t ro = (uint32_t)__shfl((int)rr, (int)ol);  // the entry's template
-            if (chk) {
-                uint32_t* slot = ck.e + ((ck.head + ck.count + rank) & 127u) * 3u;
-                slot[0] = ro;
-                slot[1] = (p + boff) | (al << 13) | (ri << 21);
-                slot[2] = lo;
-            }
-            ck.count += (uint32_t)__popcll(m);
-        }
-    };
-    uint32_t qn = 0;  // wave-uniform
-    // one walk over both reads of the lane's template: mate 0's positions, then
-    // mate 1's, each from its bucket start (records before the read are passed
-    // over); p is the position of record i, prev that of the record before it
-    const uint32_t e0 = t.x + J.L, e1 = t.x2 + J.L;
-    if (v.n == 0u) return;  // at() needs n > 0
-    uint32_t i = v.start(t.x);
-    const uint32_t j1 = J.pe ? v.start(t.x2) : 0u;
-    uint32_t p = v.pos[v.at(i)];
-    const uint32_t p1 = v.pos[v.at(j1)];
-    const bool go0 = valid && i < v.n && p < e0;
-    const bool go1 = valid && J.pe && j1 < v.n && p1 < e1;
-    if (!__ballot(go0 || go1)) return;
-    if (go0 || go1) leaf = leaf_of(J, S, t);
-    uint32_t mate = go0 ? 0u : 1u, end = go0 ? e0 : e1, x0 = go0 ? t.x : t.x2, prev = 0xFFFFFFFFu;
-    i = go0 ? i : j1;
-    p = go0 ? p : p1;
-    bool go = go0 || go1;
-    while (__ballot(go)) {
-        const uint32_t ic = go ? i : 0u;
-        const bool starts = go && p >= x0 && p != prev;
-        const unsigned long long m = __ballot(starts);
-        const uint32_t below =
-            __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        if (starts) q[qn + below] = (lane << 26) | (mate << 25) | ic;
-        qn += (uint32_t)__popcll(m);
-        i += go ? 1u : 0u;
-        const uint32_t pn = v.pos[v.at(i)];
-        prev = p;
-        go = go && i < v.n && pn < end;
-        p = pn;
-        if (!go && mate == 0u && go1) {  // mate 0 done: continue with mate 1
-            mate = 1u;
-            end = e1;
-            x0 = t.x2;
-            i = j1;
-            p = p1;
-            prev = 0xFFFFFFFFu;
-            go = true;
-        }
-        if (qn >= 64u) {
-            wave_sync();
-            drain(q + qn - 64u, 64u);
-            qn -= 64u;
-            wave_sync();
-            if (ck.count >= 64u) check_errors(J, v, tab, j, c2, ck, 64u, lane);
-        }
-    }
-    if (qn) {
-        wave_sync();
-        drain(q, qn);
-        wave_sync();
-        if (ck.count >= 64u) check_errors(J, v, tab, j, c2, ck, 64u, lane);
-    }
-}
-
 // Stratum geometry shared by both kernels.
 struct stratum {
     uint32_t b, e, wend, k0, n_win;
@@ -896,34 +658,6 @@ __device__ __forceinline__ stratum stratum_of(const job_dev& J, const seg_dev& S
 
 // The segment's first entry of the count arrays.
 __device__ __forceinline__ uint64_t out_off(const job_dev& J, const seg_dev& S) { return (uint64_t)S.so * J.n_mut; }
-
-template <int BLOCK, int CAP>
-__device__ __forceinline__ void stage_window(const job_dev& J, const stratum& s, uint32_t* s_pos, uint32_t* s_lo,
-                                             uint32_t* s_hi, uint32_t* s_info, uint32_t* s_alt, uint32_t* s_dep,
-                                             uint16_t* s_bucket, uint32_t tid) {
-    for (uint32_t i = tid; i < s.n_win; i += BLOCK) {
-        s_pos[i] = J.pos[s.k0 + i];
-        s_lo[i] = J.lo[s.k0 + i];
-        s_hi[i] = J.hi[s.k0 + i];
-        s_info[i] = J.info[s.k0 + i];
-        if (s_alt) {
-            s_alt[i] = 0;
-            s_dep[i] = 0;
-        }
-    }
-    __syncthreads();
-    const uint32_t nb = ((s.wend - s.b) >> NB_SHIFT) + 1;
-    for (uint32_t q = tid; q < nb; q += BLOCK) {
-        const uint32_t target = s.b + (q << NB_SHIFT);
-        uint32_t a = 0, z = s.n_win;
-        while (a < z) {
-            const uint32_t mid = (a + z) >> 1;
-            if (s_pos[mid] < target) a = mid + 1; else z = mid;
-        }
-        s_bucket[q] = (uint16_t)a;
-    }
-    __syncthreads();
-}
 
 // The read kernel's window: only the SNVs of [k0, k0 + n_win) that a read of
 // the segment's output sample can carry (present flags), compacted in table
@@ -978,167 +712,6 @@ __device__ __forceinline__ uint32_t stage_snvs(const job_dev& J, const seg_dev& 
     }
     __syncthreads();
     return n;
-}
-
-// ------------------------------------------------------------ count kernel
-
-// A stratum whose window exceeds the LDS capacity: reads search the global
-// records and count with global atomics (kept out of line so the LDS path's
-// code is shared by both mates).
-template <int BLOCK, bool CNA, class TAB>
-__device__ __forceinline__ void count_stratum_global(const job_dev& J, const seg_dev& S, const TAB& tab,
-                                                  const stratum& s, uint32_t t0, uint32_t nj, uint32_t j, uint32_t c2,
-                                                  uint32_t* list, uint32_t lane, uint32_t wave, uint32_t* acc) {
-    const glb_view v{J.pos + s.k0, J.lo + s.k0, J.hi + s.k0, J.info + s.k0, J.alt + out_off(J, S) + s.k0,
-                     J.depth + out_off(J, S) + s.k0, s.n_win};
-    for (uint32_t base = t0 + wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
-        const uint32_t r = base + lane;
-        bool valid = r < nj;
-        tmpl t = make_template<CNA>(J, S, tab, valid ? r : base, j, s.b, s.e);
-        if (CNA) {
-            valid = valid && t.ok;
-            *acc += valid ? 1u : 0u;
-        }
-        const terr e = J.err_n ? template_errors(J, tab, valid ? r : base, j, c2, valid) : terr{0u, 0u};
-        bool hit = false;  // errors only matter where a read covers a record
-        for (uint32_t mate = 0; mate <= J.pe; ++mate)
-            hit |= count_read(J, S, v, t, e, valid, mate ? t.x2 : t.x, mate);
-        if (J.err_n && hit) count_slow_errors(J, v, tab, t, e, valid, r, j, c2, list, lane);
-    }
-}
-
-// Jobs whose reads cover few positions: errors are checked per covered
-// position (deferred checks, one draw per 64 positions). The others' reads are
-// counted by windows (k_count_dense); both give the same counts. On a 1.6e9-read
-// run the two take the same time where 64 templates cover about 30 positions
-// (19: 5.9 against 6.2 ms; 48: 6.8 by windows). CNA: some job has copy-number
-// events (templates may be rejected and are counted); the plain instantiation
-// carries none of that code. Held to 6 waves per SIMD (80 VGPRs; a few spill).
-template <int BLOCK, int CAP, bool CNA>
-__global__ void __launch_bounds__(BLOCK, 6) k_seq_count(const seq_launch L) {
-    __shared__ uint32_t s_pos[CAP], s_lo[CAP], s_hi[CAP], s_info[CAP], s_alt[CAP], s_dep[CAP];
-    __shared__ uint16_t s_bucket[NB_MAX];
-    __shared__ lds_tables_t<8u> s_tab;  // a 256-entry guide: the LDS also holds the error-check rings
-    __shared__ uint32_t s_run, s_acc;
-    // per wave: the (lane, record) queue of a mate (also a slow template's errors on
-    // the global path), and the deferred error checks
-    __shared__ uint32_t s_wave[BLOCK / 64][ELIST];
-    __shared__ uint32_t s_chk[BLOCK / 64][3 * 128];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    uint32_t in_tab = UNRESOLVED;  // the job whose tables s_tab holds
-    for (uint32_t run = blockIdx.x;;) {
-      const item_run R = run_of(L, run);
-      if (R.first == R.end) break;
-      if (tid == 0) s_run = gridDim.x + (uint32_t)atomicAdd(L.queue, 1ull);  // the block's next run
-      for (uint32_t item = R.first; item < R.end; ++item) {
-        const item_dev it = uniform_at(L.items, item);
-        // the segment's and the job's fields are read where they are used (scalar
-        // loads from the constant address space) instead of being held in SGPRs
-        // all along, which spilled them to VGPR lanes
-        const seg_dev& S = *(const seg_dev*)((const __attribute__((address_space(4))) seg_dev*)L.segs + it.seg);
-        const job_dev& J = *(const job_dev*)((const __attribute__((address_space(4))) job_dev*)L.jobs + S.job);
-        const uint32_t c2 = (S.chr << 16) | S.so;
-        uint32_t acc = 0;  // accepted templates (copy-number events)
-        if (CNA && tid == 0) s_acc = 0;
-        if (in_tab != S.job) {
-            in_tab = S.job;
-            load_tables(J, s_tab, tid, BLOCK);
-        }
-        __syncthreads();
-        for (uint32_t j = it.j0; j < it.j1; ++j) {
-            const stratum s = stratum_of(J, S, j);
-            // the item's part of the stratum's templates
-            const uint32_t share = ((uint32_t)s.nj + seg_parts(S) - 1u) / seg_parts(S);
-            const uint32_t t0 = min((uint32_t)s.nj, it.part * share), nj = min((uint32_t)s.nj, t0 + share);
-            if (s.n_win <= (uint32_t)CAP) {
-                stage_window<BLOCK, CAP>(J, s, s_pos, s_lo, s_hi, s_info, s_alt, s_dep, s_bucket, tid);
-                const lds_view v{s_pos, s_lo, s_hi, s_info, s_alt, s_dep, s_bucket, s.n_win, s.b};
-                chk_ring ck{s_chk[wave], 0u, 0u};
-                if (!CNA) {
-                    for (uint32_t base = t0 + wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
-                        const uint32_t r = base + lane;
-                        const bool valid = r < nj;
-                        tmpl t = make_template<CNA>(J, S, s_tab, valid ? r : base, j, s.b, s.e);
-                        count_mates_wave(J, S, v, s_tab, t, valid, valid ? r : base, j, c2, s_wave[wave], ck, lane);
-                    }
-                } else {
-                    // copy-number draws reject templates: the accepted ones are packed
-                    // into the lanes [0, pc) of a pending set and counted once the next
-                    // group would overflow it, so the walks run on nearly full waves
-                    uint32_t pc = 0;  // wave-uniform
-                    uint32_t px = 0, pad = 0, pleaf = 0, pr = 0;  // x; x2 - x | allele << 13; leaf; index
-                    auto flush = [&]() {
-                        const bool on = lane < pc;
-                        tmpl t;
-                        t.x = on ? px : s.b;  // idle lanes keep a start inside the stratum
-                        t.x2 = on ? px + (pad & 0x1FFFu) : s.b;
-                        t.allele = pad >> 13;
-                        t.leaf = pleaf;
-                        t.cell = 0;
-                        t.ok = 1;
-                        count_mates_wave(J, S, v, s_tab, t, on, pr, j, c2, s_wave[wave], ck, lane);
-                        pc = 0;
-                    };
-                    for (uint32_t base = t0 + wave * 64u; base < nj; base += BLOCK) {  // wave-uniform
-                        const uint32_t r = base + lane;
-                        bool valid = r < nj;
-                        tmpl t = make_template<CNA>(J, S, s_tab, valid ? r : base, j, s.b, s.e);
-                        valid = valid && t.ok;
-                        acc += valid ? 1u : 0u;
-                        const unsigned long long m = __ballot(valid);
-                        const uint32_t n = (uint32_t)__popcll(m);
-                        if (pc + n > 64u) flush();
-                        // a permutation of the lanes: accepted ones to [pc, pc + n) in lane
-                        // order, the others to the remaining lanes
-                        const uint32_t below =
-                            __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                        const uint32_t dst = valid ? pc + below : (pc + n + (lane - below)) & 63u;
-                        const int a4 = (int)(dst * 4u);
-                        const uint32_t nx = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)t.x);
-                        const uint32_t nad = (uint32_t)__builtin_amdgcn_ds_permute(
-                            a4, (int)((t.x2 - t.x) | (t.allele << 13)));
-                        const uint32_t nleaf = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)t.leaf);
-                        const uint32_t nr = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)r);
-                        const bool recv = lane >= pc && lane < pc + n;
-                        px = recv ? nx : px;
-                        pad = recv ? nad : pad;
-                        pleaf = recv ? nleaf : pleaf;
-                        pr = recv ? nr : pr;
-                        pc += n;
-                        if (pc == 64u) flush();
-                    }
-                    if (pc) flush();
-                }
-                if (J.err_n && ck.count) check_errors(J, v, s_tab, j, c2, ck, ck.count, lane);
-                __syncthreads();
-                int32_t* ga = J.alt + out_off(J, S) + s.k0;
-                int32_t* gd = J.depth + out_off(J, S) + s.k0;
-                for (uint32_t i = tid; i < s.n_win; i += BLOCK) {
-                    const uint32_t d = s_dep[i];
-                    if (d) {
-                        atomicAdd(&gd[i], (int32_t)d);
-                        const uint32_t a = s_alt[i];
-                        if (a) atomicAdd(&ga[i], (int32_t)a);
-                    }
-                }
-                __syncthreads();
-            } else {
-                count_stratum_global<BLOCK, CNA>(J, S, s_tab, s, t0, nj, j, c2, s_wave[wave], lane, wave, &acc);
-                __syncthreads();  // s_tab may be reloaded next
-            }
-        }
-        if (CNA && S.n_cna) {
-            if (acc) atomicAdd(&s_acc, acc);
-            __syncthreads();
-            if (tid == 0 && s_acc) atomicAdd(J.acc, (unsigned long long)s_acc * (J.pe + 1u));
-            __syncthreads();
-        }
-      }
-      __syncthreads();
-      run = __builtin_amdgcn_readfirstlane(s_run);
-      __syncthreads();  // read by every wave before it is written again
-    }
 }
 
 // Presence (the sample holds the mutation) and zeroed counters; also resets
@@ -1450,7 +1023,7 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
                 if (n_t == 0) continue;
                 const bool valid = lane < n_t;
                 const uint32_t tr0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)tr);  // lane 0 holds a template
-                const terr te = J.err_n ? template_errors(J, s_tab, valid ? tr : tr0, j, c2, valid) : terr{0u, 0u};
+                const terr te = J.err_n ? template_errors(J, J.seed, s_tab.err, valid ? tr : tr0, j, c2, valid) : terr{0u, 0u};
                 for (uint32_t p = 0; p < rpt; ++p) {
                     const uint32_t src = p * tpp + lane / rpt;
                     const uint32_t mate = lane & (rpt - 1u);
