@@ -108,3 +108,36 @@ def test_id_signatures_through_the_engine(ctx):
     assert {"ID1", "ID8"} <= causes and {"SBS1", "SBS5"} & causes
     with pytest.raises(ValueError, match='Unknown ID signature "ID9"'):
         eng.place_mutations(sf, 0, 2, seed=1, preneoplastic_indel_signature_name="ID9")
+
+
+@pytest.mark.parametrize("n_indels", [1, 3, 63, 65, 300])
+def test_searches_of_rare_classes_share_a_wave(ctx, n_indels):
+    """Indels whose class is found by rejection after hundreds of tries (the
+    rarest classes that are not listed), one to many of them in a wave, alone
+    and among the jobs of a batch whose waves hold several jobs, with and
+    without the infinite-sites redraws: every table is the oracle's."""
+    rng = np.random.default_rng(31)
+    ref, _ = genome(rng)
+    lens, packed = ref.lengths, ref.packed
+    g = core.Genome(ctx, lens, packed=packed)
+    ix = O.id_index(lens, packed)
+    dense = np.nonzero(~ix["listed"].astype(bool) & (ix["counts"] > 0))[0]
+    rare = dense[np.argsort(ix["counts"][dense])[:3]]
+    sig = np.zeros((1, A.PSX_ID_CLASSES))
+    sig[0, rare] = 1.0 / len(rare)
+    fs, es, seeds = [], [], []
+    for k in range(4):
+        fd = cases.forest(n_cells=60 + 20 * k, n_samples=1, sample_size=20, seed=40 + k)
+        of = O.Forest(fd["cell_id"], fd["parent"], fd["species"], fd["sample"], fd["birth"], fd["n_samples"])
+        f = core.Forest(ctx, fd["cell_id"], fd["parent"], fd["species"], fd["sample"], fd["birth"], fd["n_samples"])
+        eng = cases.engine(packed, lens, snv=2e-7, indel=1e-6, pre_snv=k, pre_indel=n_indels, infinite_sites=k != 2)
+        eng.update(id_sig=sig, id_exposure=[[1.0], [1.0]], pre_id=0)
+        fs.append((f, of))
+        es.append(eng)
+        seeds.append(70 + k)
+    batch = core.Mutations.place_batch(ctx, g, [f for f, _ in fs], seeds, es)
+    for k, ((f, of), eng, sd) in enumerate(zip(fs, es, seeds)):
+        om = O.place_mutations(lens, packed, of, sd, **eng)
+        assert (om["kind"] != A.PSX_SNV).sum() >= n_indels
+        assert batch[k].download().tobytes() == om.tobytes(), k
+        assert core.Mutations.place(ctx, g, f, sd, **eng).download().tobytes() == om.tobytes(), k
