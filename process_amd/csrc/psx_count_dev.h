@@ -181,6 +181,31 @@ __device__ __forceinline__ void wave_share(const seg_dev& S, uint32_t part, uint
     }
 }
 
+// The descriptor a wave-uniform pointer argument names, read with scalar loads.
+template <class T>
+__device__ __forceinline__ const T& uniform_ref(const T* p) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(const T*)(const __attribute__((address_space(4))) T*)((uint64_t)hi << 32 | lo);
+#else
+    return *(const T*)(uintptr_t)((uint64_t)hi << 32 | lo);
+#endif
+}
+
+// A template of any ploidy and any copy-number events; out of line, so that its registers are not the loops'.
+struct general_draw {
+    uint32_t x, cell, allele, ins;  // allele | (kept) << 8
+};
+template <bool CNA>
+__device__ __attribute__((noinline)) general_draw draw_general(const job_dev* J, const seg_dev* S, uint32_t r, uint32_t j,
+                                                               uint32_t b, uint32_t e) {
+    psx_u4 w;
+    const tmpl t = template_source<CNA, false>(uniform_ref(J), uniform_ref(S), r, j, b, e, w);
+    return general_draw{t.x, t.cell, t.allele | t.ok << 8, w.w};
+}
+
 // What a segment's template draws use, read once per item. A diploid source
 // without copy-number events is drawn here, any other by template_source.
 struct source_draw {
@@ -191,15 +216,21 @@ struct source_draw {
         : n_cells(S.n_cells), copies(S.n_cells ? 2u * S.n_cells : 2u), normal_below((uint32_t)(J.thr_normal - 1u)),
           starts_end(S.len - J.L), RL(J.L), ins_past((int)J.ins_k0 - (int)J.L),
           diploid(J.ploidy == 2u && !(cna && S.n_cna != 0u)), normal_some(S.n_cells != 0u && J.thr_normal != 0u) {}
-    // Template r of stratum j = [b, e): start in the window that begins at wb, mate 2's offset, source cell (n_cells: the
-    // normal genome) and allele; false when a copy-number draw rejects it.
+    // Template r of stratum j = [b, e): start in the window that begins at wb, source cell (n_cells: the normal genome)
+    // and allele, and the word that gives its insert size; false when a copy-number draw rejects it. cw: the window's
+    // n_ev copy-number events (CN_GENERAL: none listed).
     template <bool CNA>
-    __device__ __forceinline__ bool draw(const job_dev& J, const seg_dev& S, const count_tables& tab, uint32_t r, uint32_t j,
-                                         uint32_t c2, uint32_t b, uint32_t e, uint32_t wb, uint32_t& x, uint32_t& d,
-                                         uint32_t& cell, uint32_t& al) const {
+    __device__ __forceinline__ bool draw(const job_dev& J, const seg_dev& S, const cn_window* cw, uint32_t n_ev, uint32_t r,
+                                         uint32_t j, uint32_t c2, uint32_t b, uint32_t e, uint32_t wb, uint32_t& x,
+                                         uint32_t& ins, uint32_t& cell, uint32_t& al) const {
         psx_u4 w;
         bool ok = true;
-        if (diploid) {
+        if (CNA && n_ev != CN_GENERAL) {
+            w = psx_draw_u(J.seed, r, j, c2, PSX_P_TEMPLATE << 24);
+            x = b + psx_uniform32(w.x, e - b);
+            ok = cn_source(S, *cw, n_ev, normal_some && w.y <= normal_below, w.z, x, cell, al);
+            x -= wb;
+        } else if (diploid) {
             w = psx_draw_u(J.seed, r, j, c2, PSX_P_TEMPLATE << 24);
             x = b - wb + psx_uniform32(w.x, e - b);
             uint32_t v = psx_uniform32(w.z, copies);
@@ -211,18 +242,55 @@ struct source_draw {
             }
             al = v & 1u;
         } else {
-            const tmpl t = template_source<CNA, false>(J, S, r, j, b, e, w);
+            const general_draw t = draw_general<CNA>(&J, &S, r, j, b, e);
             x = t.x - wb;
             cell = t.cell;
-            al = t.allele;
-            if (CNA) ok = t.ok != 0u;
+            al = t.allele & 0xFFu;
+            ok = (t.allele >> 8) != 0u;
+            w.w = t.ins;
         }
-        d = 0;
-        if (J.pe) {
-            const int I = (int)pick_insert(tab, w.w) + ins_past;
-            d = min((uint32_t)max(I, 0), starts_end - wb - x);
-        }
+        ins = w.w;
         return ok;
+    }
+    // Mate 2's offset from the start.
+    __device__ __forceinline__ uint32_t offset(const job_dev& J, const count_tables& tab, uint32_t ins, uint32_t wb,
+                                               uint32_t x) const {
+        if (!J.pe) return 0;
+        const int I = (int)pick_insert(tab, ins) + ins_past;
+        return min((uint32_t)max(I, 0), starts_end - wb - x);
+    }
+};
+
+// Copy-number draws reject templates: the accepted ones are packed into the lanes of a pending set, which takes the
+// place of a group when the next would overflow it (and at the end).
+struct pending {
+    uint32_t n = 0, x = 0, ins = 0, copy = 0, r = 0;
+    // The group's values (of the lanes that are on) go in; true: the set's come out, of its first lanes, and x is 0 in
+    // the others.
+    __device__ __forceinline__ bool pack(bool more, bool& on, uint32_t lane, uint32_t& gx, uint32_t& gi, uint32_t& gc,
+                                         uint32_t& gr) {
+        const unsigned long long m = __ballot(on);
+        const uint32_t k = (uint32_t)__popcll(m), had = n;
+        const bool out = n + k > 64u || !more;
+        const uint32_t at = out ? 0u : n;
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        const int to = (int)((on ? at + below : (at + k + (lane - below)) & 63u) * 4u);
+        const uint32_t nx = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)gx);
+        const uint32_t ni = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)gi);
+        const uint32_t nc = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)gc);
+        const uint32_t nr = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)gr);
+        on = out && lane < had;
+        gx = on ? x : 0u;
+        gi = ins;
+        gc = copy;
+        gr = on ? r : (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
+        const bool recv = lane - at < k;
+        x = recv ? nx : x;
+        ins = recv ? ni : ins;
+        copy = recv ? nc : copy;
+        r = recv ? nr : r;
+        n = at + k;
+        return out && had != 0u;
     }
 };
 
@@ -383,6 +451,7 @@ template <int BLOCK, int CAP, bool CNA>
 __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
     using LDS = sparse_lds<BLOCK, CAP>;
     __shared__ LDS lds;
+    __shared__ cn_window s_cn;  // copy numbers
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     sparse_read* const queue = lds.queue[wave];
@@ -416,6 +485,7 @@ __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
                 const uint32_t k0 = uniform_at(J.bucket, S.bucket_off + jw);
                 const uint32_t n_win = window_records(J, S, k0, wend);
                 const uint32_t n_lds = n_win <= (uint32_t)CAP ? n_win : 0u;
+                if (CNA && S.n_cna && wave == 0) cn_fill(J, S, wb, starts, lane, s_cn);
                 // the records, and the starts from which a read reaches one
                 for (uint32_t i = tid; i < n_win; i += BLOCK) {
                     const uint32_t p = J.pos[k0 + i] - wb;
@@ -433,11 +503,13 @@ __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
                 uint32_t t0 = 0, t1 = 0;
                 if (j < je) wave_share(S, it.part, b, e, lane, t0, t1);
                 uint32_t qn = 0;
+                const uint32_t n_ev = CNA && S.n_cna ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s_cn.n) : CN_GENERAL;
                 for (uint32_t g = t0 + slot * 64u; g < t1; g += nslot * 64u) {  // wave-uniform
                     bool on = g + lane < t1;
                     const uint32_t r = on ? g + lane : g;
-                    uint32_t x, d, cell, al;
-                    on = D.draw<CNA>(J, S, lds.tab, r, j, c2, b, e, wb, x, d, cell, al) && on;
+                    uint32_t x, ins, cell, al;
+                    on = D.draw<CNA>(J, S, &s_cn, n_ev, r, j, c2, b, e, wb, x, ins, cell, al) && on;
+                    const uint32_t d = D.offset(J, lds.tab, ins, wb, x);
                     if (CNA) acc += (uint32_t)__popcll(__ballot(on));
                     for (uint32_t m = 0; m <= pe; ++m) {
                         const uint32_t xm = m ? x + d : x;
@@ -521,6 +593,7 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
     __shared__ uint32_t s_run, s_acc, s_neff, s_todo_n[2];
     __shared__ uint32_t s_list[DENSE_WAVES][ELIST];  // per wave: a slow template's errors
     __shared__ todo s_todo[TODO_CAP];
+    __shared__ cn_window s_cn;  // copy numbers
     uint32_t* const s_bits = (uint32_t*)s_dyn;
     uint32_t* const s_bin = s_bits + L.bit_words;
     uint32_t* const s_cnt = s_bin + L.bins * BIN_STRIDE;  // two sets: one fills while the other is cleared
@@ -561,6 +634,12 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                     for (uint32_t i = tid; i < (wend - wb + 31u) >> 5; i += DENSE_BLOCK) s_bits[i] = 0;
                 for (uint32_t i = tid; i < L.bins; i += DENSE_BLOCK) s_cnt[i] = 0;
                 if (tid == 0) s_neff = s_todo_n[0] = 0;
+                if (CNA && S.n_cna && wave == 0) {
+                    const uint32_t starts = min(je * PSX_STRATUM, S.W);
+                    cn_fill(J, S, wb, starts, lane, s_cn);
+                    wave_sync();
+                    cn_share(J, S, wb, starts, lane, s_cn);
+                }
                 __syncthreads();
                 for (uint32_t i0 = 0; i0 < n_win; i0 += DENSE_BLOCK) {
                     const uint32_t i = i0 + tid;
@@ -578,63 +657,50 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                 const uint32_t sub = tid & ((1u << lgt) - 1u), step = 1u << lgt;
                 const uint32_t per_pass = DENSE_BLOCK >> lgt;
                 const bool one_pass = n_rec <= per_pass;
+                const uint32_t n_ev = CNA && S.n_cna ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s_cn.n) : CN_GENERAL;
                 // the wave's stratum: its templates [t0, t1)
                 const uint32_t j = jw + wave / nslot;
                 const uint32_t b = j * PSX_STRATUM, e = min(b + PSX_STRATUM, S.W);
                 uint32_t t0 = 0, t1 = 0;
                 if (j < je) wave_share(S, it.part, b, e, lane, t0, t1);
                 // rounds: the same number for every wave, from a bound on any stratum's share
-                const uint32_t most = S.most, round_t = S.round_t;
+                const uint32_t most = S.most;
+                uint32_t round_t = S.round_t;
+                if (CNA && S.n_cna) {
+                    // of a round's templates only a share has reads: rounds of more templates, as many in each
+                    const uint32_t fit = __float2uint_rz(fminf((float)round_t * 1024.0f /
+                                                               (float)__builtin_amdgcn_readfirstlane((int)s_cn.share),
+                                                               (float)most));
+                    const uint32_t rounds = (most + fit - 1u) / max(fit, 1u);
+                    round_t = ((most + rounds - 1u) / max(rounds, 1u) + 63u) & ~63u;
+                }
                 scan_rec R{0, 0, 0, REC_NONE};
                 uint32_t dep = 0, alt = 0, set = 0;
                 for (uint32_t q0 = 0; q0 < most; q0 += round_t) {
                     uint32_t* const cnt = s_cnt + set * L.bins;
                     // ---- draw the round's templates, drop their reads into bins
-                    uint32_t pc = 0, px = 0, pd = 0, pX = 0, pr = 0;  // copy numbers: pending accepted templates
+                    pending P;  // copy numbers: accepted templates
                     const uint32_t end = min(t0 + q0 + round_t, t1);
                     for (uint32_t g = t0 + q0 + slot * 64u;; g += nslot * 64u) {  // wave-uniform
                         const bool more = g < end;
                         bool have = more, on = false;
-                        uint32_t x = 0, d = 0, X = 0, r = g;  // start in the window, mate 2's offset, copy, index
+                        uint32_t x = 0, ins = 0, X = 0, r = g;  // start in the window, insert draw, copy, index
                         if (more) {
                             on = g + lane < end;
                             r = on ? g + lane : g;
                             uint32_t cell, al;
-                            const bool ok = D.draw<CNA>(J, S, s_tab, r, j, c2, b, e, wb, x, d, cell, al);
+                            const bool ok = D.draw<CNA>(J, S, &s_cn, n_ev, r, j, c2, b, e, wb, x, ins, cell, al);
                             X = (al << cb) | cell;
                             if (CNA) on = on && ok;
                         }
                         if (CNA) {
-                            // copy-number draws reject templates: the accepted ones are packed into the lanes of a
-                            // pending set, counted when the next group would overflow it (and at the end)
                             acc += on ? 1u : 0u;
-                            const unsigned long long m = __ballot(on);
-                            const uint32_t n = (uint32_t)__popcll(m);
-                            const uint32_t cx = px, cd = pd, cX = pX, cr = pr, cn = pc;
-                            have = pc + n > 64u || (!more && pc);
-                            pc = have ? 0u : pc;
-                            const uint32_t below =
-                                __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                            const int a4 = (int)((on ? pc + below : (pc + n + (lane - below)) & 63u) * 4u);
-                            const uint32_t nx = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)x);
-                            const uint32_t nd = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)d);
-                            const uint32_t nX = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)X);
-                            const uint32_t nr = (uint32_t)__builtin_amdgcn_ds_permute(a4, (int)r);
-                            const bool recv = lane >= pc && lane < pc + n;
-                            px = recv ? nx : px;
-                            pd = recv ? nd : pd;
-                            pX = recv ? nX : pX;
-                            pr = recv ? nr : pr;
-                            pc += n;
-                            on = have && lane < cn;
-                            x = on ? cx : 0u;
-                            d = on ? cd : 0u;
-                            X = cX;
-                            r = on ? cr : (uint32_t)__builtin_amdgcn_readfirstlane((int)cr);
+                            have = P.pack(more, on, lane, x, ins, X, r);
                         }
                         uint32_t ev = 0;  // the lane's rare events: full bins (bits 0, 1), errors at records (2, 3, 4)
                         uint32_t P0 = 0, P1 = 0, P2 = 0, subs = 0;
                         unsigned long long slow = 0;
+                        const uint32_t d = have ? D.offset(J, s_tab, ins, wb, x) : 0u;
                         if (have) {
                             auto put = [&](uint32_t xr) {  // whether the bin is full
                                 const uint32_t bin = xr >> lw;

@@ -719,11 +719,16 @@ namespace {
 // of those strata's first reads; after it (finish) the kept templates of each
 // stratum are counted (k_cn_accept), every segment's first read and each such
 // stratum's first read are set in output order, and the segments are
-// uploaded again. Without events nothing changes.
+// uploaded again. With masks, k_cn_accept also leaves a bit per template, and
+// such a segment's descriptor has the index of its first mask word in place of
+// its first read. Without events nothing changes.
 struct cn_rows {
-    dbuf buf;                    // kept | first read (uint64 per stratum) | segment list | first strata
+    dbuf buf;                    // kept | first read (uint64 per stratum) | first masks | masks | segment list | first strata
     std::vector<uint32_t> seg, first;
-    uint64_t n = 0;
+    std::vector<uint64_t> mask;  // per segment with events: its first mask word (empty: no masks)
+    uint64_t n = 0, n_mask = 0;
+    explicit cn_rows(bool masks) : masks_(masks) {}
+    const uint64_t* kept_masks() const { return masks_ && n ? buf.as<uint64_t>() + 2 * n + mask.size() : nullptr; }
     std::vector<uint64_t> seg_reads;  // reads of each segment (finish)
     bool prepare(seq_batch& P) {
         seg_dev* hs = (seg_dev*)(P.sb.host.data() + P.o_segs);
@@ -734,22 +739,32 @@ struct cn_rows {
                 seg.push_back(k);
                 n += hs[k].J;
                 first.push_back((uint32_t)n);
+                if (masks_) {
+                    mask.push_back(n_mask);
+                    // templates_below(S, a stratum), the largest share less one
+                    const uint64_t most = (uint64_t)((unsigned __int128)hs[k].T * std::min(PSX_STRATUM, hs[k].W) / hs[k].W);
+                    n_mask += (uint64_t)hs[k].J * (most + 64u >> 6);
+                }
             }
         if (!n) return false;
         if (n >= (uint64_t(1) << 32)) psx_throw(PSX_EINVAL, "too many strata with copy-number events");
-        buf.alloc(16 * n + 4 * (seg.size() + first.size()) + 256);
+        buf.alloc(16 * n + 8 * (mask.size() + n_mask) + 4 * (seg.size() + first.size()) + 256);
         job_dev* hj = (job_dev*)(P.sb.host.data() + P.o_jobs);
         for (size_t k = 0; k < P.jobs.size(); ++k) hj[k].cn_row = buf.as<uint64_t>() + n;
         return true;
     }
     void finish(psx_ctx* ctx, seq_batch& P, const seq_lane& lane) {
         uint64_t* d_kept = buf.as<uint64_t>();
-        uint32_t* d_seg = (uint32_t*)(d_kept + 2 * n);
+        uint64_t* d_mask_first = d_kept + 2 * n;
+        uint64_t* d_mask = d_mask_first + mask.size();
+        uint32_t* d_seg = (uint32_t*)(d_mask + n_mask);
         uint32_t* d_first = d_seg + seg.size();
         PSX_HIP(hipMemcpyAsync(d_seg, seg.data(), 4 * seg.size(), hipMemcpyHostToDevice, lane.stream));
         PSX_HIP(hipMemcpyAsync(d_first, first.data(), 4 * first.size(), hipMemcpyHostToDevice, lane.stream));
         psxk::accept_args a{(const job_dev*)(lane.desc + P.o_jobs), (const seg_dev*)(lane.desc + P.o_segs), d_seg,
-                            d_first, (uint32_t)seg.size(), d_kept};
+                            d_first, (uint32_t)seg.size(), d_kept, d_mask, masks_ ? d_mask_first : nullptr};
+        if (masks_)
+            PSX_HIP(hipMemcpyAsync(d_mask_first, mask.data(), 8 * mask.size(), hipMemcpyHostToDevice, lane.stream));
         hipLaunchKernelGGL(psxk::k_cn_accept, dim3((uint32_t)((n + 3) / 4)), dim3(256), 0, lane.stream, a);
         PSX_HIP(hipGetLastError());
         std::vector<uint64_t> kept(n), row(n);
@@ -783,11 +798,15 @@ struct cn_rows {
             P.job_reads[S.job] += reads;
         }
         P.n_reads = at;
+        for (size_t k = 0; k < mask.size(); ++k) hs[seg[k]].read_base = mask[k];
         PSX_HIP(hipMemcpyAsync(d_kept + n, row.data(), 8 * n, hipMemcpyHostToDevice, lane.stream));
         PSX_HIP(hipMemcpyAsync(lane.desc + P.o_segs, hs, sizeof(seg_dev) * P.segs.size(), hipMemcpyHostToDevice,
                                lane.stream));
         PSX_HIP(hipStreamSynchronize(lane.stream));  // the host arrays above go out of scope
     }
+
+private:
+    bool masks_;
 };
 
 // Read materialisation of jobs in one persistent launch: job k's reads start
@@ -813,7 +832,7 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
     }
     std::unique_ptr<seq_batch, void (*)(seq_batch*)> B(batch_prepare(ctx, in.data(), in.size(), 1, false, false), batch_free);
     seq_batch& P = *B;
-    cn_rows cn;
+    cn_rows cn(true);
     const bool with_cn = cn.prepare(P);
     // presence flags per (output sample, mutation): the read kernel stages
     // only the SNVs a read of the sample can carry. Kernels index a job's
@@ -845,6 +864,7 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
                            (uint32_t)P.pres.size(), P.pres_total);
     }
     L.reads_out = d_reads;
+    L.cn_kept = cn.kept_masks();
     L.read_words = rw;
     L.out_vec4 = (L.read_words % 4 == 0 && ((uintptr_t)d_reads & 15) == 0) ? 1u : 0u;
     // 64 rows of read_words words per wave staged in LDS; the block is the
@@ -889,7 +909,7 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
 std::vector<uint64_t> psxh::segment_reads(psx_ctx* ctx, const job_in& in) {
     std::unique_ptr<seq_batch, void (*)(seq_batch*)> B(batch_prepare(ctx, &in, 1, 1, false, false), batch_free);
     seq_batch& P = *B;
-    cn_rows cn;
+    cn_rows cn(false);
     if (cn.prepare(P)) {
         const seq_lane lane = ctx_lane(ctx, batch_desc_bytes(&P));
         batch_upload(&P, lane);

@@ -139,6 +139,7 @@ struct seq_launch {
     uint32_t* reads_out;     // materialisation only
     uint32_t read_words;
     uint32_t out_vec4;       // read_words % 4 == 0 and reads_out 16-byte aligned
+    const uint64_t* cn_kept; // segments with copy-number events: which templates are kept (cn_groups words a stratum)
 };
 
 // The items of a persistent launch are handed out in runs of L.chunk: block b
@@ -267,41 +268,122 @@ __device__ __forceinline__ uint32_t cna_copies(const psx_cna_dev* ev, uint32_t n
     return total;
 }
 
-// cna_copies for ploidy 2: copies of lineage 0 | lineage 1 << 16 (copy
-// numbers stay below 2^16: the host bounds them by the largest copy number).
-__device__ __forceinline__ uint32_t cna_copies2(const psx_cna_dev* ev, uint32_t n, uint32_t leaf, uint32_t x) {
-    uint32_t c0 = 1u, c1 = 1u;
-    for (uint32_t i = 0; i < n; ++i) {
-        const psx_cna_dev e = uniform_at(ev, i);
-        const bool hit = leaf >= e.lo && leaf < e.hi && x >= e.start && x < e.end;
-        const uint32_t a = e.code & 0xFFu, kind = (e.code >> 8) & 0xFFu, c = e.code >> 16;
-        uint32_t n0, n1;
-        if (kind == PSX_CNA_WGD) {  // uniform branches: the event is the same for every lane
-            n0 = 2u * c0;
-            n1 = 2u * c1;
-        } else if (kind == PSX_CNA_AMP) {
-            n0 = a == 0u ? c0 + c : c0;
-            n1 = a == 1u ? c1 + c : c1;
-        } else {
-            n0 = a == 0u ? 0u : c0;
-            n1 = a == 1u ? 0u : c1;
-        }
-        c0 = hit ? n0 : c0;
-        c1 = hit ? n1 : c1;
-    }
-    return c0 | (c1 << 16);
-}
-
-__device__ __forceinline__ uint32_t leaf_of(const job_dev& J, const seg_dev& S, tmpl& t) {
-    if (t.leaf == UNRESOLVED) t.leaf = J.sample_leaves[S.leaf_off + t.cell];
-    return t.leaf;
-}
-
 // Cells of the sample with leaf ranks below x, from the sample's running counts.
 __device__ __forceinline__ uint32_t cells_below(const job_dev& J, uint32_t sample, uint32_t x) {
     const uint4 e = J.leaf_count[(uint64_t)sample * J.leaf_blocks + (x >> 6)];
     const uint64_t bits = (uint64_t)e.y | ((uint64_t)e.z << 32);
     return e.x + (uint32_t)__popcll(bits & ((1ull << (x & 63u)) - 1ull));
+}
+
+// The copy-number events of a diploid segment that touch a window of starts,
+// with their leaf ranges as ranges of the sample's cells: [cell, cell + cells),
+// [start, start + starts), and what they do to the packed copies of the two
+// lineages, ((C & keep) << twice) + add. A template needs no look-up of its
+// leaf and no division, and walks the events of its window alone, in LDS: the
+// counts of 3.3e8 templates of 9e8 draws (500x, 13 events on 10 chromosomes)
+// 4.8 -> 4.1 ms. Bound by vector instruction issue: 120 instructions a group of
+// 64 draws, 43 of them Philox, and 6 for each read queued.
+struct cn_event {
+    uint32_t cell, cells, start, starts;
+    uint32_t keep, twice, add, pad;
+};
+constexpr uint32_t CN_EVENTS = 16;
+constexpr uint32_t CN_DOUBLINGS = 3;  // an event adds at most 255: (1 + 16 * 255) << 3 < 2^16, no lineage overflows its half
+struct cn_window {
+    cn_event ev[CN_EVENTS];
+    uint32_t n;
+    uint32_t share;  // about the largest share of the templates, of any quarter of the window, that is kept, times 2^10
+};
+constexpr uint32_t CN_GENERAL = 0xFFFFFFFFu;  // not in this form: drawn by template_source
+
+// One wave fills w with the events of S that touch the starts [b, e).
+__device__ __forceinline__ void cn_fill(const job_dev& J, const seg_dev& S, uint32_t b, uint32_t e, uint32_t lane,
+                                        cn_window& w) {
+    uint32_t n = 0, doubled = 0;
+    const bool general = J.ploidy != 2u;
+    for (uint32_t i0 = 0; S.n_cells && i0 < S.n_cna; i0 += 64u) {
+        const uint32_t i = i0 + lane;
+        cn_event q{};
+        uint32_t kind = 0;
+        bool on = i < S.n_cna;
+        if (on) {
+            const psx_cna_dev d = J.cna[S.cna_off + i];
+            const uint32_t a = d.code & 0xFFu;
+            kind = (d.code >> 8) & 0xFFu;
+            const uint32_t c = kind == PSX_CNA_AMP ? d.code >> 16 : 0u;
+            q.cell = cells_below(J, S.sample, d.lo);
+            q.cells = cells_below(J, S.sample, d.hi) - q.cell;
+            q.start = d.start;
+            q.starts = d.end - d.start;
+            q.keep = kind == PSX_CNA_DEL ? (a == 0u ? 0xFFFF0000u : 0xFFFFu) : 0xFFFFFFFFu;
+            q.twice = kind == PSX_CNA_WGD ? 1u : 0u;
+            q.add = a == 0u ? c : c << 16;
+            on = d.start < e && d.end > b && q.cells != 0u;
+        }
+        const unsigned long long m = __ballot(on);
+        const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (on && at < CN_EVENTS) w.ev[at] = q;
+        n += (uint32_t)__popcll(m);
+        doubled += (uint32_t)__popcll(__ballot(on && kind == PSX_CNA_WGD));
+    }
+    if (lane == 0) w.n = general || n > CN_EVENTS || doubled > CN_DOUBLINGS ? CN_GENERAL : n;
+}
+
+// The packed copies of a cell at start x.
+__device__ __forceinline__ uint32_t cn_copies(const cn_window& w, uint32_t n_ev, uint32_t cell, uint32_t x) {
+    uint32_t C = 0x10001u;  // lineage 0 | lineage 1 << 16
+    for (uint32_t i = 0; i < n_ev; ++i) {
+        const cn_event& q = w.ev[i];
+        const bool hit = (cell - q.cell < q.cells) & (x - q.start < q.starts);
+        const uint32_t D = ((C & q.keep) << q.twice) + q.add;
+        C = hit ? D : C;
+    }
+    return C;
+}
+
+// The share of templates kept, by one wave after cn_fill: 64 cells in the
+// middle of each quarter of the window. It only sizes the rounds.
+__device__ __forceinline__ void cn_share(const job_dev& J, const seg_dev& S, uint32_t b, uint32_t e, uint32_t lane,
+                                         cn_window& w) {
+    const uint32_t n_ev = (uint32_t)__builtin_amdgcn_readfirstlane((int)w.n);
+    float most = 0.0f;
+    for (uint32_t q = 0; n_ev != CN_GENERAL && q < 4u; ++q) {
+        const uint32_t C = cn_copies(w, n_ev, (uint32_t)(((uint64_t)S.n_cells * (2u * lane + 1u)) >> 7),
+                                     b + (uint32_t)(((uint64_t)(e - b) * (2u * q + 1u)) >> 3));
+        float sum = (float)((C & 0xFFFFu) + (C >> 16));
+        for (uint32_t m = 1; m < 64u; m <<= 1) sum += __shfl_xor(sum, (int)m);
+        most = fmaxf(most, sum);
+    }
+    const float normal = S.n_cells ? (float)J.thr_normal * 0x1p-32f : 1.0f;
+    const float kept = n_ev == CN_GENERAL ? 1.0f : ((1.0f - normal) * most * 0x1p-6f + normal * 2.0f) / (float)S.kmax;
+    if (lane == 0) w.share = (uint32_t)fminf(fmaxf(kept, 0x1p-6f) * 1024.0f, 1024.0f);
+}
+
+// The source of a template that starts at x, from word z of its draw: cell
+// (n_cells: the normal genome) and lineage; whether the drawn slot is one of
+// its copies. The slot X = floor(z cells K / 2^32) belongs to cell
+// floor(X / K) = floor(z cells / 2^32). normal: a tumour sample's template is
+// the normal genome's.
+__device__ __forceinline__ bool cn_source(const seg_dev& S, const cn_window& w, uint32_t n_ev, bool normal, uint32_t z,
+                                          uint32_t x, uint32_t& cell, uint32_t& al) {
+    const uint32_t K = S.kmax, n = S.n_cells;
+    cell = n;
+    if (n == 0u) {  // the normal sample (the same branch for every lane)
+        al = psx_uniform32(z, K);
+        return al < 2u;
+    }
+    const uint32_t c = psx_uniform32(z, normal ? 1u : n);
+    const uint32_t k = psx_uniform32(z, normal ? K : n * K) - c * K;
+    cell = normal ? n : c;
+    const uint32_t C = cn_copies(w, n_ev, cell, x);
+    const uint32_t c0 = C & 0xFFFFu;
+    al = k >= c0 ? 1u : 0u;
+    return k < c0 + (C >> 16);
+}
+
+__device__ __forceinline__ uint32_t leaf_of(const job_dev& J, const seg_dev& S, tmpl& t) {
+    if (t.leaf == UNRESOLVED) t.leaf = J.sample_leaves[S.leaf_off + t.cell];
+    return t.leaf;
 }
 
 __device__ __forceinline__ bool carried(const job_dev& J, uint32_t info, uint32_t lo, uint32_t hi, uint32_t leaf) {
@@ -347,8 +429,8 @@ __device__ __forceinline__ tmpl template_source(const job_dev& J, const seg_dev&
         // a copy of a cell, or of the normal genome (cell n_cells)
         const bool normal = S.n_cells == 0 || (uint64_t)w.y < J.thr_normal;
         const uint32_t X = psx_uniform32(w.z, normal ? J.ploidy : S.n_cells * J.ploidy);
-        if (J.ploidy == 2) { t.cell = X >> 1; t.allele = X & 1u; }
-        else { t.cell = X / J.ploidy; t.allele = X - t.cell * J.ploidy; }
+        t.cell = normal ? 0u : psx_uniform32(w.z, S.n_cells);  // floor(X / ploidy)
+        t.allele = X - t.cell * J.ploidy;
         if (LEAF) {
             t.leaf = J.n_leaves;
             if (!normal) t.leaf = J.sample_leaves[S.leaf_off + t.cell];  // issued early: its latency overlaps the draws
@@ -365,48 +447,97 @@ __device__ __forceinline__ tmpl template_source(const job_dev& J, const seg_dev&
             t.allele = k;
             t.ok = k < J.ploidy;
         } else {
-            const uint32_t X = psx_uniform32(w.z, S.n_cells * K);
-            t.cell = X / K;
-            const uint32_t k = X - t.cell * K;
+            t.cell = psx_uniform32(w.z, S.n_cells);  // floor(floor(z cells K / 2^32) / K)
+            const uint32_t k = psx_uniform32(w.z, S.n_cells * K) - t.cell * K;
             t.leaf = J.sample_leaves[S.leaf_off + t.cell];
-            if (J.ploidy == 2u) {
-                // diploid: the two lineages' copy numbers in two registers
-                const uint32_t C0 = cna_copies2(J.cna + S.cna_off, S.n_cna, t.leaf, t.x);
-                const uint32_t c0 = C0 & 0xFFFFu, c1 = C0 >> 16;
-                t.allele = k >= c0 ? 1u : 0u;
-                t.ok = k < c0 + c1;
-            } else {
-                uint32_t cn[PSX_MAX_CNA_PLOIDY];
-                const uint32_t C = cna_copies(J.cna + S.cna_off, S.n_cna, t.leaf, t.x, J.ploidy, cn);
-                uint32_t cum = 0, al = 0;
+            uint32_t cn[PSX_MAX_CNA_PLOIDY];
+            const uint32_t C = cna_copies(J.cna + S.cna_off, S.n_cna, t.leaf, t.x, J.ploidy, cn);
+            uint32_t cum = 0, al = 0;
 #pragma unroll
-                for (uint32_t a = 0; a < PSX_MAX_CNA_PLOIDY; ++a) {
-                    cum += cn[a];
-                    al += (a + 1 < J.ploidy && k >= cum) ? 1u : 0u;
-                }
-                t.allele = al;
-                t.ok = k < C;
+            for (uint32_t a = 0; a < PSX_MAX_CNA_PLOIDY; ++a) {
+                cum += cn[a];
+                al += (a + 1 < J.ploidy && k >= cum) ? 1u : 0u;
             }
+            t.allele = al;
+            t.ok = k < C;
         }
     }
     t.x2 = t.x;
     return t;
 }
 
-// Template r of stratum j (oracle: the template loop of orc_simulate_seq).
-template <bool CNA = false, class TAB>
+// Start of mate 2 of a template that starts at x, from the insert word of its draw.
+template <class TAB>
+__device__ __forceinline__ uint32_t mate_start(const job_dev& J, const seg_dev& S, const TAB& tab, uint32_t x, uint32_t ins) {
+    if (!J.pe) return x;
+    uint32_t I = J.ins_k0 + guided_pick_u<TAB::GUIDE_BITS>(tab.ins, tab.guide, J.ins_n, ins);
+    if (I < J.L) I = J.L;
+    const uint64_t x2 = (uint64_t)x + I - J.L;
+    return x2 > S.len - J.L ? S.len - J.L : (uint32_t)x2;
+}
+
+// Template r of stratum j of a segment without copy-number events (oracle:
+// the template loop of orc_simulate_seq).
+template <class TAB>
 __device__ __forceinline__ tmpl make_template(const job_dev& J, const seg_dev& S, const TAB& tab, uint32_t r,
                                               uint32_t j, uint32_t b, uint32_t e) {
     psx_u4 w;
-    tmpl t = template_source<CNA>(J, S, r, j, b, e, w);
-    if (J.pe) {
-        uint32_t I = J.ins_k0 + guided_pick_u<TAB::GUIDE_BITS>(tab.ins, tab.guide, J.ins_n, w.w);
-        if (I < J.L) I = J.L;
-        uint64_t x2 = (uint64_t)t.x + I - J.L;
-        if (x2 > S.len - J.L) x2 = S.len - J.L;
-        t.x2 = (uint32_t)x2;
-    }
+    tmpl t = template_source(J, S, r, j, b, e, w);
+    t.x2 = mate_start(J, S, tab, t.x, w.w);
     return t;
+}
+
+// Templates that start below x: floor(T x / W) (T W < 2^64, x <= W) by a
+// double quotient and its exact remainder; a 64-bit integer division is over
+// a hundred instructions.
+__device__ __forceinline__ uint64_t templates_below(const seg_dev& S, uint32_t x) {
+    const uint64_t n = S.T * x, W = S.W;
+    uint64_t q = (uint64_t)((double)n / (double)W);
+    int64_t r = (int64_t)(n - q * W);
+    while (r < 0) {
+        --q;
+        r += (int64_t)W;
+    }
+    while (r >= (int64_t)W) {
+        ++q;
+        r -= (int64_t)W;
+    }
+    return q;
+}
+
+// Whether template r of stratum [b, e) is kept and its draw, start, cell and
+// lineage; a segment with copy-number events.
+__device__ __forceinline__ bool cn_template(const job_dev& J, const seg_dev& S, const cn_window& cw, uint32_t n_ev,
+                                            uint32_t r, uint32_t j, uint32_t b, uint32_t e, psx_u4& w, tmpl& t) {
+    if (n_ev == CN_GENERAL) {
+        t = template_source<true, false>(J, S, r, j, b, e, w);
+        return t.ok != 0u;
+    }
+    w = psx_draw_u(J.seed, r, j, (S.chr << 16) | S.so, PSX_P_TEMPLATE << 24);
+    t.x = b + psx_uniform32(w.x, e - b);
+    return cn_source(S, cw, n_ev, (uint64_t)w.y < J.thr_normal, w.z, t.x, t.cell, t.allele);
+}
+
+// Groups of 64 templates of a segment's strata (the largest of them).
+__device__ __forceinline__ uint32_t cn_groups(const seg_dev& S) {
+    return (uint32_t)((templates_below(S, min(PSX_STRATUM, S.W)) + 64u) >> 6);
+}
+constexpr uint32_t CN_CHUNK = 256;  // groups whose kept templates a block of the read kernel numbers at a time
+
+// Position of set bit n of m (n < the number of set bits).
+__device__ __forceinline__ uint32_t nth_set(uint64_t m, uint32_t n) {
+    uint32_t w = (uint32_t)m, at = 0;
+    const uint32_t c = (uint32_t)__popc(w);
+    if (n >= c) { n -= c; w = (uint32_t)(m >> 32); at = 32; }
+#pragma unroll
+    for (uint32_t s = 16; s; s >>= 1) {
+        const uint32_t k = (uint32_t)__popc(w & ((1u << s) - 1u));
+        const bool up = n >= k;
+        n -= up ? k : 0u;
+        w >>= up ? s : 0u;
+        at += up ? s : 0u;
+    }
+    return at;
 }
 
 // Sequencing errors of a template (oracle: template_errors). Most templates
@@ -618,24 +749,6 @@ struct stratum {
     uint32_t b, e, wend, k0, n_win;
     uint64_t nj, before;
 };
-
-// Templates that start below x: floor(T x / W) (T W < 2^64, x <= W) by a
-// double quotient and its exact remainder; a 64-bit integer division is over
-// a hundred instructions.
-__device__ __forceinline__ uint64_t templates_below(const seg_dev& S, uint32_t x) {
-    const uint64_t n = S.T * x, W = S.W;
-    uint64_t q = (uint64_t)((double)n / (double)W);
-    int64_t r = (int64_t)(n - q * W);
-    while (r < 0) {
-        --q;
-        r += (int64_t)W;
-    }
-    while (r >= (int64_t)W) {
-        ++q;
-        r -= (int64_t)W;
-    }
-    return q;
-}
 
 // Records of the stratum index from stratum j's first to the last that a read
 // below wend can reach (up to the end of wend's stratum).
@@ -899,7 +1012,9 @@ __device__ __forceinline__ void apply_error(uint32_t* row, uint32_t o, uint32_t 
 // their source (their reads from J.cn_row on); the others as without. The
 // 512-thread forms are held to 80 VGPRs (the copy-number one spills two), so
 // that 3 blocks run per CU instead of 2: 5e7 single-end 100 bp reads 737 ->
-// 615 us, 2.7e7 reads with copy numbers 1290 -> 1100 us.
+// 615 us. Reads with copy numbers (2.7e7 of 3.3e7 templates' draws): a lane
+// per draw, the kept ones packed between two barriers, 1,100 us; a lane per
+// kept template, numbered by the bits of the pass that counts them, 450 us.
 template <int BLOCK, int CAP, bool STAGE, int NW, bool CNA = false>
 __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const seq_launch L) {
     constexpr uint32_t WAVES = BLOCK / 64;
@@ -910,7 +1025,9 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
     __shared__ uint32_t s_run;
     __shared__ uint32_t s_cnt[WAVES];
     __shared__ uint32_t s_elist[WAVES][ELIST];  // per wave: errors of a slow template
-    __shared__ uint32_t s_kept[WAVES];          // CNA: kept templates per wave in a round
+    __shared__ cn_window s_cn;                  // CNA: the stratum's events; the chunk's kept templates per group and
+    __shared__ uint64_t s_mask[CNA ? CN_CHUNK : 1u];      // those of the groups before
+    __shared__ uint32_t s_below[CNA ? CN_CHUNK + 1u : 1u];
     extern __shared__ uint4 s_stage4[];  // STAGE: per wave 64 rows of read_words words
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
@@ -944,27 +1061,53 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
             const uint32_t ref_w0 = s.b >> 4;
             const uint32_t n_ref = min(chr_words, ((s.wend + 15u) >> 4) + 1u) - ref_w0;
             for (uint32_t i = tid; i <= n_ref; i += BLOCK) s_ref[i] = i < n_ref ? J.packed[S.chr_woff + ref_w0 + i] : 0u;
+            if (CNA && S.n_cna && wave == 0) cn_fill(J, S, s.b, s.e, lane, s_cn);
             uint32_t n_snv = 0;
             if (fits) n_snv = stage_snvs<BLOCK, CAP>(J, S, s, s_pos, s_lo, s_hi, s_info, s_bucket, s_cnt, tid);
             else __syncthreads();
             const lds_view lv{s_pos, s_lo, s_hi, s_info, nullptr, nullptr, s_bucket, n_snv, s.b};
             const glb_view gv{J.pos + s.k0, J.lo + s.k0, J.hi + s.k0, J.info + s.k0, nullptr, nullptr, s.n_win};
             const uint32_t nj = (uint32_t)s.nj;
-            // Rounds of WAVES x 64 templates, 64 per wave. Without copy-number events wave w takes templates
-            // [base + 64 w, base + 64 w + 64). With them only the templates whose copy slot is a copy of their
-            // source have reads, in template order: each wave counts its kept templates, one block barrier
-            // orders the waves, and each wave moves its kept templates to its first lanes (forward lane
-            // permutation). Either way lanes [0, n_t) then hold the templates (start tx, mate start tx2,
-            // leaf | allele << 26, template index tr) whose reads start at read index first0.
+            // Rounds of WAVES x 64 templates, 64 per wave: lanes [0, n_t) hold the templates (start tx, mate start tx2,
+            // leaf | allele << 26, template index tr) whose reads start at read index first0. With copy-number events
+            // only the templates whose copy slot is a copy of their source have reads: k_cn_accept left a bit for each;
+            // they are numbered by chunks of CN_CHUNK groups of 64, and a lane finds its template by its number.
             const bool cn = CNA && S.n_cna != 0u;
-            const uint64_t row0 = cn ? uniform_at(J.cn_row, S.st_off + j) : 0ull;
-            // Without copy-number events the chunks of 64 templates are shifted by o so that every pass after
-            // the stratum's first chunk starts on a 1024-byte boundary of the output (else 512, 256, 128): the
-            // first chunk holds the templates before the first aligned row. A 16-byte offset of such 3 KiB
-            // passes costs about 10 % of the write rate (partly written lines at every pass boundary).
+            uint64_t row = cn ? uniform_at(J.cn_row, S.st_off + j) : S.read_base + s.before * rpt;
+            const uint32_t n_grp = cn ? (nj + 63u) >> 6 : 1u;
+            for (uint32_t g0 = 0; g0 < n_grp; g0 += CN_CHUNK) {
+            uint32_t nk = nj;  // templates with reads (of the chunk)
+            if (CNA && cn) {
+                __syncthreads();  // the chunk before is done
+                const uint64_t* const mask = L.cn_kept + S.read_base + (uint64_t)j * cn_groups(S) + g0;
+                uint64_t m = 0;
+                uint32_t n = 0;
+                if (tid < CN_CHUNK) {
+                    m = g0 + tid < n_grp ? mask[tid] : 0u;
+                    s_mask[tid] = m;
+                    n = (uint32_t)__popcll(m);
+                    for (uint32_t k = 1; k < 64u; k <<= 1) {
+                        const uint32_t v = (uint32_t)__shfl_up((int)n, k);
+                        n += lane >= k ? v : 0u;
+                    }
+                    if (lane == 63u) s_cnt[wave] = n;
+                }
+                __syncthreads();
+                if (tid < CN_CHUNK) {
+                    for (uint32_t k = 0; k < wave; ++k) n += s_cnt[k];
+                    s_below[tid + 1u] = n;
+                    if (tid == 0) s_below[0] = 0;
+                }
+                __syncthreads();
+                nk = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_below[CN_CHUNK]);
+            }
+            // The chunks of 64 templates are shifted by o so that every pass after the first chunk starts on a
+            // 1024-byte boundary of the output (else 512, 256, 128): the first chunk holds the templates before the
+            // first aligned row. A 16-byte offset of such 3 KiB passes costs about 10 % of the write rate (partly
+            // written lines at every pass boundary).
             uint32_t o = 0;
-            if (!cn && STAGE && vec4) {
-                const uint64_t a0 = (uint64_t)(uintptr_t)(L.reads_out + (S.read_base + s.before * rpt) * RW);
+            if (STAGE && vec4) {
+                const uint64_t a0 = (uint64_t)(uintptr_t)(L.reads_out + row * RW);
                 const uint64_t step = (uint64_t)rpt * RW * 4u;  // bytes per template
                 for (uint32_t A = 1024u; A >= 128u; A >>= 1) {
                     const unsigned long long m = __ballot(((a0 + lane * step) & (A - 1u)) == 0u);
@@ -974,51 +1117,31 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
                     }
                 }
             }
-            uint32_t kept = 0;  // copy-number events: kept templates of the stratum's earlier rounds
-            for (uint32_t base = 0; base < nj + o; base += WAVES * 64u) {
+            for (uint32_t base = 0; base < nk + o; base += WAVES * 64u) {
                 // the wave's chunk: templates [c0, cend) (virtual templates [vb, vb + 64) less o)
                 const uint32_t vb = base + wave * 64u;
                 const uint32_t c0 = vb == 0u ? 0u : vb - o;
-                const uint32_t cend = min(vb + 64u - o, nj);
-                const uint32_t rt = c0 + lane;
-                uint32_t tx = 0, tx2 = 0, tla = 0, tr = rt, n_t;
-                uint64_t first0;
-                if (cn) {
-                    tmpl t{};
-                    bool ok = false;
-                    if (rt < nj) {
-                        t = make_template<true>(J, S, s_tab, rt, j, s.b, s.e);
-                        ok = t.ok != 0u;
-                    }
-                    const unsigned long long bal = __ballot(ok);
-                    if (lane == 0) s_kept[wave] = (uint32_t)__popcll(bal);
-                    __syncthreads();
-                    uint32_t before = kept, total = 0;
-                    for (uint32_t w2 = 0; w2 < WAVES; ++w2) {
-                        const uint32_t c = s_kept[w2];
-                        before += w2 < wave ? c : 0u;
-                        total += c;
-                    }
-                    __syncthreads();  // every wave has read s_kept before the next round writes it
-                    kept += total;
-                    n_t = (uint32_t)__popcll(bal);
-                    const uint32_t mine = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-                    const int to = (int)(ok ? mine : n_t + (lane - mine)) << 2;
-                    tla = leaf_of(J, S, t) | (t.allele << 26);
-                    tx = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)t.x);
-                    tx2 = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)t.x2);
-                    tla = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)tla);
-                    tr = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)rt);
-                    first0 = row0 + (uint64_t)before * rpt;
-                } else {
-                    n_t = cend > c0 ? cend - c0 : 0u;
+                const uint32_t cend = min(vb + 64u - o, nk);
+                const uint32_t n_t = cend > c0 ? cend - c0 : 0u;
+                const uint64_t first0 = row + (uint64_t)c0 * rpt;
+                uint32_t tx = 0, tx2 = 0, tla = 0, tr = c0 + lane;
+                if (CNA && cn) {
                     if (lane < n_t) {
-                        tmpl t = make_template(J, S, s_tab, rt, j, s.b, s.e);
+                        uint32_t a = 0;  // the group of kept template tr
+                        for (uint32_t h = CN_CHUNK / 2u; h; h >>= 1) a += s_below[a + h] <= tr ? h : 0u;
+                        tr = ((g0 + a) << 6) + nth_set(s_mask[a], tr - s_below[a]);
+                        psx_u4 w;
+                        tmpl t;
+                        cn_template(J, S, s_cn, (uint32_t)__builtin_amdgcn_readfirstlane((int)s_cn.n), tr, j, s.b, s.e, w, t);
                         tx = t.x;
-                        tx2 = t.x2;
-                        tla = leaf_of(J, S, t) | (t.allele << 26);
+                        tx2 = mate_start(J, S, s_tab, t.x, w.w);
+                        tla = (t.cell == S.n_cells ? J.n_leaves : J.sample_leaves[S.leaf_off + t.cell]) | (t.allele << 26);
                     }
-                    first0 = S.read_base + (s.before + c0) * rpt;
+                } else if (lane < n_t) {
+                    tmpl t = make_template(J, S, s_tab, tr, j, s.b, s.e);
+                    tx = t.x;
+                    tx2 = t.x2;
+                    tla = leaf_of(J, S, t) | (t.allele << 26);
                 }
                 if (n_t == 0) continue;
                 const bool valid = lane < n_t;
@@ -1090,6 +1213,8 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
                     }
                 }
             }
+            row += (uint64_t)nk * rpt;
+            }
             __syncthreads();
         }
       }
@@ -1100,8 +1225,11 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
 }
 
 // Kept templates of every stratum of the segments with copy-number events
-// (the read kernel's draws, so its row order follows): one wave per stratum,
-// 64 templates at a time.
+// (the read kernel's draws, so its row order follows), and a bit for each
+// template: one wave per stratum, 64 templates at a time. Bound by vector
+// instruction issue, 43 of them the draw's: a template's copies by a walk of
+// the chromosome's events with its leaf's rank 261 us for 3.3e7 draws, by the
+// stratum's events with ranges of cells 154 us.
 struct accept_args {
     const job_dev* jobs;
     const seg_dev* segs;
@@ -1109,6 +1237,8 @@ struct accept_args {
     const uint32_t* cn_first;  // its first stratum (index into kept), n_seg + 1 entries
     uint32_t n_seg;
     uint64_t* kept;            // per stratum
+    uint64_t* mask;            // with cn_mask: which templates are kept, 64 a word, cn_groups words a stratum
+    const uint64_t* cn_mask;   // the first word of each segment with events (null: no masks)
 };
 
 __global__ void __launch_bounds__(256) k_cn_accept(const accept_args a) {
@@ -1125,15 +1255,22 @@ __global__ void __launch_bounds__(256) k_cn_accept(const accept_args a) {
     const uint32_t j = g - uniform_at(a.cn_first, lo);
     const uint32_t b = j * PSX_STRATUM, e = min(b + PSX_STRATUM, S.W);
     const uint64_t nj = templates_below(S, e) - templates_below(S, b);
-    uint64_t cnt = 0;
-    for (uint64_t r0 = 0; r0 < nj; r0 += 64u) {
-        const uint64_t r = r0 + lane;
-        bool ok = false;
-        if (r < nj) {
-            psx_u4 w;
-            ok = template_source<true>(J, S, (uint32_t)r, j, b, e, w).ok != 0u;
-        }
-        cnt += (uint64_t)__popcll(__ballot(ok));
+    __shared__ cn_window s_cn[4];
+    cn_window& cw = s_cn[threadIdx.x >> 6];
+    cn_fill(J, S, b, e, lane, cw);
+    wave_sync();
+    const uint32_t n_ev = (uint32_t)__builtin_amdgcn_readfirstlane((int)cw.n);
+    uint64_t* const mask = a.cn_mask ? a.mask + uniform_at(a.cn_mask, lo) + (uint64_t)j * cn_groups(S) : nullptr;
+    uint64_t cnt = 0, mine = 0;  // 64 groups' masks, one per lane, stored together
+    for (uint32_t q = 0; (uint64_t)q * 64u < nj; ++q) {
+        const uint32_t r = q * 64u + lane;
+        psx_u4 w;
+        tmpl t;
+        const bool ok = cn_template(J, S, cw, n_ev, r, j, b, e, w, t) && r < nj;
+        const uint64_t m = __ballot(ok);
+        cnt += (uint64_t)__popcll(m);
+        mine = lane == (q & 63u) ? m : mine;
+        if (mask && ((q & 63u) == 63u || (uint64_t)(q + 1u) * 64u >= nj) && lane <= (q & 63u)) mask[(q & ~63u) + lane] = mine;
     }
     if (lane == 0) a.kept[g] = cnt;
 }

@@ -96,6 +96,36 @@ def test_windows_with_copy_numbers(ctx):
         assert n == on and np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op)
 
 
+AMP, DEL, WGD = 0, 1, 2  # (species, chromosome, start, length, lineage, kind, copies)
+
+
+@pytest.mark.parametrize("snv", [3e-7, 6e-5])
+@pytest.mark.parametrize("cov,ploidy,cna", [
+    # a listed window; its edges at a stratum's; more templates in a stratum than the read kernel numbers at a time
+    (700.0, 2, [(0, 0, 8192, 8192, 1, AMP, 255), (1, 0, 100, 30_000, 0, DEL, 0), (0, 0, 0, 0, 0, WGD, 0)]),
+    # what a listed window does not hold: a 17th event, a fourth doubling, three lineages
+    (60.0, 2, [(0, 0, 500 * k, 20_000, k & 1, DEL if k % 5 == 0 else AMP, 1) for k in range(17)]),
+    (20.0, 2, [(0, 0, 0, 0, 0, WGD, 0)] * 4),
+    (60.0, 3, [(0, 0, 9_000, 20_000, 2, AMP, 2), (1, 1, 0, 4_000, 0, DEL, 0), (1, 0, 0, 0, 0, WGD, 0)]),
+    # both lineages gone where every read would start
+    (30.0, 2, [(0, 1, 0, 5_000, 0, DEL, 0), (0, 1, 0, 5_000, 1, DEL, 0)])])
+def test_copy_number_draws(ctx, snv, cov, ploidy, cna):
+    """Counts and reads of segments with copy numbers, sparse and dense tables, with and without a normal share."""
+    from process_amd import _abi as A
+    kinds = [A.PSX_CNA_AMP, A.PSX_CNA_DEL, A.PSX_CNA_WGD]
+    w = World(ctx, [40_000, 5_000], dict(n_cells=500, n_samples=1, sample_size=90, seed=2), snv,
+              cna=[(sp, c, at, ln, a, kinds[k], n) for sp, c, at, ln, a, k, n in cna], ploidy=ploidy)
+    for kw in (dict(read_size=75, error_rate=2e-3, purity=0.7),
+               dict(read_size=100, insert_size_mean=250, insert_size_stddev=10, error_rate=1e-3)):
+        kw["coverage"] = cov
+        a, d, p, _ = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)
+        oa, od, op, on = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), ploidy=ploidy, **kw)
+        assert np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op)
+        rows, m = core.simulate_seq_reads(ctx, w.g, w.pf, w.pm, 3, **kw)
+        ref = O.simulate_reads(w.lens, w.g.download(), w.of, w.recs, 3, m, cna=w.pm.cna(), ploidy=ploidy, **kw)
+        assert m == on and np.array_equal(rows.numpy()[:m], ref)
+
+
 def test_parts_of_few_strata(ctx):
     """Few strata with many templates: items are cut into parts, in both count kernels."""
     forest = dict(n_cells=300, n_samples=1, sample_size=60, seed=4)
