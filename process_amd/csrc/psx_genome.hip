@@ -276,9 +276,7 @@ void psx_mutations_build(psx_ctx* ctx, psx_mutations* m, std::vector<psx_mutatio
     }
     m->n = n;
     m->chr_len = chr_len;
-    auto block = std::make_shared<dbuf>();
-    block->alloc(psx_mutations_bytes(n));
-    psx_mutations_carve(m, block, 0);
+    psx_mutations_carve(m, psx_block(psx_mutations_bytes(n)), 0);
     if (n)
         PSX_HIP(hipMemcpyAsync(m->recs, recs.data(), n * sizeof(psx_mutation), hipMemcpyHostToDevice,
                                ctx->stream));

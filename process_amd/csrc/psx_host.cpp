@@ -41,6 +41,8 @@ extern "C" psx_status psx_ctx_create(int device, psx_ctx** out) {
         PSX_HIP(hipEventCreate(&ctx->ev0));
         PSX_HIP(hipEventCreate(&ctx->ev1));
         ctx->noalloc_scratch = psx_noalloc_scratch_init(device);
+        psx_blocks_open(device);
+        ctx->blocks = true;
     });
     if (st != PSX_OK) {
         // keep the context so the caller can read the message
@@ -85,6 +87,7 @@ extern "C" void psx_ctx_destroy(psx_ctx* ctx) {
         (void)hipEventDestroy(ctx->ev1);
         (void)hipStreamDestroy(ctx->stream);
     }
+    if (ctx->blocks) psx_blocks_close(ctx->device);
     delete ctx;
 }
 
@@ -123,9 +126,144 @@ extern "C" psx_status psx_ctx_mem_info(psx_ctx* ctx, uint64_t* free_bytes, uint6
         PSX_HIP(hipSetDevice(ctx->device));
         size_t f = 0, t = 0;
         PSX_HIP(hipMemGetInfo(&f, &t));
-        *free_bytes = f;
+        *free_bytes = f + psx_blocks_idle(ctx->device);  // given back when an allocation needs them
         *total_bytes = t;
     });
+}
+
+// ------------------------------------------------------------ device blocks
+
+namespace {
+
+constexpr size_t BLOCKS_IDLE = size_t(1) << 30, BLOCK_LARGEST = BLOCKS_IDLE / 2, BLOCKS_COUNT = 16;
+
+struct block_pool {
+    struct idle_block {
+        void* p;
+        size_t bytes;
+    };
+    int contexts = 0;
+    size_t bytes = 0, n = 0;
+    idle_block idle[BLOCKS_COUNT + 1];  // oldest first
+    idle_block take(size_t k) {
+        const idle_block b = idle[k];
+        std::copy(idle + k + 1, idle + n, idle + k);
+        --n;
+        bytes -= b.bytes;
+        return b;
+    }
+};
+
+std::mutex blocks_mu;
+
+std::map<int, block_pool>& block_pools() {
+    static auto* const pools = new std::map<int, block_pool>();  // tables may be freed while the process ends
+    return *pools;
+}
+
+// Blocks taken out of a pool, to be freed without its lock.
+struct taken_blocks {
+    void* p[BLOCKS_COUNT + 1];
+    size_t n = 0;
+    // oldest first, until at most `keep` bytes and `count` blocks are idle
+    void oldest(block_pool& P, size_t keep, size_t count) {
+        while (P.bytes > keep || P.n > count) p[n++] = P.take(0).p;
+    }
+    ~taken_blocks() {
+        for (size_t k = 0; k < n; ++k) (void)hipFree(p[k]);
+    }
+};
+
+void give_block(dbuf* b, int device) {
+    int now = device;
+    (void)hipGetDevice(&now);
+    if (now != device) (void)hipSetDevice(device);
+    taken_blocks out;
+    // launches in flight may read the block, on any stream
+    if (b->bytes <= BLOCK_LARGEST && hipDeviceSynchronize() == hipSuccess) {
+        std::lock_guard<std::mutex> g(blocks_mu);
+        block_pool& P = block_pools()[device];
+        if (P.contexts) {
+            P.idle[P.n++] = {b->p, b->bytes};
+            P.bytes += b->bytes;
+            b->p = nullptr;
+            out.oldest(P, BLOCKS_IDLE, BLOCKS_COUNT);
+        }
+    }
+    delete b;
+    if (now != device) (void)hipSetDevice(now);
+}
+
+}  // namespace
+
+hipError_t psx_dev_malloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    int device = 0;
+    if (e != hipErrorOutOfMemory || hipGetDevice(&device) != hipSuccess) return e;
+    bool any = false;
+    {
+        taken_blocks out;
+        std::lock_guard<std::mutex> g(blocks_mu);
+        auto P = block_pools().find(device);
+        if (P != block_pools().end()) out.oldest(P->second, 0, 0);
+        any = out.n != 0;
+    }
+    if (!any) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
+std::shared_ptr<dbuf> psx_block(size_t n) {
+    if (n == 0) n = 256;
+    int device = 0;
+    PSX_HIP(hipGetDevice(&device));
+    auto b = std::make_unique<dbuf>();
+    {
+        // the smallest that fits, unless it is half as large again
+        std::lock_guard<std::mutex> g(blocks_mu);
+        block_pool& P = block_pools()[device];
+        size_t best = P.n;
+        for (size_t k = 0; k < P.n; ++k)
+            if (P.idle[k].bytes >= n && P.idle[k].bytes <= n + n / 2 + 4096 &&
+                (best == P.n || P.idle[k].bytes < P.idle[best].bytes))
+                best = k;
+        if (best != P.n) {
+            const block_pool::idle_block k = P.take(best);
+            b->p = k.p;
+            b->bytes = k.bytes;
+        }
+    }
+    if (!b->p) {
+        // rounded up by a sixteenth at most, so that the next call's table, of about this size, fits too
+        size_t step = 4096;
+        while (step * 32 <= n) step *= 2;
+        const size_t whole = n <= BLOCK_LARGEST ? (n + step - 1) / step * step : n;
+        if (whole != n && psx_dev_malloc(&b->p, whole) == hipSuccess) {
+            b->bytes = whole;
+        } else {
+            (void)hipGetLastError();
+            b->p = nullptr;
+            b->alloc(n);
+        }
+    }
+    return std::shared_ptr<dbuf>(b.release(), [device](dbuf* d) { give_block(d, device); });
+}
+
+void psx_blocks_open(int device) {
+    std::lock_guard<std::mutex> g(blocks_mu);
+    ++block_pools()[device].contexts;
+}
+
+void psx_blocks_close(int device) {
+    taken_blocks out;
+    std::lock_guard<std::mutex> g(blocks_mu);
+    block_pool& P = block_pools()[device];
+    if (--P.contexts == 0) out.oldest(P, 0, 0);
+}
+
+size_t psx_blocks_idle(int device) {
+    std::lock_guard<std::mutex> g(blocks_mu);
+    return block_pools()[device].bytes;
 }
 
 // ----------------------------------------------------------- device buffers

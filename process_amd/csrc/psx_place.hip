@@ -1725,8 +1725,7 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
         t_off[k] = block_bytes;
         block_bytes += psx_mutations_bytes(jobs[k].M);
     }
-    auto block = std::make_shared<dbuf>();
-    block->alloc(block_bytes);
+    const std::shared_ptr<dbuf> block = psx_block(block_bytes);
     PSX_HIP(hipStreamSynchronize(s));
     // status of every job's placement launches, the moved mutations and the losers of the last check run
     uint32_t round = 1, spec_end = 1, n_lose = 0, n_moved = 0;
@@ -1810,8 +1809,7 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
     ia.n_chr = g->n_chr;
     ia.nb = ix_off[g->n_chr];
     for (uint32_t c = 0; c <= g->n_chr; ++c) ia.boff[c] = ix_off[c];
-    auto ix_block = std::make_shared<dbuf>();
-    ix_block->alloc(ia.nb * nj * 4u);
+    const std::shared_ptr<dbuf> ix_block = psx_block(ia.nb * nj * 4u);
     for (uint32_t k = 0; k < nj; ++k) tab[k].bucket = ix_block->as<uint32_t>() + ia.nb * k;
     upload_table();
     if (Mt) {

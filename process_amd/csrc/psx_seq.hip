@@ -723,12 +723,12 @@ namespace {
 // such a segment's descriptor has the index of its first mask word in place of
 // its first read. Without events nothing changes.
 struct cn_rows {
-    dbuf buf;                    // kept | first read (uint64 per stratum) | first masks | masks | segment list | first strata
+    std::shared_ptr<dbuf> buf;   // kept | first read (uint64 per stratum) | first masks | masks | segment list | first strata
     std::vector<uint32_t> seg, first;
     std::vector<uint64_t> mask;  // per segment with events: its first mask word (empty: no masks)
     uint64_t n = 0, n_mask = 0;
     explicit cn_rows(bool masks) : masks_(masks) {}
-    const uint64_t* kept_masks() const { return masks_ && n ? buf.as<uint64_t>() + 2 * n + mask.size() : nullptr; }
+    const uint64_t* kept_masks() const { return masks_ && n ? buf->as<uint64_t>() + 2 * n + mask.size() : nullptr; }
     std::vector<uint64_t> seg_reads;  // reads of each segment (finish)
     bool prepare(seq_batch& P) {
         seg_dev* hs = (seg_dev*)(P.sb.host.data() + P.o_segs);
@@ -748,13 +748,13 @@ struct cn_rows {
             }
         if (!n) return false;
         if (n >= (uint64_t(1) << 32)) psx_throw(PSX_EINVAL, "too many strata with copy-number events");
-        buf.alloc(16 * n + 8 * (mask.size() + n_mask) + 4 * (seg.size() + first.size()) + 256);
+        buf = psx_block(16 * n + 8 * (mask.size() + n_mask) + 4 * (seg.size() + first.size()) + 256);
         job_dev* hj = (job_dev*)(P.sb.host.data() + P.o_jobs);
-        for (size_t k = 0; k < P.jobs.size(); ++k) hj[k].cn_row = buf.as<uint64_t>() + n;
+        for (size_t k = 0; k < P.jobs.size(); ++k) hj[k].cn_row = buf->as<uint64_t>() + n;
         return true;
     }
     void finish(psx_ctx* ctx, seq_batch& P, const seq_lane& lane) {
-        uint64_t* d_kept = buf.as<uint64_t>();
+        uint64_t* d_kept = buf->as<uint64_t>();
         uint64_t* d_mask_first = d_kept + 2 * n;
         uint64_t* d_mask = d_mask_first + mask.size();
         uint32_t* d_seg = (uint32_t*)(d_mask + n_mask);
@@ -838,13 +838,12 @@ void run_reads(psx_ctx* ctx, const std::vector<job_in>& in, uint32_t* d_reads, u
     // only the SNVs a read of the sample can carry. Kernels index a job's
     // flags from its own base (so * n_mut + m), so each job gets the slice
     // that starts at its first (job, output sample) entry.
-    dbuf d_present;
-    d_present.alloc(P.pres_total);
+    const std::shared_ptr<dbuf> d_present = psx_block(P.pres_total);
     std::vector<uint64_t> pres_base(P.jobs.size(), 0);
     for (const pres_dev& q : P.pres)
         if (q.so == 0) pres_base[q.job] = q.begin;
     job_dev* hj = (job_dev*)(P.sb.host.data() + P.o_jobs);  // the uploaded descriptors
-    for (size_t k = 0; k < P.jobs.size(); ++k) hj[k].present = d_present.as<uint8_t>() + pres_base[k];
+    for (size_t k = 0; k < P.jobs.size(); ++k) hj[k].present = d_present->as<uint8_t>() + pres_base[k];
     const seq_lane lane = ctx_lane(ctx, batch_desc_bytes(&P));
     batch_upload(&P, lane);
     if (with_cn) cn.finish(ctx, P, lane);

@@ -123,3 +123,45 @@ def test_many_tiny_jobs_share_waves(ctx):
         if k % 8 == 0:
             assert got.tobytes() == O.place_mutations(LENS, packed, of, sd, **eng).tobytes(), k
     assert sum(sizes) > 48 * 5 and min(sizes) < 64
+
+
+def test_tables_in_blocks_used_before(ctx):
+    """A table's memory goes to a later table: sizes that fit an idle block and sizes that do not, tables freed in any
+    order, from two threads with a context each and from a third context's; every table is the oracle's."""
+    import threading
+    g = core.Genome(ctx, LENS, seed=5)
+    packed = g.download()
+    fs = forests(ctx, [(400, 1, True), (900, 2, True)])
+    rates = [1e-6, 1.2e-6, 5e-6, 2e-5]
+    want = {}
+    for k, (f, of, _) in enumerate(fs):
+        for r in rates:
+            want[k, r] = O.place_mutations(LENS, packed, of, 9, **cases.engine(packed, LENS, snv=r)).tobytes()
+    errors = []
+
+    def work(seed, own):
+        try:
+            c = core.Context(0) if own else ctx
+            gc = core.Genome(c, LENS, packed=packed)
+            rng = np.random.default_rng(seed)
+            held = []
+            for _ in range(24):
+                k, r = int(rng.integers(2)), rates[int(rng.integers(4))]
+                m = core.Mutations.place(c, gc, fs[k][0], 9, **cases.engine(packed, LENS, snv=r))
+                held.append((m, want[k, r]))
+                if len(held) > 3:
+                    m, w = held.pop(int(rng.integers(4)))
+                    assert m.download().tobytes() == w
+                    m.close()
+            for m, w in held:
+                assert m.download().tobytes() == w
+        except Exception as e:  # reported by the caller's thread
+            errors.append(e)
+
+    ts = [threading.Thread(target=work, args=(s, True)) for s in (1, 2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    work(3, False)
+    assert not errors, errors
