@@ -472,6 +472,7 @@ struct fjob {
     uint32_t *pos, *lo, *hi, *info;  // and the kernels' arrays of them
     uint64_t* chr_begin;  // its table's chromosome ranges (PSX_MAX_CHROMOSOMES + 1)
     uint32_t* bucket;     // its table's stratum index
+    uint32_t sort_first, sort_n;  // its sort buckets
 };
 
 struct batch {
@@ -620,9 +621,34 @@ __device__ __forceinline__ bool fp_touch(uint64_t sa, uint32_t la, uint64_t sb, 
     return sb <= sa + la + 1u && sa <= sb + lb + 1u;
 }
 
-// One thread per mutation of every job, first attempt, and its sort entry.
+// Sort of the first attempts by (key, creation order): a job's padded
+// positions are cut into buckets of equal length, one for every SORT_MEAN
+// mutations, which k_place counts; a scan, a scatter and one block per bucket
+// follow. A bucket's entries are spread over SORT_SUBS parts of its length in
+// LDS (one or two to a part) and ordered by insertion, or all together where
+// many crowd a part. 1.49e6 entries 85 us, 26 of them the counts' atomics, 26
+// the scattered 16-byte stores, against 175 for four radix passes of 8 bits
+// and their clears; a table of 100 to 200 thousand 35 us against 78 for the
+// library's merges. Up to SORT_FEW entries that is one launch, 8 us, and these
+// four 15. Mutations crowded in a small part of the genome overfill a bucket
+// (SORT_MOST): the scan then sets io->skew, the kernels after it do nothing,
+// and the caller sorts by radix.
+constexpr uint32_t SORT_MEAN = 256, SORT_MOST = 2048, SORT_SUB_BITS = 9, SORT_SUBS = 1u << SORT_SUB_BITS,
+                   SORT_FEW = 1024;
+constexpr uint32_t SORT_PAD = 16;  // words from counter to counter: atomics on one 128-byte line queue (k_place 94 -> 160 us)
+
+// A key's bucket among its job's, and the part of the bucket.
+__device__ __forceinline__ uint32_t sort_bucket(const batch& B, uint32_t sort_n, uint64_t key, uint32_t& sub) {
+    const uint64_t in_job = (1ull << B.pbits) - 1ull, q = (key & in_job) * sort_n;
+    sub = (uint32_t)((q & in_job) >> (B.pbits - SORT_SUB_BITS));
+    return (uint32_t)(q >> B.pbits);
+}
+
+// One thread per mutation of every job, first attempt, its sort entry and its
+// place among its bucket's.
 __global__ void __launch_bounds__(256) k_place(const batch B, uint64_t n, uint64_t* __restrict__ fkey,
-                                               uint32_t* __restrict__ fval) {
+                                               uint32_t* __restrict__ fval, uint32_t* __restrict__ count,
+                                               uint32_t* __restrict__ rank) {
     const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= n) return;
     per_job(job_of_seq(B.mbase, B.nj, g), [&](uint32_t j) {
@@ -634,9 +660,136 @@ __global__ void __launch_bounds__(256) k_place(const batch B, uint64_t n, uint64
         finish_searches([&](int) -> const place_args& { return a; }, search, r, st);
         if (st != ST_OK) atomicOr(a.status, st);
         a.recs[id] = r;
-        fkey[g] = jkey(B, j, r);
+        const uint64_t key = jkey(B, j, r);
+        fkey[g] = key;
         fval[g] = fp_val((uint32_t)id, r);
+        uint32_t sub;
+        if (rank) rank[g] = atomicAdd(&count[(size_t)(cjob(B, j).sort_first + sort_bucket(B, cjob(B, j).sort_n, key, sub)) * SORT_PAD], 1u);
     });
+}
+
+// Each bucket's first entry from the counts, first[nb] the total; one block.
+__global__ void __launch_bounds__(1024) k_sort_scan(const uint32_t* __restrict__ count, uint32_t nb,
+                                                    uint32_t* __restrict__ first, uint32_t* __restrict__ skew) {
+    using scan = hipcub::BlockScan<uint32_t, 1024>;
+    __shared__ typename scan::TempStorage tmp;
+    uint32_t carry = 0, most = 0;
+    for (uint32_t b0 = 0; b0 < nb; b0 += 4096u) {
+        uint32_t c[4], total;
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const uint32_t b = b0 + threadIdx.x * 4u + k;
+            c[k] = b < nb ? count[(size_t)b * SORT_PAD] : 0u;
+            most = max(most, c[k]);
+        }
+        scan(tmp).ExclusiveSum(c, c, total);
+        __syncthreads();  // tmp
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const uint32_t b = b0 + threadIdx.x * 4u + k;
+            if (b < nb) first[b] = carry + c[k];
+        }
+        carry += total;
+    }
+    if (threadIdx.x == 0) first[nb] = carry;
+    if (most > SORT_MOST) *skew = 1u;
+}
+
+__global__ void __launch_bounds__(256) k_sort_scatter(const batch B, uint64_t n, const uint64_t* __restrict__ fkey,
+                                                      const uint32_t* __restrict__ fval, const uint32_t* __restrict__ first,
+                                                      const uint32_t* __restrict__ rank, uint4* __restrict__ entry,
+                                                      const uint32_t* __restrict__ skew) {
+    const uint64_t g = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (g >= n || *skew) return;
+    const uint64_t key = fkey[g];
+    const fjob& J = B.jobs[(uint32_t)(key >> B.pbits)];
+    uint32_t sub;
+    const uint32_t b = J.sort_first + sort_bucket(B, J.sort_n, key, sub);
+    entry[first[b] + rank[g]] = uint4{(uint32_t)key, (uint32_t)(key >> 32), fval[g], sub};
+}
+
+__global__ void __launch_bounds__(256) k_sort_buckets(const uint32_t* __restrict__ first, const uint4* __restrict__ entries,
+                                                      uint64_t* __restrict__ okey, uint32_t* __restrict__ oval,
+                                                      const uint32_t* __restrict__ skew) {
+    __shared__ struct {
+        uint64_t key[SORT_MOST];
+        uint32_t val[SORT_MOST], at[SORT_SUBS];
+        hipcub::BlockScan<uint32_t, 256>::TempStorage tmp;
+    } l;
+    const uint32_t o = first[blockIdx.x], n = first[blockIdx.x + 1u] - o;
+    if (n == 0u || *skew) return;  // the whole block
+    const uint4* const entry = entries + o;
+    const uint32_t tid = threadIdx.x;
+    constexpr uint32_t PER = SORT_SUBS / 256u, CROWD = 32u;  // parts per thread; entries of a part sorted by insertion
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k) l.at[tid * PER + k] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += 256u) atomicAdd(&l.at[entry[i].w], 1u);
+    __syncthreads();
+    uint32_t c[PER], at[PER];
+    bool crowd = false;
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k) {
+        c[k] = l.at[tid * PER + k];
+        crowd = crowd || c[k] > CROWD;
+    }
+    hipcub::BlockScan<uint32_t, 256>(l.tmp).ExclusiveSum(c, at);
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k) l.at[tid * PER + k] = at[k];
+    crowd = __syncthreads_or(crowd);
+    for (uint32_t i = tid; i < n; i += 256u) {
+        const uint4 e = entry[i];
+        const uint32_t q = atomicAdd(&l.at[e.w], 1u);
+        l.key[q] = (uint64_t)e.y << 32 | e.x;
+        l.val[q] = e.z;
+    }
+    auto after = [&](uint64_t ka, uint32_t va, uint64_t kb, uint32_t vb) {
+        return ka > kb || (ka == kb && (va & ID_MASK) > (vb & ID_MASK));
+    };
+    __syncthreads();
+    if (crowd) {  // many of one part: a bitonic sort of the whole block
+        uint32_t N = 2;
+        while (N < n) N *= 2;
+        for (uint32_t i = n + tid; i < N; i += 256u) {
+            l.key[i] = ~0ull;
+            l.val[i] = NO_ENTRY;
+        }
+        for (uint32_t w = 2; w <= N; w *= 2)
+            for (uint32_t d = w / 2; d; d /= 2) {
+                __syncthreads();
+                for (uint32_t t = tid; t < N / 2; t += 256u) {
+                    const uint32_t i = 2u * t - (t & (d - 1u)), q = i + d;
+                    const uint64_t ki = l.key[i], kq = l.key[q];
+                    const uint32_t vi = l.val[i], vq = l.val[q];
+                    if (after(ki, vi, kq, vq) == ((i & w) == 0u)) {
+                        l.key[i] = kq;
+                        l.val[i] = vq;
+                        l.key[q] = ki;
+                        l.val[q] = vi;
+                    }
+                }
+            }
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < PER; ++k)
+            for (uint32_t i = at[k] + 1u; i < at[k] + c[k]; ++i) {
+                const uint64_t key = l.key[i];
+                const uint32_t val = l.val[i];
+                uint32_t q = i;
+                while (q > at[k] && after(l.key[q - 1u], l.val[q - 1u], key, val)) {
+                    l.key[q] = l.key[q - 1u];
+                    l.val[q] = l.val[q - 1u];
+                    --q;
+                }
+                l.key[q] = key;
+                l.val[q] = val;
+            }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += 256u) {
+        okey[o + i] = l.key[i];
+        oval[o + i] = l.val[i];
+    }
 }
 
 // A loser of check number `stamp` (1 for the first): lose[gid] holds the
@@ -704,7 +857,9 @@ __device__ __forceinline__ bool loses(const batch& B, const uint64_t* __restrict
 __global__ void __launch_bounds__(256) k_conflicts(const batch B, const uint64_t* __restrict__ fkey,
                                                    const uint32_t* __restrict__ fval, uint64_t n,
                                                    uint32_t* __restrict__ lose, uint32_t* __restrict__ list,
-                                                   uint32_t* __restrict__ apos, uint32_t* __restrict__ n_lose) {
+                                                   uint32_t* __restrict__ apos, uint32_t* __restrict__ n_lose,
+                                                   const uint32_t* __restrict__ skew) {
+    if (*skew) return;
     const uint64_t b = (uint64_t)blockIdx.x * 256u * APPEND_ITEMS + threadIdx.x;
     uint32_t mask = 0, c = 0, gids[APPEND_ITEMS];
 #pragma unroll
@@ -770,7 +925,7 @@ struct round_io {
     uint32_t n_moved;   // mutations moved so far (entries of the moved list)
     uint32_t tab_used;  // table entries since it was last cleared
     uint32_t halt;      // first round that found the table too full to run (0: none)
-    uint32_t pad;
+    uint32_t skew;      // some sort bucket holds more than SORT_MOST mutations
     uint32_t n_lose[IS_ROUNDS + 1];  // losers of check r (0: the first check)
 };
 
@@ -1517,7 +1672,7 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
     auto at = [&](size_t off) { return (void*)(base + off); };
     // sort keys: the padded position below bit pbits (at least 16 to spare), the job above
     const uint64_t p_max = pstart[g->n_chr - 1] + g->len[g->n_chr - 1];
-    const uint32_t pbits = (uint32_t)bits_for(p_max + 16), kbits = pbits + (uint32_t)bits_for(nj - 1);
+    const uint32_t pbits = std::max<uint32_t>((uint32_t)bits_for(p_max + 16), SORT_SUB_BITS), kbits = pbits + (uint32_t)bits_for(nj - 1);
     if (kbits > 64) psx_throw(PSX_EINVAL, "too many jobs for one call (%u)", nj);
 
     // node bases, the job table and the batch's round state (one device buffer)
@@ -1636,22 +1791,31 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
     PSX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, rank_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr,
                                              (int)Mt + 1, s));
     sort_bytes = std::max(sort_bytes, rank_bytes);
-    // per-mutation arrays of the whole batch from the context's placement pool: attempt counters, moved flags
-    // and loser stamps first (cleared together)
+    // per-mutation arrays of the whole batch from the context's placement pool: attempt counters, moved flags,
+    // loser stamps and the sort buckets' counts first (cleared together)
     const uint64_t tab_slots_max = tab_max(Mt);
     carver cm;
-    const size_t c_zero = cm.take(Mt * 12), c_sort = cm.take(sort_bytes), c_recs = cm.take(Mt * sizeof(psx_mutation)),
+    uint64_t n_sort = 0;  // sort buckets
+    for (uint32_t k = 0; k < nj; ++k) {
+        tab[k].sort_first = (uint32_t)n_sort;
+        tab[k].sort_n = (uint32_t)(jobs[k].M ? std::max<uint64_t>(1, jobs[k].M / SORT_MEAN) : 0);
+        n_sort += tab[k].sort_n;
+    }
+    const bool few = Mt <= SORT_FEW;
+    const size_t zero_bytes = Mt * 12 + n_sort * SORT_PAD * 4;
+    const size_t c_zero = cm.take(zero_bytes), c_sort = cm.take(sort_bytes), c_recs = cm.take(Mt * sizeof(psx_mutation)),
                  c_list0 = cm.take(Mt * 4), c_list1 = cm.take(Mt * 4), c_lap0 = cm.take(Mt * 4),
                  c_lap1 = cm.take(Mt * 4), c_ids = cm.take(Mt * 4), c_ids2 = cm.take(Mt * 4), c_ml = cm.take(Mt * 4),
                  c_map = cm.take(Mt * 4), c_w = cm.take((Mt + 1) * 4), c_S = cm.take((Mt + 1) * 4),
                  c_nof = cm.take(n_pass_all * 4), c_key = cm.take(Mt * 8), c_key2 = cm.take(Mt * 8),
-                 c_tab = cm.take(tab_slots_max * 4), c_head = cm.take(Mt);
+                 c_tab = cm.take(tab_slots_max * 4), c_head = cm.take(Mt), c_first = cm.take((n_sort + 1) * 4);
     ctx->place_muts.reserve(cm.bytes);
     uint8_t* pm = (uint8_t*)ctx->place_muts.p;
     void* d_sort = pm + c_sort;
     uint32_t* d_att = (uint32_t*)(pm + c_zero);
     uint32_t* d_moved = d_att + Mt;
     uint32_t* d_lose = d_att + 2 * Mt;
+    uint32_t *d_count = d_att + 3 * Mt, *d_first = (uint32_t*)(pm + c_first);
     psx_mutation* d_recs = (psx_mutation*)(pm + c_recs);
     uint32_t* d_list[2] = {(uint32_t*)(pm + c_list0), (uint32_t*)(pm + c_list1)};
     uint32_t* d_lapos[2] = {(uint32_t*)(pm + c_lap0), (uint32_t*)(pm + c_lap1)};
@@ -1701,21 +1865,41 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
     }
     upload_table();
     PSX_HIP(hipMemsetAsync(dt + t_state, 0, sizeof(round_io) + 4 * nj, s));
-    PSX_HIP(hipMemsetAsync(pm + c_zero, 0, Mt * 12, s));
+    PSX_HIP(hipMemsetAsync(pm + c_zero, 0, zero_bytes, s));
     if (N) {
         hipLaunchKernelGGL(k_node_expand, dim3(grid_of(N)), dim3(256), 0, s, B, N, d_off, d_node_of);
         PSX_HIP(hipGetLastError());
     }
+    auto radix_sort = [&] {
+        PSX_HIP(hipcub::DeviceRadixSort::SortPairs(d_sort, sort_bytes, d_key, d_key2, d_ids, d_ids2, (int)Mt, 0,
+                                                   (int)kbits, s));
+    };
+    auto first_check = [&] {
+        hipLaunchKernelGGL(k_conflicts, dim3(grid_append(Mt)), dim3(256), 0, s, B, d_key2, d_ids2, Mt, d_lose,
+                           d_list[0], d_lapos[0], &d_io->n_lose[0], &d_io->skew);
+        PSX_HIP(hipGetLastError());
+    };
     if (Mt) {
         // first attempts and sort entries; one sort of every job's footprints (job-major, the sorted entries stay
         // as the reference of later rounds and give the position order); the first check
-        hipLaunchKernelGGL(k_place, dim3(grid_of(Mt)), dim3(256), 0, s, B, Mt, d_key, d_ids);
+        // (the entries' ranks and the scattered entries in memory that the later rounds use)
+        uint32_t* const rank = few ? nullptr : d_mlist;
+        uint4* const entry = (uint4*)d_tab;
+        hipLaunchKernelGGL(k_place, dim3(grid_of(Mt)), dim3(256), 0, s, B, Mt, d_key, d_ids, d_count, rank);
         PSX_HIP(hipGetLastError());
-        PSX_HIP(hipcub::DeviceRadixSort::SortPairs(d_sort, sort_bytes, d_key, d_key2, d_ids, d_ids2, (int)Mt, 0,
-                                                   (int)kbits, s));
-        hipLaunchKernelGGL(k_conflicts, dim3(grid_append(Mt)), dim3(256), 0, s, B, d_key2, d_ids2, Mt, d_lose,
-                           d_list[0], d_lapos[0], &d_io->n_lose[0]);
+        if (few) {
+            radix_sort();
+        } else {
+            hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(1024), 0, s, d_count, (uint32_t)n_sort, d_first, &d_io->skew);
+            PSX_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_sort_scatter, dim3(grid_of(Mt)), dim3(256), 0, s, B, Mt, d_key, d_ids, d_first, rank,
+                               entry, &d_io->skew);
+            PSX_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_sort_buckets, dim3((uint32_t)n_sort), dim3(256), 0, s, d_first, entry, d_key2, d_ids2,
+                               &d_io->skew);
+        }
         PSX_HIP(hipGetLastError());
+        first_check();
     }
     PSX_HIP(hipMemcpyAsync(io, dt + t_state, io_state, hipMemcpyDeviceToHost, s));
     // the tables' block, allocated while the GPU runs the placement
@@ -1727,6 +1911,13 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
     }
     const std::shared_ptr<dbuf> block = psx_block(block_bytes);
     PSX_HIP(hipStreamSynchronize(s));
+    if (h_io->skew) {
+        PSX_HIP(hipMemsetAsync(&d_io->skew, 0, 4, s));
+        radix_sort();
+        first_check();
+        PSX_HIP(hipMemcpyAsync(io, dt + t_state, io_state, hipMemcpyDeviceToHost, s));
+        PSX_HIP(hipStreamSynchronize(s));
+    }
     // status of every job's placement launches, the moved mutations and the losers of the last check run
     uint32_t round = 1, spec_end = 1, n_lose = 0, n_moved = 0;
     bool halted = false;

@@ -165,3 +165,45 @@ def test_tables_in_blocks_used_before(ctx):
         t.join()
     work(3, False)
     assert not errors, errors
+
+
+@pytest.mark.parametrize("lens,share,pre,infinite", [
+    ([400_000], 1.0, 1024, True), ([400_000], 1.0, 1025, True),  # one launch of the library; the bucket sort
+    ([700_000, 90_000, 37], 1.0, 6000, True),                    # a chromosome shorter than a bucket
+    ([3000], 1.0, 3000, False),                                  # several mutations at every position
+    ([2_000_000], 0.004, 5000, False),                           # all in 8 kb: a bucket overfilled, sorted by radix
+    ([2_000_000], 0.0008, 1900, False),                          # a bucket's entries in few of its parts
+    ([2_000_000], 1e-5, 1500, False)])                           # at 20 positions
+def test_order_of_crowded_tables(ctx, lens, share, pre, infinite):
+    """The bucket sort of the first attempts over table sizes and densities, alone and in a batch: mutations confined to
+    the first bases of a reference that is one letter elsewhere."""
+    rng = np.random.default_rng(7)
+    seqs = []
+    for k, n in enumerate(lens):
+        s = np.full(n, "A")
+        m = int(n * share)
+        s[:m] = rng.choice(list("CG") if share < 1.0 else list("ACGT"), m)
+        seqs.append("".join(s))
+    import process_amd as pa
+    names = [str(k + 1) for k in range(len(lens))]
+    ref = pa.ReferenceGenome(dict(zip(names, lens)), sequences=dict(zip(names, seqs)))
+    packed = ref.packed
+    g = core.Genome(ctx, ref.lengths, packed=packed)
+    sbs = np.zeros((1, 96))
+    sbs[0, :48] = 1.0 / 48  # C>N
+    if share < 1.0:  # of C and G neighbours only
+        sbs[0] = 0.0
+        for sub in range(3):
+            for five in (1, 2):
+                for three in (1, 2):
+                    sbs[0, sub * 16 + five * 4 + three] = 1.0 / 12
+    fs, es = forests(ctx, [(300, 4, False), (200, 5, False)]), []
+    for k in range(2):
+        es.append(dict(snv_rate=[1e-9], indel_rate=[0.0], sbs=sbs, epoch_start=[0.0], exposure=[[1.0]],
+                       n_pre_snv=pre >> k, n_pre_indel=0, pre_sbs=0, indel_max_len=10, indel_len_p=0.5,
+                       infinite_sites=infinite, ploidy=2, drivers=[], germline=[]))
+    want = [O.place_mutations(ref.lengths, packed, of, 3 + k, **es[k]).tobytes() for k, (_, of, _) in enumerate(fs)]
+    batch = core.Mutations.place_batch(ctx, g, [f for f, _, _ in fs], [3, 4], es)
+    for k, (f, of, _) in enumerate(fs):
+        assert batch[k].download().tobytes() == want[k], k
+        assert core.Mutations.place(ctx, g, f, 3 + k, **es[k]).download().tobytes() == want[k], k
