@@ -350,7 +350,8 @@ __device__ uint32_t draw_indel_id(const place_args& a, uint32_t v, uint32_t k, u
 // same for every caller. Bound by the chain of dependent reads of one pass
 // (bases of the word, the homopolymer's ends), once in 64 tries instead of once
 // in each: a forest of 7,128 nodes on 10 Mb with ID signatures: k_place 80 us
-// (2,775 us with one lane's own loop), k_redraw's four rounds 73 us (430 us).
+// (2,775 us with one lane's own loop), k_redraw's four rounds 73 us (430 us),
+// before the searches were spread over more waves (search_lanes_log2).
 template <class JOB>
 __device__ __forceinline__ void finish_searches(const JOB& job, const id_search& mine, psx_mutation& r, uint32_t& st) {
     uint64_t left = __ballot(mine.on);
@@ -384,6 +385,48 @@ __device__ __forceinline__ void finish_searches(const JOB& job, const id_search&
         }
         if (!found && lane == (uint32_t)ln) st |= ST_NO_SITE;
     }
+}
+
+// The search that the first thread of a block left, by all its 256 threads
+// (every one calls it): 256 tries at a time.
+__device__ __forceinline__ void finish_search_block(const place_args& a, const id_search& mine, psx_mutation& r,
+                                                    uint32_t& st) {
+    __shared__ uint32_t s_search[5];
+    __shared__ uint32_t s_hit[2][4][4];  // per pass (two in turn) and wave: found, then the site
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (tid == 0) {
+        s_search[0] = mine.on;
+        s_search[1] = mine.v;
+        s_search[2] = mine.k;
+        s_search[3] = mine.att;
+        s_search[4] = mine.cls;
+    }
+    __syncthreads();
+    const id_search s{s_search[0] != 0u, s_search[1], s_search[2], s_search[3], s_search[4]};
+    bool found = false;
+    if (s.on)
+        for (uint32_t t0 = LANE_TRIES, pass = 0; t0 < SITE_TRIES && !found; t0 += 256u, pass ^= 1u) {
+            uint32_t c = 0, q = 0, payload = 0;
+            const uint32_t t = t0 + tid;
+            const bool ok = t < SITE_TRIES && try_site(a, s, t, c, q, payload);
+            const uint64_t hits = __ballot(ok);
+            uint32_t* const h = s_hit[pass][wave];
+            if (hits && lane == (uint32_t)__builtin_ctzll(hits)) {
+                h[1] = c;
+                h[2] = q;
+                h[3] = payload;
+            }
+            if (lane == 0) h[0] = hits ? 1u : 0u;
+            __syncthreads();
+            for (uint32_t w = 0; w < 4u && !found; ++w)
+                if (s_hit[pass][w][0]) {
+                    const uint32_t* const f = s_hit[pass][w];
+                    if (tid == 0) id_record(a, s.cls, f[1], f[2], f[3], r);
+                    found = true;
+                }
+        }
+    if (s.on && !found && tid == 0) st |= ST_NO_SITE;
+    __syncthreads();  // s_search and s_hit are written again
 }
 
 __device__ uint32_t place_one(const place_args& a, uint64_t id, uint32_t att, psx_mutation& r, id_search& search) {
@@ -644,20 +687,39 @@ __device__ __forceinline__ uint32_t sort_bucket(const batch& B, uint32_t sort_n,
     return (uint32_t)(q >> B.pbits);
 }
 
-// One thread per mutation of every job, first attempt, its sort entry and its
-// place among its bucket's.
+// With ID signatures a mutation of a small table gets several lanes, so that
+// the searches of a wave, served one after another, spread over more waves: as
+// many as leave the GPU SEARCH_LANES in all, and up to SEARCH_BLOCKS mutations
+// a block each, whose four waves search together. 1,500 mutations: k_place 36
+// us (84 with a lane each, 71 with 32: one search's chain of passes), the
+// first redraw round 24 (67).
+constexpr uint64_t SEARCH_LANES = 1u << 17, SEARCH_BLOCKS = 2048;
+constexpr uint32_t BLOCK_LOG2 = 8;
+inline uint32_t search_lanes_log2(bool use_id, uint64_t n) {
+    if (use_id && n <= SEARCH_BLOCKS) return BLOCK_LOG2;
+    uint32_t lg = 0;
+    while (use_id && lg < 5u && (n << (lg + 1u)) <= SEARCH_LANES) ++lg;
+    return lg;
+}
+
+// One lane (the first of 1 << lanes_log2) per mutation of every job: its first
+// attempt, its sort entry and its place among its bucket's.
 __global__ void __launch_bounds__(256) k_place(const batch B, uint64_t n, uint64_t* __restrict__ fkey,
                                                uint32_t* __restrict__ fval, uint32_t* __restrict__ count,
-                                               uint32_t* __restrict__ rank) {
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                               uint32_t* __restrict__ rank, uint32_t lanes_log2) {
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, g = t >> lanes_log2;
+    const bool own = (t & ((1u << lanes_log2) - 1u)) == 0u;
     if (g >= n) return;
     per_job(job_of_seq(B.mbase, B.nj, g), [&](uint32_t j) {
         const place_args& a = cjob(B, j).pa;
         const uint64_t id = g - B.mbase[j];
         psx_mutation r;
         id_search search;
-        uint32_t st = place_one(a, id, 0u, r, search);
-        finish_searches([&](int) -> const place_args& { return a; }, search, r, st);
+        uint32_t st = ST_OK;
+        if (own) st = place_one(a, id, 0u, r, search);
+        if (lanes_log2 == BLOCK_LOG2) finish_search_block(a, search, r, st);
+        else finish_searches([&](int) -> const place_args& { return a; }, search, r, st);
+        if (!own) return;
         if (st != ST_OK) atomicOr(a.status, st);
         a.recs[id] = r;
         const uint64_t key = jkey(B, j, r);
@@ -931,6 +993,7 @@ struct round_io {
 
 struct redraw_args {
     uint32_t round;          // r >= 1: redraws the losers of check r - 1
+    uint32_t lanes_log2;     // lanes per loser
     const uint32_t* list;    // losers of check r - 1 (gids)
     const uint32_t* lapos;   // and their first-check entries (NO_ENTRY once moved)
     uint32_t* moved;         // set for every redrawn gid
@@ -955,9 +1018,10 @@ __global__ void __launch_bounds__(256) k_redraw(const batch B, const redraw_args
         if (blockIdx.x == 0 && threadIdx.x == 0) io->halt = b.round;
         return;
     }
-    for (uint32_t base = blockIdx.x * 256u; base < n; base += gridDim.x * 256u) {
-        const uint32_t t = base + threadIdx.x;
-        const bool on = t < n;
+    const uint32_t per_block = 256u >> b.lanes_log2;
+    for (uint32_t base = blockIdx.x * per_block; base < n; base += gridDim.x * per_block) {
+        const uint32_t t = base + (threadIdx.x >> b.lanes_log2);
+        const bool on = t < n && (threadIdx.x & ((1u << b.lanes_log2) - 1u)) == 0u;
         const uint32_t gid = on ? b.list[t] : 0u;
         const bool first = on && atomicExch(&b.moved[gid], 1u) == 0u;
         const uint32_t slot = block_reserve(first ? 1u : 0u, &io->n_moved);
@@ -983,9 +1047,14 @@ __global__ void __launch_bounds__(256) k_redraw(const batch B, const redraw_args
             a.attempt[id] = att;
             st = place_one(a, id, att, r, search);
         }
-        finish_searches(
-            [&](int ln) -> const place_args& { return cjob(B, (uint32_t)__builtin_amdgcn_readlane((int)j, ln)).pa; },
-            search, r, st);
+        if (b.lanes_log2 == BLOCK_LOG2) {  // one loser: thread 0's
+            const uint32_t jb = job_of(B.mbase, B.nj, b.list[base]);
+            finish_search_block(cjob(B, (uint32_t)__builtin_amdgcn_readfirstlane((int)jb)).pa, search, r, st);
+        } else {
+            finish_searches(
+                [&](int ln) -> const place_args& { return cjob(B, (uint32_t)__builtin_amdgcn_readlane((int)j, ln)).pa; },
+                search, r, st);
+        }
         if (on) {
             const place_args& a = B.jobs[j].pa;
             if (st != ST_OK) atomicOr(a.status, st);
@@ -1870,6 +1939,8 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
         hipLaunchKernelGGL(k_node_expand, dim3(grid_of(N)), dim3(256), 0, s, B, N, d_off, d_node_of);
         PSX_HIP(hipGetLastError());
     }
+    bool use_id = false;
+    for (const place_job& J : jobs) use_id = use_id || J.use_id;
     auto radix_sort = [&] {
         PSX_HIP(hipcub::DeviceRadixSort::SortPairs(d_sort, sort_bytes, d_key, d_key2, d_ids, d_ids2, (int)Mt, 0,
                                                    (int)kbits, s));
@@ -1885,7 +1956,8 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
         // (the entries' ranks and the scattered entries in memory that the later rounds use)
         uint32_t* const rank = few ? nullptr : d_mlist;
         uint4* const entry = (uint4*)d_tab;
-        hipLaunchKernelGGL(k_place, dim3(grid_of(Mt)), dim3(256), 0, s, B, Mt, d_key, d_ids, d_count, rank);
+        const uint32_t lg = search_lanes_log2(use_id, Mt);
+        hipLaunchKernelGGL(k_place, dim3(grid_of(Mt << lg)), dim3(256), 0, s, B, Mt, d_key, d_ids, d_count, rank, lg);
         PSX_HIP(hipGetLastError());
         if (few) {
             radix_sort();
@@ -1958,11 +2030,12 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
                                n_moved, d_tab, (uint32_t)(tab_slots - 1), d_io);
             PSX_HIP(hipGetLastError());
         }
-        const uint32_t grid = std::min<uint32_t>(1024, grid_of(n_lose));
+        const uint32_t lg = search_lanes_log2(use_id, n_lose);
+        const uint32_t grid = std::min<uint32_t>(1024, grid_of((uint64_t)n_lose << lg));
         spec_end = std::min<uint32_t>(round + SPEC_ROUNDS, IS_ROUNDS);
         for (uint32_t r = round; r < spec_end; ++r) {
             redraw_args rd{};
-            rd.round = r; rd.list = d_list[(r - 1) & 1]; rd.lapos = d_lapos[(r - 1) & 1];
+            rd.round = r; rd.lanes_log2 = lg; rd.list = d_list[(r - 1) & 1]; rd.lapos = d_lapos[(r - 1) & 1];
             rd.moved = d_moved; rd.mlist = d_mlist; rd.mapos = d_mapos;
             rd.akey = d_key2; rd.aval = d_ids2; rd.n = Mt; rd.io = d_io;
             rd.tab = d_tab; rd.tab_mask = (uint32_t)(tab_slots - 1);

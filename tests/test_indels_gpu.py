@@ -110,12 +110,13 @@ def test_id_signatures_through_the_engine(ctx):
         eng.place_mutations(sf, 0, 2, seed=1, preneoplastic_indel_signature_name="ID9")
 
 
-@pytest.mark.parametrize("n_indels", [1, 3, 63, 65, 300])
+@pytest.mark.parametrize("n_indels", [1, 3, 63, 65, 300, 3000, 20_000])
 def test_searches_of_rare_classes_share_a_wave(ctx, n_indels):
     """Indels whose class is found by rejection after hundreds of tries (the
-    rarest classes that are not listed), one to many of them in a wave, alone
-    and among the jobs of a batch whose waves hold several jobs, with and
-    without the infinite-sites redraws: every table is the oracle's."""
+    rarest classes that are not listed): with a block, several lanes or one
+    lane for each mutation, alone and among the jobs of a batch whose waves
+    hold several jobs, with and without the infinite-sites redraws (as far as
+    the classes have sites): every table is the oracle's."""
     rng = np.random.default_rng(31)
     ref, _ = genome(rng)
     lens, packed = ref.lengths, ref.packed
@@ -130,7 +131,8 @@ def test_searches_of_rare_classes_share_a_wave(ctx, n_indels):
         fd = cases.forest(n_cells=60 + 20 * k, n_samples=1, sample_size=20, seed=40 + k)
         of = O.Forest(fd["cell_id"], fd["parent"], fd["species"], fd["sample"], fd["birth"], fd["n_samples"])
         f = core.Forest(ctx, fd["cell_id"], fd["parent"], fd["species"], fd["sample"], fd["birth"], fd["n_samples"])
-        eng = cases.engine(packed, lens, snv=2e-7, indel=1e-6, pre_snv=k, pre_indel=n_indels, infinite_sites=k != 2)
+        eng = cases.engine(packed, lens, snv=2e-7, indel=1e-6, pre_snv=k, pre_indel=n_indels,
+                           infinite_sites=k != 2 and n_indels <= 300)
         eng.update(id_sig=sig, id_exposure=[[1.0], [1.0]], pre_id=0)
         fs.append((f, of))
         es.append(eng)
