@@ -589,8 +589,9 @@ __device__ __forceinline__ uint64_t jkey(const batch& B, uint32_t j, const psx_m
 }
 
 // Passenger counts of the edge into every node of every job (none for roots).
-__global__ void __launch_bounds__(256) k_edge_counts(const batch B, uint64_t n) {
+__global__ void __launch_bounds__(256) k_edge_counts(const batch B, uint64_t n, uint64_t* __restrict__ cnt_tot) {
     const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g == n) cnt_tot[n] = 0;  // the end of the scan
     if (g >= n) return;
     per_job(job_of_seq(B.nbase, B.nj, g), [&](uint32_t j) {
         const edge_args& a = cjob(B, j).ea;
@@ -624,8 +625,17 @@ __global__ void __launch_bounds__(256) k_node_bases(const batch B, uint64_t n, c
 // entries together, 64 consecutive entries a pass: each lane finds its
 // entry's node among the 64 first offsets in LDS, so nodes with many
 // passengers need no long loop of one lane.
+// It also clears the rounds' state (io, io_words) and the zeros, whole 16
+// bytes: on small tables a launch is a few microseconds of the placement, and
+// the clears were three.
 __global__ void __launch_bounds__(256) k_node_expand(const batch B, uint64_t n, const uint64_t* __restrict__ off,
-                                                     uint32_t* __restrict__ node_of) {
+                                                     uint32_t* __restrict__ node_of, uint32_t* __restrict__ io,
+                                                     uint32_t io_words, uint4* __restrict__ zeros, uint64_t n_zeros) {
+    {
+        const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, all = (uint64_t)gridDim.x * blockDim.x;
+        for (uint64_t i = t; i < io_words; i += all) io[i] = 0;
+        for (uint64_t i = t; i < n_zeros; i += all) zeros[i] = uint4{0, 0, 0, 0};
+    }
     __shared__ uint64_t s_off[4][64];
     __shared__ uint32_t s_v[4][64];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
@@ -868,11 +878,14 @@ __device__ __forceinline__ void mark_loser(uint32_t* lose, uint32_t stamp, uint3
     }
 }
 
-// Appending kernels take APPEND_ITEMS items per thread (item k of thread t of
-// block b: b * 256 * APPEND_ITEMS + t + 256 k) and reserve their output slots
-// with one atomic per block: atomics on one address serialise (about 12 ns
-// each), so one per item or per wave would cost more than the scan itself.
-constexpr uint32_t APPEND_ITEMS = 16;
+// k_conflicts takes ITEMS items per thread (item k of thread t of block b:
+// b * 256 * ITEMS + t + 256 k) and reserves its output slots with one atomic
+// per block: atomics on one address serialise (about 12 ns each), so one per
+// item or per wave would cost more than the scan itself. An item is a chain of
+// dependent reads of its neighbours, so below APPEND_FEW items, where there are
+// few waves, a thread takes 4: 1.6e5 entries 29 -> 10 us, 1.5e6 34 -> 28; from
+// there on 16, since more blocks' atomics take longer than the reads.
+constexpr uint64_t APPEND_FEW = 2u << 20;
 
 // The calling thread's first slot for n items (every thread of the block calls it).
 __device__ __forceinline__ uint32_t block_reserve(uint32_t n, uint32_t* counter) {
@@ -916,16 +929,17 @@ __device__ __forceinline__ bool loses(const batch& B, const uint64_t* __restrict
     return false;
 }
 
+template <uint32_t ITEMS>
 __global__ void __launch_bounds__(256) k_conflicts(const batch B, const uint64_t* __restrict__ fkey,
                                                    const uint32_t* __restrict__ fval, uint64_t n,
                                                    uint32_t* __restrict__ lose, uint32_t* __restrict__ list,
                                                    uint32_t* __restrict__ apos, uint32_t* __restrict__ n_lose,
                                                    const uint32_t* __restrict__ skew) {
     if (*skew) return;
-    const uint64_t b = (uint64_t)blockIdx.x * 256u * APPEND_ITEMS + threadIdx.x;
-    uint32_t mask = 0, c = 0, gids[APPEND_ITEMS];
+    const uint64_t b = (uint64_t)blockIdx.x * 256u * ITEMS + threadIdx.x;
+    uint32_t mask = 0, c = 0, gids[ITEMS];
 #pragma unroll
-    for (uint32_t k = 0; k < APPEND_ITEMS; ++k) {
+    for (uint32_t k = 0; k < ITEMS; ++k) {
         const uint64_t t = b + 256u * k;
         gids[k] = 0;
         if (t < n && loses(B, fkey, fval, n, t, gids[k])) {
@@ -935,7 +949,7 @@ __global__ void __launch_bounds__(256) k_conflicts(const batch B, const uint64_t
     }
     uint32_t slot = block_reserve(c, n_lose);
 #pragma unroll
-    for (uint32_t k = 0; k < APPEND_ITEMS; ++k)
+    for (uint32_t k = 0; k < ITEMS; ++k)
         if (mask & (1u << k)) {
             lose[gids[k]] = 1u;
             list[slot] = gids[k];
@@ -1067,13 +1081,18 @@ __global__ void __launch_bounds__(256) k_redraw(const batch B, const redraw_args
 
 // The table rebuilt (after the host cleared it) from the moved mutations'
 // current footprints; the halt, if any, is lifted.
-__global__ void __launch_bounds__(256) k_tab_fill(const batch B, const uint32_t* __restrict__ mlist, uint32_t n,
-                                                  uint32_t* tab, uint32_t mask, round_io* io) {
+__global__ void __launch_bounds__(256) k_tab_clear(uint4* __restrict__ tab, uint32_t n16, uint32_t used, round_io* io) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
-        io->tab_used = n;
+        io->tab_used = used;
         io->halt = 0;
     }
+    for (uint32_t i = t; i < n16; i += gridDim.x * blockDim.x) tab[i] = uint4{NO_ENTRY, NO_ENTRY, NO_ENTRY, NO_ENTRY};
+}
+
+__global__ void __launch_bounds__(256) k_tab_fill(const batch B, const uint32_t* __restrict__ mlist, uint32_t n,
+                                                  uint32_t* tab, uint32_t mask) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const uint32_t gid = mlist[t];
     tab_insert(tab, mask, jkey(B, job_of(B.mbase, B.nj, gid), B.recs[gid]), gid);
@@ -1145,8 +1164,10 @@ __global__ void __launch_bounds__(256) k_check(const batch B, const check_args a
 
 // SID order: the moved mutations' current keys (sorted next) ...
 __global__ void __launch_bounds__(256) k_moved_keys(const batch B, const uint32_t* __restrict__ mlist, uint32_t n,
-                                                    uint64_t* __restrict__ key, uint32_t* __restrict__ gids) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+                                                    uint64_t* __restrict__ key, uint32_t* __restrict__ gids,
+                                                    uint32_t* __restrict__ w, uint64_t M) {
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t <= M) w[t] = t < M ? 1u : 0u;  // k_merge_marks' counts
     if (t >= n) return;
     const uint32_t gid = mlist[t];
     key[t] = jkey(B, job_of(B.mbase, B.nj, gid), B.recs[gid]);
@@ -1208,11 +1229,6 @@ __global__ void __launch_bounds__(256) k_merge(const batch B, const merge_args a
         a.okey[o] = a.bkey[k];
         a.ogid[o] = a.bval[k];
     }
-}
-
-__global__ void __launch_bounds__(256) k_fill_u32(uint32_t* __restrict__ p, uint64_t n, uint32_t v, uint32_t last) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = i + 1 == n ? last : v;
 }
 
 // SID order within runs of one key: after the position order (stable: ties
@@ -1329,7 +1345,6 @@ inline int bits_for(uint64_t x) {
 }
 
 inline uint32_t grid_of(uint64_t n) { return (uint32_t)((n + 255) / 256); }
-inline uint32_t grid_append(uint64_t n) { return (uint32_t)((n + 256 * APPEND_ITEMS - 1) / (256 * APPEND_ITEMS)); }
 
 inline uint64_t next_pow2(uint64_t x) {
     uint64_t p = 1;
@@ -1815,11 +1830,8 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
         ea.T = (uint64_t*)at(J.o_T); ea.cnt_snv = d_cnt_snv + nbase[k]; ea.cnt_tot = d_cnt_tot + nbase[k];
     }
     upload_table();
-    PSX_HIP(hipMemsetAsync(d_cnt_tot + N, 0, 8, s));
-    if (N) {
-        hipLaunchKernelGGL(k_edge_counts, dim3(grid_of(N)), dim3(256), 0, s, B, N);
-        PSX_HIP(hipGetLastError());
-    }
+    hipLaunchKernelGGL(k_edge_counts, dim3(grid_of(N + 1)), dim3(256), 0, s, B, N, d_cnt_tot);
+    PSX_HIP(hipGetLastError());
     PSX_HIP(hipcub::DeviceScan::ExclusiveSum(pn + c_scan, scan_bytes, d_cnt_tot, d_off, (int)(N + 1), s));
     hipLaunchKernelGGL(k_node_bases, dim3(grid_of(std::max<uint64_t>(N, nj))), dim3(256), 0, s, B, N, d_off,
                        d_off_job, d_pcount);
@@ -1933,12 +1945,10 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
         tab[k].n_chr = g->n_chr;
     }
     upload_table();
-    PSX_HIP(hipMemsetAsync(dt + t_state, 0, sizeof(round_io) + 4 * nj, s));
-    PSX_HIP(hipMemsetAsync(pm + c_zero, 0, zero_bytes, s));
-    if (N) {
-        hipLaunchKernelGGL(k_node_expand, dim3(grid_of(N)), dim3(256), 0, s, B, N, d_off, d_node_of);
-        PSX_HIP(hipGetLastError());
-    }
+    const uint64_t n_zeros = (zero_bytes + 15) / 16;
+    hipLaunchKernelGGL(k_node_expand, dim3(grid_of(std::max<uint64_t>({N, n_zeros / 8, 1}))), dim3(256), 0, s, B, N, d_off,
+                       d_node_of, (uint32_t*)d_io, (uint32_t)(sizeof(round_io) / 4 + nj), (uint4*)(pm + c_zero), n_zeros);
+    PSX_HIP(hipGetLastError());
     bool use_id = false;
     for (const place_job& J : jobs) use_id = use_id || J.use_id;
     auto radix_sort = [&] {
@@ -1946,8 +1956,9 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
                                                    (int)kbits, s));
     };
     auto first_check = [&] {
-        hipLaunchKernelGGL(k_conflicts, dim3(grid_append(Mt)), dim3(256), 0, s, B, d_key2, d_ids2, Mt, d_lose,
-                           d_list[0], d_lapos[0], &d_io->n_lose[0], &d_io->skew);
+        const uint32_t items = Mt < APPEND_FEW ? 4u : 16u;
+        hipLaunchKernelGGL(items == 4u ? k_conflicts<4> : k_conflicts<16>, dim3((uint32_t)((Mt + 256 * items - 1) / (256 * items))),
+                           dim3(256), 0, s, B, d_key2, d_ids2, Mt, d_lose, d_list[0], d_lapos[0], &d_io->n_lose[0], &d_io->skew);
         PSX_HIP(hipGetLastError());
     };
     if (Mt) {
@@ -2025,10 +2036,14 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
         if (!tab_slots || halted) {
             // cleared, sized for a few rounds of this many losers, refilled with the moved footprints
             tab_slots = std::min(tab_slots_max, next_pow2(std::max<uint64_t>(1024, 8 * ((uint64_t)n_moved + n_lose))));
-            PSX_HIP(hipMemsetAsync(d_tab, 0xFF, tab_slots * 4, s));
-            hipLaunchKernelGGL(k_tab_fill, dim3(std::max<uint32_t>(1, grid_of(n_moved))), dim3(256), 0, s, B, d_mlist,
-                               n_moved, d_tab, (uint32_t)(tab_slots - 1), d_io);
+            hipLaunchKernelGGL(k_tab_clear, dim3(std::min<uint32_t>(2048, grid_of(tab_slots / 4))), dim3(256), 0, s,
+                               (uint4*)d_tab, (uint32_t)(tab_slots / 4), n_moved, d_io);
             PSX_HIP(hipGetLastError());
+            if (n_moved) {
+                hipLaunchKernelGGL(k_tab_fill, dim3(grid_of(n_moved)), dim3(256), 0, s, B, d_mlist, n_moved, d_tab,
+                                   (uint32_t)(tab_slots - 1));
+                PSX_HIP(hipGetLastError());
+            }
         }
         const uint32_t lg = search_lanes_log2(use_id, n_lose);
         const uint32_t grid = std::min<uint32_t>(1024, grid_of((uint64_t)n_lose << lg));
@@ -2084,13 +2099,11 @@ void place_batch(psx_ctx* ctx, const psx_genome* g, std::vector<place_job>& jobs
             // the first loser list's
             uint64_t* bkey = (uint64_t*)d_tab;
             uint32_t* bval = (uint32_t*)(bkey + n_moved);
-            hipLaunchKernelGGL(k_moved_keys, dim3(grid_of(n_moved)), dim3(256), 0, s, B, d_mlist, n_moved, d_key,
-                               d_ids);
+            hipLaunchKernelGGL(k_moved_keys, dim3(grid_of(Mt + 1)), dim3(256), 0, s, B, d_mlist, n_moved, d_key, d_ids,
+                               d_w, Mt);
             PSX_HIP(hipGetLastError());
             PSX_HIP(hipcub::DeviceRadixSort::SortPairs(d_sort, sort_bytes, d_key, bkey, d_ids, bval, (int)n_moved, 0,
                                                        (int)kbits, s));
-            hipLaunchKernelGGL(k_fill_u32, dim3(grid_of(Mt + 1)), dim3(256), 0, s, d_w, Mt + 1, 1u, 0u);
-            PSX_HIP(hipGetLastError());
             hipLaunchKernelGGL(k_merge_marks, dim3(grid_of(n_moved)), dim3(256), 0, s, d_mapos, d_key2, Mt, bkey,
                                n_moved, d_w, d_list[0]);
             PSX_HIP(hipGetLastError());
