@@ -22,6 +22,11 @@
 // 7.11 ms per 1.6e9 reads, 4.5 ms without errors; 10x single-end reads over
 // 300 Mb in windows of 8 strata 1.05 -> 0.57 ms.
 //
+// A template whose errors its first draw does not settle (more than three of
+// them, or two at one base) takes the whole wave 250 instructions; where such
+// templates are more than a few in a thousand (the form with MANY) they wait
+// in LDS until 48 are there, and each lane makes one's errors.
+//
 // Sources are cells of the sample, not leaves: the cells that carry a record
 // are a range of the sample's cells (cells_below of its leaf range), so a
 // template needs no look-up of its leaf. Sequencing errors are drawn per
@@ -139,7 +144,7 @@ __device__ __attribute__((noinline)) void dense_todo(const job_dev* Jp, const se
 }
 
 // Errors of a slow template into list; returns their number (all lanes of a wave call it).
-__device__ __attribute__((noinline)) uint32_t dense_slow(const job_dev* Jp, uint32_t r, uint32_t j, uint32_t c2,
+__device__ __attribute__((noinline)) uint32_t dense_one_slow(const job_dev* Jp, uint32_t r, uint32_t j, uint32_t c2,
                                                          uint32_t* list) {
     const job_dev& J = *Jp;
     wave_sync();
@@ -149,6 +154,113 @@ __device__ __attribute__((noinline)) uint32_t dense_slow(const job_dev* Jp, uint
         wave_template_errors((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, r, j, c2, list, threadIdx.x & 63u);
     wave_sync();
     return n;
+}
+
+// The errors of a slow template per lane (template r, lanes with on): the
+// first K words of its stream that name different bases, in order, f(base
+// index, substitution) for each. Returns the lanes with more than LANE_ERRORS,
+// whose errors the wave has to make (wave_template_errors). A wave's lanes take
+// about 60 vector instructions a word, so some ten for each slow template of
+// 48, where the wave's own pass takes 250 for one.
+constexpr uint32_t LANE_ERRORS = 8;
+template <class F>
+__device__ __forceinline__ unsigned long long lane_errors(const job_dev& J, uint64_t seed, uint32_t r, uint32_t j, uint32_t c2,
+                                                          bool on, const F& f) {
+    psx_u4 w = psx_draw_u(seed, r, j, c2, PSX_P_ERROR << 24);
+    uint32_t lo = 0, hi = on ? J.err_n - 1u : 0u;  // thresholds at or below the count's word
+    while (__ballot(lo < hi)) {
+        if (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (w.y >= J.err_T[mid]) lo = mid + 1u; else hi = mid;
+        }
+    }
+    const uint32_t all = on ? J.err_k0 + lo : 0u, K = all > LANE_ERRORS ? 0u : all;
+    uint32_t c[LANE_ERRORS], cnt = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < LANE_ERRORS; ++i) c[i] = 0xFFFFFFFFu;
+    for (uint32_t t = 0; t < 4u * PSX_ERR_KCAP && __ballot(cnt < K); ++t) {
+        const uint32_t i4 = (t - 3u) & 3u;
+        if (t >= 3u && i4 == 0u) w = psx_draw_u(seed, r, j, c2, (PSX_P_ERROR << 24) | (1u + ((t - 3u) >> 2)));
+        const uint32_t word = t < 3u ? (t == 0u ? w.x : (t == 1u ? w.z : w.w))
+                                     : (i4 == 0u ? w.x : (i4 == 1u ? w.y : (i4 == 2u ? w.z : w.w)));
+        const uint32_t x = psx_mulhi32(word, J.err_N);
+        bool take = cnt < K;
+#pragma unroll
+        for (uint32_t i = 0; i < LANE_ERRORS; ++i) take = take & (c[i] != x);
+#pragma unroll
+        for (uint32_t i = 0; i < LANE_ERRORS; ++i) c[i] = take & (i == cnt) ? x : c[i];
+        cnt += take ? 1u : 0u;
+        if (take) f(x, ((word & 0xFFFFu) * 3u) >> 16);
+    }
+    return __ballot(all > LANE_ERRORS);
+}
+
+// A wave's slow templates that wait (index, copy, start, mate 2's offset of each), and its stratum and window, kept in LDS
+// so that the calls below take no registers of the hot loop.
+constexpr uint32_t SLOW_CAP = 48;
+static_assert(4 * SLOW_CAP <= ELIST, "the waiting templates take the place of one's errors");
+struct slow_list {
+    uint32_t list[ELIST];
+    uint32_t n, j, c2, wb, k0, n_win, cb, pad;
+    const uint32_t* bits;
+    uint64_t pad2;
+};
+
+struct one_list {
+    uint32_t list[ELIST];
+};
+
+// The errors of the waiting templates, corrected where they meet a record of the window; all lanes of a wave call it.
+__device__ __attribute__((noinline)) void dense_slow(const job_dev* Jp, const seg_dev* Sp, slow_list* l) {
+    wave_sync();
+    const uint32_t n = l->n, j = l->j, c2 = l->c2, wb = l->wb, k0 = l->k0, n_win = l->n_win, cb = l->cb;
+    const uint32_t* const bits = l->bits;
+    uint32_t* const list = l->list;
+    const job_dev& J = *Jp;
+    const uint32_t lane = threadIdx.x & 63u;
+    const bool on = lane < n;
+    const uint4 T = ((const uint4*)list)[on ? lane : 0u];  // index, copy, start, offset
+    wave_sync();  // every entry read: the list is free
+    if (lane == 0) l->n = 0;
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)J.seed);
+    const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(J.seed >> 32));
+    const uint64_t seed = (uint64_t)s1 << 32 | s0;
+    const uint32_t RL = J.L;
+    auto error = [&](uint32_t x, uint32_t d, uint32_t X, uint32_t bi, uint32_t sub) {
+        const uint32_t p = bi + (bi >= RL ? x + d - RL : x);
+        if ((bits[p >> 5] >> (p & 31u)) & 1u) dense_todo(Jp, Sp, todo{p | sub << 18, X}, wb, k0, n_win, cb);
+    };
+    unsigned long long big =
+        lane_errors(J, seed, T.x, j, c2, on, [&](uint32_t bi, uint32_t sub) { error(T.z, T.w, T.y, bi, sub); });
+    while (big) {
+        const int ln = __ffsll((long long)big) - 1;
+        big &= big - 1ull;
+        const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)T.x, ln), Xs = (uint32_t)__builtin_amdgcn_readlane((int)T.y, ln);
+        const uint32_t xs = (uint32_t)__builtin_amdgcn_readlane((int)T.z, ln), ds = (uint32_t)__builtin_amdgcn_readlane((int)T.w, ln);
+        const uint32_t ne = wave_template_errors(seed, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane);
+        wave_sync();
+        for (uint32_t k = lane; k < ne; k += 64u) error(xs, ds, Xs, list[k] & 0xFFFFFu, list[k] >> 20);
+        wave_sync();
+    }
+}
+
+// The slow templates of a group (lanes of the mask) wait until SLOW_CAP are there.
+__device__ __attribute__((noinline)) void dense_wait(const job_dev* Jp, const seg_dev* Sp, slow_list* l, unsigned long long slow,
+                                                     uint32_t r, uint32_t X, uint32_t x, uint32_t d) {
+    const uint32_t lane = threadIdx.x & 63u;
+    while (slow) {
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)l->n);
+        const uint32_t at =
+            n + __builtin_amdgcn_mbcnt_hi((uint32_t)(slow >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)slow, 0u));
+        const bool in = ((slow >> lane) & 1ull) && at < SLOW_CAP;
+        if (in) ((uint4*)l->list)[at] = uint4{r, X, x, d};
+        const unsigned long long m = __ballot(in);
+        slow &= ~m;
+        if (lane == 0) l->n = n + (uint32_t)__popcll(m);
+        wave_sync();
+        if (n + (uint32_t)__popcll(m) == SLOW_CAP) dense_slow(Jp, Sp, l);
+        wave_sync();
+    }
 }
 
 // The reads of one bin over a record that shares its position (or has no single range of carriers).
@@ -586,12 +698,13 @@ __device__ __forceinline__ scan_rec load_rec(const job_dev& J, const seg_dev& S,
 }
 
 
-template <bool CNA>
+template <bool CNA, bool MANY>
 __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch L) {
     extern __shared__ uint4 s_dyn[];
     __shared__ count_tables s_tab;
     __shared__ uint32_t s_run, s_acc, s_neff, s_todo_n[2];
-    __shared__ uint32_t s_list[DENSE_WAVES][ELIST];  // per wave: a slow template's errors
+    using slow_store = std::conditional_t<MANY, slow_list, one_list>;
+    __shared__ __align__(16) slow_store s_slow[DENSE_WAVES];  // per wave: a slow template's errors, or those that wait
     __shared__ todo s_todo[TODO_CAP];
     __shared__ cn_window s_cn;  // copy numbers
     uint32_t* const s_bits = (uint32_t*)s_dyn;
@@ -599,7 +712,8 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
     uint32_t* const s_cnt = s_bin + L.bins * BIN_STRIDE;  // two sets: one fills while the other is cleared
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    uint32_t* const list = s_list[wave];
+    slow_store* const sl = &s_slow[wave];
+    uint32_t* const list = sl->list;
     uint32_t in_tab = UNRESOLVED;
     for (uint32_t run = blockIdx.x;;) {
         const item_run R0 = run_of(L, run);
@@ -676,6 +790,18 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                 }
                 scan_rec R{0, 0, 0, REC_NONE};
                 uint32_t dep = 0, alt = 0, set = 0;
+                if constexpr (MANY) {
+                    if (lane == 0) {
+                        sl->n = 0;
+                        sl->j = j;
+                        sl->c2 = c2;
+                        sl->wb = wb;
+                        sl->k0 = k0;
+                        sl->n_win = n_win;
+                        sl->cb = cb;
+                        sl->bits = s_bits;
+                    }
+                }
                 for (uint32_t q0 = 0; q0 < most; q0 += round_t) {
                     uint32_t* const cnt = s_cnt + set * L.bins;
                     // ---- draw the round's templates, drop their reads into bins
@@ -752,41 +878,59 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                             }
                         }
                         // the group's rare events
-                        uint32_t sl_n = 0, sl_k = 0;  // the current slow template's errors and the next one
-                        uint32_t sx = 0, sd = 0, sX = 0;
-                        while (__ballot(ev != 0u) || slow || sl_k < sl_n) {
-                            bool add = false;
-                            todo q{0, 0};
-                            if (__ballot(ev != 0u)) {
-                                add = ev != 0u;
+                        if constexpr (MANY) {
+                            if (slow) dense_wait(&J, &S, sl, slow, r, X, x, d);
+                            while (__ballot(ev != 0u)) {
+                                const bool add = ev != 0u;
                                 const uint32_t f = add ? (uint32_t)__ffs((int)ev) - 1u : 0u;
                                 ev &= ev - 1u;
+                                todo q;
                                 q.at = f < 2u ? (x + (f ? d : 0u)) | TODO_READ
                                               : (f == 2u ? P0 : (f == 3u ? P1 : P2)) | ((subs >> (2u * (f - 2u))) & 3u) << 18;
                                 q.copy = X;
-                            } else if (sl_k < sl_n) {
-                                const uint32_t k = sl_k + lane;
-                                const uint32_t w = k < sl_n ? list[k] : 0u, bi = w & 0xFFFFFu;
-                                const uint32_t p = bi + (bi >= RL ? sx + sd - RL : sx);
-                                add = k < sl_n && ((s_bits[p >> 5] >> (p & 31u)) & 1u);
-                                q.at = p | (w >> 20) << 18;
-                                q.copy = sX;
-                                sl_k += 64u;
-                            } else {  // wave-uniform
-                                const int ln = __ffsll((long long)slow) - 1;
-                                slow &= slow - 1ull;
-                                sx = (uint32_t)__builtin_amdgcn_readlane((int)x, ln);
-                                sd = (uint32_t)__builtin_amdgcn_readlane((int)d, ln);
-                                sX = (uint32_t)__builtin_amdgcn_readlane((int)X, ln);
-                                const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)r, ln);
-                                sl_n = (uint32_t)__builtin_amdgcn_readfirstlane((int)dense_slow(&J, rs, j, c2, list));
-                                sl_k = 0;
-                                continue;
+                                if (add) {
+                                    const uint32_t k = atomicAdd(&s_todo_n[set], 1u);
+                                    if (k < TODO_CAP) s_todo[k] = q;
+                                    else dense_todo(&J, &S, q, wb, k0, n_win, cb);
+                                }
                             }
-                            if (add) {
-                                const uint32_t k = atomicAdd(&s_todo_n[set], 1u);
-                                if (k < TODO_CAP) s_todo[k] = q;
-                                else dense_todo(&J, &S, q, wb, k0, n_win, cb);
+                        } else {
+                            uint32_t sl_n = 0, sl_k = 0;  // the current slow template's errors and the next one
+                            uint32_t sx = 0, sd = 0, sX = 0;
+                            while (__ballot(ev != 0u) || slow || sl_k < sl_n) {
+                                bool add = false;
+                                todo q{0, 0};
+                                if (__ballot(ev != 0u)) {
+                                    add = ev != 0u;
+                                    const uint32_t f = add ? (uint32_t)__ffs((int)ev) - 1u : 0u;
+                                    ev &= ev - 1u;
+                                    q.at = f < 2u ? (x + (f ? d : 0u)) | TODO_READ
+                                                  : (f == 2u ? P0 : (f == 3u ? P1 : P2)) | ((subs >> (2u * (f - 2u))) & 3u) << 18;
+                                    q.copy = X;
+                                } else if (sl_k < sl_n) {
+                                    const uint32_t k = sl_k + lane;
+                                    const uint32_t w = k < sl_n ? list[k] : 0u, bi = w & 0xFFFFFu;
+                                    const uint32_t p = bi + (bi >= RL ? sx + sd - RL : sx);
+                                    add = k < sl_n && ((s_bits[p >> 5] >> (p & 31u)) & 1u);
+                                    q.at = p | (w >> 20) << 18;
+                                    q.copy = sX;
+                                    sl_k += 64u;
+                                } else {  // wave-uniform
+                                    const int ln = __ffsll((long long)slow) - 1;
+                                    slow &= slow - 1ull;
+                                    sx = (uint32_t)__builtin_amdgcn_readlane((int)x, ln);
+                                    sd = (uint32_t)__builtin_amdgcn_readlane((int)d, ln);
+                                    sX = (uint32_t)__builtin_amdgcn_readlane((int)X, ln);
+                                    const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)r, ln);
+                                    sl_n = (uint32_t)__builtin_amdgcn_readfirstlane((int)dense_one_slow(&J, rs, j, c2, list));
+                                    sl_k = 0;
+                                    continue;
+                                }
+                                if (add) {
+                                    const uint32_t k = atomicAdd(&s_todo_n[set], 1u);
+                                    if (k < TODO_CAP) s_todo[k] = q;
+                                    else dense_todo(&J, &S, q, wb, k0, n_win, cb);
+                                }
                             }
                         }
                         if (!more) break;
@@ -845,6 +989,9 @@ __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch
                         }
                     }
                     __syncthreads();
+                }
+                if constexpr (MANY) {
+                    if (__builtin_amdgcn_readfirstlane((int)sl->n)) dense_slow(&J, &S, sl);
                 }
                 __syncthreads();
             }

@@ -23,6 +23,14 @@ namespace psxh {
 // Covered positions per 64 templates from which a job counts by windows: on 1.6e9 reads with errors k_count_sparse takes
 // 3.8 ms at 10 and 5.2 at 19, k_count_dense 6.0 and 6.2; without errors 3.5 (10) and 4.7 (19) against 3.7 and 3.8.
 constexpr double DENSE_COVER = 28.0, DENSE_COVER_NO_ERRORS = 8.0;
+// Share of templates with more than three errors from which the dense kernel lets them wait and makes their errors 48
+// templates at a time (5.6e7 templates of 250 bases: 0.013 % of them 0.46 ms by one after another, 0.53 by 48; 1.7 %
+// 1.01 and 0.90; 14 % 3.85 and 1.55; of 150 bases: 0.33 % 1.05 and 1.06).
+constexpr double MANY_SLOW = 0.006;
+// And from which share on it takes jobs of fewer covered positions: the sparse kernel makes the errors of each such read
+// one after another (14 %, 250 bases: 1.80 ms at 23 covered
+// positions, 1.48 at 17, against 1.42 and 1.42).
+constexpr double SLOW_READS = 0.06, DENSE_COVER_SLOW = 15.0;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
 // templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves.
 constexpr uint64_t FEW_ITEMS = 2048, MANY_ITEMS = 4096;
@@ -43,6 +51,8 @@ struct seq_batch {
     std::vector<size_t> tab_off;  // per job: insert thresholds, insert guide, error thresholds
     std::vector<size_t> cna_off;  // per job: copy-number events (SIZE_MAX: none)
     std::vector<uint64_t> job_reads;  // per job: reads of the sampling model without copy-number events
+    std::vector<double> job_slow;   // per job: share of its templates with more than three errors
+    double slow_templates = 0.0;    // such templates of the dense jobs
     std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
     std::vector<uint8_t> job_fits;  // per job: its source copies fit the dense count kernel's words
     bool cna_sparse = false, cna_dense = false;  // copy-number events among the sparse / the other jobs
@@ -236,6 +246,8 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
         if (bases > 0.0) cover = 64.0 * (pe ? 2.0 : 1.0) * L * recs / bases * kept / bases;
     }
     P.job_cover.push_back(cover);
+    const uint32_t past = err.k0 > 3u ? 0u : 3u - err.k0;  // K > 3: the draw at or past this threshold
+    P.job_slow.push_back(err.k0 > 3u ? 1.0 : past + 1u < err.T.size() ? 1.0 - (double)err.T[past] * 0x1p-32 : 0.0);
     P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;
     for (uint32_t so = 0; so < n_out; ++so) {
@@ -282,7 +294,9 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
 // A job whose reads cover few positions queues the reads that cover any
 // (k_count_sparse), the others count by windows (k_count_dense).
 bool job_sparse(const seq_batch& P, uint32_t job) {
-    return !P.job_fits[job] || P.job_cover[job] < (P.jobs[job].err_n ? DENSE_COVER : DENSE_COVER_NO_ERRORS);
+    return !P.job_fits[job] || P.job_cover[job] < (!P.jobs[job].err_n           ? DENSE_COVER_NO_ERRORS
+                                                   : P.job_slow[job] > SLOW_READS ? DENSE_COVER_SLOW
+                                                                                  : DENSE_COVER);
 }
 
 // Strata, bins and items of a segment in the count kernels (parts: layout). A
@@ -342,6 +356,7 @@ void layout(seq_batch& P) {
         } else {
             const job_dev& J = P.jobs[S.job];
             const uint64_t starts = std::min<uint64_t>(S.W, (uint64_t)PSX_STRATUM << seg_lns(S));  // of a window
+            P.slow_templates += (double)S.T * P.job_slow[S.job];
             if (P.count) {
                 // a stratum's share, rounded up, in rounds of whole groups of 64 templates
                 const uint64_t stratum =
@@ -483,10 +498,10 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
         Ld.bins = P->dense_bins;
         Ld.bit_words = dense_bit_words(P->dense_bits);
         const uint32_t lds = dense_lds(P->dense_bins, P->dense_bits);
-        if (P->cna_dense)
-            hipLaunchKernelGGL(k_count_dense<true>, dim3((uint32_t)grid), dim3(DENSE_BLOCK), lds, lane.stream, Ld);
-        else
-            hipLaunchKernelGGL(k_count_dense<false>, dim3((uint32_t)grid), dim3(DENSE_BLOCK), lds, lane.stream, Ld);
+        const bool many = P->slow_templates > MANY_SLOW * (double)(P->templates - P->templates_sparse);
+        auto* const kernel = P->cna_dense ? (many ? k_count_dense<true, true> : k_count_dense<true, false>)
+                                          : (many ? k_count_dense<false, true> : k_count_dense<false, false>);
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(DENSE_BLOCK), lds, lane.stream, Ld);
     }
     PSX_HIP(hipGetLastError());
     if (timed) PSX_HIP(hipEventRecord(lane.ev1, lane.stream));

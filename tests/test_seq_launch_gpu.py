@@ -126,6 +126,24 @@ def test_copy_number_draws(ctx, snv, cov, ploidy, cna):
         assert m == on and np.array_equal(rows.numpy()[:m], ref)
 
 
+@pytest.mark.parametrize("kw", [
+    # shares of templates with more than three errors below and above the rule; more than eight errors; reads of few bases
+    dict(read_size=150, error_rate=3e-3), dict(read_size=250, error_rate=4e-3),
+    dict(read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=1e-2, purity=0.5),
+    dict(read_size=200, error_rate=6e-2), dict(read_size=5, error_rate=0.6)])
+@pytest.mark.parametrize("cna", [False, True])
+def test_templates_of_many_errors(ctx, kw, cna):
+    """Templates whose errors the first draw does not settle, on dense tables: waiting ones counted 48 at a time, the
+    last ones of a window, with and without copy numbers."""
+    from process_amd import _abi as A
+    eng = dict(cna=[(0, 0, 5_000, 30_000, 0, A.PSX_CNA_AMP, 2), (1, 0, 0, 0, 0, A.PSX_CNA_WGD, 0)]) if cna else {}
+    w = World(ctx, [60_000, 20_000], dict(n_cells=500, n_samples=1, sample_size=90, seed=2), 2e-4, **eng)
+    kw = dict(kw, coverage=150)
+    a, d, p, _ = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)
+    oa, od, op, _ = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), **kw)
+    assert np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op) and d.sum() > 0
+
+
 def test_parts_of_few_strata(ctx):
     """Few strata with many templates: items are cut into parts, in both count kernels."""
     forest = dict(n_cells=300, n_samples=1, sample_size=60, seed=4)
