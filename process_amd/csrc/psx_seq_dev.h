@@ -72,7 +72,7 @@ struct job_dev {
 struct seg_dev {
     uint64_t T;             // templates of the segment
     uint32_t sample;        // the forest sample (tumour samples)
-    uint32_t shape;         // count kernels: seg_cb | seg_lns << 8 | seg_lw << 12 | seg_parts << 16
+    uint32_t shape;         // seg_parts << 16, and for the count kernels seg_cb | seg_lns << 8 | seg_lw << 12
     union {
         uint64_t read_base;  // materialisation: first read index of the segment
         struct {             // dense count kernel: most templates of an item's part of a stratum, and of a round of it
@@ -1073,10 +1073,17 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
             // only the templates whose copy slot is a copy of their source have reads: k_cn_accept left a bit for each;
             // they are numbered by chunks of CN_CHUNK groups of 64, and a lane finds its template by its number.
             const bool cn = CNA && S.n_cna != 0u;
-            uint64_t row = cn ? uniform_at(J.cn_row, S.st_off + j) : S.read_base + s.before * rpt;
+            // the item's part of the stratum's templates (one part with copy numbers): [p0, p0 + part_n)
+            uint32_t p0 = 0, part_n = nj;
+            if (seg_parts(S) != 1u) {
+                const uint32_t share = ((nj + seg_parts(S) - 1u) / seg_parts(S) + 63u) & ~63u;
+                p0 = min(nj, it.part * share);
+                part_n = min(share, nj - p0);
+            }
+            uint64_t row = cn ? uniform_at(J.cn_row, S.st_off + j) : S.read_base + (s.before + p0) * rpt;
             const uint32_t n_grp = cn ? (nj + 63u) >> 6 : 1u;
             for (uint32_t g0 = 0; g0 < n_grp; g0 += CN_CHUNK) {
-            uint32_t nk = nj;  // templates with reads (of the chunk)
+            uint32_t nk = part_n;  // templates with reads (of the chunk)
             if (CNA && cn) {
                 __syncthreads();  // the chunk before is done
                 const uint64_t* const mask = L.cn_kept + S.read_base + (uint64_t)j * cn_groups(S) + g0;
@@ -1124,7 +1131,7 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
                 const uint32_t cend = min(vb + 64u - o, nk);
                 const uint32_t n_t = cend > c0 ? cend - c0 : 0u;
                 const uint64_t first0 = row + (uint64_t)c0 * rpt;
-                uint32_t tx = 0, tx2 = 0, tla = 0, tr = c0 + lane;
+                uint32_t tx = 0, tx2 = 0, tla = 0, tr = p0 + c0 + lane;
                 if (CNA && cn) {
                     if (lane < n_t) {
                         uint32_t a = 0;  // the group of kept template tr

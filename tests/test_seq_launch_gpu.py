@@ -145,10 +145,13 @@ def test_templates_of_many_errors(ctx, kw, cna):
 
 
 def test_parts_of_few_strata(ctx):
-    """Few strata with many templates: items are cut into parts, in both count kernels."""
+    """Few strata with many templates: items are cut into parts, in both count kernels and the read kernel."""
     forest = dict(n_cells=300, n_samples=1, sample_size=60, seed=4)
     for snv in (2e-7, 1e-4):
         w = World(ctx, [20_000, 5_000], forest, snv)
         for kw in (dict(coverage=6000, read_size=101, error_rate=5e-3, purity=0.7),
                    dict(coverage=4000, read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=1e-3)):
-            w.check(core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 5, **kw)[:3], 5, kw)
+            n = w.check(core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 5, **kw)[:3], 5, kw)
+            rows, m = core.simulate_seq_reads(ctx, w.g, w.pf, w.pm, 5, **kw)
+            assert m == n and np.array_equal(rows.numpy()[:m],
+                                             O.simulate_reads(w.lens, w.g.download(), w.of, w.recs, 5, m, **kw))
