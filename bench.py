@@ -36,7 +36,7 @@ SERVE_OVERLAP_US = 250
 # rocprofv3 summaries under profiles/, named for the kernel and workload). Count-only sequencing is bound by
 # vector instruction issue, not HBM; the probe kernels' instruction counts per lane-iteration come from the
 # same counter (profiles/k_probe_valu.md).
-PROFILED = {"k_seq_count": dict(traffic=302.1e6, valu_insts=6.206e9),
+PROFILED = {"k_count_dense": dict(valu_insts=4.068e9),
             "k_seq_reads": dict(traffic=77.42e9),
             # batched read materialisation of the 256-job batched workload's leading 19 jobs
             "k_seq_reads_batched": dict(traffic=72.54e9),
@@ -658,9 +658,9 @@ def main() -> int:
     leaves = int(sum(int((w.forest["sample"] == s).sum()) for s in range(w.forest["n_samples"])))
     algo_bytes = 16 * M + 8 * M * S + 4 * leaves
     achieved = algo_bytes / (kernel_ms / 1e3) / 1e9
-    prof = PROFILED["k_seq_count"] if args.cells == 1_000_000 else {}
+    prof = PROFILED["k_count_dense"] if args.cells == 1_000_000 else {}
     roofline = dict(bound="hbm", achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s", frac=achieved / HBM_PEAK_GBS,
-                    traffic=prof.get("traffic"), kernel="k_seq_count", kernel_ms=kernel_ms, algo_bytes=algo_bytes)
+                    traffic=prof.get("traffic"), kernel="k_count_dense", kernel_ms=kernel_ms, algo_bytes=algo_bytes)
     # the bound that applies: vector instruction issue, against the probe kernels' rate on this GPU
     ceil = valu_ceiling(ctx)
     valu = dict(probe=ceil, note="count-only moves ~0.04 B per read; vector instruction issue bounds it")
