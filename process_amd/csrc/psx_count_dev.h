@@ -308,14 +308,15 @@ __device__ __forceinline__ const T& uniform_ref(const T* p) {
 
 // A template of any ploidy and any copy-number events; out of line, so that its registers are not the loops'.
 struct general_draw {
-    uint32_t x, cell, allele, ins;  // allele | (kept) << 8
+    uint32_t x, cell, allele, ins;
+    uint32_t kept;  // a word of its own: the allele of a draw that is not kept is any copy slot
 };
 template <bool CNA>
 __device__ __attribute__((noinline)) general_draw draw_general(const job_dev* J, const seg_dev* S, uint32_t r, uint32_t j,
                                                                uint32_t b, uint32_t e) {
     psx_u4 w;
     const tmpl t = template_source<CNA, false>(uniform_ref(J), uniform_ref(S), r, j, b, e, w);
-    return general_draw{t.x, t.cell, t.allele | t.ok << 8, w.w};
+    return general_draw{t.x, t.cell, t.allele, w.w, t.ok};
 }
 
 // What a segment's template draws use, read once per item. A diploid source
@@ -357,8 +358,8 @@ struct source_draw {
             const general_draw t = draw_general<CNA>(&J, &S, r, j, b, e);
             x = t.x - wb;
             cell = t.cell;
-            al = t.allele & 0xFFu;
-            ok = (t.allele >> 8) != 0u;
+            al = t.allele;
+            ok = t.kept != 0u;
             w.w = t.ins;
         }
         ins = w.w;

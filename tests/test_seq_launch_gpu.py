@@ -126,6 +126,31 @@ def test_copy_number_draws(ctx, snv, cov, ploidy, cna):
         assert m == on and np.array_equal(rows.numpy()[:m], ref)
 
 
+@pytest.mark.parametrize("snv", [3e-7, 6e-5])
+@pytest.mark.parametrize("cov,ploidy,cna", [
+    # draws of the general form with hundreds of copy slots: eight doublings, three lineages, more events than are listed
+    (4.0, 2, [(0, 0, 0, 0, 0, WGD, 0)] * 8),
+    (8.0, 3, [(0, 1, 0, 9_000, 0, AMP, 255), (0, 1, 0, 9_000, 1, AMP, 255)]),
+    (2.0, 2, [(0, 1, 300 * k, 5_000, k & 1, AMP, 255) for k in range(17)])])
+def test_copy_number_draws_of_many_slots(ctx, snv, cov, ploidy, cna):
+    """A template of the normal genome draws one of the chromosome's copy slots, of which only the first ploidy are its
+    copies, however many slots there are: sparse and dense tables, a tumour sample with a normal share and the normal
+    sample; the materialised reads are as many."""
+    from process_amd import _abi as A
+    kinds = [A.PSX_CNA_AMP, A.PSX_CNA_DEL, A.PSX_CNA_WGD]
+    w = World(ctx, [40_000, 10_000], dict(n_cells=500, n_samples=1, sample_size=90, seed=2), snv,
+              cna=[(sp, c, at, ln, a, kinds[k], n) for sp, c, at, ln, a, k, n in cna], ploidy=ploidy,
+              infinite_sites=False, n_pre_snv=6_000 if snv > 1e-6 else 8)
+    for kw in (dict(read_size=75, error_rate=2e-3, purity=0.7), dict(read_size=250, insert_size_mean=600,
+                                                                    insert_size_stddev=10, purity=0.7)):
+        kw["coverage"] = cov
+        a, d, p, _ = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)
+        oa, od, op, on = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), ploidy=ploidy, **kw)
+        assert np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op)
+        _, m = core.simulate_seq_reads(ctx, w.g, w.pf, w.pm, 3, **kw)
+        assert m == on
+
+
 @pytest.mark.parametrize("kw", [
     # shares of templates with more than three errors below and above the rule; more than eight errors; reads of few bases
     dict(read_size=150, error_rate=3e-3), dict(read_size=250, error_rate=4e-3),
