@@ -109,22 +109,34 @@ static psx_ctable error_ctable(uint32_t N, double e, uint32_t L) {
     return t;
 }
 
-// Largest copy number of any leaf on a chromosome (at least the ploidy): the
-// copy numbers change only at event boundaries, in leaf rank and position.
-static uint32_t cna_kmax(const std::vector<psx_cna_dev>& ev, uint32_t n_leaves, uint32_t len, uint32_t ploidy) {
-    std::vector<uint32_t> leaves{0}, xs{0};
+// Copy numbers on a chromosome: the largest of any leaf (at least the ploidy) and the mean over leaves and positions.
+// They change only at event boundaries, in leaf rank and position.
+struct cna_numbers {
+    uint32_t most;
+    double mean;
+};
+static cna_numbers cna_range(const std::vector<psx_cna_dev>& ev, uint32_t n_leaves, uint32_t len, uint32_t ploidy) {
+    std::vector<uint32_t> leaves{0, n_leaves}, xs{0, len};
     for (const psx_cna_dev& e : ev) {
-        leaves.push_back(e.lo);
-        if (e.hi < n_leaves) leaves.push_back(e.hi);
-        xs.push_back(e.start);
-        if (e.end < len) xs.push_back(e.end);
+        leaves.push_back(std::min(e.lo, n_leaves));
+        leaves.push_back(std::min(e.hi, n_leaves));
+        xs.push_back(std::min(e.start, len));
+        xs.push_back(std::min(e.end, len));
     }
-    uint32_t best = ploidy, cn[PSX_MAX_CNA_PLOIDY];
-    for (uint32_t l : leaves) {
-        if (l >= n_leaves) continue;
-        for (uint32_t x : xs) best = std::max(best, psx_cna_copies(ev.data(), (uint32_t)ev.size(), l, x, ploidy, cn));
+    for (std::vector<uint32_t>* v : {&leaves, &xs}) {
+        std::sort(v->begin(), v->end());
+        v->erase(std::unique(v->begin(), v->end()), v->end());
     }
-    return best;
+    cna_numbers r{ploidy, 0.0};
+    uint32_t cn[PSX_MAX_CNA_PLOIDY];
+    for (size_t a = 0; a + 1 < leaves.size(); ++a)
+        for (size_t b = 0; b + 1 < xs.size(); ++b) {
+            const uint32_t c = psx_cna_copies(ev.data(), (uint32_t)ev.size(), leaves[a], xs[b], ploidy, cn);
+            r.most = std::max(r.most, c);
+            r.mean += (double)c * (double)(leaves[a + 1] - leaves[a]) * (double)(xs[b + 1] - xs[b]);
+        }
+    r.mean /= std::max(1.0, (double)n_leaves * (double)len);
+    return r;
 }
 
 bool batch_has_cna(const seq_batch* b);
@@ -215,6 +227,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     // copy-number events per chromosome (doublings on every chromosome), in DFS order
     std::vector<psx_cna_dev> cdev;
     std::vector<uint32_t> c_off(g->n_chr, 0), c_n(g->n_chr, 0), c_kmax(g->n_chr, ploidy);
+    std::vector<double> c_mean(g->n_chr, (double)ploidy);
     for (uint32_t c = 0; c < g->n_chr && !m->cna.empty(); ++c) {
         std::vector<psx_cna_dev> ev;
         for (const psx_cna_event& e : m->cna)
@@ -223,7 +236,9 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
                                          e.chr == c ? e.end : g->len[c], psx_cna_code(e)});
         c_off[c] = (uint32_t)cdev.size();
         c_n[c] = (uint32_t)ev.size();
-        c_kmax[c] = cna_kmax(ev, f->n_leaves, g->len[c], ploidy);
+        const cna_numbers cn = cna_range(ev, f->n_leaves, g->len[c], ploidy);
+        c_kmax[c] = cn.most;
+        c_mean[c] = cn.mean;
         if ((uint64_t)f->n_leaves * c_kmax[c] >= (uint64_t(1) << 32))
             psx_throw(PSX_EINVAL, "too many cell copies (%u copies on chromosome %u)", c_kmax[c], c);
         if (c_kmax[c] > 0xFFFFu)
@@ -234,14 +249,18 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     P.jobs.push_back(J);
     double cover = 0.0;
     {
-        // expected positions covered by 64 templates: records per base x bases read, times the share of
-        // templates kept under copy numbers (ploidy / kmax, length-weighted)
+        // expected positions covered by 64 templates: records per base x bases read, times the share of templates
+        // kept under copy numbers (length-weighted): the source's copies among kmax slots, a cell's (their mean over
+        // the leaves) or the normal genome's. With ploidy / kmax for the share, a table of 200,000 records at 60x under
+        // four doublings, 220 positions, was taken for one of 14: 2,740 -> 1,000 us
+        const double normal = std::min(1.0, (double)J.thr_normal * 0x1p-32);
+        const double tumour = n_out ? (double)n_req / (double)n_out * (1.0 - normal) : 0.0;
         double recs = 0.0, bases = 0.0, kept = 0.0;
         for (uint32_t c = 0; c < g->n_chr; ++c) {
             if (!sel[c] || g->len[c] < L) continue;
             recs += (double)(m->chr_begin[c + 1] - m->chr_begin[c]);
             bases += (double)g->len[c];
-            kept += (double)g->len[c] * (double)ploidy / (double)c_kmax[c];
+            kept += (double)g->len[c] * (tumour * c_mean[c] + (1.0 - tumour) * (double)ploidy) / (double)c_kmax[c];
         }
         if (bases > 0.0) cover = 64.0 * (pe ? 2.0 : 1.0) * L * recs / bases * kept / bases;
     }
