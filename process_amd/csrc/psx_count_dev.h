@@ -151,21 +151,20 @@ __device__ __attribute__((noinline)) uint32_t dense_one_slow(const job_dev* Jp, 
     const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)J.seed);
     const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(J.seed >> 32));
     const uint32_t n =
-        wave_template_errors((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, r, j, c2, list, threadIdx.x & 63u);
+        wave_template_errors<true>((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, r, j, c2, list, threadIdx.x & 63u);
     wave_sync();
     return n;
 }
 
 // The errors of a slow template per lane (template r, lanes with on): the
 // first K words of its stream that name different bases, in order, f(base
-// index, substitution) for each. Returns the lanes with more than LANE_ERRORS,
+// index, substitution) for each. Returns the lanes with more than MOST (number),
 // whose errors the wave has to make (wave_template_errors). A wave's lanes take
-// about 60 vector instructions a word, so some ten for each slow template of
-// 48, where the wave's own pass takes 250 for one.
-constexpr uint32_t LANE_ERRORS = 8;
-template <class F>
+// about 44 + 2 MOST vector instructions a word, so some ten for each slow
+// template of 48, where the wave's own pass takes 250 for one.
+template <uint32_t MOST, class F>
 __device__ __forceinline__ unsigned long long lane_errors(const job_dev& J, uint64_t seed, uint32_t r, uint32_t j, uint32_t c2,
-                                                          bool on, const F& f) {
+                                                          bool on, uint32_t& number, const F& f) {
     psx_u4 w = psx_draw_u(seed, r, j, c2, PSX_P_ERROR << 24);
     uint32_t lo = 0, hi = on ? J.err_n - 1u : 0u;  // thresholds at or below the count's word
     while (__ballot(lo < hi)) {
@@ -174,10 +173,11 @@ __device__ __forceinline__ unsigned long long lane_errors(const job_dev& J, uint
             if (w.y >= J.err_T[mid]) lo = mid + 1u; else hi = mid;
         }
     }
-    const uint32_t all = on ? J.err_k0 + lo : 0u, K = all > LANE_ERRORS ? 0u : all;
-    uint32_t c[LANE_ERRORS], cnt = 0;
+    const uint32_t all = on ? J.err_k0 + lo : 0u, K = all > MOST ? 0u : all;
+    number = all;
+    uint32_t c[MOST], cnt = 0;
 #pragma unroll
-    for (uint32_t i = 0; i < LANE_ERRORS; ++i) c[i] = 0xFFFFFFFFu;
+    for (uint32_t i = 0; i < MOST; ++i) c[i] = 0xFFFFFFFFu;
     for (uint32_t t = 0; t < 4u * PSX_ERR_KCAP && __ballot(cnt < K); ++t) {
         const uint32_t i4 = (t - 3u) & 3u;
         if (t >= 3u && i4 == 0u) w = psx_draw_u(seed, r, j, c2, (PSX_P_ERROR << 24) | (1u + ((t - 3u) >> 2)));
@@ -186,13 +186,13 @@ __device__ __forceinline__ unsigned long long lane_errors(const job_dev& J, uint
         const uint32_t x = psx_mulhi32(word, J.err_N);
         bool take = cnt < K;
 #pragma unroll
-        for (uint32_t i = 0; i < LANE_ERRORS; ++i) take = take & (c[i] != x);
+        for (uint32_t i = 0; i < MOST; ++i) take = take & (c[i] != x);
 #pragma unroll
-        for (uint32_t i = 0; i < LANE_ERRORS; ++i) c[i] = take & (i == cnt) ? x : c[i];
+        for (uint32_t i = 0; i < MOST; ++i) c[i] = take & (i == cnt) ? x : c[i];
         cnt += take ? 1u : 0u;
         if (take) f(x, ((word & 0xFFFFu) * 3u) >> 16);
     }
-    return __ballot(all > LANE_ERRORS);
+    return __ballot(all > MOST);
 }
 
 // A wave's slow templates that wait (index, copy, start, mate 2's offset of each), and its stratum and window, kept in LDS
@@ -230,14 +230,16 @@ __device__ __attribute__((noinline)) void dense_slow(const job_dev* Jp, const se
         const uint32_t p = bi + (bi >= RL ? x + d - RL : x);
         if ((bits[p >> 5] >> (p & 31u)) & 1u) dense_todo(Jp, Sp, todo{p | sub << 18, X}, wb, k0, n_win, cb);
     };
+    uint32_t number;
     unsigned long long big =
-        lane_errors(J, seed, T.x, j, c2, on, [&](uint32_t bi, uint32_t sub) { error(T.z, T.w, T.y, bi, sub); });
+        lane_errors<8>(J, seed, T.x, j, c2, on, number, [&](uint32_t bi, uint32_t sub) { error(T.z, T.w, T.y, bi, sub); });
     while (big) {
         const int ln = __ffsll((long long)big) - 1;
         big &= big - 1ull;
         const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)T.x, ln), Xs = (uint32_t)__builtin_amdgcn_readlane((int)T.y, ln);
         const uint32_t xs = (uint32_t)__builtin_amdgcn_readlane((int)T.z, ln), ds = (uint32_t)__builtin_amdgcn_readlane((int)T.w, ln);
-        const uint32_t ne = wave_template_errors(seed, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane);
+        const uint32_t ne = wave_template_errors<true>(seed, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane,
+                                                 (uint32_t)__builtin_amdgcn_readlane((int)number, ln));
         wave_sync();
         for (uint32_t k = lane; k < ne; k += 64u) error(xs, ds, Xs, list[k] & 0xFFFFFu, list[k] >> 20);
         wave_sync();
@@ -448,6 +450,12 @@ __device__ __forceinline__ bool plain_record(uint32_t info) {
 // one record per 13,000 bases 559 -> 357 us, 1.5 Mb at 2000x 500 -> 447 us.
 // With a bit per 32 starts instead of 8 (more reads queued in vain) 362 and
 // 486 us.
+//
+// A queued read whose template's errors its first draw does not settle is
+// counted without them, and the wave makes them, 250 vector instructions a
+// template; where such templates are many (the form with MANY) the reads wait
+// until 48 do, and each lane makes one's: 2.8e7 reads of 250 bases at 0.8 %
+// 1.38 -> 0.50 ms, pairs of 150 at 2 % 6.6 -> 1.4 ms.
 
 // An entry of a wave's queue: a read.
 struct sparse_read {
@@ -457,10 +465,13 @@ struct sparse_read {
 };
 
 constexpr uint32_t START_SHIFT = 3;  // starts per bit of the reach bitmap
+constexpr uint32_t WAIT_FULL = 48;  // reads that wait before their templates' errors are made, and room for a queue's more
+constexpr uint32_t WAIT_READS = WAIT_FULL + 64;
 
-template <int BLOCK, int CAP>
+template <int BLOCK, int CAP, bool MANY>
 struct sparse_lds {
     static constexpr uint32_t WAVES = BLOCK / 64;
+    static constexpr bool SLOW_WAIT = MANY;
     static constexpr uint32_t START_BITS = ((PSX_STRATUM * WAVES + MAX_READ) >> START_SHIFT) + 1u;
     count_tables tab;
     uint32_t err[4];                         // thresholds of 1 to 4 errors, padded
@@ -468,6 +479,8 @@ struct sparse_lds {
     uint32_t dep[CAP], alt[CAP];
     uint32_t bits[(START_BITS + 31u) / 32u];
     sparse_read queue[WAVES][128];
+    sparse_read wait[WAVES][MANY ? WAIT_READS : 1u];  // counted reads of slow templates, whose errors are not made yet
+    uint32_t wait_n[WAVES];
     uint32_t run, acc;
 };
 static_assert(64 * sizeof(sparse_read) >= 4 * ELIST, "a slow template's errors take the place of the entries counted");
@@ -491,6 +504,71 @@ __device__ __forceinline__ void stage_record(const job_dev& J, const seg_dev& S,
     lds.low[i] = lo;
     lds.len[i] = len;
     lds.info[i] = (info & ~(REC_SKIP | REC_SHARED)) | flag;
+}
+
+// The errors of the slow templates of the last 64 reads that wait: each lane makes one's, up to 16 of them (lane_errors), and corrects
+// the counts at those on the read that meet a record; the wave makes the others', one template after another (in list,
+// ELIST words). All lanes of a wave call it.
+template <class LDS>
+__device__ __attribute__((noinline)) void count_slow(const job_dev* Jp, const seg_dev* Sp, LDS* lds, uint32_t* list,
+                                                     uint32_t wb, uint32_t k0, uint32_t n_win, uint32_t n_lds, uint32_t j,
+                                                     uint32_t c2) {
+    const job_dev& J = *Jp;
+    const seg_dev& S = *Sp;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    wave_sync();
+    const uint32_t n = lds->wait_n[wave], from = n > 64u ? n - 64u : 0u;
+    const bool on = from + lane < n;
+    const sparse_read R = on ? lds->wait[wave][from + lane] : sparse_read{0u, 0u, 0u};
+    wave_sync();  // every lane has read its entry
+    if (lane == 0) lds->wait_n[wave] = from;
+    const uint32_t RL = J.L;
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)J.seed);
+    const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(J.seed >> 32));
+    const uint64_t seed = (uint64_t)s1 << 32 | s0;
+    const glb_view gv = window_view(J, S, k0, n_win);
+    uint32_t a0 = 0;  // the read's first record
+    for (uint32_t z = on ? n_lds : 0u; a0 < z;) {
+        const uint32_t mid = (a0 + z) >> 1;
+        if (lds->p[mid] < (R.at & 0x3FFFFu)) a0 = mid + 1u; else z = mid;
+    }
+    // base index bi of the template of the read (at, cell), whose first record is `first`, substituted
+    auto error = [&](uint32_t at, uint32_t cell, uint32_t first, uint32_t bi, uint32_t sub) {
+        const uint32_t mate = (at >> 18) & 1u, al = at >> 19;
+        if ((bi >= RL ? 1u : 0u) != mate) return;
+        const uint32_t p = (at & 0x3FFFFu) + bi - mate * RL;
+        if (n_lds) {
+            uint32_t a = first;
+            while (a < n_lds && lds->p[a] < p) ++a;
+            if (a == n_lds || lds->p[a] != p) return;
+            const uint32_t in = lds->info[a];
+            if (in & REC_SHARED) {
+                error_fix(J, gv, a, al, leaf_of_cell(J, S, cell), sub);
+            } else if (PSX_INFO_KIND(in) == PSX_SNV) {
+                const bool car = PSX_INFO_ALLELE(in) == al && cell - lds->low[a] < lds->len[a];
+                const uint32_t alt = PSX_INFO_ALT(in), tb = car ? alt : PSX_INFO_REF(in), ob = sub < tb ? sub : sub + 1u;
+                if ((ob == alt) != (tb == alt)) atomicAdd(&lds->alt[a], ob == alt ? 1u : 0xFFFFFFFFu);
+            }
+        } else {
+            const uint32_t a = gv.first(wb + p);
+            if (a < n_win && gv.pos[a] == wb + p) error_fix(J, gv, a, al, leaf_of_cell(J, S, cell), sub);
+        }
+    };
+    uint32_t number;
+    unsigned long long big = lane_errors<16>(J, seed, R.r, j, c2, on, number,
+                                             [&](uint32_t bi, uint32_t sub) { error(R.at, R.cell, a0, bi, sub); });
+    while (big) {
+        const int ln = __ffsll((long long)big) - 1;
+        big &= big - 1ull;
+        const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)R.at, ln), cell = (uint32_t)__builtin_amdgcn_readlane((int)R.cell, ln);
+        const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)R.r, ln), first = (uint32_t)__builtin_amdgcn_readlane((int)a0, ln);
+        wave_sync();
+        const uint32_t ne = wave_template_errors<true>(seed, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane,
+                                                 (uint32_t)__builtin_amdgcn_readlane((int)number, ln));
+        wave_sync();
+        for (uint32_t k = lane; k < ne; k += 64u) error(at, cell, first, list[k] & 0xFFFFFu, list[k] >> 20);
+    }
+    wave_sync();
 }
 
 template <class LDS>
@@ -537,9 +615,22 @@ __device__ __attribute__((noinline)) void count_queued(const job_dev* Jp, const 
         uint32_t i = gv.first(wb + xr);
         while (i < n_win && gv.pos[i] < wb + end) i = count_group(J, gv, i, al, leaf, e, boff - wb);
     }
-    // slow templates counted without errors: the wave generates each one's and corrects the counts at those of this mate
-    uint32_t* list = (uint32_t*)q;  // every lane has read its entry
+    // slow templates counted without errors
     unsigned long long sm = __ballot(on && e.slow());
+    if constexpr (LDS::SLOW_WAIT) {  // wait (count_slow); there is room for 64
+        if (sm) {
+            const uint32_t wave = threadIdx.x >> 6, had = lds->wait_n[wave];
+            const uint32_t at =
+                had + __builtin_amdgcn_mbcnt_hi((uint32_t)(sm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)sm, 0u));
+            if ((sm >> lane) & 1ull) lds->wait[wave][at] = R;
+            wave_sync();
+            if (lane == 0) lds->wait_n[wave] = had + (uint32_t)__popcll(sm);
+        }
+        wave_sync();
+        return;
+    }
+    // the wave generates each one's and corrects the counts at those of this mate
+    uint32_t* list = (uint32_t*)q;  // every lane has read its entry
     while (sm) {
         const int ln = __ffsll((long long)sm) - 1;
         sm &= sm - 1ull;
@@ -547,7 +638,7 @@ __device__ __attribute__((noinline)) void count_queued(const job_dev* Jp, const 
         const uint32_t as = (uint32_t)__builtin_amdgcn_readlane((int)al, ln), ls = (uint32_t)__builtin_amdgcn_readlane((int)leaf, ln);
         const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)R.r, ln);
         wave_sync();
-        const uint32_t ne = wave_template_errors((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane);
+        const uint32_t ne = wave_template_errors<true>((uint64_t)s1 << 32 | s0, J.err_n, J.err_k0, J.err_N, J.err_T, rs, j, c2, list, lane);
         wave_sync();
         for (uint32_t k = lane; k < ne; k += 64u) {
             const uint32_t w = list[k], bi = w & 0xFFFFFu;
@@ -560,9 +651,9 @@ __device__ __attribute__((noinline)) void count_queued(const job_dev* Jp, const 
     wave_sync();
 }
 
-template <int BLOCK, int CAP, bool CNA>
+template <int BLOCK, int CAP, bool CNA, bool MANY>
 __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
-    using LDS = sparse_lds<BLOCK, CAP>;
+    using LDS = sparse_lds<BLOCK, CAP, MANY>;
     __shared__ LDS lds;
     __shared__ cn_window s_cn;  // copy numbers
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -571,6 +662,7 @@ __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
     uint32_t in_tab = UNRESOLVED;
     for (uint32_t i = tid; i < (uint32_t)CAP; i += BLOCK) lds.dep[i] = lds.alt[i] = 0;
     for (uint32_t i = tid; i < (LDS::START_BITS + 31u) / 32u; i += BLOCK) lds.bits[i] = 0;
+    if (MANY && lane == 0) lds.wait_n[wave] = 0;
     __syncthreads();
     for (uint32_t run = blockIdx.x;;) {
         const item_run R0 = run_of(L, run);
@@ -639,6 +731,8 @@ __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
                             qn -= 64u;
                             wave_sync();
                             count_queued(&J, &S, &lds, queue + qn, 64u, wb, k0, n_win, n_lds, j, c2);
+                            if (MANY && __builtin_amdgcn_readfirstlane((int)lds.wait_n[wave]) >= WAIT_FULL)
+                                count_slow(&J, &S, &lds, (uint32_t*)(queue + qn), wb, k0, n_win, n_lds, j, c2);
                         }
                     }
                 }
@@ -646,6 +740,8 @@ __global__ void __launch_bounds__(BLOCK, 6) k_count_sparse(const seq_launch L) {
                     wave_sync();
                     count_queued(&J, &S, &lds, queue, qn, wb, k0, n_win, n_lds, j, c2);
                 }
+                while (MANY && __builtin_amdgcn_readfirstlane((int)lds.wait_n[wave]))
+                    count_slow(&J, &S, &lds, (uint32_t*)queue, wb, k0, n_win, n_lds, j, c2);
                 __syncthreads();
                 for (uint32_t i = tid; i < n_lds; i += BLOCK) {
                     const uint32_t dep = lds.dep[i], alt = lds.alt[i];

@@ -20,17 +20,17 @@ using namespace psxk;
 
 namespace psxh {
 
-// Covered positions per 64 templates from which a job counts by windows: on 1.6e9 reads with errors k_count_sparse takes
-// 3.8 ms at 10 and 5.2 at 19, k_count_dense 6.0 and 6.2; without errors 3.5 (10) and 4.7 (19) against 3.7 and 3.8.
-constexpr double DENSE_COVER = 28.0, DENSE_COVER_NO_ERRORS = 8.0;
+// Covered positions per 64 templates from which a job counts by windows (k_count_dense) rather than by queued reads
+// (k_count_sparse): see dense_from.
+constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 12.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0;
 // Share of templates with more than three errors from which the dense kernel lets them wait and makes their errors 48
 // templates at a time (5.6e7 templates of 250 bases: 0.013 % of them 0.46 ms by one after another, 0.53 by 48; 1.7 %
 // 1.01 and 0.90; 14 % 3.85 and 1.55; of 150 bases: 0.33 % 1.05 and 1.06).
 constexpr double MANY_SLOW = 0.006;
-// And from which share on it takes jobs of fewer covered positions: the sparse kernel makes the errors of each such read
-// one after another (14 %, 250 bases: 1.80 ms at 23 covered
-// positions, 1.48 at 17, against 1.42 and 1.42).
-constexpr double SLOW_READS = 0.06, DENSE_COVER_SLOW = 15.0;
+// And the same of the sparse kernel, with 5 blocks per CU in place of 6 then (5.6e7 templates of 150 bases, 11 covered
+// positions: 0.34 % of them 0.47 ms by one after another, 0.49 waiting; 1.35 % 0.56 and 0.50; 3.4 % 0.74 and 0.51; 15 %
+// 1.33 and 0.57).
+constexpr double MANY_SLOW_SPARSE = 0.005;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
 // templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves.
 constexpr uint64_t FEW_ITEMS = 2048, MANY_ITEMS = 4096;
@@ -52,8 +52,9 @@ struct seq_batch {
     std::vector<size_t> cna_off;  // per job: copy-number events (SIZE_MAX: none)
     std::vector<uint64_t> job_reads;  // per job: reads of the sampling model without copy-number events
     std::vector<double> job_slow;   // per job: share of its templates with more than three errors
-    double slow_templates = 0.0;    // such templates of the dense jobs
+    double slow_templates = 0.0, slow_sparse = 0.0;  // such templates of the dense jobs, of the sparse ones
     std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
+    std::vector<double> job_dense_from;  // and of how many it counts by windows
     std::vector<uint8_t> job_fits;  // per job: its source copies fit the dense count kernel's words
     bool cna_sparse = false, cna_dense = false;  // copy-number events among the sparse / the other jobs
     size_t o_jobs = 0, o_segs = 0, o_items = 0, o_pres = 0, o_acc = 0;
@@ -153,6 +154,18 @@ uint32_t bits_of(uint32_t x) {  // bits that represent x (at least 1)
     return b;
 }
 
+// Covered positions per 64 templates from which a job counts by windows, by the errors of an average template (draws
+// that are not kept have none). The windows form makes the errors of every template, the other those of the reads that
+// can reach a record, so the line moves with the errors. Measured crossings on 4.7e7 to 1.4e8 templates of 100 to 250
+// bases: 12 covered positions at 0.05 errors, 15 at 0.12, 18 at 0.2, 25 at 0.5, 29 at 0.6; with more than
+// MANY_SLOW_SPARSE slow templates, where those wait, 51 at 0.9, 60 at 1, 83 at 1.5, 120 at 2, 190 at 3. A line at 28, and
+// at 15 for many slow templates, lost up to 1.8 times the time: 1.3e7 pairs of 150 bases at 2 %, 16 covered, 4.08 -> 1.29
+// ms; 2.8e7 single ones at 0.8 %, 18 covered, 1.20 -> 0.50 ms; pairs of 36 at 0.1 %, 26 covered, 0.96 -> 0.72 ms.
+double dense_from(double errors, double slow) {
+    if (errors <= 0.0) return DENSE_COVER_NO_ERRORS;
+    return slow > MANY_SLOW_SPARSE ? DENSE_COVER_SLOW * errors : DENSE_COVER + DENSE_COVER_ERROR * errors;
+}
+
 // Validates one job and appends its descriptors; the ordering of output
 // samples and chromosomes follows the oracle. Nothing is appended when the
 // job is invalid.
@@ -247,7 +260,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     }
     P.cna_off.push_back(cdev.empty() ? SIZE_MAX : P.sb.put_vec(cdev));
     P.jobs.push_back(J);
-    double cover = 0.0;
+    double cover = 0.0, share = 1.0;
     {
         // expected positions covered by 64 templates: records per base x bases read, times the share of templates
         // kept under copy numbers (length-weighted): the source's copies among kmax slots, a cell's (their mean over
@@ -262,11 +275,13 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
             bases += (double)g->len[c];
             kept += (double)g->len[c] * (tumour * c_mean[c] + (1.0 - tumour) * (double)ploidy) / (double)c_kmax[c];
         }
+        if (bases > 0.0) share = kept / bases;
         if (bases > 0.0) cover = 64.0 * (pe ? 2.0 : 1.0) * L * recs / bases * kept / bases;
     }
     P.job_cover.push_back(cover);
     const uint32_t past = err.k0 > 3u ? 0u : 3u - err.k0;  // K > 3: the draw at or past this threshold
     P.job_slow.push_back(err.k0 > 3u ? 1.0 : past + 1u < err.T.size() ? 1.0 - (double)err.T[past] * 0x1p-32 : 0.0);
+    P.job_dense_from.push_back(dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back()));
     P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;
     for (uint32_t so = 0; so < n_out; ++so) {
@@ -312,11 +327,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
 
 // A job whose reads cover few positions queues the reads that cover any
 // (k_count_sparse), the others count by windows (k_count_dense).
-bool job_sparse(const seq_batch& P, uint32_t job) {
-    return !P.job_fits[job] || P.job_cover[job] < (!P.jobs[job].err_n           ? DENSE_COVER_NO_ERRORS
-                                                   : P.job_slow[job] > SLOW_READS ? DENSE_COVER_SLOW
-                                                                                  : DENSE_COVER);
-}
+bool job_sparse(const seq_batch& P, uint32_t job) { return !P.job_fits[job] || P.job_cover[job] < P.job_dense_from[job]; }
 
 // Strata, bins and items of a segment in the count kernels (parts: layout). A
 // dense window takes 2, 4 or 8 strata while their reads fit one round, in 64
@@ -377,6 +388,7 @@ void layout(seq_batch& P) {
         if (sparse) {
             P.n_items_sparse = P.n_items;
             P.templates_sparse = P.templates;
+            P.slow_sparse += (double)S.T * P.job_slow[S.job];
         } else {
             const job_dev& J = P.jobs[S.job];
             const uint64_t starts = std::min<uint64_t>(S.W, (uint64_t)PSX_STRATUM << seg_lns(S));  // of a window
@@ -406,14 +418,16 @@ void layout(seq_batch& P) {
 }
 
 template <int BLOCK, int CAP>
-void launch_count_t(const seq_lane& lane, const seq_launch& L, uint32_t grid, bool cna) {
-    if (cna) hipLaunchKernelGGL((k_count_sparse<BLOCK, CAP, true>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
-    else hipLaunchKernelGGL((k_count_sparse<BLOCK, CAP, false>), dim3(grid), dim3(BLOCK), 0, lane.stream, L);
+void launch_count_t(const seq_lane& lane, const seq_launch& L, uint32_t grid, bool cna, bool many) {
+    auto* const kernel = cna ? (many ? k_count_sparse<BLOCK, CAP, true, true> : k_count_sparse<BLOCK, CAP, true, false>)
+                             : (many ? k_count_sparse<BLOCK, CAP, false, true> : k_count_sparse<BLOCK, CAP, false, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(BLOCK), 0, lane.stream, L);
 }
 
-void launch_count(const seq_lane& lane, const psx_launch_config& c, const seq_launch& L, uint32_t grid, bool cna) {
+void launch_count(const seq_lane& lane, const psx_launch_config& c, const seq_launch& L, uint32_t grid, bool cna,
+                  bool many) {
 #define PSX_CASE(B, C) \
-    if (c.block_threads == B && c.lds_records == C) return launch_count_t<B, C>(lane, L, grid, cna);
+    if (c.block_threads == B && c.lds_records == C) return launch_count_t<B, C>(lane, L, grid, cna, many);
     PSX_CASE(256, 512) PSX_CASE(256, 1024) PSX_CASE(256, 2048)
     PSX_CASE(512, 512) PSX_CASE(512, 1024) PSX_CASE(512, 2048)
 #undef PSX_CASE
@@ -510,7 +524,8 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
         const uint64_t grid = std::max<uint64_t>(1, std::min(want, ns));
         Ls.n_items = ns;
         Ls.chunk = run_items(ns, P->templates_sparse, grid, 8192, 4);
-        launch_count(lane, cfg, Ls, (uint32_t)grid, P->cna_sparse);
+        const bool many = P->slow_sparse > MANY_SLOW_SPARSE * (double)P->templates_sparse;
+        launch_count(lane, cfg, Ls, (uint32_t)grid, P->cna_sparse, many);
     }
     if (nd) {
         seq_launch Ld = L;

@@ -652,13 +652,18 @@ constexpr uint32_t ELIST = PSX_ERR_KCAP + 64u;
 // t0 + l (x, z, w of w_0, then the four words of w_1, w_2, ...). A word is new
 // when no earlier stream word gives the same base index (an earlier equal
 // index was taken or was itself a repeat of a taken one), and the first K new
-// words are the errors. Repeats are rare: the bitmap flags a batch that may
-// hold one, and only such a batch runs the exact check. Writes the errors to
+// words are the errors. Repeats are rare: the bitmap flags the lanes that may
+// be one, and only such a batch runs the exact check: of every index, or with
+// FLAGGED of the flagged lanes' (tens of errors flag a lane of most batches: 7e6
+// reads of 1,000 bases at 5 %, counted, 9.5 -> 4.7 ms; the read kernel, whose
+// registers are few, keeps the other: 5e7 single-end reads of 100 bases 610 us,
+// 625 with FLAGGED). Writes the errors to
 // list[0 .. K) as b | sub << 20 and returns K (wave-uniform); every lane
-// steps through the same loops.
+// steps through the same loops. known: K, if the caller has it (above 0).
+template <bool FLAGGED = false>
 __device__ __forceinline__ uint32_t wave_template_errors(uint64_t seed, uint32_t err_n, uint32_t err_k0, uint32_t err_N,
                                                       const uint32_t* err_T, uint32_t r, uint32_t j, uint32_t c2,
-                                                      uint32_t* list, uint32_t lane) {
+                                                      uint32_t* list, uint32_t lane, uint32_t known = UNRESOLVED) {
     constexpr uint32_t TMAX = 4u * PSX_ERR_KCAP;  // stream words available
     uint32_t* bits = list + PSX_ERR_KCAP;
     uint32_t K = 0, cnt = 0;
@@ -667,7 +672,11 @@ __device__ __forceinline__ uint32_t wave_template_errors(uint64_t seed, uint32_t
         const uint32_t call = t < 3u ? 0u : 1u + ((t - 3u) >> 2);
         const psx_u4 w = psx_draw_u(seed, r, j, c2, (PSX_P_ERROR << 24) | call);
         const uint32_t word = psx_word(w, t < 3u ? (t == 0u ? 0 : (int)t + 1) : (int)((t - 3u) & 3u));
-        if (t0 == 0) {
+        if (t0 == 0 && known != UNRESOLVED) {
+            K = known;
+            bits[lane] = 0u;
+            wave_sync();
+        } else if (t0 == 0) {
             // K - err_k0 = the number of thresholds k < err_n - 1 with u >= T[k]
             const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)w.y);  // lane 0 drew w_0
             uint32_t k = 0;
@@ -686,7 +695,17 @@ __device__ __forceinline__ uint32_t wave_template_errors(uint64_t seed, uint32_t
         const uint32_t h = (x * 0x9E3779B1u) >> 21;
         const uint32_t seen = live ? atomicOr(&bits[h >> 5], 1u << (h & 31u)) & (1u << (h & 31u)) : 0u;
         unsigned long long dupm = 0;
-        if (__ballot(seen != 0u)) {  // exact check against the batch and the earlier batches
+        if constexpr (FLAGGED) {
+            // lanes that found their bit set: of the lanes that name one index all but one did
+            for (unsigned long long left = __ballot(seen != 0u); left;) {
+                const uint32_t xq = (uint32_t)__builtin_amdgcn_readlane((int)x, __ffsll((long long)left) - 1);
+                const unsigned long long same = __ballot(live && x == xq);
+                left &= ~same;
+                bool d = false;
+                for (uint32_t q = lane; q < cnt; q += 64u) d |= (list[q] & 0xFFFFFu) == xq;
+                dupm |= __ballot(d) ? same : same & (same - 1ull);
+            }
+        } else if (__ballot(seen != 0u)) {  // the batch's and the earlier batches'
             for (uint32_t q = 0; q + 1u < B; ++q) {
                 const uint32_t xq = (uint32_t)__builtin_amdgcn_readlane((int)x, (int)q);
                 dupm |= __ballot(live && x == xq) & (~0ull << (q + 1u));

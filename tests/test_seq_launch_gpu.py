@@ -180,3 +180,25 @@ def test_parts_of_few_strata(ctx):
             rows, m = core.simulate_seq_reads(ctx, w.g, w.pf, w.pm, 5, **kw)
             assert m == n and np.array_equal(rows.numpy()[:m],
                                              O.simulate_reads(w.lens, w.g.download(), w.of, w.recs, 5, m, **kw))
+
+
+@pytest.mark.parametrize("n,kw", [
+    # few records: reads that wait, some windows' last ones alone; more errors than a lane makes, on either mate
+    (300, dict(coverage=150, read_size=100, error_rate=2e-2)),
+    (300, dict(coverage=6, read_size=100, error_rate=3e-2)),
+    (300, dict(coverage=150, read_size=400, insert_size_mean=900, insert_size_stddev=20, error_rate=3e-2, purity=0.5)),
+    # more records in a window than are staged, several of them at one position
+    (8000, dict(coverage=60, read_size=100, error_rate=0.12)),
+    # by windows: templates that wait
+    (8000, dict(coverage=60, read_size=250, error_rate=8e-3)),
+    (8000, dict(coverage=60, read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=6e-3, purity=0.5))])
+@pytest.mark.parametrize("cna", [False, True])
+def test_reads_of_many_errors(ctx, n, kw, cna):
+    """Reads and templates of more than three errors that wait, in both count kernels, with and without copy numbers."""
+    from process_amd import _abi as A
+    eng = dict(cna=[(0, 0, 5_000, 30_000, 0, A.PSX_CNA_AMP, 2), (1, 0, 0, 0, 0, A.PSX_CNA_WGD, 0)]) if cna else {}
+    w = World(ctx, [60_000, 20_000], dict(n_cells=500, n_samples=1, sample_size=90, seed=2), 1e-7, n_pre_snv=n,
+              infinite_sites=False, **eng)
+    a, d, p, _ = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)
+    oa, od, op, _ = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), **kw)
+    assert np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op) and d.sum() > 0
