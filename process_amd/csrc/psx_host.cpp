@@ -273,7 +273,7 @@ extern "C" psx_status psx_dev_alloc(psx_ctx* ctx, uint64_t bytes, void** out) {
     return psx_guard(ctx, [&] {
         PSX_HIP(hipSetDevice(ctx->device));
         *out = nullptr;
-        PSX_HIP(hipMalloc(out, bytes ? bytes : 1));
+        PSX_HIP(psx_dev_malloc(out, bytes ? bytes : 1));
     });
 }
 

@@ -166,7 +166,7 @@ extern "C" psx_status psx_write_sam(psx_ctx* ctx, const psx_genome* g, const psx
         const uint64_t chunk = std::min<uint64_t>(CHUNK_READS, std::max<uint64_t>(max_reads, 1));
         const size_t chunk_bytes = (size_t)chunk * rw * 4u;
         PSX_HIP(hipHostMalloc(&staging, 2 * chunk_bytes, hipHostMallocDefault));
-        if (max_reads) PSX_HIP(hipMalloc((void**)&d_reads, (size_t)max_reads * rw * 4u));
+        if (max_reads) PSX_HIP(psx_dev_malloc((void**)&d_reads, (size_t)max_reads * rw * 4u));
         const uint32_t n_threads = std::max(1u, std::min(MAX_THREADS, std::thread::hardware_concurrency()));
         uint64_t total = 0;
         for (size_t ci = 0; ci < chrs.size(); ++ci) {
