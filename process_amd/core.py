@@ -66,8 +66,9 @@ class Context:
         return f.value, t.value
 
     def trim(self) -> None:
-        """Frees the buffers the context keeps grown between calls; later calls
-        grow them again (psx_ctx_trim)."""
+        """Frees the buffers the context keeps grown between calls and the
+        memory of closed tables that the device keeps for later ones; later
+        calls grow them again (psx_ctx_trim)."""
         check(lib().psx_ctx_trim(self.h), self.h)
 
 

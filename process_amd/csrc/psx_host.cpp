@@ -69,6 +69,7 @@ extern "C" psx_status psx_ctx_trim(psx_ctx* ctx) {
         if (ctx->host_stage) PSX_HIP(hipHostFree(ctx->host_stage));
         ctx->host_stage = nullptr;
         ctx->host_stage_bytes = 0;
+        psx_blocks_trim(ctx->device);
     });
 }
 
@@ -259,6 +260,12 @@ void psx_blocks_close(int device) {
     std::lock_guard<std::mutex> g(blocks_mu);
     block_pool& P = block_pools()[device];
     if (--P.contexts == 0) out.oldest(P, 0, 0);
+}
+
+void psx_blocks_trim(int device) {
+    taken_blocks out;
+    std::lock_guard<std::mutex> g(blocks_mu);
+    out.oldest(block_pools()[device], 0, 0);
 }
 
 size_t psx_blocks_idle(int device) {

@@ -78,11 +78,12 @@ struct dbuf {
 // takes 260 us at 75 MB and its hipMalloc 50 us, a third of the placement that
 // fills it: 1.49e6 mutations placed and sequenced at 10x 1,340 us, 1,605 without.
 // At most BLOCKS_IDLE bytes stay idle on a device; they go back with its last
-// context, and when an allocation fails. psx_blocks_open and psx_blocks_close
-// count the contexts.
+// context, when an allocation of this library fails and by psx_blocks_trim.
+// psx_blocks_open and psx_blocks_close count the contexts.
 std::shared_ptr<dbuf> psx_block(size_t n);
 void psx_blocks_open(int device);
 void psx_blocks_close(int device);
+void psx_blocks_trim(int device);
 size_t psx_blocks_idle(int device);
 
 // ------------------------------------------------------------------- handles

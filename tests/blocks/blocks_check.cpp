@@ -93,11 +93,21 @@ static void alloc(psx_ctx* ctx) {
     CHECK(used == 0);
 }
 
+// Trimming a context gives the device's idle blocks back, and nothing that is in use.
+static void trim(psx_ctx* ctx) {
+    const std::shared_ptr<dbuf> held = psx_block(64 * MIB);
+    idle_blocks(128, 2);
+    CHECK(used == 320 * MIB);
+    CHECK(psx_ctx_trim(ctx) == PSX_OK);
+    CHECK(used == 64 * MIB);
+}
+
 int main(int argc, char** argv) {
     psx_ctx* ctx = nullptr;
     CHECK(psx_ctx_create(0, &ctx) == PSX_OK);
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "alloc") alloc(ctx);
+    else if (what == "trim") trim(ctx);
     else return 2;
     psx_ctx_destroy(ctx);
     CHECK(used == 0 && live.empty());

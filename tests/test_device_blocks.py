@@ -34,6 +34,10 @@ def test_callers_buffers_take_the_memory_of_idle_blocks(check):
     check("alloc")
 
 
+def test_trim_gives_idle_blocks_back(check):
+    check("trim")
+
+
 def test_device_memory_is_allocated_in_one_place():
     """psx_dev_malloc gives idle blocks back when memory runs out; nothing allocates past it."""
     calls = [f"{f.name}: {line.strip()}" for f in sorted(CSRC.iterdir()) for line in f.read_text().splitlines()
