@@ -78,7 +78,9 @@ psx_status psx_ctx_synchronize(psx_ctx* ctx);
 /* Milliseconds of the dominant kernel(s) of the last sequencing call, timed
  * with HIP events on the context stream. */
 psx_status psx_ctx_last_kernel_ms(const psx_ctx* ctx, double* ms);
-/* Free and total HBM of the context device, in bytes. */
+/* Free and total HBM of the context device, in bytes. The memory of freed
+ * tables that the device keeps for later ones is not free: an allocation of
+ * this library that needs it takes it, psx_ctx_trim gives it to others. */
 psx_status psx_ctx_mem_info(psx_ctx* ctx, uint64_t* free_bytes, uint64_t* total_bytes);
 /* Frees the buffers a context keeps grown between calls (placement
  * temporaries, psx_simulate_seq's device tables, launch descriptors, pinned

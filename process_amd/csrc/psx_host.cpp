@@ -127,7 +127,7 @@ extern "C" psx_status psx_ctx_mem_info(psx_ctx* ctx, uint64_t* free_bytes, uint6
         PSX_HIP(hipSetDevice(ctx->device));
         size_t f = 0, t = 0;
         PSX_HIP(hipMemGetInfo(&f, &t));
-        *free_bytes = f + psx_blocks_idle(ctx->device);  // given back when an allocation needs them
+        *free_bytes = f;
         *total_bytes = t;
     });
 }
@@ -266,11 +266,6 @@ void psx_blocks_trim(int device) {
     taken_blocks out;
     std::lock_guard<std::mutex> g(blocks_mu);
     out.oldest(block_pools()[device], 0, 0);
-}
-
-size_t psx_blocks_idle(int device) {
-    std::lock_guard<std::mutex> g(blocks_mu);
-    return block_pools()[device].bytes;
 }
 
 // ----------------------------------------------------------- device buffers

@@ -84,7 +84,6 @@ std::shared_ptr<dbuf> psx_block(size_t n);
 void psx_blocks_open(int device);
 void psx_blocks_close(int device);
 void psx_blocks_trim(int device);
-size_t psx_blocks_idle(int device);
 
 // ------------------------------------------------------------------- handles
 

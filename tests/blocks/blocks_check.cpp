@@ -102,12 +102,22 @@ static void trim(psx_ctx* ctx) {
     CHECK(used == 64 * MIB);
 }
 
+// The free memory reported is the device's: idle blocks are not free to others.
+static void info(psx_ctx* ctx) {
+    uint64_t f = 0, t = 0;
+    idle_blocks(256, 2);
+    CHECK(psx_ctx_mem_info(ctx, &f, &t) == PSX_OK && f == 512 * MIB && t == DEVICE);
+    CHECK(psx_ctx_trim(ctx) == PSX_OK);
+    CHECK(psx_ctx_mem_info(ctx, &f, &t) == PSX_OK && f == DEVICE);
+}
+
 int main(int argc, char** argv) {
     psx_ctx* ctx = nullptr;
     CHECK(psx_ctx_create(0, &ctx) == PSX_OK);
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "alloc") alloc(ctx);
     else if (what == "trim") trim(ctx);
+    else if (what == "info") info(ctx);
     else return 2;
     psx_ctx_destroy(ctx);
     CHECK(used == 0 && live.empty());
