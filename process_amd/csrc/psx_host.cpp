@@ -181,7 +181,9 @@ void give_block(dbuf* b, int device) {
     if (now != device) (void)hipSetDevice(device);
     taken_blocks out;
     // launches in flight may read the block, on any stream
-    if (b->bytes <= BLOCK_LARGEST && hipDeviceSynchronize() == hipSuccess) {
+    const bool idle = b->bytes <= BLOCK_LARGEST && hipDeviceSynchronize() == hipSuccess;
+    if (!idle && b->bytes <= BLOCK_LARGEST) (void)hipGetLastError();  // during a capture: not the next launch's error
+    if (idle) {
         std::lock_guard<std::mutex> g(blocks_mu);
         block_pool& P = block_pools()[device];
         if (P.contexts) {

@@ -111,6 +111,15 @@ static void info(psx_ctx* ctx) {
     CHECK(psx_ctx_mem_info(ctx, &f, &t) == PSX_OK && f == DEVICE);
 }
 
+// A table freed while the device cannot be synchronised (another stream is being captured) is freed at once, and leaves
+// no error for the next launch's check.
+static void capture(psx_ctx*) {
+    sync_result = hipErrorStreamCaptureUnsupported;
+    idle_blocks(128, 2);
+    sync_result = hipSuccess;
+    CHECK(used == 0 && last == hipSuccess);
+}
+
 int main(int argc, char** argv) {
     psx_ctx* ctx = nullptr;
     CHECK(psx_ctx_create(0, &ctx) == PSX_OK);
@@ -118,6 +127,7 @@ int main(int argc, char** argv) {
     if (what == "alloc") alloc(ctx);
     else if (what == "trim") trim(ctx);
     else if (what == "info") info(ctx);
+    else if (what == "capture") capture(ctx);
     else return 2;
     psx_ctx_destroy(ctx);
     CHECK(used == 0 && live.empty());

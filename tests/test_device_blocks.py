@@ -42,6 +42,10 @@ def test_idle_blocks_are_not_reported_free(check):
     check("info")
 
 
+def test_a_table_freed_during_a_capture_leaves_no_error(check):
+    check("capture")
+
+
 def test_device_memory_is_allocated_in_one_place():
     """psx_dev_malloc gives idle blocks back when memory runs out; nothing allocates past it."""
     calls = [f"{f.name}: {line.strip()}" for f in sorted(CSRC.iterdir()) for line in f.read_text().splitlines()
