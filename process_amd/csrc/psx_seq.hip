@@ -51,6 +51,7 @@ struct seq_batch {
     std::vector<size_t> tab_off;  // per job: insert thresholds, insert guide, error thresholds
     std::vector<size_t> cna_off;  // per job: copy-number events (SIZE_MAX: none)
     std::vector<uint64_t> job_reads;  // per job: reads of the sampling model without copy-number events
+    std::vector<uint64_t> job_plain;  // those of its segments without events
     std::vector<double> job_slow;   // per job: share of its templates with more than three errors
     double slow_templates = 0.0, slow_sparse = 0.0;  // such templates of the dense jobs, of the sparse ones
     std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
@@ -284,6 +285,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     P.job_dense_from.push_back(dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back()));
     P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;
+    uint64_t plain = 0;
     for (uint32_t so = 0; so < n_out; ++so) {
         const bool normal = so == n_req;
         const uint32_t leaf_off = normal ? 0u : f->sample_begin[req[so]];
@@ -315,6 +317,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
             S.bucket_off = (uint32_t)ix->bucket_off[c];
             S.leaf_off = leaf_off; S.n_cells = n_cells;
             P.n_reads += S.T * (pe ? 2u : 1u);  // template draws: an upper bound with copy-number events
+            if (!S.n_cna) plain += S.T * (pe ? 2u : 1u);
             // bits of a cell index (the sample's number of cells included) and of an allele in a 25-bit copy field
             const uint32_t cb = bits_of(n_cells + 1u);
             if (cb + bits_of(ploidy - 1u) > 32u - BIN_SHIFT) P.job_fits[job] = 0;
@@ -323,6 +326,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
         }
     }
     P.job_reads.push_back(P.n_reads - reads_before);
+    P.job_plain.push_back(plain);
 }
 
 // A job whose reads cover few positions queues the reads that cover any
@@ -479,7 +483,7 @@ std::vector<uint64_t> batch_job_reads(const seq_batch* b, const seq_lane& lane) 
     PSX_HIP(hipMemcpyAsync(acc.data(), lane.desc + b->o_acc, 8 * acc.size(), hipMemcpyDeviceToHost, lane.stream));
     PSX_HIP(hipStreamSynchronize(lane.stream));
     for (size_t k = 0; k < r.size(); ++k)
-        if (b->cna_off[k] != SIZE_MAX) r[k] = acc[k];
+        if (b->cna_off[k] != SIZE_MAX) r[k] = b->job_plain[k] + acc[k];
     return r;
 }
 size_t batch_items(const seq_batch* b) { return b->n_items; }

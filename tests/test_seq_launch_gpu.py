@@ -202,3 +202,22 @@ def test_reads_of_many_errors(ctx, n, kw, cna):
     a, d, p, _ = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)
     oa, od, op, _ = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), **kw)
     assert np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op) and d.sum() > 0
+
+
+@pytest.mark.parametrize("snv", [3e-7, 6e-5])
+def test_reads_of_chromosomes_with_and_without_events(ctx, snv):
+    """The number of reads of a count-only call is that of all its chromosomes, those without copy-number events too:
+    the plain call, a batched launch, a plan and a server."""
+    from process_amd import _abi as A
+    w = World(ctx, [40_000, 30_000, 5_000], dict(n_cells=500, n_samples=2, sample_size=90, seed=2), snv,
+              cna=[(0, 1, 2_000, 20_000, 1, A.PSX_CNA_AMP, 2)])
+    kw = dict(coverage=30, read_size=75, insert_size_mean=200, insert_size_stddev=8, error_rate=2e-3, purity=0.7)
+    on = O.simulate_seq(w.lens, w.of, w.recs, 3, cna=w.pm.cna(), **kw)[3]
+    assert core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, **kw)[3] == on
+    assert core.num_reads_table(ctx, w.g, w.pf, w.pm, 3, **kw) == on
+    jobs = [core.SeqJob(ctx, w.g, w.pf, w.pm, 3, **kw) for _ in range(2)]
+    assert core.simulate_seq_batch(ctx, jobs) == 2 * on
+    assert core.SeqPlan(ctx, jobs).run() == 2 * on
+    server = core.Server(ctx, 1 << 20)
+    assert server.wait(server.submit(w.g, w.pf, w.pm, 3, **kw))[3]["n_reads"] == on
+    server.close()
