@@ -47,8 +47,9 @@ constexpr uint32_t BIN_READS = 88;    // expected reads of a bin in a round
 constexpr uint32_t MAX_BINS = (PSX_STRATUM + MAX_READ) >> BIN_SHIFT;
 
 // Dynamic LDS of a launch: the bitmap of record positions, the bins, their counts (two sets).
-__host__ __device__ __forceinline__ uint32_t dense_bit_words(uint32_t bits) { return (bits + 127u) / 128u * 4u; }
-__host__ __device__ __forceinline__ uint32_t dense_lds(uint32_t bins, uint32_t bits) {
+constexpr uint32_t MAX_BITS = (PSX_STRATUM << 2) + MAX_READ;  // jobs with errors: windows of at most 4 strata
+__host__ __device__ constexpr uint32_t dense_bit_words(uint32_t bits) { return (bits + 127u) / 128u * 4u; }
+__host__ __device__ constexpr uint32_t dense_lds(uint32_t bins, uint32_t bits) {
     return 4u * (dense_bit_words(bits) + bins * (BIN_STRIDE + 2u));
 }
 
@@ -794,6 +795,10 @@ __device__ __forceinline__ scan_rec load_rec(const job_dev& J, const seg_dev& S,
     return R;
 }
 
+
+static_assert(dense_lds(MAX_BINS, MAX_BITS) + sizeof(count_tables) + DENSE_WAVES * sizeof(slow_list) + TODO_CAP * sizeof(todo) +
+                      sizeof(cn_window) + 64 <= 160 * 1024,
+              "the widest window (71 KB: mates 4,000 bases away) fits a compute unit's LDS");
 
 template <bool CNA, bool MANY>
 __global__ void __launch_bounds__(DENSE_BLOCK, 6) k_count_dense(const seq_launch L) {

@@ -409,6 +409,10 @@ void layout(seq_batch& P) {
             }
             P.dense_bins = std::max(P.dense_bins, (uint32_t)((starts - 1 + J.reach - J.L) >> seg_lw(S)) + 1u);
             if (J.err_n) P.dense_bits = std::max(P.dense_bits, (PSX_STRATUM << seg_lns(S)) + J.reach);
+            // the launch's dynamic LDS (the largest is checked against the CU's when the kernel is compiled)
+            if (P.count && (P.dense_bins > MAX_BINS || P.dense_bits > MAX_BITS))
+                psx_throw(PSX_EINVAL, "a window of %u bins and %u positions does not fit the count kernel", P.dense_bins,
+                          P.dense_bits);
         }
     }
     for (uint32_t k = 0; k < (uint32_t)P.jobs.size(); ++k)

@@ -221,3 +221,21 @@ def test_reads_of_chromosomes_with_and_without_events(ctx, snv):
     server = core.Server(ctx, 1 << 20)
     assert server.wait(server.submit(w.g, w.pf, w.pm, 3, **kw))[3]["n_reads"] == on
     server.close()
+
+
+@pytest.mark.parametrize("kw", [
+    # windows of four strata and of one; one job's templates wait for their errors; no errors: eight strata
+    dict(coverage=2, error_rate=1e-3), dict(coverage=300, error_rate=1e-3, purity=0.5),
+    dict(coverage=2, error_rate=2e-2), dict(coverage=300, error_rate=2e-2, purity=0.5), dict(coverage=2)])
+@pytest.mark.parametrize("cna", [False, True])
+def test_widest_windows(ctx, kw, cna):
+    """Mates as far from their reads as the library takes them (4,096 bases): the most bins and the largest bitmap of
+    the windows form, 71 KB of LDS."""
+    from process_amd import _abi as A
+    eng = dict(cna=[(0, 0, 5_000, 30_000, 0, A.PSX_CNA_AMP, 2)]) if cna else {}
+    w = World(ctx, [60_000, 9_000, 4_200], dict(n_cells=500, n_samples=1, sample_size=90, seed=2), 1e-7, n_pre_snv=8000,
+              infinite_sites=False, **eng)
+    kw = dict(kw, read_size=60, insert_size_mean=4000, insert_size_stddev=10)
+    a, d, p, n = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 17, **kw)
+    oa, od, op, on = O.simulate_seq(w.lens, w.of, w.recs, 17, cna=w.pm.cna(), **kw)
+    assert n == on and np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op) and d.sum() > 0
