@@ -482,18 +482,19 @@ typedef struct psx_seq_job {
 } psx_seq_job;
 
 typedef struct psx_launch_config {
-    uint32_t block_threads;    /* 64..1024, multiple of 64 */
-    uint32_t lds_records;      /* mutation records staged in LDS per block */
-    uint32_t strata_per_item;  /* strata processed by one work item */
-    uint32_t blocks_per_cu;    /* persistent blocks per compute unit */
+    uint32_t block_threads;    /* 256 or 512; of the launch of sparse jobs (below) */
+    uint32_t lds_records;      /* 512, 1024 or 2048 mutation records staged in LDS per block, likewise */
+    uint32_t strata_per_item;  /* at least so many strata processed by one work item */
+    uint32_t blocks_per_cu;    /* persistent blocks per compute unit, 1..64 */
     int32_t use_graph;         /* capture the launch sequence in a hipGraph */
 } psx_launch_config;
 
 /* All jobs in persistent launches pulling (job, sample, chromosome, strata)
- * items from device queues: one launch for the jobs whose reads cover few
- * mutation positions (errors checked per covered position) and one for the
- * others (errors drawn per template); the same counts either way. cfg = NULL
- * uses the tuned default. */
+ * items from device queues: one launch for the sparse jobs, whose reads cover
+ * few mutation positions (the reads that can cover one are queued, and only
+ * their errors are drawn), and one for the others (counted by windows, errors
+ * drawn for every template); the same counts either way. cfg = NULL uses the
+ * tuned default. */
 psx_status psx_simulate_seq_batch(psx_ctx* ctx, const psx_seq_job* jobs, uint32_t n_jobs,
                                   const psx_launch_config* cfg, uint64_t* n_reads);
 /* Read materialisation of many jobs in one persistent launch (the batched
@@ -518,7 +519,8 @@ psx_status psx_seq_plan_create(psx_ctx* ctx, const psx_seq_job* jobs, uint32_t n
 psx_status psx_seq_plan_run(psx_seq_plan* plan, uint64_t* n_reads);
 void psx_seq_plan_free(psx_seq_plan* plan);
 /* Times candidate launch configurations on the jobs and returns the fastest
- * (results are identical for every configuration). */
+ * (results are identical for every configuration), which the context then
+ * uses. block_threads and lds_records vary where some job is sparse. */
 psx_status psx_autotune_seq(psx_ctx* ctx, const psx_seq_job* jobs, uint32_t n_jobs,
                             psx_launch_config* best, double* best_ms);
 

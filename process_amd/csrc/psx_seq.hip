@@ -1138,11 +1138,16 @@ extern "C" psx_status psx_autotune_seq(psx_ctx* ctx, const psx_seq_job* jobs, ui
         const uint32_t bpcs[] = {2, 4, 8, 16};
         double best_t = 1e300;
         psx_launch_config bc = default_config();
+        // threads and staged records are k_count_sparse's: without jobs for it they would be the noise's choice, and the
+        // context's for later calls
+        const std::unique_ptr<seq_batch, void (*)(seq_batch*)> P(batch_prepare(ctx, in.data(), in.size(), 1), batch_free);
+        const bool sparse = P->n_items_sparse != 0;
         for (uint32_t b : blocks)
             for (uint32_t cap : caps)
                 for (uint32_t spi : spis)
                     for (uint32_t bpc : bpcs) {
                         if (b == 512 && bpc > 8) continue;
+                        if (!sparse && (b != default_config().block_threads || cap != default_config().lds_records)) continue;
                         const psx_launch_config c{b, cap, spi, bpc, 0};
                         psx_check_cancel(ctx);
                         double t = 0.0;

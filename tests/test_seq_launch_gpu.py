@@ -239,3 +239,20 @@ def test_widest_windows(ctx, kw, cna):
     a, d, p, n = core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 17, **kw)
     oa, od, op, on = O.simulate_seq(w.lens, w.of, w.recs, 17, cna=w.pm.cna(), **kw)
     assert n == on and np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op) and d.sum() > 0
+
+
+def test_autotuner_varies_what_the_jobs_use(ctx):
+    """Jobs counted by windows alone leave the block size and the staged records, which that form does not have, at the
+    default; with a sparse job every configuration is timed."""
+    own = core.Context(0)  # the tuned configuration is the context's
+    forest = dict(n_cells=500, n_samples=1, sample_size=90, seed=2)
+    kw = dict(coverage=20, read_size=150, insert_size_mean=350, insert_size_stddev=10, error_rate=1e-3)
+    dense, sparse = World(own, [300_000], forest, 6e-5), World(own, [300_000], forest, 1e-8)
+    for worlds in ([dense], [dense, sparse]):
+        jobs = [core.SeqJob(own, w.g, w.pf, w.pm, 3, **kw) for w in worlds]
+        cfg, ms = core.autotune(own, jobs)
+        assert ms > 0 and cfg.block_threads in (256, 512) and cfg.lds_records in (512, 1024, 2048)
+        if worlds == [dense]:
+            assert (cfg.block_threads, cfg.lds_records) == (256, 512)
+        for w, j in zip(worlds, jobs):
+            w.check(j.results(), 3, kw)
