@@ -231,7 +231,6 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     J.err_n = (uint32_t)err.T.size();
     J.err_k0 = err.k0;
     J.err_N = (pe ? 2u : 1u) * L;
-    J.inv_L = (uint32_t)(((uint64_t(1) << 32) + L - 1) / L);
     J.L = L; J.pe = pe ? 1u : 0u; J.ploidy = ploidy; J.n_leaves = f->n_leaves;
     J.preneo = p->preneoplastic_in_normal ? 1u : 0u; J.reach = reach; J.n_out = n_out;
     J.purity_lt1 = p->purity < 1.0 ? 1u : 0u;
@@ -490,7 +489,6 @@ std::vector<uint64_t> batch_job_reads(const seq_batch* b, const seq_lane& lane) 
         if (b->cna_off[k] != SIZE_MAX) r[k] = b->job_plain[k] + acc[k];
     return r;
 }
-size_t batch_items(const seq_batch* b) { return b->n_items; }
 
 void batch_upload(seq_batch* P, const seq_lane& lane) {
     if (lane.desc_bytes < batch_desc_bytes(P)) psx_throw(PSX_EINVAL, "descriptor buffer too small");
@@ -524,8 +522,7 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
     hipLaunchKernelGGL(k_seq_init, dim3(init_grid), dim3(256), 0, lane.stream, L.jobs, ps, (uint32_t)P->pres.size(),
                        P->pres_total, L.queue, (uint32_t)P->jobs.size());
     if (timed) PSX_HIP(hipEventRecord(lane.ev0, lane.stream));
-    // the sparse jobs' items (errors checked per covered position), then the others' (errors per template), each
-    // range from its own counter
+    // the sparse jobs' items (k_count_sparse), then the others' (k_count_dense), each range from its own counter
     const uint64_t ns = P->n_items_sparse, nd = P->n_items - ns;
     if (ns || !nd) {
         seq_launch Ls = L;

@@ -1,5 +1,6 @@
-// Device side of simulate_seq on gfx950: descriptors, the count-only kernel
-// and the read-materialising kernel. Included once, by psx_seq.hip.
+// Device side of simulate_seq on gfx950: descriptors, the draws of templates
+// and their errors, and the read-materialising kernel (the count-only kernels:
+// psx_count_dev.h). Included once, by psx_seq.hip.
 //
 // Work decomposition. A segment is one (job, output sample, chromosome); its
 // W = len - L + 1 template starts are cut into strata of PSX_STRATUM starts,
@@ -7,11 +8,9 @@
 // so results do not depend on the launch). A work item is a run of strata of
 // one segment; persistent blocks pull runs of items from a device counter.
 //
-// Per stratum a block stages in LDS the mutation records the stratum's reads
-// can reach (pos, leaf range, packed info) with a 32-base bucket index, plus
-// the job's inversion tables; reads are generated from counters and looked up
-// in LDS, counts go to LDS counters and the block flushes them with one global
-// atomic per touched record. All counting is integer.
+// Per stratum the read kernel stages in LDS the SNVs that the stratum's reads
+// can carry, with a 32-base bucket index, the reference under them and the job's
+// inversion tables; reads are generated from counters and built from there.
 #pragma once
 #include "psx_cna.h"
 #include "psx_internal.h"
@@ -59,10 +58,9 @@ struct job_dev {
     uint32_t ins_k0, ins_n;
     uint32_t err_n, err_k0;      // error table (err_n == 0: no sequencing errors)
     uint32_t err_N;              // bases per template: (pe + 1) L
-    uint32_t inv_L;              // ceil(2^32 / L): b / L = mulhi(b, inv_L) for b < 2^20
+    uint32_t purity_lt1;
     uint32_t L, pe, ploidy, n_leaves, preneo, reach;
     uint32_t n_out;
-    uint32_t purity_lt1;
     uint32_t leaf_blocks;        // leaf_count entries per sample
     const psx_cna_dev* cna;      // copy-number events of every chromosome, per segment ranges
     unsigned long long* acc;     // reads of accepted templates (jobs with copy-number events)
@@ -158,25 +156,17 @@ __device__ __forceinline__ item_run run_of(const seq_launch& L, uint32_t run) {
     return item_run{(uint32_t)first, (uint32_t)(first + (left < L.chunk ? left : L.chunk))};
 }
 
-// The job's inversion tables in LDS; the insert-size guide keeps 2^GB of the
-// host table's PSX_GUIDE entries (every 2^(PSX_GUIDE_BITS - GB)-th, the same
-// guide at a coarser step), so a kernel short of LDS can hold a smaller one.
-template <uint32_t GB>
-struct lds_tables_t {
-    static constexpr uint32_t GUIDE_BITS = GB;
+// The job's inversion tables in LDS (the read kernel's; the count kernels': count_tables).
+struct lds_tables {
     uint32_t ins[MAX_INS];
-    uint16_t guide[1u << GB];
+    uint16_t guide[PSX_GUIDE];
     uint32_t err[MAX_ERRT];
 };
-using lds_tables = lds_tables_t<PSX_GUIDE_BITS>;
 
-template <class TAB>
-__device__ __forceinline__ void load_tables(const job_dev& J, TAB& t, uint32_t tid, uint32_t block) {
-    constexpr uint32_t GB = TAB::GUIDE_BITS;
-    static_assert(GB <= PSX_GUIDE_BITS, "the host guide is the finest");
+__device__ __forceinline__ void load_tables(const job_dev& J, lds_tables& t, uint32_t tid, uint32_t block) {
     if (J.pe) {
         for (uint32_t i = tid; i < J.ins_n; i += block) t.ins[i] = J.ins_T[i];
-        for (uint32_t i = tid; i < (1u << GB); i += block) t.guide[i] = J.ins_guide[i << (PSX_GUIDE_BITS - GB)];
+        for (uint32_t i = tid; i < PSX_GUIDE; i += block) t.guide[i] = J.ins_guide[i];
     }
     for (uint32_t i = tid; i < J.err_n; i += block) t.err[i] = J.err_T[i];
     // the error-count pick reads thresholds 0..3 whatever the table's length
@@ -192,29 +182,19 @@ __device__ __forceinline__ void wave_sync() {
 
 // ------------------------------------------------------------- record views
 
-struct lds_view {
+struct lds_view {  // the read kernel's staged records
     const uint32_t* pos;
     const uint32_t* lo;
     const uint32_t* hi;
     const uint32_t* info;
-    uint32_t* alt;
-    uint32_t* dep;
     const uint16_t* bucket;
     uint32_t n, b;
-    __device__ __forceinline__ uint32_t first(uint32_t x) const {
-        uint32_t i = bucket[(x - b) >> NB_SHIFT];
-        while (i < n && pos[i] < x) ++i;
-        return i;
-    }
     // a record index at or before the first record at or after x
     __device__ __forceinline__ uint32_t start(uint32_t x) const { return bucket[(x - b) >> NB_SHIFT]; }
     __device__ __forceinline__ uint32_t at(uint32_t i) const { return min(i, n - 1u); }  // n > 0
-    __device__ __forceinline__ void add_dep(uint32_t q) const { atomicAdd(&dep[q], 1u); }
-    __device__ __forceinline__ void add_alt(uint32_t q) const { atomicAdd(&alt[q], 1u); }
-    __device__ __forceinline__ void add_alt_n(uint32_t q, int d) const { atomicAdd(&alt[q], (uint32_t)d); }
 };
 
-struct glb_view {  // window larger than the LDS capacity
+struct glb_view {  // records in global memory
     const uint32_t* pos;
     const uint32_t* lo;
     const uint32_t* hi;
@@ -230,7 +210,6 @@ struct glb_view {  // window larger than the LDS capacity
         }
         return a;
     }
-    __device__ __forceinline__ uint32_t first_u(uint32_t x) const { return first(x); }
     __device__ __forceinline__ uint32_t start(uint32_t x) const { return first(x); }
     __device__ __forceinline__ uint32_t at(uint32_t i) const { return min(i, n - 1u); }  // n > 0
     __device__ __forceinline__ void add_dep(uint32_t q) const { atomicAdd(&dep[q], 1); }
@@ -423,11 +402,10 @@ __device__ __forceinline__ bool carried(const job_dev& J, uint32_t info, uint32_
 // the answer lies in [guide[g], guide[g + 1]] (the last bucket ends at n - 1),
 // and the tail buckets of a peaked distribution hold tens of entries, which a
 // linear scan would walk for the whole wave. Same result as psx_guided_pick.
-template <uint32_t GB>
 __device__ __forceinline__ uint32_t guided_pick_u(const uint32_t* T32, const uint16_t* guide, uint32_t n, uint32_t u) {
-    const uint32_t g = u >> (32u - GB);
+    const uint32_t g = u >> (32u - PSX_GUIDE_BITS);
     uint32_t lo = guide[g];
-    uint32_t hi = g < (1u << GB) - 1u ? guide[g + 1u] : n - 1u;
+    uint32_t hi = g < PSX_GUIDE - 1u ? guide[g + 1u] : n - 1u;
     while (__ballot(lo < hi)) {
         const uint32_t mid = (lo + hi) >> 1;
         const bool below = u < T32[mid];
@@ -499,10 +477,10 @@ __device__ __forceinline__ tmpl template_source(const job_dev& J, const seg_dev&
 }
 
 // Start of mate 2 of a template that starts at x, from the insert word of its draw.
-template <class TAB>
-__device__ __forceinline__ uint32_t mate_start(const job_dev& J, const seg_dev& S, const TAB& tab, uint32_t x, uint32_t ins) {
+__device__ __forceinline__ uint32_t mate_start(const job_dev& J, const seg_dev& S, const lds_tables& tab, uint32_t x,
+                                               uint32_t ins) {
     if (!J.pe) return x;
-    uint32_t I = J.ins_k0 + guided_pick_u<TAB::GUIDE_BITS>(tab.ins, tab.guide, J.ins_n, ins);
+    uint32_t I = J.ins_k0 + guided_pick_u(tab.ins, tab.guide, J.ins_n, ins);
     if (I < J.L) I = J.L;
     const uint64_t x2 = (uint64_t)x + I - J.L;
     return x2 > S.len - J.L ? S.len - J.L : (uint32_t)x2;
@@ -510,8 +488,7 @@ __device__ __forceinline__ uint32_t mate_start(const job_dev& J, const seg_dev& 
 
 // Template r of stratum j of a segment without copy-number events (oracle:
 // the template loop of orc_simulate_seq).
-template <class TAB>
-__device__ __forceinline__ tmpl make_template(const job_dev& J, const seg_dev& S, const TAB& tab, uint32_t r,
+__device__ __forceinline__ tmpl make_template(const job_dev& J, const seg_dev& S, const lds_tables& tab, uint32_t r,
                                               uint32_t j, uint32_t b, uint32_t e) {
     psx_u4 w;
     tmpl t = template_source(J, S, r, j, b, e, w);
@@ -628,18 +605,6 @@ __device__ __forceinline__ uint32_t observe(const terr& e, uint32_t b, uint32_t 
     sub = n > 1u && (e1 & 0x1FFFu) == b ? e1 >> 13 : sub;
     sub = n > 2u && (e2 & 0x1FFFu) == b ? e2 >> 13 : sub;
     return sub == 4u ? tb : (sub < tb ? sub : sub + 1u);
-}
-
-// The substitution index of the summary's error at template base index b, or
-// 4 when b has none.
-__device__ __forceinline__ uint32_t error_sub(const terr& e, uint32_t b) {
-    const uint32_t n = e.n();
-    const uint32_t e0 = e.w01 & 0xFFFFu, e1 = e.w01 >> 16, e2 = e.w2n & 0xFFFFu;
-    uint32_t sub = 4u;
-    sub = n > 0u && (e0 & 0x1FFFu) == b ? e0 >> 13 : sub;
-    sub = n > 1u && (e1 & 0x1FFFu) == b ? e1 >> 13 : sub;
-    sub = n > 2u && (e2 & 0x1FFFu) == b ? e2 >> 13 : sub;
-    return sub;
 }
 
 // Per-wave LDS of a slow template's errors: the list, then a 2048-bit hashed
@@ -1116,7 +1081,7 @@ __global__ void __launch_bounds__(BLOCK, BLOCK == 512 ? 6 : 1) k_seq_reads(const
             uint32_t n_snv = 0;
             if (fits) n_snv = stage_snvs<BLOCK, CAP>(J, S, s, s_pos, s_lo, s_hi, s_info, s_bucket, s_cnt, tid);
             else __syncthreads();
-            const lds_view lv{s_pos, s_lo, s_hi, s_info, nullptr, nullptr, s_bucket, n_snv, s.b};
+            const lds_view lv{s_pos, s_lo, s_hi, s_info, s_bucket, n_snv, s.b};
             const glb_view gv{J.pos + s.k0, J.lo + s.k0, J.hi + s.k0, J.info + s.k0, nullptr, nullptr, s.n_win};
             const uint32_t nj = (uint32_t)s.nj;
             // Rounds of WAVES x 64 templates, 64 per wave: lanes [0, n_t) hold the templates (start tx, mate start tx2,

@@ -44,7 +44,6 @@ seq_batch* batch_prepare(psx_ctx* ctx, const job_in* jobs, size_t n_jobs, uint32
 void batch_free(seq_batch* b);
 size_t batch_desc_bytes(const seq_batch* b);
 uint64_t batch_reads(const seq_batch* b);
-size_t batch_items(const seq_batch* b);
 // Reads simulated per job once the launch has finished (jobs with
 // copy-number events: the device count of accepted templates).
 std::vector<uint64_t> batch_job_reads(const seq_batch* b, const seq_lane& lane);
