@@ -23,9 +23,10 @@ namespace psxh {
 // Covered positions per 64 templates from which a job counts by windows (k_count_dense) rather than by queued reads
 // (k_count_sparse): see dense_from.
 constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 12.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0;
-// Share of templates with more than three errors from which the dense kernel lets them wait and makes their errors 48
-// templates at a time (5.6e7 templates of 250 bases: 0.013 % of them 0.46 ms by one after another, 0.53 by 48; 1.7 %
-// 1.01 and 0.90; 14 % 3.85 and 1.55; of 150 bases: 0.33 % 1.05 and 1.06).
+// Share of slow templates (slow_share) from which the dense kernel lets them wait and makes their errors 48 templates at a
+// time (5.6e7 templates of 250 bases: 0.013 % of them with more than three errors 0.46 ms by one after another, 0.53 by
+// 48; 1.7 % 1.01 and 0.90; 14 % 3.85 and 1.55; of 150 bases: 0.33 % 1.05 and 1.06; 2.8e8 of 36 bases, 0.7 % slow in all,
+// 2.52 and 2.34).
 constexpr double MANY_SLOW = 0.006;
 // And the same of the sparse kernel, with 5 blocks per CU in place of 6 then (5.6e7 templates of 150 bases, 11 covered
 // positions: 0.34 % of them 0.47 ms by one after another, 0.49 waiting; 1.35 % 0.56 and 0.50; 3.4 % 0.74 and 0.51; 15 %
@@ -52,7 +53,7 @@ struct seq_batch {
     std::vector<size_t> cna_off;  // per job: copy-number events (SIZE_MAX: none)
     std::vector<uint64_t> job_reads;  // per job: reads of the sampling model without copy-number events
     std::vector<uint64_t> job_plain;  // those of its segments without events
-    std::vector<double> job_slow;   // per job: share of its templates with more than three errors
+    std::vector<double> job_slow;   // per job: share of its slow templates (slow_share)
     double slow_templates = 0.0, slow_sparse = 0.0;  // such templates of the dense jobs, of the sparse ones
     std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
     std::vector<double> job_dense_from;  // and of how many it counts by windows
@@ -153,6 +154,15 @@ uint32_t bits_of(uint32_t x) {  // bits that represent x (at least 1)
     uint32_t b = 1;
     while (b < 32 && (x >> b) != 0) ++b;
     return b;
+}
+
+// Share of templates whose errors their first draw does not settle: more than three, or two or three at one base of N.
+double slow_share(const psx_ctable& err, double N) {
+    if (err.T.empty()) return 0.0;
+    auto below = [&](uint32_t k) {  // share of templates of at most k errors
+        return k < err.k0 ? 0.0 : k - err.k0 + 1u < err.T.size() ? (double)err.T[k - err.k0] * 0x1p-32 : 1.0;
+    };
+    return 1.0 - below(3) + (below(2) - below(1)) / N + (below(3) - below(2)) * (3.0 - 2.0 / N) / N;
 }
 
 // Covered positions per 64 templates from which a job counts by windows, by the errors of an average template (draws
@@ -279,8 +289,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
         if (bases > 0.0) cover = 64.0 * (pe ? 2.0 : 1.0) * L * recs / bases * kept / bases;
     }
     P.job_cover.push_back(cover);
-    const uint32_t past = err.k0 > 3u ? 0u : 3u - err.k0;  // K > 3: the draw at or past this threshold
-    P.job_slow.push_back(err.k0 > 3u ? 1.0 : past + 1u < err.T.size() ? 1.0 - (double)err.T[past] * 0x1p-32 : 0.0);
+    P.job_slow.push_back(slow_share(err, J.err_N));
     P.job_dense_from.push_back(dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back()));
     P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;

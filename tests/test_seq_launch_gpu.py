@@ -187,6 +187,8 @@ def test_parts_of_few_strata(ctx):
     (300, dict(coverage=150, read_size=100, error_rate=2e-2)),
     (300, dict(coverage=6, read_size=100, error_rate=3e-2)),
     (300, dict(coverage=150, read_size=400, insert_size_mean=900, insert_size_stddev=20, error_rate=3e-2, purity=0.5)),
+    # some twenty errors, many of them drawn again
+    (300, dict(coverage=40, read_size=40, error_rate=0.5)),
     # more records in a window than are staged, several of them at one position
     (8000, dict(coverage=60, read_size=100, error_rate=0.12)),
     # by windows: templates that wait
