@@ -33,10 +33,10 @@ SERVE_OVERLAP_US = 250
 
 # HBM bytes per launch of the dominant kernels on the plain_large workload, from rocprofv3 FETCH_SIZE and
 # WRITE_SIZE runs calibrated against a device copy, and vector instructions per launch from SQ_INSTS_VALU (the
-# rocprofv3 summaries under profiles/, named for the kernel and workload). Count-only sequencing is bound by
+# rocprofv3 summaries under profiles/: k_cases.md, and those named for a kernel and workload). Count-only sequencing is bound by
 # vector instruction issue, not HBM; the probe kernels' instruction counts per lane-iteration come from the
 # same counter (profiles/k_probe_valu.md).
-PROFILED = {"k_count_dense": dict(valu_insts=4.068e9),
+PROFILED = {"k_count_dense": dict(traffic=1.81e9, valu_insts=4.066e9),
             "k_seq_reads": dict(traffic=77.42e9),
             # batched read materialisation of the 256-job batched workload's leading 19 jobs
             "k_seq_reads_batched": dict(traffic=72.54e9),

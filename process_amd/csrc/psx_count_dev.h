@@ -15,7 +15,7 @@
 //
 // Bound by vector instruction issue (4.4 cycles each; 6 waves per SIMD by
 // 80 VGPRs and 52 KB of LDS per block; 4 waves: 8.8 ms): on the plain-large
-// workload (200x, one record per 200 bases) 322 instructions per 64 templates
+// workload (200x, one record per 200 bases) 325 instructions per 64 templates
 // against 497 of a form that walked each read's records and queued (read,
 // record) pairs: 80 of them Philox, 80 the rest of the draw and the bins, 35
 // the window's set-up, 45 the scan, 80 the errors past their draw. 9.10 ->
@@ -444,7 +444,7 @@ __device__ __forceinline__ bool plain_record(uint32_t info) {
 // reach a record. The reads that can are queued by the wave and counted 64 at
 // a time, one per lane: the records each covers, found in LDS, the carriers as
 // ranges of the sample's cells, and the errors of its template, drawn only
-// then. Bound by vector instruction issue: 132 instructions per 64 templates
+// then. Bound by vector instruction issue: 115 instructions per 64 templates
 // where nothing is covered (43 Philox, 20 the source, 20 the insert size, 20
 // the tests; 4.4-4.7 cycles each), and about 390 per 64 queued reads. The form
 // before walked every read's records and queued positions: 200 Mb at 30x with

@@ -285,8 +285,8 @@ __device__ __forceinline__ uint32_t cells_below(const job_dev& J, uint32_t sampl
 // lineages, ((C & keep) << twice) + add. A template needs no look-up of its
 // leaf and no division, and walks the events of its window alone, in LDS: the
 // counts of 3.3e8 templates of 9e8 draws (500x, 13 events on 10 chromosomes)
-// 4.8 -> 4.1 ms. Bound by vector instruction issue: 120 instructions a group of
-// 64 draws, 43 of them Philox, and 6 for each read queued.
+// 4.8 -> 4.1 ms. Bound by vector instruction issue: 173 instructions a group of
+// 64 draws with the reads queued, 43 of them Philox.
 struct cn_event {
     uint32_t cell, cells, start, starts;
     uint32_t keep, twice, add, pad;
