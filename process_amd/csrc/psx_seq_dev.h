@@ -58,9 +58,10 @@ struct job_dev {
     uint32_t ins_k0, ins_n;
     uint32_t err_n, err_k0;      // error table (err_n == 0: no sequencing errors)
     uint32_t err_N;              // bases per template: (pe + 1) L
-    uint32_t purity_lt1;
+    uint32_t pad;                // the fields from here on start at 16 bytes: without it every small count takes 0.5-1 % longer
     uint32_t L, pe, ploidy, n_leaves, preneo, reach;
     uint32_t n_out;
+    uint32_t purity_lt1;
     uint32_t leaf_blocks;        // leaf_count entries per sample
     const psx_cna_dev* cna;      // copy-number events of every chromosome, per segment ranges
     unsigned long long* acc;     // reads of accepted templates (jobs with copy-number events)
