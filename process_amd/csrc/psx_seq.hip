@@ -33,7 +33,8 @@ constexpr double MANY_SLOW = 0.006;
 // 1.33 and 0.57).
 constexpr double MANY_SLOW_SPARSE = 0.005;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
-// templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves.
+// templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves, and
+// 1,116 such 73 -> 84.
 constexpr uint64_t FEW_ITEMS = 2048, MANY_ITEMS = 4096;
 
 struct seq_batch {
@@ -384,7 +385,7 @@ void layout(seq_batch& P) {
         const bool sparse = job_sparse(P, S.job);
         const uint64_t own = (S.J + S.spi - 1) / S.spi, all = items[sparse ? 0 : 1];
         if (P.count && S.T && all < FEW_ITEMS) {
-            const uint64_t per_item = S.T / own, least = sparse ? 1024 : 32 * BIN_READS;
+            const uint64_t per_item = S.T / own, least = sparse ? 2048 : 32 * BIN_READS;
             const uint64_t parts = std::min<uint64_t>((MANY_ITEMS + all - 1) / all, per_item / least);
             S.shape = (S.shape & 0xFFFFu) | (uint32_t)std::max<uint64_t>(parts, 1) << 16;
         }
