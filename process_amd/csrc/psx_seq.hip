@@ -22,16 +22,19 @@ namespace psxh {
 
 // Covered positions per 64 templates from which a job counts by windows (k_count_dense) rather than by queued reads
 // (k_count_sparse): see dense_from.
-constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 12.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0;
+constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 13.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0,
+                 DENSE_WINDOW = 30000.0;
 // Share of slow templates (slow_share) from which the dense kernel lets them wait and makes their errors 48 templates at a
 // time (5.6e7 templates of 250 bases: 0.013 % of them with more than three errors 0.46 ms by one after another, 0.53 by
 // 48; 1.7 % 1.01 and 0.90; 14 % 3.85 and 1.55; of 150 bases: 0.33 % 1.05 and 1.06; 2.8e8 of 36 bases, 0.7 % slow in all,
 // 2.52 and 2.34).
 constexpr double MANY_SLOW = 0.006;
-// And the same of the sparse kernel, with 5 blocks per CU in place of 6 then (5.6e7 templates of 150 bases, 11 covered
-// positions: 0.34 % of them 0.47 ms by one after another, 0.49 waiting; 1.35 % 0.56 and 0.50; 3.4 % 0.74 and 0.51; 15 %
-// 1.33 and 0.57).
-constexpr double MANY_SLOW_SPARSE = 0.005;
+// And the slow templates' covered positions per 64 templates from which reads wait in the sparse kernel, with 5 blocks
+// per CU in place of 6 then (one after another / waiting: 0.02 448 / 481 us, 0.05 474 / 488, 0.1 757 / 726, 0.2 280 / 267,
+// 0.4 558 / 499, 0.8 737 / 506); of windows with at least 12 of them, three a wave: fewer never fill the list.
+constexpr double MANY_SLOW_COVERED = 0.08, MANY_SLOW_WINDOW = 12.0;
+// Share of slow templates from which the sparse form's advantage at high error rates moves the line between the forms.
+constexpr double SLOW_ERRORS = 0.005;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
 // templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves, and
 // 1,116 such 73 -> 84.
@@ -55,7 +58,9 @@ struct seq_batch {
     std::vector<uint64_t> job_reads;  // per job: reads of the sampling model without copy-number events
     std::vector<uint64_t> job_plain;  // those of its segments without events
     std::vector<double> job_slow;   // per job: share of its slow templates (slow_share)
-    double slow_templates = 0.0, slow_sparse = 0.0;  // such templates of the dense jobs, of the sparse ones
+    double slow_templates = 0.0;    // such templates of the dense jobs
+    double slow_covered = 0.0;      // and 64 times those of the sparse ones by the positions that a template covers, of
+                                    // windows with enough of them
     std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
     std::vector<double> job_dense_from;  // and of how many it counts by windows
     std::vector<uint8_t> job_fits;  // per job: its source copies fit the dense count kernel's words
@@ -166,16 +171,28 @@ double slow_share(const psx_ctable& err, double N) {
     return 1.0 - below(3) + (below(2) - below(1)) / N + (below(3) - below(2)) * (3.0 - 2.0 / N) / N;
 }
 
+// log2 of the strata of a window of the dense count kernel: 2, 4 or 8 (4 with errors) while their reads fit one round.
+uint32_t window_strata_log2(double reads, bool errors, uint32_t strata, uint32_t copy_bits) {
+    uint32_t lns = 0;
+    while (lns < (errors ? 2u : 3u) && reads * (double)(2u << lns) <= 64.0 * BIN_READS * 0.9 && (1u << lns) < strata &&
+           copy_bits + BIN_SHIFT + lns + 1u <= 32u)
+        ++lns;
+    return lns;
+}
+
 // Covered positions per 64 templates from which a job counts by windows, by the errors of an average template (draws
-// that are not kept have none). The windows form makes the errors of every template, the other those of the reads that
-// can reach a record, so the line moves with the errors. Measured crossings on 4.7e7 to 1.4e8 templates of 100 to 250
-// bases: 12 covered positions at 0.05 errors, 15 at 0.12, 18 at 0.2, 25 at 0.5, 29 at 0.6; with more than
-// MANY_SLOW_SPARSE slow templates, where those wait, 51 at 0.9, 60 at 1, 83 at 1.5, 120 at 2, 190 at 3. A line at 28, and
-// at 15 for many slow templates, lost up to 1.8 times the time: 1.3e7 pairs of 150 bases at 2 %, 16 covered, 4.08 -> 1.29
-// ms; 2.8e7 single ones at 0.8 %, 18 covered, 1.20 -> 0.50 ms; pairs of 36 at 0.1 %, 26 covered, 0.96 -> 0.72 ms.
-double dense_from(double errors, double slow) {
+// that are not kept have none) and the templates of a window. The windows form makes the errors of every template, the
+// other those of the reads that can reach a record, and a window's set-up is the dearer the fewer its templates.
+// Measured crossings, 100 to 250 bases: at 10,000 and more templates a window 12 covered positions at 0.05 errors, 15 at
+// 0.12, 18 at 0.2, 25 at 0.5, 29 at 0.6; at 0.15 errors 23 with 5,400, 22 with 4,400, 31 with 2,700, 28 with 2,200, 40
+// with 1,100; pairs at 0.3 errors 20 with 11,000, 31 with 2,700, 45 with 1,400. With more than SLOW_ERRORS slow templates,
+// where those wait, 51 at 0.9, 60 at 1, 83 at 1.5, 120 at 2, 190 at 3. A line at 28, and at 15 for many slow templates, lost
+// up to 1.8 times the time: 1.3e7 pairs of 150 bases at 2 %, 16 covered, 4.08 -> 1.05 ms; 2.8e7 single ones at 0.8 %, 18
+// covered, 1.20 -> 0.55 ms; pairs of 36 at 0.1 %, 26 covered, 0.96 -> 0.72 ms.
+double dense_from(double errors, double slow, double window) {
     if (errors <= 0.0) return DENSE_COVER_NO_ERRORS;
-    return slow > MANY_SLOW_SPARSE ? DENSE_COVER_SLOW * errors : DENSE_COVER + DENSE_COVER_ERROR * errors;
+    return (slow > SLOW_ERRORS ? DENSE_COVER_SLOW * errors : DENSE_COVER + DENSE_COVER_ERROR * errors) +
+           DENSE_WINDOW / std::max(window, 1.0);
 }
 
 // Validates one job and appends its descriptors; the ordering of output
@@ -291,7 +308,6 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     }
     P.job_cover.push_back(cover);
     P.job_slow.push_back(slow_share(err, J.err_N));
-    P.job_dense_from.push_back(dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back()));
     P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;
     uint64_t plain = 0;
@@ -334,6 +350,15 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
             P.segs.push_back(S);  // its work items are numbered in layout()
         }
     }
+    double templates = 0.0, strata = 0.0;  // those of a stratum give those of a window
+    for (size_t k = P.segs.size(); k-- > 0 && P.segs[k].job == job;) {
+        templates += (double)P.segs[k].T;
+        strata += (double)P.segs[k].J;
+    }
+    const double stratum = templates / std::max(strata, 1.0);
+    const uint32_t lns = window_strata_log2(stratum * (pe ? 2.0 : 1.0), J.err_n != 0, 4u, 0u);
+    P.job_dense_from.push_back(
+        dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back(), stratum * (double)(1u << lns)));
     P.job_reads.push_back(P.n_reads - reads_before);
     P.job_plain.push_back(plain);
 }
@@ -354,9 +379,7 @@ void shape_segment(const seq_batch& P, seg_dev& S, uint64_t strata) {
     uint32_t lns = 0, lw = BIN_SHIFT;
     if (P.count && !job_sparse(P, S.job)) {
         const double reads = (double)S.T * (J.pe + 1u) * PSX_STRATUM / (double)S.W;  // of a stratum
-        while (lns < (J.err_n ? 2u : 3u) && reads * (double)(2u << lns) <= 64.0 * BIN_READS * 0.9 &&
-               (1u << lns) < S.J && copy_bits + BIN_SHIFT + lns + 1u <= 32u)
-            ++lns;
+        lns = window_strata_log2(reads, J.err_n != 0, S.J, copy_bits);
         lw += lns;
         while (lw > 1 && (S.W >> lw) < 32u && ((S.W + past) >> (lw - 1u)) < MAX_BINS) --lw;
     } else if (P.count) {
@@ -401,7 +424,9 @@ void layout(seq_batch& P) {
         if (sparse) {
             P.n_items_sparse = P.n_items;
             P.templates_sparse = P.templates;
-            P.slow_sparse += (double)S.T * P.job_slow[S.job];
+            const double slow = P.job_slow[S.job] * P.job_cover[S.job];
+            if (slow / 64.0 * (double)(S.T << seg_lns(S)) / ((double)S.J * seg_parts(S)) >= MANY_SLOW_WINDOW)
+                P.slow_covered += (double)S.T * slow;
         } else {
             const job_dev& J = P.jobs[S.job];
             const uint64_t starts = std::min<uint64_t>(S.W, (uint64_t)PSX_STRATUM << seg_lns(S));  // of a window
@@ -539,7 +564,7 @@ void batch_launch(const seq_batch* P, const seq_lane& lane, const psx_launch_con
         const uint64_t grid = std::max<uint64_t>(1, std::min(want, ns));
         Ls.n_items = ns;
         Ls.chunk = run_items(ns, P->templates_sparse, grid, 8192, 4);
-        const bool many = P->slow_sparse > MANY_SLOW_SPARSE * (double)P->templates_sparse;
+        const bool many = P->slow_covered > MANY_SLOW_COVERED * (double)P->templates_sparse;
         launch_count(lane, cfg, Ls, (uint32_t)grid, P->cna_sparse, many);
     }
     if (nd) {
