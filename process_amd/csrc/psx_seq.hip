@@ -24,6 +24,7 @@ namespace psxh {
 // (k_count_sparse): see dense_from.
 constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 13.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0,
                  DENSE_WINDOW = 30000.0;
+constexpr double STAGED = 512.0;  // records that a sparse window stages (by default)
 // Share of slow templates (slow_share) from which the dense kernel lets them wait and makes their errors 48 templates at a
 // time (5.6e7 templates of 250 bases: 0.013 % of them with more than three errors 0.46 ms by one after another, 0.53 by
 // 48; 1.7 % 1.01 and 0.90; 14 % 3.85 and 1.55; of 150 bases: 0.33 % 1.05 and 1.06; 2.8e8 of 36 bases, 0.7 % slow in all,
@@ -37,8 +38,11 @@ constexpr double MANY_SLOW_COVERED = 0.08, MANY_SLOW_WINDOW = 12.0;
 constexpr double SLOW_ERRORS = 0.005;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
 // templates (a 1.5 Mb panel at 2000x) 1390 -> 520 us, but 2,442 strata of 2,200 templates 93 -> 105 us in halves, and
-// 1,116 such 73 -> 84.
+// 1,116 such 73 -> 84. With less than an item per CU smaller parts gain (50 strata of 6,140 templates of pairs in parts of
+// 512 57 -> 34 us; 490 of them in 3 parts instead of 2 66 -> 77).
 constexpr uint64_t FEW_ITEMS = 2048, MANY_ITEMS = 4096;
+// Windows that a launch keeps when its sparse windows take several strata.
+constexpr uint64_t LEAST_WINDOWS = 128;
 
 struct seq_batch {
     std::vector<job_dev> jobs;
@@ -63,6 +67,7 @@ struct seq_batch {
                                     // windows with enough of them
     std::vector<double> job_cover;  // per job: expected covered positions per 64 templates
     std::vector<double> job_dense_from;  // and of how many it counts by windows
+    std::vector<double> job_records;  // per job: records of a stratum
     std::vector<uint8_t> job_fits;  // per job: its source copies fit the dense count kernel's words
     bool cna_sparse = false, cna_dense = false;  // copy-number events among the sparse / the other jobs
     size_t o_jobs = 0, o_segs = 0, o_items = 0, o_pres = 0, o_acc = 0;
@@ -288,7 +293,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     }
     P.cna_off.push_back(cdev.empty() ? SIZE_MAX : P.sb.put_vec(cdev));
     P.jobs.push_back(J);
-    double cover = 0.0, share = 1.0;
+    double cover = 0.0, share = 1.0, records = 0.0;
     {
         // expected positions covered by 64 templates: records per base x bases read, times the share of templates
         // kept under copy numbers (length-weighted): the source's copies among kmax slots, a cell's (their mean over
@@ -303,10 +308,11 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
             bases += (double)g->len[c];
             kept += (double)g->len[c] * (tumour * c_mean[c] + (1.0 - tumour) * (double)ploidy) / (double)c_kmax[c];
         }
-        if (bases > 0.0) share = kept / bases;
+        if (bases > 0.0) share = kept / bases, records = recs / bases * PSX_STRATUM;
         if (bases > 0.0) cover = 64.0 * (pe ? 2.0 : 1.0) * L * recs / bases * kept / bases;
     }
     P.job_cover.push_back(cover);
+    P.job_records.push_back(records);
     P.job_slow.push_back(slow_share(err, J.err_N));
     P.job_fits.push_back(1);
     const uint64_t reads_before = P.n_reads;
@@ -372,7 +378,11 @@ bool job_sparse(const seq_batch& P, uint32_t job) { return !P.job_fits[job] || P
 // bins of starts and as many more as mates reach past the window; on a
 // chromosome of less than a stratum the bins are narrower, at least 2 starts.
 // Sparse windows take 2 or 4 strata where a wave would have fewer than 16
-// groups of 64 templates of one, as long as the launch keeps MANY_ITEMS.
+// groups of 64 templates of one, as long as the launch keeps MANY_ITEMS; with
+// fewer, where one has few templates for the windows left: the strata share a
+// window's set-up, but fewer windows end less evenly. 7,320 strata of 33
+// templates 112 -> 58 us, of 820 124 -> 92; 2,450 of 33 78 -> 33, but of 3,300
+// two by two 91 -> 103.
 void shape_segment(const seq_batch& P, seg_dev& S, uint64_t strata) {
     const job_dev& J = P.jobs[S.job];
     const uint32_t cb = seg_cb(S), copy_bits = cb + bits_of(J.ploidy - 1u), past = J.reach - J.L;
@@ -384,8 +394,12 @@ void shape_segment(const seq_batch& P, seg_dev& S, uint64_t strata) {
         while (lw > 1 && (S.W >> lw) < 32u && ((S.W + past) >> (lw - 1u)) < MAX_BINS) --lw;
     } else if (P.count) {
         const double templates = (double)S.T * PSX_STRATUM / (double)S.W;  // of a stratum
-        while (lns < 2u && templates * (double)(1u << lns) < 4096.0 && (1u << lns) < S.J && strata >> (lns + 1u) >= MANY_ITEMS)
-            ++lns;
+        for (; lns < 2u && (1u << lns) < S.J; ++lns) {
+            const uint64_t windows = strata >> (lns + 1u);  // that the launch would have
+            const double most = windows >= MANY_ITEMS ? 4096.0 : (double)windows / 2.0;
+            const double staged = P.job_records[S.job] * (double)((2u << lns) + 1u);  // the next stratum's too
+            if (windows < LEAST_WINDOWS || templates * (double)(1u << lns) >= most || staged > STAGED) break;
+        }
     }
     S.spi = std::max(P.spi, 1u << lns);
     S.shape = cb | lns << 8 | lw << 12 | 1u << 16;
@@ -408,7 +422,8 @@ void layout(seq_batch& P) {
         const bool sparse = job_sparse(P, S.job);
         const uint64_t own = (S.J + S.spi - 1) / S.spi, all = items[sparse ? 0 : 1];
         if (P.count && S.T && all < FEW_ITEMS) {
-            const uint64_t per_item = S.T / own, least = sparse ? 2048 : 32 * BIN_READS;
+            const uint64_t per_item = S.T / own;
+            const uint64_t least = sparse ? std::min<uint64_t>(std::max<uint64_t>(8 * all, 512), 2048) : 32 * BIN_READS;
             const uint64_t parts = std::min<uint64_t>((MANY_ITEMS + all - 1) / all, per_item / least);
             S.shape = (S.shape & 0xFFFFu) | (uint32_t)std::max<uint64_t>(parts, 1) << 16;
         }

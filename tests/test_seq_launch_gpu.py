@@ -243,6 +243,22 @@ def test_widest_windows(ctx, kw, cna):
     assert n == on and np.array_equal(d, od) and np.array_equal(a, oa) and np.array_equal(p, op) and d.sum() > 0
 
 
+@pytest.mark.parametrize("cov,kw", [
+    # few templates for the launch's windows: four strata each, two, one
+    (0.5, dict(read_size=150, error_rate=3e-2)),
+    (0.6, dict(read_size=250, insert_size_mean=600, insert_size_stddev=10, error_rate=8e-3, purity=0.6)),
+    (1.0, dict(read_size=150, error_rate=1e-3)),
+    (2.0, dict(read_size=150, error_rate=3e-2, purity=0.5)),
+    (3.0, dict(read_size=100))])
+@pytest.mark.parametrize("n", [300, 20_000, 60_000])
+def test_queued_reads_of_several_strata(ctx, n, cov, kw):
+    """Windows of queued reads of one, two and four strata in a launch of 600, with few records, with as many as are
+    staged of two strata but not of four, and with more than are staged of one."""
+    w = World(ctx, [600_000] * 4 + [8_192 + 149, 20_000, 5_000, 400], dict(n_cells=500, n_samples=1, sample_size=90, seed=2),
+              1e-8, n_pre_snv=n, infinite_sites=False)
+    w.check(core.simulate_seq_arrays(ctx, w.g, w.pf, w.pm, 3, coverage=cov, **kw)[:3], 3, dict(kw, coverage=cov))
+
+
 def test_autotuner_varies_what_the_jobs_use(ctx):
     """Jobs counted by windows alone leave the block size and the staged records, which that form does not have, at the
     default; with a sparse job every configuration is timed."""
