@@ -23,7 +23,7 @@ namespace psxh {
 // Covered positions per 64 templates from which a job counts by windows (k_count_dense) rather than by queued reads
 // (k_count_sparse): see dense_from.
 constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 13.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0,
-                 DENSE_WINDOW = 30000.0;
+                 DENSE_COVER_SLOW_PAIRS = 34.0, DENSE_WINDOW = 30000.0;
 constexpr double STAGED = 512.0;  // records that a sparse window stages (by default)
 // Share of slow templates (slow_share) from which the dense kernel lets them wait and makes their errors 48 templates at a
 // time (5.6e7 templates of 250 bases: 0.013 % of them with more than three errors 0.46 ms by one after another, 0.53 by
@@ -32,8 +32,9 @@ constexpr double STAGED = 512.0;  // records that a sparse window stages (by def
 constexpr double MANY_SLOW = 0.006;
 // And the slow templates' covered positions per 64 templates from which reads wait in the sparse kernel, with 5 blocks
 // per CU in place of 6 then (one after another / waiting: 0.02 448 / 481 us, 0.05 474 / 488, 0.1 757 / 726, 0.2 280 / 267,
-// 0.4 558 / 499, 0.8 737 / 506); of windows with at least 12 of them, three a wave: fewer never fill the list.
-constexpr double MANY_SLOW_COVERED = 0.08, MANY_SLOW_WINDOW = 12.0;
+// 0.4 558 / 499, 0.8 737 / 506); of windows with at least 10 of them, which lanes make at once (7 of them 118 / 130 us, 9
+// 130 / 134, 11 50 / 27, 14 158 / 145, 17 155 / 143).
+constexpr double MANY_SLOW_COVERED = 0.08, MANY_SLOW_WINDOW = 10.0;
 // Share of slow templates from which the sparse form's advantage at high error rates moves the line between the forms.
 constexpr double SLOW_ERRORS = 0.005;
 // Items below which a launch cuts them into parts, and about how many parts it then has: 368 strata of 16,000
@@ -191,12 +192,16 @@ uint32_t window_strata_log2(double reads, bool errors, uint32_t strata, uint32_t
 // Measured crossings, 100 to 250 bases: at 10,000 and more templates a window 12 covered positions at 0.05 errors, 15 at
 // 0.12, 18 at 0.2, 25 at 0.5, 29 at 0.6; at 0.15 errors 23 with 5,400, 22 with 4,400, 31 with 2,700, 28 with 2,200, 40
 // with 1,100; pairs at 0.3 errors 20 with 11,000, 31 with 2,700, 45 with 1,400. With more than SLOW_ERRORS slow templates,
-// where those wait, 51 at 0.9, 60 at 1, 83 at 1.5, 120 at 2, 190 at 3. A line at 28, and at 15 for many slow templates, lost
-// up to 1.8 times the time: 1.3e7 pairs of 150 bases at 2 %, 16 covered, 4.08 -> 1.05 ms; 2.8e7 single ones at 0.8 %, 18
-// covered, 1.20 -> 0.55 ms; pairs of 36 at 0.1 %, 26 covered, 0.96 -> 0.72 ms.
-double dense_from(double errors, double slow, double window) {
+// where those wait, 51 at 0.9, 60 at 1, 83 at 1.5, 120 at 2, 190 at 3, and past 200 at 4.5; pairs, whose reads each make
+// their template's errors, 55 at 1.2, 105 at 3, 110 at 4, 150 at 4.8. Where a window has more records than are staged its
+// reads look them up in global memory: 100 positions at 1.8 errors 6.2 ms by windows, 14.0 queued. A line at 28, and at 15
+// for many slow templates, lost up to 1.8 times the time: 1.3e7 pairs of 150 bases at 2 %, 16 covered, 4.08 -> 1.05 ms;
+// 2.8e7 single ones at 0.8 %, 18 covered, 1.20 -> 0.55 ms; pairs of 36 at 0.1 %, 26 covered, 0.96 -> 0.72 ms.
+double dense_from(double errors, double slow, double window, bool pairs, double records) {
     if (errors <= 0.0) return DENSE_COVER_NO_ERRORS;
-    return (slow > SLOW_ERRORS ? DENSE_COVER_SLOW * errors : DENSE_COVER + DENSE_COVER_ERROR * errors) +
+    if (2.0 * records > STAGED) return DENSE_COVER;  // of a window of one stratum, with the next one's
+    const double by_slow = pairs ? DENSE_COVER_SLOW_PAIRS : DENSE_COVER_SLOW;
+    return (slow > SLOW_ERRORS ? by_slow * errors : DENSE_COVER + DENSE_COVER_ERROR * errors) +
            DENSE_WINDOW / std::max(window, 1.0);
 }
 
@@ -364,7 +369,7 @@ void prepare_job(psx_ctx* ctx, seq_batch& P, const job_in& in, uint32_t spi) {
     const double stratum = templates / std::max(strata, 1.0);
     const uint32_t lns = window_strata_log2(stratum * (pe ? 2.0 : 1.0), J.err_n != 0, 4u, 0u);
     P.job_dense_from.push_back(
-        dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back(), stratum * (double)(1u << lns)));
+        dense_from(p->error_rate * (double)J.err_N * share, P.job_slow.back(), stratum * (double)(1u << lns), pe, records));
     P.job_reads.push_back(P.n_reads - reads_before);
     P.job_plain.push_back(plain);
 }
