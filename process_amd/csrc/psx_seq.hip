@@ -23,7 +23,7 @@ namespace psxh {
 // Covered positions per 64 templates from which a job counts by windows (k_count_dense) rather than by queued reads
 // (k_count_sparse): see dense_from.
 constexpr double DENSE_COVER_NO_ERRORS = 8.0, DENSE_COVER = 13.0, DENSE_COVER_ERROR = 26.0, DENSE_COVER_SLOW = 60.0,
-                 DENSE_COVER_SLOW_PAIRS = 34.0, DENSE_WINDOW = 30000.0;
+                 DENSE_COVER_PAIRS = 25.0, DENSE_WINDOW = 30000.0;
 constexpr double STAGED = 512.0;  // records that a sparse window stages (by default)
 // Share of slow templates (slow_share) from which the dense kernel lets them wait and makes their errors 48 templates at a
 // time (5.6e7 templates of 250 bases: 0.013 % of them with more than three errors 0.46 ms by one after another, 0.53 by
@@ -200,8 +200,8 @@ uint32_t window_strata_log2(double reads, bool errors, uint32_t strata, uint32_t
 double dense_from(double errors, double slow, double window, bool pairs, double records) {
     if (errors <= 0.0) return DENSE_COVER_NO_ERRORS;
     if (2.0 * records > STAGED) return DENSE_COVER;  // of a window of one stratum, with the next one's
-    const double by_slow = pairs ? DENSE_COVER_SLOW_PAIRS : DENSE_COVER_SLOW;
-    return (slow > SLOW_ERRORS ? by_slow * errors : DENSE_COVER + DENSE_COVER_ERROR * errors) +
+    const bool many = slow > SLOW_ERRORS;
+    return (many && !pairs ? DENSE_COVER_SLOW * errors : (many ? DENSE_COVER_PAIRS : DENSE_COVER) + DENSE_COVER_ERROR * errors) +
            DENSE_WINDOW / std::max(window, 1.0);
 }
 
